@@ -119,7 +119,7 @@ __device__ __forceinline__ Lds2D<R> carve2d(unsigned char* smem, int nvt, int nc
 template <typename R>
 struct Tissue2DCtx {
   int c0, nc, v0, nvt;  // first cell, cells, first vertex, vertices
-  R L;
+  R L, invL;            // box length and 1 / L
   int pbc;
   R Kre, Kat;
 };
@@ -132,6 +132,7 @@ __device__ __forceinline__ Tissue2DCtx<R> tissue_ctx(const Geom2D<R>& g, int t) 
   T.v0 = g.cell_vert_begin[T.c0];
   T.nvt = g.cell_vert_begin[T.c0 + T.nc] - T.v0;
   T.L = g.tL[t];
+  T.invL = R(1) / T.L;
   T.pbc = g.tpbc[t];
   T.Kre = (R)g.tKre[t];
   T.Kat = (R)g.tKat[t];
@@ -197,11 +198,13 @@ __device__ void cell_pass(const Geom2D<R>& g, const Tissue2DCtx<R>& T, const Lds
 //  - distance predicates (attraction d < l0[ci], vertex repulsion
 //    d < (l0[ci] + l0[cj])/2, both under the per-pair minimum image): per
 //    axis the minimum-image gap between the two boxes exceeds the cut-off
-//    and the boxes are small against L (then no other image comes closer);
+//    and the boxes are small against L (then no other image comes closer;
+//    the image is rounded from a product with 1/L, which can name the other
+//    of two images only where both are half a box away);
 //  - repulsion (crossing parity of raw differences, transformed only where a
-//    difference exceeds L): the raw boxes are disjoint and no raw
-//    difference can exceed L (then the parity of a point outside cj's box
-//    is even).
+//    difference exceeds L): ci's box lies above or below cj's with no y
+//    difference beyond L, or left of it with no x difference beyond L, or
+//    right of it with neither (outside_box_even's argument, box for point).
 template <typename R>
 __device__ bool maybe_pair(const Geom2D<R>& g, const Tissue2DCtx<R>& T, const Lds2D<R>& l, int ci, int cj) {
   const R L = T.L;
@@ -209,12 +212,11 @@ __device__ bool maybe_pair(const Geom2D<R>& g, const Tissue2DCtx<R>& T, const Ld
   const R spanx = fmax(l.ax1[ci] - l.ax0[cj], l.ax1[cj] - l.ax0[ci]);
   const R spany = fmax(l.ay1[ci] - l.ay0[cj], l.ay1[cj] - l.ay0[ci]);
   if (g.mask & M2_REPULSION) {
-    const bool raw_guard = !T.pbc || (spanx < L * R(0.999f) && spany < L * R(0.999f));
-    if (!raw_guard) return true;
+    const bool xin = !T.pbc || spanx < L * R(0.999f), yin = !T.pbc || spany < L * R(0.999f);
     const R m = tiny * (R(1) + fmax(fabs(l.ax1[cj]), fabs(l.ax0[cj])) + fmax(fabs(l.ay1[cj]), fabs(l.ay0[cj])));
-    const bool disjoint = l.ax1[ci] < l.ax0[cj] - m || l.ax0[ci] > l.ax1[cj] + m ||
-                          l.ay1[ci] < l.ay0[cj] - m || l.ay0[ci] > l.ay1[cj] + m;
-    if (!disjoint) return true;
+    const bool even = (yin && (l.ay1[ci] < l.ay0[cj] - m || l.ay0[ci] > l.ay1[cj] + m)) ||
+                      (xin && (l.ax1[ci] < l.ax0[cj] - m || (yin && l.ax0[ci] > l.ax1[cj] + m)));
+    if (!even) return true;
   }
   if (g.mask & (M2_ATTRACTION | M2_VREPULSION)) {
     const R l0i = l.l0c[ci], l0j = l.l0c[cj];
@@ -225,8 +227,8 @@ __device__ bool maybe_pair(const Geom2D<R>& g, const Tissue2DCtx<R>& T, const Ld
     R dy = R(0.5f) * (l.ay0[cj] + l.ay1[cj]) - R(0.5f) * (l.ay0[ci] + l.ay1[ci]);
     if (T.pbc) {
       if (!(hx + cut < R(0.45f) * L && hy + cut < R(0.45f) * L)) return true;
-      dx -= L * round(dx / L);
-      dy -= L * round(dy / L);
+      dx -= L * round(dx * T.invL);
+      dy -= L * round(dy * T.invL);
     }
     const R reach = cut * R(1.0001f) + tiny * (R(1) + L);
     const bool far = fabs(dx) - hx > reach || fabs(dy) - hy > reach;
@@ -295,8 +297,8 @@ __device__ __forceinline__ bool vertex_far_from_box(const Lds2D<R>& l, const Tis
   R dx = R(0.5f) * (l.ax0[cj] + l.ax1[cj]) - px, dy = R(0.5f) * (l.ay0[cj] + l.ay1[cj]) - py;
   if (T.pbc) {
     if (!(hx + cut < R(0.45f) * L && hy + cut < R(0.45f) * L)) return false;
-    dx -= L * round(dx / L);
-    dy -= L * round(dy / L);
+    dx -= L * round(dx * T.invL);
+    dy -= L * round(dy * T.invL);
   }
   const R reach = cut * R(1.0001f) + R(1e-5f) * (R(1) + L);
   return fabs(dx) - hx > reach || fabs(dy) - hy > reach;
@@ -372,19 +374,27 @@ __device__ __forceinline__ bool crossing_odd(const Lds2D<R>& l, int cj, R px, R 
   return odd;
 }
 
-// A point outside cell cj's raw bounding box by more than 1e-5 (1 + L),
-// whose raw differences to every vertex of cj stay within L (so crossing_odd
-// applies no image), has even crossing parity: above or below the box no
-// edge straddles its row; left of the box every crossing lies to its right
-// and none counts; right of the box every one counts, and a closed ring has
-// an even number of edges straddling any row.
+// True where the crossing parity of point p about cell cj is even by its
+// raw bounding box alone.  crossing_odd takes an axis's raw differences as
+// they are while all of them stay within L (subtraction is monotone, so the
+// box's ends decide that):
+//   * y taken raw and p above or below the box: no edge straddles p's row
+//     (the sign of a float difference is exact);
+//   * x taken raw and p left of the box: whatever the rows, every crossing
+//     lies to p's right (tt < 0 by the margin) and none counts;
+//   * both taken raw and p right of the box: every straddling edge counts,
+//     and a closed ring has an even number of edges straddling any row.
+// The margin in x, 1e-5 (1 + L), covers the rounding of tt.  The first rule
+// leaves a vertex at one raw side of the tissue, whose x differences to the
+// cells of the opposite side exceed L, the crossing loops of its own row
+// instead of the whole side's.
 template <typename R>
 __device__ __forceinline__ bool outside_box_even(const Lds2D<R>& l, int cj, R px, R py, int pbc, R L) {
   const R x0 = l.ax0[cj], x1 = l.ax1[cj], y0 = l.ay0[cj], y1 = l.ay1[cj];
-  if (pbc && !(fabs(px - x0) <= L && fabs(px - x1) <= L && fabs(py - y0) <= L && fabs(py - y1) <= L))
-    return false;
+  const bool xin = !pbc || (fabs(px - x0) <= L && fabs(px - x1) <= L);
+  const bool yin = !pbc || (fabs(py - y0) <= L && fabs(py - y1) <= L);
   const R m = R(1e-5f) * (R(1) + L);
-  return px < x0 - m || px > x1 + m || py < y0 - m || py > y1 + m;
+  return (yin && (py < y0 || py > y1)) || (xin && (px < x0 - m || (yin && px > x1 + m)));
 }
 
 // Crossing parity of every vertex against every candidate cell: bit k of
@@ -458,25 +468,20 @@ __device__ void over_pass(const Tissue2DCtx<R>& T, const Lds2D<R>& l, unsigned* 
   }
 }
 
-// All force terms on vertex k (tissue-local index).  With `energy`, also
-// accumulates this vertex's share of the conservative energy (perimeter edge
-// k -> k+1, bending at k, the cell's area energy at its first vertex) and
-// with `e_int` half of each vertex-repulsion pair energy.  With `over_bits`
-// the crossing parity comes from over_pass instead of the loop here, with
-// over_state (0 or 1) from k2d_wide_over.
+// The terms of vertex k (tissue-local index, of cell ci) that its own cell
+// alone decides: area, perimeter, bending.  With `energy`, also accumulates
+// this vertex's share of their energy (perimeter edge k -> k+1, bending at k,
+// the cell's area energy at its first vertex).
 template <typename R>
-__device__ __forceinline__ void force_vertex(const Geom2D<R>& g, const Tissue2DCtx<R>& T, const Lds2D<R>& l,
-                                          int k, R& Fx, R& Fy, int* n_over, int* n_attr, double* energy,
-                                          double* e_int, const unsigned* over_bits = nullptr,
-                                          unsigned* attr_key = nullptr, int over_state = -1) {
-  const int ci = cell_of(l.vb, T.nc, k);
+__device__ __forceinline__ void shape_vertex(const Geom2D<R>& g, const Tissue2DCtx<R>& T, const Lds2D<R>& l, int ci,
+                                             int k, R& fx, R& fy, double* energy) {
   const int gc = T.c0 + ci;
   const int b = l.vb[ci], e = l.vb[ci + 1], n = e - b, vi = k - b;
   const int im1 = (vi == 0) ? e - 1 : k - 1;
   const int ip1 = (vi == n - 1) ? b : k + 1;
   const R px = l.x[k], py = l.y[k];
-  const R L = T.L;
-  R fx = R(0), fy = R(0);
+  fx = R(0);
+  fy = R(0);
   const unsigned mask = g.mask;
   if (mask & M2_AREA) {
     const R Ka = (R)g.Ka[gc], a0 = (R)g.a0[gc];
@@ -529,6 +534,45 @@ __device__ __forceinline__ void force_vertex(const Geom2D<R>& g, const Tissue2DC
       *energy += 0.5 * Kb * (sx * sx + sy * sy);
     }
   }
+}
+
+// The push toward the own centre of mass of a vertex at (px, py) of cell ci
+// that lies inside another cell (Cell2D_kernel.cl:203-219), added to (fx, fy).
+template <typename R>
+__device__ __forceinline__ void repulsion_push(const Geom2D<R>& g, const Tissue2DCtx<R>& T, const Lds2D<R>& l, int ci,
+                                               R px, R py, R& fx, R& fy) {
+  const R L = T.L;
+  R dx = l.comx[ci] - px, dy = l.comy[ci] - py;
+  if (T.pbc) {
+    dx -= L * round(dx / L);
+    dy -= L * round(dy / L);
+  }
+  const R dist = sqrt(dx * dx + dy * dy);
+  const R xij = dist / (R(2) * (R)g.r0[T.c0 + ci]);
+  const R ftmp = T.Kre * (R(1) - xij);
+  const V3<R> u = vnormalize(V3<R>{dx, dy, R(0)});
+  fx += R(0.5f) * ftmp * u.x;
+  fy += R(0.5f) * ftmp * u.y;
+}
+
+// All force terms on vertex k (tissue-local index).  With `energy`, also
+// accumulates this vertex's share of the conservative energy (shape_vertex)
+// and with `e_int` half of each vertex-repulsion pair energy.  With
+// `over_bits` the crossing parity comes from over_pass instead of the loop
+// here.
+template <typename R>
+__device__ __forceinline__ void force_vertex(const Geom2D<R>& g, const Tissue2DCtx<R>& T, const Lds2D<R>& l,
+                                          int k, R& Fx, R& Fy, int* n_over, int* n_attr, double* energy,
+                                          double* e_int, const unsigned* over_bits = nullptr,
+                                          unsigned* attr_key = nullptr) {
+  const int ci = cell_of(l.vb, T.nc, k);
+  const int gc = T.c0 + ci;
+  const int n = l.vb[ci + 1] - l.vb[ci];
+  const R px = l.x[k], py = l.y[k];
+  const R L = T.L;
+  const unsigned mask = g.mask;
+  R fx, fy;
+  shape_vertex(g, T, l, ci, k, fx, fy, energy);
   const int nc = l.ncand[ci];
   const bool scan_all = nc > DPM2D_MAXCAND;
   const int ncl = scan_all ? T.nc : nc;
@@ -599,28 +643,14 @@ __device__ __forceinline__ void force_vertex(const Geom2D<R>& g, const Tissue2DC
     }
   }
   if (mask & M2_REPULSION) {
-    // the crossing parity given (over_state 0 or 1, or bit k of over_bits),
-    // else found by the loop
-    const bool given = over_state >= 0 || over_bits;
-    bool over = over_state >= 0 ? over_state != 0 : (over_bits && ((over_bits[k >> 5] >> (k & 31)) & 1u));
-    for (int q = 0; q < ncl && !over && !given; q++) {
+    // the crossing parity given (bit k of over_bits), else found by the loop
+    bool over = over_bits && ((over_bits[k >> 5] >> (k & 31)) & 1u);
+    for (int q = 0; q < ncl && !over && !over_bits; q++) {
       const int cj = scan_all ? q : (int)l.cand[ci * DPM2D_MAXCAND + q];
       if (cj == ci || outside_box_even(l, cj, px, py, T.pbc, L)) continue;
       over = crossing_odd(l, cj, px, py, T.pbc, L);
     }
-    if (over) {
-      R dx = l.comx[ci] - px, dy = l.comy[ci] - py;
-      if (T.pbc) {
-        dx -= L * round(dx / L);
-        dy -= L * round(dy / L);
-      }
-      const R dist = sqrt(dx * dx + dy * dy);
-      const R xij = dist / (R(2) * (R)g.r0[gc]);
-      const R ftmp = T.Kre * (R(1) - xij);
-      const V3<R> u = vnormalize(V3<R>{dx, dy, R(0)});
-      fx += R(0.5f) * ftmp * u.x;
-      fy += R(0.5f) * ftmp * u.y;
-    }
+    if (over) repulsion_push(g, T, l, ci, px, py, fx, fy);
     *n_over = over ? 1 : 0;
   }
   Fx = fx;
@@ -989,6 +1019,7 @@ __device__ void rescale_box(const Geom2D<R>& g, Tissue2DCtx<R>& T, const Lds2D<R
     l.y[k] += s * l.comy[c];
   }
   T.L = Lnew;
+  T.invL = R(1) / Lnew;
   __syncthreads();
 }
 
@@ -1078,6 +1109,7 @@ __device__ void k2d_relax_body(const Relax2D<R>& a) {
         }
         copy_positions(T, sx, sy, l.x, l.y);  // back to the unjammed state
         T.L = (R)sqrt(A0 / phi_lo);
+        T.invL = R(1) / T.L;
         phi = phi_lo;
       }
       if (phi_hi > 0.0 && phi_hi - phi_lo < jp.phi_tol) {
@@ -1095,6 +1127,7 @@ __device__ void k2d_relax_body(const Relax2D<R>& a) {
     if ((status == 0 || status == 3) && phi != phi_lo) {  // end on the largest unjammed state
       copy_positions(T, sx, sy, l.x, l.y);
       T.L = (R)sqrt(A0 / phi_lo);
+      T.invL = R(1) / T.L;
       phi = phi_lo;
     }
     res[RS_ITER] = iters;

@@ -158,14 +158,13 @@ struct dpm_tissue {
   hipGraphExec_t jam_graph = nullptr;
   std::vector<unsigned char> jam_key;
   // tissues beyond one workgroup: 0 automatic, 1 one workgroup per tissue,
-  // 2 the wide path (three or four launches per step over the device)
+  // 2 the wide path (three launches per step over the device)
   int wide_mode = 0;
   bool fits_wg = true;  // every tissue fits one workgroup (k2d_run)
   int max_cells = 0;    // cells of the largest tissue
   float *xw = nullptr, *yw = nullptr, *cellq = nullptr;
   int *ncand_w = nullptr, *cell_tissue2 = nullptr, *vbl = nullptr;
   short* cand_w = nullptr;
-  unsigned* over_w = nullptr;  // crossing-parity bits of the wide path
   int* vcell_w = nullptr;      // cell of each vertex
   hipGraphExec_t wide_graph = nullptr;
   float wide_graph_dt = 0.0f;
@@ -1712,7 +1711,6 @@ static int ensure_wide(dpm_tissue* h) {
   rc |= h->alloc(&h->cand_w, (size_t)C * DPM2D_MAXCAND);
   rc |= h->alloc(&h->cell_tissue2, C);
   rc |= h->alloc(&h->vbl, (size_t)C + T);
-  rc |= h->alloc(&h->over_w, ((size_t)h->V + 31) / 32);
   rc |= h->alloc(&h->vcell_w, (size_t)h->V);
   if (rc) return DPM_ENOMEM;
   std::vector<int> ct(C), vbl((size_t)C + T), vc((size_t)h->V);
@@ -1751,20 +1749,18 @@ static Wide2D wide_args(dpm_tissue* h, int in, float dt, int flags) {
   a.dt = dt;
   a.flags = flags;
   a.counters = h->counters;
-  a.over_bits = h->over_w;
   a.vcell = h->vcell_w;
   return a;
 }
 
 static int launch_wide(dpm_tissue* h, const Wide2D& a) {
-  const int bc = (h->C + 255) / 256, bv = (h->V + 255) / 256, bw = (h->C + 3) / 4;
+  const int bc = (h->C + 255) / 256, bw = (h->C + 3) / 4;
+  const int G = wide_group(h->V);
+  const unsigned bv = (unsigned)(((long long)h->V * G + 255) / 256);
+  auto step = G == 32 ? k2d_wide_step<32> : G == 16 ? k2d_wide_step<16> : k2d_wide_step<8>;
   hipLaunchKernelGGL(k2d_wide_cells, dim3(bc), dim3(256), 0, h->stream, a);
   hipLaunchKernelGGL(k2d_wide_cand, dim3(bw), dim3(256), 0, h->stream, a);  // a wave per cell
-  if (a.g.mask & M2_REPULSION) {  // (vertex, candidate slot) threads
-    const long long n = (long long)h->V * DPM2D_MAXCAND;
-    hipLaunchKernelGGL(k2d_wide_over, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, h->stream, a);
-  }
-  hipLaunchKernelGGL(k2d_wide_step, dim3(bv), dim3(256), 0, h->stream, a);
+  hipLaunchKernelGGL(step, dim3(bv), dim3(256), 0, h->stream, a);  // G lanes per vertex
   HIPCHECK(hipGetLastError());
   return DPM_OK;
 }
