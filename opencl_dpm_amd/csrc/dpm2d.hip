@@ -72,6 +72,18 @@ __host__ __device__ inline size_t lds2d_bytes(int nvt, int nc, int rs) {
   return b + sizeof(double) * DPM2D_RED;
 }
 
+// Optional LDS behind those arrays (and the pair list of k2d_run), taken
+// where it fits: the boxes of the cells' arcs of DPM2D_ARC vertices and, for
+// at most 256 cells, the cell of each vertex as a byte.
+#define DPM2D_ARC 8
+template <typename R>
+struct alignas(4 * sizeof(R)) Box4 {
+  R x0, x1, y0, y1;
+};
+__host__ __device__ inline size_t lds2d_extra_bytes(int nvt, int nc, int rs) {
+  return 32u + 4u * (size_t)rs * (size_t)(nvt / DPM2D_ARC + nc) + (nc <= 256 ? (size_t)nvt : 0u);
+}
+
 template <typename R>
 struct Lds2D {
   R *x, *y;
@@ -82,11 +94,24 @@ struct Lds2D {
   short* cand;
   unsigned* cbits;  // [nc * CSPLIT] candidate bits of one chunk of cells
   double* red;
+  bool has_arc, has_vc;  // (flags beside the pointers, which stay LDS addresses to the compiler)
+  Box4<R>* arc;          // arc boxes, cell c's from arc_base(c)
+  unsigned char* vc;     // cell of each vertex
 };
 
+// First arc box of cell c (a cell's arcs, ceil(n / DPM2D_ARC), never reach
+// the next cell's first).
+__device__ __forceinline__ int arc_base(const int* vb, int c) { return vb[c] / DPM2D_ARC + c; }
+
+// extra: byte offset of the optional arrays (0: none).
 template <typename R>
-__device__ __forceinline__ Lds2D<R> carve2d(unsigned char* smem, int nvt, int nc) {
+__device__ __forceinline__ Lds2D<R> carve2d(unsigned char* smem, int nvt, int nc, size_t extra = 0) {
   Lds2D<R> l;
+  extra = (extra + 31u) & ~(size_t)31u;
+  l.has_arc = extra != 0;
+  l.has_vc = extra != 0 && nc <= 256;
+  l.arc = reinterpret_cast<Box4<R>*>(smem + extra);
+  l.vc = smem + extra + sizeof(Box4<R>) * (size_t)(nvt / DPM2D_ARC + nc);
   l.x = reinterpret_cast<R*>(smem);
   l.y = l.x + nvt;
   size_t o = sizeof(R) * 2u * (size_t)nvt;
@@ -149,33 +174,67 @@ __device__ __forceinline__ int cell_of(const int* vb, int nc, int k) {
   return lo;
 }
 
-// Per-cell quantities of the current positions: area strain (double area),
-// orientation, centre of mass, axis-aligned bounds, of tissue-local cell c.
 template <typename R>
-__device__ __forceinline__ void cell_one(const Geom2D<R>& g, const Tissue2DCtx<R>& T, const Lds2D<R>& l, int c) {
+__device__ __forceinline__ int vertex_cell(const Lds2D<R>& l, int nc, int k) {
+  return l.has_vc ? (int)l.vc[k] : cell_of(l.vb, nc, k);
+}
+
+__device__ __forceinline__ float dpp8(float v, int step) {
+  return step == 1 ? dpp_f<0xB1, 0xF>(v) : step == 2 ? dpp_f<0x4E, 0xF>(v) : dpp_f<0x141, 0xF>(v);
+}
+__device__ __forceinline__ double dpp8(double v, int step) {
+  return step == 1 ? dpp_d<0xB1, 0xF>(v) : step == 2 ? dpp_d<0x4E, 0xF>(v) : dpp_d<0x141, 0xF>(v);
+}
+
+// Per-cell quantities of the current positions: area strain (double area),
+// orientation, centre of mass, axis-aligned bounds, of tissue-local cell c,
+// by an aligned group of eight lanes (sub = 0..7, all calling with the same
+// c).  A lane takes every eighth arc of DPM2D_ARC vertices, in order; the
+// group's sums are added in a fixed tree (swaps within quads, then the two
+// quads), the same in every kernel that calls this.  With l.has_arc the arcs'
+// boxes are kept: arc a holds vertices 8a - 1 (the last one for arc 0) to
+// 8a + 7, both ends of each of its edges.
+template <typename R>
+__device__ __forceinline__ void cell_group(const Geom2D<R>& g, const Tissue2DCtx<R>& T, const Lds2D<R>& l, int c,
+                                           int sub) {
   const int b = l.vb[c], e = l.vb[c + 1], n = e - b;
   double area = 0.0, sx = 0.0, sy = 0.0;
-  R x0 = l.x[b], x1 = l.x[b], y0 = l.y[b], y1 = l.y[b];
-  // vertex k's predecessor (the last vertex before the first) carried in
-  // registers, the loads of several vertices issued ahead: the same
-  // operations in the same order as one vertex after the other
-  R xp = l.x[e - 1], yp = l.y[e - 1];
+  R x0 = l.x[b], x1 = x0, y0 = l.y[b], y1 = y0;
+  for (int a = sub; DPM2D_ARC * a < n; a += 8) {
+    const int i0 = b + DPM2D_ARC * a, i1 = min(i0 + DPM2D_ARC, e);
+    const int ip = a == 0 ? e - 1 : i0 - 1;
+    R xp = l.x[ip], yp = l.y[ip];
+    R bx0 = xp, bx1 = xp, by0 = yp, by1 = yp;
 #pragma unroll 4
-  for (int j = 0; j < n; j++) {
-    const int k = b + j;
-    const R xk = l.x[k], yk = l.y[k];
-    const double xs = (double)xp + (double)xk;
-    const double yd = (double)yp - (double)yk;
-    area += xs * yd;
-    sx += (double)xk;
-    sy += (double)yk;
-    x0 = fmin(x0, xk);
-    x1 = fmax(x1, xk);
-    y0 = fmin(y0, yk);
-    y1 = fmax(y1, yk);
-    xp = xk;
-    yp = yk;
+    for (int k = i0; k < i1; k++) {
+      const R xk = l.x[k], yk = l.y[k];
+      area += ((double)xp + (double)xk) * ((double)yp - (double)yk);
+      sx += (double)xk;
+      sy += (double)yk;
+      bx0 = fmin(bx0, xk);
+      bx1 = fmax(bx1, xk);
+      by0 = fmin(by0, yk);
+      by1 = fmax(by1, yk);
+      xp = xk;
+      yp = yk;
+    }
+    if (l.has_arc) l.arc[arc_base(l.vb, c) + a] = Box4<R>{bx0, bx1, by0, by1};
+    x0 = fmin(x0, bx0);
+    x1 = fmax(x1, bx1);
+    y0 = fmin(y0, by0);
+    y1 = fmax(y1, by1);
   }
+#pragma unroll
+  for (int s = 1; s <= 4; s *= 2) {
+    area += dpp8(area, s);
+    sx += dpp8(sx, s);
+    sy += dpp8(sy, s);
+    x0 = fmin(x0, dpp8(x0, s));
+    x1 = fmax(x1, dpp8(x1, s));
+    y0 = fmin(y0, dpp8(y0, s));
+    y1 = fmax(y1, dpp8(y1, s));
+  }
+  if (sub != 0) return;
   l.strain[c] = (R)(0.5 * fabs(area) / (double)g.a0[T.c0 + c] - 1.0);
   // the shoelace sum in this order is negative for counter-clockwise cells
   l.orient[c] = area < 0.0 ? R(-1) : R(1);
@@ -187,10 +246,10 @@ __device__ __forceinline__ void cell_one(const Geom2D<R>& g, const Tissue2DCtx<R
   l.ay1[c] = y1;
 }
 
-// cell_one for every cell of the tissue, one thread per cell.
+// cell_group for every cell of the tissue.
 template <typename R>
 __device__ void cell_pass(const Geom2D<R>& g, const Tissue2DCtx<R>& T, const Lds2D<R>& l) {
-  for (int c = threadIdx.x; c < T.nc; c += blockDim.x) cell_one(g, T, l, c);
+  for (int c = threadIdx.x / 8; c < T.nc; c += blockDim.x / 8) cell_group(g, T, l, c, threadIdx.x & 7);
 }
 
 // Cell-level candidate lists: cell cj is a candidate of ci unless every
@@ -284,24 +343,92 @@ __device__ void cand_pass(const Geom2D<R>& g, const Tissue2DCtx<R>& T, const Lds
   for (int ci = threadIdx.x; ci < nc; ci += NT) cand_one(g, T, l, ci);
 }
 
-// True when no vertex of cell cj can lie within `cut` of point p under the
-// per-pair minimum image: per axis the minimum-image gap between p and cj's
-// axis-aligned box exceeds the cut-off, and the box is small against L (then
-// no other image comes closer) — maybe_pair's argument with a point for the
-// first box.  Skipping such a cell leaves every sum unchanged.
+// Where cell cj lies from point p under the per-pair minimum image, for
+// vertices within `cut` of p.  far: per axis the minimum-image gap between p
+// and cj's axis-aligned box exceeds the cut-off, and the box is small against
+// L (then no other image comes closer) — maybe_pair's argument with a point
+// for the first box.  Else, with small: cj's vertices that can be within the
+// cut-off lie at raw position - (sx, sy), so an arc's box decides for its
+// vertices the same way (far_from).  Skipping what is far leaves every sum
+// unchanged.
+template <typename R>
+struct CellImage {
+  bool far, small;
+  R sx, sy, reach;
+  __device__ __forceinline__ CellImage(R x0, R x1, R y0, R y1, const Tissue2DCtx<R>& T, R px, R py, R cut)
+      : far(false), small(true), sx(R(0)), sy(R(0)) {
+    const R L = T.L;
+    const R hx = R(0.5f) * (x1 - x0), hy = R(0.5f) * (y1 - y0);
+    R dx = R(0.5f) * (x0 + x1) - px, dy = R(0.5f) * (y0 + y1) - py;
+    reach = cut * R(1.0001f) + R(1e-5f) * (R(1) + L);
+    if (T.pbc) {
+      small = hx + cut < R(0.45f) * L && hy + cut < R(0.45f) * L;
+      sx = L * round(dx * T.invL);
+      sy = L * round(dy * T.invL);
+      dx -= sx;
+      dy -= sy;
+    }
+    far = small && (fabs(dx) - hx > reach || fabs(dy) - hy > reach);
+  }
+  __device__ __forceinline__ bool far_from(const Box4<R>& b, R px, R py) const {
+    const R dx = (R(0.5f) * (b.x0 + b.x1) - px) - sx, dy = (R(0.5f) * (b.y0 + b.y1) - py) - sy;
+    return fabs(dx) - R(0.5f) * (b.x1 - b.x0) > reach || fabs(dy) - R(0.5f) * (b.y1 - b.y0) > reach;
+  }
+};
+template <typename R>
+__device__ __forceinline__ CellImage<R> cell_image(const Lds2D<R>& l, const Tissue2DCtx<R>& T, int cj, R px, R py,
+                                                   R cut) {
+  return CellImage<R>(l.ax0[cj], l.ax1[cj], l.ay0[cj], l.ay1[cj], T, px, py, cut);
+}
 template <typename R>
 __device__ __forceinline__ bool vertex_far_from_box(const Lds2D<R>& l, const Tissue2DCtx<R>& T, int cj, R px, R py,
                                                     R cut) {
-  const R L = T.L;
-  const R hx = R(0.5f) * (l.ax1[cj] - l.ax0[cj]), hy = R(0.5f) * (l.ay1[cj] - l.ay0[cj]);
-  R dx = R(0.5f) * (l.ax0[cj] + l.ax1[cj]) - px, dy = R(0.5f) * (l.ay0[cj] + l.ay1[cj]) - py;
-  if (T.pbc) {
-    if (!(hx + cut < R(0.45f) * L && hy + cut < R(0.45f) * L)) return false;
-    dx -= L * round(dx * T.invL);
-    dy -= L * round(dy * T.invL);
+  return cell_image(l, T, cj, px, py, cut).far;
+}
+
+// Candidate loops of one vertex.  A lane first tests all candidates of its
+// cell (up to 64 at a time) into a bit mask, then walks its own bits: a wave
+// runs as many rounds as its lane with most near cells (two or three), not
+// one for every candidate that is near some lane.  Ascending cell order.
+template <typename R, typename Keep, typename Cell>
+__device__ __forceinline__ void each_candidate(const Lds2D<R>& l, int ci, int nc, Keep keep, Cell cell) {
+  const int ncd = l.ncand[ci];
+  const bool scan_all = ncd > DPM2D_MAXCAND;
+  const int ncl = scan_all ? nc : ncd;
+  for (int q0 = 0; q0 < ncl; q0 += 64) {
+    const int q1 = min(ncl, q0 + 64);
+    unsigned long long m = 0ull;
+    for (int q = q0; q < q1; q++) {
+      const int cj = scan_all ? q : (int)l.cand[ci * DPM2D_MAXCAND + q];
+      if (cj != ci && keep(cj)) m |= 1ull << (q - q0);
+    }
+    for (; m; m &= m - 1ull) {
+      const int q = q0 + __ffsll((long long)m) - 1;
+      if (!cell(scan_all ? q : (int)l.cand[ci * DPM2D_MAXCAND + q])) return;
+    }
   }
-  const R reach = cut * R(1.0001f) + R(1e-5f) * (R(1) + L);
-  return fabs(dx) - hx > reach || fabs(dy) - hy > reach;
+}
+// The vertices [j0, j1) of cell cj, arc by arc where the boxes are kept
+// (arcs with skip(box) left out), ascending.
+template <typename R, typename Skip, typename Arc>
+__device__ __forceinline__ void each_arc(const Lds2D<R>& l, int cj, Skip skip, Arc arc) {
+  const int b = l.vb[cj], e = l.vb[cj + 1];
+  if (!l.has_arc) {  // block-uniform
+    arc(b, e);
+    return;
+  }
+  const int na = (e - b + DPM2D_ARC - 1) / DPM2D_ARC;
+  const Box4<R>* box = l.arc + arc_base(l.vb, cj);
+  for (int a0 = 0; a0 < na; a0 += 32) {
+    const int a1 = min(na, a0 + 32);
+    unsigned m = 0u;
+    for (int a = a0; a < a1; a++)
+      if (!skip(box[a])) m |= 1u << (a - a0);
+    for (; m; m &= m - 1u) {
+      const int i = b + DPM2D_ARC * (a0 + __ffs((int)m) - 1);
+      arc(i, min(i + DPM2D_ARC, e));
+    }
+  }
 }
 
 // floor(x / L) and round(x / L) as the reference evaluates them (a
@@ -335,12 +462,21 @@ __device__ __forceinline__ R round_quot(R x, R L, R invL) {
 // rounded sum of two floats is 0 only when the exact sum is, so the sign of
 // tt is the sign of q + dix for the rounded quotient q.)
 template <typename R>
-__device__ __forceinline__ bool crossing_odd(const Lds2D<R>& l, int cj, R px, R py, int pbc, R L,
+__device__ __forceinline__ bool edge_counts(R dix, R diy, R djx, R djy) {
+  if ((diy > R(0)) == (djy > R(0))) return false;
+  const R a = (djx - dix) * (R(0) - diy), c = djy - diy;
+  if constexpr (sizeof(R) == 4) {
+    const R qa = a * __builtin_amdgcn_rcpf(c), ta = qa + dix;
+    if (fabs(ta) > R(1e-6f) * (fabs(qa) + fabs(dix))) return ta > R(0);
+  }
+  return R(0) < a / c + dix;
+}
+template <typename R>
+__device__ __forceinline__ bool crossing_odd(const Lds2D<R>& l, int cj, R px, R py, int pbc, R L, R invL,
                                              int first = 0, int stride = 1) {
   // the edges (i, i - 1) for i = first, first + stride, ... (all of them by
   // default; a share of them when several lanes split one polygon)
   const int b = l.vb[cj], e = l.vb[cj + 1], n = e - b;
-  const R invL = R(1) / L;
   bool odd = false;
   for (int i = first; i < n; i += stride) {
     const int j = i == 0 ? n - 1 : i - 1;
@@ -356,20 +492,7 @@ __device__ __forceinline__ bool crossing_odd(const Lds2D<R>& l, int cj, R px, R 
         djy -= L * round_quot(djy, L, invL);
       }
     }
-    if ((diy > R(0)) != (djy > R(0))) {
-      const R a = (djx - dix) * (R(0) - diy), c = djy - diy;
-      bool pos;
-      if constexpr (sizeof(R) == 4) {
-        const R qa = a * __builtin_amdgcn_rcpf(c), ta = qa + dix;
-        if (fabs(ta) > R(1e-6f) * (fabs(qa) + fabs(dix)))
-          pos = ta > R(0);
-        else
-          pos = R(0) < a / c + dix;
-      } else {
-        pos = R(0) < a / c + dix;
-      }
-      if (pos) odd = !odd;
-    }
+    odd ^= edge_counts(dix, diy, djx, djy);
   }
   return odd;
 }
@@ -395,6 +518,33 @@ __device__ __forceinline__ bool outside_box_even(const Lds2D<R>& l, int cj, R px
   const bool yin = !pbc || (fabs(py - y0) <= L && fabs(py - y1) <= L);
   const R m = R(1e-5f) * (R(1) + L);
   return (yin && (py < y0 || py > y1)) || (xin && (px < x0 - m || (yin && px > x1 + m)));
+}
+
+// crossing_odd of a whole cell by one lane.  Where both axes are taken raw
+// (outside_box_even's tests of the cell's box) an arc whose box, with both
+// ends of its edges, lies above or below p straddles no row, and one that lies
+// right of p by the margin has no crossing that counts: only the others' edges
+// are tested.
+template <typename R>
+__device__ __forceinline__ bool crossing_odd_cell(const Lds2D<R>& l, int cj, R px, R py, const Tissue2DCtx<R>& T) {
+  const R L = T.L;
+  const bool raw = !T.pbc || (fabs(px - l.ax0[cj]) <= L && fabs(px - l.ax1[cj]) <= L &&
+                              fabs(py - l.ay0[cj]) <= L && fabs(py - l.ay1[cj]) <= L);
+  if (!raw || !l.has_arc) return crossing_odd(l, cj, px, py, T.pbc, L, T.invL);
+  const R m = R(1e-5f) * (R(1) + L);
+  const int b = l.vb[cj], e = l.vb[cj + 1];
+  bool odd = false;
+  each_arc(l, cj, [&](const Box4<R>& q) { return py < q.y0 || py > q.y1 || px < q.x0 - m; }, [&](int j0, int j1) {
+    const int p = j0 == b ? e - 1 : j0 - 1;
+    R djx = px - l.x[p], djy = py - l.y[p];
+    for (int j = j0; j < j1; j++) {
+      const R dix = px - l.x[j], diy = py - l.y[j];
+      odd ^= edge_counts(dix, diy, djx, djy);
+      djx = dix;
+      djy = diy;
+    }
+  });
+  return odd;
 }
 
 // Crossing parity of every vertex against every candidate cell: bit k of
@@ -423,7 +573,7 @@ __device__ void over_pass(const Tissue2DCtx<R>& T, const Lds2D<R>& l, unsigned* 
       k -= nvt;
       q++;
     }
-    const int ci = cell_of(l.vb, nc, k);
+    const int ci = vertex_cell(l, nc, k);
     const int ncd = l.ncand[ci];
     const bool scan_all = ncd > DPM2D_MAXCAND;
     bool pass = false;
@@ -436,7 +586,7 @@ __device__ void over_pass(const Tissue2DCtx<R>& T, const Lds2D<R>& l, unsigned* 
       pass = cj != ci && !outside_box_even(l, cj, px, py, T.pbc, T.L);
     }
     if (cap == 0) {  // block-uniform: no list (count and list are not allocated)
-      if (pass && crossing_odd(l, cj, px, py, T.pbc, T.L)) atomicOr(&bits[k >> 5], 1u << (k & 31));
+      if (pass && crossing_odd_cell(l, cj, px, py, T)) atomicOr(&bits[k >> 5], 1u << (k & 31));
       continue;
     }
     const unsigned long long m = __ballot(pass);
@@ -449,7 +599,7 @@ __device__ void over_pass(const Tissue2DCtx<R>& T, const Lds2D<R>& l, unsigned* 
       const int slot = base + (int)__popcll(m & ((1ull << lane) - 1ull));
       if (slot < cap)
         list[slot] = k | (cj << 16);
-      else if (crossing_odd(l, cj, px, py, T.pbc, T.L))
+      else if (crossing_odd_cell(l, cj, px, py, T))
         atomicOr(&bits[k >> 5], 1u << (k & 31));
     }
   }
@@ -460,7 +610,7 @@ __device__ void over_pass(const Tissue2DCtx<R>& T, const Lds2D<R>& l, unsigned* 
   const int n = min(*count, cap);
   for (int i = threadIdx.x; i < 8 * n; i += blockDim.x) {
     const int e = list[i >> 3], g = i & 7, k = e & 0xffff, cj = e >> 16;
-    int odd = crossing_odd(l, cj, l.x[k], l.y[k], T.pbc, T.L, g, 8) ? 1 : 0;
+    int odd = crossing_odd(l, cj, l.x[k], l.y[k], T.pbc, T.L, T.invL, g, 8) ? 1 : 0;
     odd ^= __shfl_xor(odd, 1);
     odd ^= __shfl_xor(odd, 2);
     odd ^= __shfl_xor(odd, 4);
@@ -565,91 +715,91 @@ __device__ __forceinline__ void force_vertex(const Geom2D<R>& g, const Tissue2DC
                                           int k, R& Fx, R& Fy, int* n_over, int* n_attr, double* energy,
                                           double* e_int, const unsigned* over_bits = nullptr,
                                           unsigned* attr_key = nullptr) {
-  const int ci = cell_of(l.vb, T.nc, k);
+  const int ci = vertex_cell(l, T.nc, k);
   const int gc = T.c0 + ci;
-  const int n = l.vb[ci + 1] - l.vb[ci];
   const R px = l.x[k], py = l.y[k];
   const R L = T.L;
   const unsigned mask = g.mask;
   R fx, fy;
   shape_vertex(g, T, l, ci, k, fx, fy, energy);
-  const int nc = l.ncand[ci];
-  const bool scan_all = nc > DPM2D_MAXCAND;
-  const int ncl = scan_all ? T.nc : nc;
   const R half_l = R(0.49f) * L;
   // With Kat = 0 the attraction adds exact zeros: it is evaluated only where
   // its partners are asked for (n_attr, attr_key).
   if ((mask & M2_ATTRACTION) && (T.Kat != R(0) || n_attr || attr_key)) {
     const R l0 = (R)g.l0[gc];
-    const R kat = T.Kat / (R)n;
+    const R kat = T.Kat / (R)(l.vb[ci + 1] - l.vb[ci]);
     const R lim = l0 * l0 * R(1.00001f);
     const double kk = (double)kat / (double)l0;  // ftmp/d = kat/l0 of an accepted pair
     int cnt = 0;
-    for (int q = 0; q < ncl; q++) {
-      const int cj = scan_all ? q : (int)l.cand[ci * DPM2D_MAXCAND + q];
-      if (cj == ci || vertex_far_from_box(l, T, cj, px, py, l0)) continue;
-      for (int j = l.vb[cj]; j < l.vb[cj + 1]; j++) {
-        R rx = l.x[j] - px, ry = l.y[j] - py;
-        R nx = R(0), ny = R(0);
-        // minimum image; a component below 0.49 L rounds to image 0, which
-        // leaves it unchanged, so the division is skipped there
-        if (T.pbc && !(fabs(rx) < half_l && fabs(ry) < half_l)) {
-          nx = round(rx / L);
-          ny = round(ry / L);
-          rx -= L * nx;
-          ry -= L * ny;
+    each_candidate(l, ci, T.nc, [&](int cj) { return !cell_image(l, T, cj, px, py, l0).far; }, [&](int cj) {
+      const CellImage<R> im = cell_image(l, T, cj, px, py, l0);
+      each_arc(l, cj, [&](const Box4<R>& q) { return im.small && im.far_from(q, px, py); }, [&](int j0, int j1) {
+        for (int j = j0; j < j1; j++) {
+          R rx = l.x[j] - px, ry = l.y[j] - py;
+          R nx = R(0), ny = R(0);
+          // minimum image; a component below 0.49 L rounds to image 0, which
+          // leaves it unchanged, so the division is skipped there
+          if (T.pbc && !(fabs(rx) < half_l && fabs(ry) < half_l)) {
+            nx = round(rx / L);
+            ny = round(ry / L);
+            rx -= L * nx;
+            ry -= L * ny;
+          }
+          const R d2 = rx * rx + ry * ry;
+          if (!(d2 < lim)) continue;  // sqrt(d2) < l0 needs d2 < l0^2 (1 + 1e-5)
+          const R dist = sqrt(d2);
+          if (dist < l0) {
+            // the reference's decision; the force (kat d/l0 along r) in
+            // double on the same image, as a short image vector keeps few
+            // digits in float
+            const double ddx = ((double)l.x[j] - (double)px) - (double)L * (double)nx;
+            const double ddy = ((double)l.y[j] - (double)py) - (double)L * (double)ny;
+            fx += (R)(kk * ddx);
+            fy += (R)(kk * ddy);
+            cnt++;
+            if (attr_key) atomicAdd(attr_key, vertex_key(l.x[j], l.y[j]));
+          }
         }
-        const R d2 = rx * rx + ry * ry;
-        if (!(d2 < lim)) continue;  // sqrt(d2) < l0 needs d2 < l0^2 (1 + 1e-5)
-        const R dist = sqrt(d2);
-        if (dist < l0) {
-          // the reference's decision; the force (kat d/l0 along r) in
-          // double on the same image, as a short image vector keeps few
-          // digits in float
-          const double ddx = ((double)l.x[j] - (double)px) - (double)L * (double)nx;
-          const double ddy = ((double)l.y[j] - (double)py) - (double)L * (double)ny;
-          fx += (R)(kk * ddx);
-          fy += (R)(kk * ddy);
-          cnt++;
-          if (attr_key) atomicAdd(attr_key, vertex_key(l.x[j], l.y[j]));
-        }
-      }
-    }
+      });
+      return true;
+    });
     if (n_attr) *n_attr = cnt;
   }
   if (mask & M2_VREPULSION) {
     // U = Kre/2 (1 - d/sigma)^2 for d < sigma = (l0_i + l0_j)/2
     const R l0i = (R)g.l0[gc];
-    for (int q = 0; q < ncl; q++) {
-      const int cj = scan_all ? q : (int)l.cand[ci * DPM2D_MAXCAND + q];
-      if (cj == ci) continue;
-      const R sig = R(0.5f) * (l0i + (R)g.l0[T.c0 + cj]);
-      if (vertex_far_from_box(l, T, cj, px, py, sig)) continue;
-      for (int j = l.vb[cj]; j < l.vb[cj + 1]; j++) {
-        R rx = l.x[j] - px, ry = l.y[j] - py;
-        if (T.pbc && !(fabs(rx) < half_l && fabs(ry) < half_l)) {
-          rx -= L * round(rx / L);
-          ry -= L * round(ry / L);
+    auto sigma = [&](int cj) { return R(0.5f) * (l0i + l.l0c[cj]); };
+    each_candidate(l, ci, T.nc, [&](int cj) { return !cell_image(l, T, cj, px, py, sigma(cj)).far; }, [&](int cj) {
+      const R sig = sigma(cj);
+      const CellImage<R> im = cell_image(l, T, cj, px, py, sig);
+      each_arc(l, cj, [&](const Box4<R>& q) { return im.small && im.far_from(q, px, py); }, [&](int j0, int j1) {
+        for (int j = j0; j < j1; j++) {
+          R rx = l.x[j] - px, ry = l.y[j] - py;
+          if (T.pbc && !(fabs(rx) < half_l && fabs(ry) < half_l)) {
+            rx -= L * round(rx / L);
+            ry -= L * round(ry / L);
+          }
+          const R d2 = rx * rx + ry * ry;
+          if (!(d2 < sig * sig) || d2 == R(0)) continue;
+          const R dist = sqrt(d2);
+          const R ov = R(1) - dist / sig;
+          const R ft = T.Kre / sig * ov / dist;
+          fx -= ft * rx;
+          fy -= ft * ry;
+          if (e_int) *e_int += 0.25 * (double)T.Kre * (double)ov * (double)ov;  // half of the pair
         }
-        const R d2 = rx * rx + ry * ry;
-        if (!(d2 < sig * sig) || d2 == R(0)) continue;
-        const R dist = sqrt(d2);
-        const R ov = R(1) - dist / sig;
-        const R ft = T.Kre / sig * ov / dist;
-        fx -= ft * rx;
-        fy -= ft * ry;
-        if (e_int) *e_int += 0.25 * (double)T.Kre * (double)ov * (double)ov;  // half of the pair
-      }
-    }
+      });
+      return true;
+    });
   }
   if (mask & M2_REPULSION) {
     // the crossing parity given (bit k of over_bits), else found by the loop
     bool over = over_bits && ((over_bits[k >> 5] >> (k & 31)) & 1u);
-    for (int q = 0; q < ncl && !over && !over_bits; q++) {
-      const int cj = scan_all ? q : (int)l.cand[ci * DPM2D_MAXCAND + q];
-      if (cj == ci || outside_box_even(l, cj, px, py, T.pbc, L)) continue;
-      over = crossing_odd(l, cj, px, py, T.pbc, L);
-    }
+    if (!over_bits)
+      each_candidate(l, ci, T.nc, [&](int cj) { return !outside_box_even(l, cj, px, py, T.pbc, L); }, [&](int cj) {
+        over = crossing_odd_cell(l, cj, px, py, T);
+        return !over;
+      });
     if (over) repulsion_push(g, T, l, ci, px, py, fx, fy);
     *n_over = over ? 1 : 0;
   }
@@ -662,7 +812,12 @@ __device__ __forceinline__ void stage_tissue(const Geom2D<R>& g, const Tissue2DC
                                              const R* x, const R* y) {
   for (int c = threadIdx.x; c <= T.nc; c += blockDim.x) {
     l.vb[c] = g.cell_vert_begin[T.c0 + c] - T.v0;
-    if (c < T.nc) l.l0c[c] = (R)g.l0[T.c0 + c];
+    if (c < T.nc) {
+      l.l0c[c] = (R)g.l0[T.c0 + c];
+      if (l.has_vc)
+        for (int k = g.cell_vert_begin[T.c0 + c], e = g.cell_vert_begin[T.c0 + c + 1]; k < e; k++)
+          l.vc[k - T.v0] = (unsigned char)c;
+    }
   }
   for (int k = threadIdx.x; k < T.nvt; k += blockDim.x) {
     l.x[k] = x[T.v0 + k];
@@ -686,6 +841,7 @@ struct Run2D {
   int* p_attr;
   unsigned* p_attr_key;  // attraction partner-set key sums (vertex_key)
   int over_cap;          // entries of the crossing-parity pair list after the LDS arrays (0: none)
+  int extra;             // the optional LDS arrays fit (arc boxes, vertex cells)
 };
 
 // The crossing-parity pair list of k2d_run (a count, the largest candidate
@@ -694,32 +850,50 @@ struct Run2D {
 #define DPM2D_OVER_CAP 2048
 __host__ __device__ inline size_t lds2d_over_bytes() { return sizeof(int) * (size_t)(DPM2D_OVER_CAP + 2); }
 
-// Forces stay in registers: up to DPM2D_VPT vertices per thread.
+// Vertices per thread at most.
 #define DPM2D_VPT 16
+
+// Whether a tissue takes the crossing parity in its own pass on NT threads:
+// its (vertex, candidate) pairs are at most 16 per thread and one bit per
+// vertex fits the candidate-bit words (nc * DPM2D_CSPLIT of them, unused
+// between the candidate and the next step's cell pass).
+__host__ __device__ inline bool over_split(int nvt, int nc, int NT) {
+  return nvt <= 32 * DPM2D_CSPLIT * nc && (long long)nvt * nc <= 16LL * NT;
+}
+// k2d_run's LDS of one tissue: the arrays, the pair list where the tissue
+// takes the pass, the optional arrays.
+__host__ __device__ inline size_t run2d_list_bytes(int nvt, int nc, int NT, int over_cap) {
+  return over_cap > 0 && over_split(nvt, nc, NT) ? lds2d_over_bytes() : 0u;
+}
 
 extern "C" __global__ void __launch_bounds__(1024) k2d_run(const Run2D a) {
   extern __shared__ __align__(16) unsigned char smem[];
   const Geom2D<float>& g = a.g;
   const Tissue2DCtx<float> T = tissue_ctx(g, blockIdx.x);
-  const Lds2D<float> l = carve2d<float>(smem, T.nvt, T.nc);
   const int tid = threadIdx.x, NT = blockDim.x;
+  const size_t base = lds2d_bytes(T.nvt, T.nc, (int)sizeof(float));
+  const Lds2D<float> l = carve2d<float>(
+      smem, T.nvt, T.nc, a.extra ? base + run2d_list_bytes(T.nvt, T.nc, NT, a.over_cap) : 0);
   stage_tissue(g, T, l, a.x, a.y);
 
   const int nsteps = a.nsteps;
   const int nevals = nsteps > 0 ? nsteps : 1;
   unsigned long long n_over_total = 0;
-  // Crossing parity in its own pass when the (vertex, candidate) pairs are at
-  // most 16 per thread and one bit per vertex fits the candidate-bit words
-  // (nc * DPM2D_CSPLIT of them, unused between the candidate and the next
-  // step's cell pass).
-  const bool split_over = (g.mask & M2_REPULSION) && T.nvt <= 32 * DPM2D_CSPLIT * T.nc &&
-                          T.nvt * T.nc <= 16 * NT;
+  const bool split_over = (g.mask & M2_REPULSION) && over_split(T.nvt, T.nc, NT);
   unsigned* obits = l.cbits;
-  int* ocount = reinterpret_cast<int*>(smem + lds2d_bytes(T.nvt, T.nc, (int)sizeof(float)));
+  int* ocount = reinterpret_cast<int*>(smem + base);
   int* oqmax = ocount + 1;
   int* olist = ocount + 2;
-  if (tid == 0 && a.over_cap > 0) *oqmax = 0;  // (the first step's barriers precede its use)
-  float rfx[DPM2D_VPT], rfy[DPM2D_VPT];
+  const bool listed = split_over && a.over_cap > 0;  // block-uniform
+  if (tid == 0 && listed) *oqmax = 0;  // (the first step's barriers precede its use)
+  auto force = [&](int k, float& fx, float& fy) {
+    int no = 0, na = 0;
+    force_vertex(g, T, l, k, fx, fy, &no, a.p_attr ? &na : nullptr, (double*)nullptr, (double*)nullptr,
+                 split_over ? obits : nullptr, a.p_attr_key ? a.p_attr_key + T.v0 + k : nullptr);
+    n_over_total += no;
+    if (a.p_overlap) a.p_overlap[T.v0 + k] = no;
+    if (a.p_attr) a.p_attr[T.v0 + k] = na;
+  };
   for (int s = 0; s < nevals; s++) {
     cell_pass(g, T, l);
     __syncthreads();
@@ -727,7 +901,7 @@ extern "C" __global__ void __launch_bounds__(1024) k2d_run(const Run2D a) {
     __syncthreads();
     if (split_over) {  // block-uniform; the candidate bits are dead here
       for (int i = tid; i < (T.nvt + 31) / 32; i += NT) obits[i] = 0u;
-      if (a.over_cap > 0) {
+      if (listed) {
         if (tid == 0) *ocount = 0;
         for (int c = tid; c < T.nc; c += NT) {
           const int nd = l.ncand[c];
@@ -735,47 +909,31 @@ extern "C" __global__ void __launch_bounds__(1024) k2d_run(const Run2D a) {
         }
       }
       __syncthreads();
-      over_pass(T, l, obits, olist, a.over_cap, ocount, a.over_cap > 0 ? *oqmax : T.nc);
+      over_pass(T, l, obits, olist, a.over_cap, ocount, listed ? *oqmax : T.nc);
       __syncthreads();
-      if (tid == 0 && a.over_cap > 0) *oqmax = 0;  // every thread read it before the barrier above
+      if (tid == 0 && listed) *oqmax = 0;  // every thread read it before the barrier above
     }
-#pragma unroll
-    for (int r = 0; r < DPM2D_VPT; r++) {
-      const int k = tid + r * NT;
-      rfx[r] = 0.0f;
-      rfy[r] = 0.0f;
-      if (k < T.nvt) {
-        int no = 0, na = 0;
-        force_vertex(g, T, l, k, rfx[r], rfy[r], &no, a.p_attr ? &na : nullptr, (double*)nullptr, (double*)nullptr,
-                     split_over ? obits : nullptr, a.p_attr_key ? a.p_attr_key + T.v0 + k : nullptr);
-        n_over_total += no;
-        if (a.p_overlap) a.p_overlap[T.v0 + k] = no;
-        if (a.p_attr) a.p_attr[T.v0 + k] = na;
-      }
+    // The forces wait in global memory (written and read by the same thread)
+    // for the barrier before the move: in registers, up to DPM2D_VPT per
+    // thread, they need the loop unrolled, sixteen copies of force_vertex.
+    for (int k = tid; k < T.nvt; k += NT) {
+      float fx, fy;
+      force(k, fx, fy);
+      a.fx[T.v0 + k] = fx;
+      a.fy[T.v0 + k] = fy;
     }
     __syncthreads();
     if (nsteps > 0) {
-      const float dt = a.dt;
-#pragma unroll
-      for (int r = 0; r < DPM2D_VPT; r++) {
-        const int k = tid + r * NT;
-        if (k < T.nvt) {
-          l.x[k] = fmaf(rfx[r], dt, l.x[k]);
-          l.y[k] = fmaf(rfy[r], dt, l.y[k]);
-        }
+      for (int k = tid; k < T.nvt; k += NT) {
+        l.x[k] = fmaf(a.fx[T.v0 + k], a.dt, l.x[k]);
+        l.y[k] = fmaf(a.fy[T.v0 + k], a.dt, l.y[k]);
       }
       __syncthreads();
     }
   }
-#pragma unroll
-  for (int r = 0; r < DPM2D_VPT; r++) {
-    const int k = tid + r * NT;
-    if (k < T.nvt) {
-      a.x[T.v0 + k] = l.x[k];
-      a.y[T.v0 + k] = l.y[k];
-      a.fx[T.v0 + k] = rfx[r];
-      a.fy[T.v0 + k] = rfy[r];
-    }
+  for (int k = tid; k < T.nvt; k += NT) {
+    a.x[T.v0 + k] = l.x[k];
+    a.y[T.v0 + k] = l.y[k];
   }
   if (a.counters) {
     const double c = block_sum((double)n_over_total, l.red);
@@ -844,13 +1002,13 @@ struct Relax2D {
   R* tLout;              // [T] box length at the end (jamming changes it)
   double* res;           // [T * RS_COUNT]
   const double* sum_a0;  // [T]
-  int mode;
   int nsteps;
   R dt;
   FireParams fire;
   JamParams jam;
   int jam_start;   // 1: begin a jamming protocol; 0: continue the one in res
   int jam_stages;  // minimisations this launch may run
+  int extra;       // the optional LDS arrays fit (arc boxes, vertex cells)
 };
 
 // Reduction of five doubles (four sums, one max) over the workgroup; every
@@ -1014,7 +1172,7 @@ __device__ void rescale_box(const Geom2D<R>& g, Tissue2DCtx<R>& T, const Lds2D<R
   __syncthreads();
   const R s = Lnew / T.L - R(1);
   for (int k = threadIdx.x; k < T.nvt; k += blockDim.x) {
-    const int c = cell_of(l.vb, T.nc, k);
+    const int c = vertex_cell(l, T.nc, k);
     l.x[k] += s * l.comx[c];
     l.y[k] += s * l.comy[c];
   }
@@ -1032,19 +1190,21 @@ __device__ void copy_positions(const Tissue2DCtx<R>& T, const R* fx, const R* fy
   __syncthreads();
 }
 
-template <typename R>
-__device__ void k2d_relax_body(const Relax2D<R>& a) {
+// MODE: one RELAX_* (an instance each: the registers of one mode's state do
+// not weigh on another's force loops).
+template <typename R, int MODE>
+__global__ void __launch_bounds__(1024) k2d_relax(const Relax2D<R> a) {
   extern __shared__ __align__(16) unsigned char smem[];
   const Geom2D<R>& g = a.g;
   Tissue2DCtx<R> T = tissue_ctx(g, blockIdx.x);
-  const Lds2D<R> l = carve2d<R>(smem, T.nvt, T.nc);
+  const Lds2D<R> l = carve2d<R>(smem, T.nvt, T.nc, a.extra ? lds2d_bytes(T.nvt, T.nc, (int)sizeof(R)) : 0);
   const int tid = threadIdx.x, NT = blockDim.x;
   stage_tissue(g, T, l, a.x, a.y);
   double res[RS_COUNT];
   for (int i = 0; i < RS_COUNT; i++) res[i] = 0.0;
   const double A0 = a.sum_a0[blockIdx.x];
 
-  if (a.mode == RELAX_EULER) {
+  if constexpr (MODE == RELAX_EULER) {
     for (int s = 0; s < a.nsteps; s++) {
       prepare_forces(g, T, l);
       for (int k = tid; k < T.nvt; k += NT) {
@@ -1062,11 +1222,11 @@ __device__ void k2d_relax_body(const Relax2D<R>& a) {
       __syncthreads();
     }
     res[RS_ITER] = a.nsteps;
-  } else if (a.mode == RELAX_FIRE) {
+  } else if constexpr (MODE == RELAX_FIRE) {
     bool conv, cleared;
     res[RS_ITER] = fire_min(a, T, l, -1.0, conv, cleared);
     res[RS_UNCONVERGED] = !conv;
-  } else if (a.mode == RELAX_JAM) {
+  } else if constexpr (MODE == RELAX_JAM) {
     // The protocol state lives in res (and the saved positions in sx, sy),
     // so a protocol can run over several launches with the same result.
     const JamParams& jp = a.jam;
@@ -1138,7 +1298,7 @@ __device__ void k2d_relax_body(const Relax2D<R>& a) {
     res[RS_STATUS] = status;
     res[RS_PHI_TARGET] = phi;
   }
-  if (a.mode != RELAX_EULER) {
+  if constexpr (MODE != RELAX_EULER) {
     // final state: forces at the final positions, energy (Euler keeps the
     // forces of its last step, as the reference's Forces)
     double U, Ui, fm;
@@ -1159,6 +1319,3 @@ __device__ void k2d_relax_body(const Relax2D<R>& a) {
     a.tLout[blockIdx.x] = T.L;
   }
 }
-
-extern "C" __global__ void __launch_bounds__(1024) k2d_relax_f32(const Relax2D<float> a) { k2d_relax_body(a); }
-extern "C" __global__ void __launch_bounds__(1024) k2d_relax_f64(const Relax2D<double> a) { k2d_relax_body(a); }

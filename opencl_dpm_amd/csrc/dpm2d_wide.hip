@@ -6,7 +6,7 @@
 // per step on global arrays laid out as k2d_run's LDS (the same Lds2D view,
 // pointing at global memory, and the same per-cell, candidate and per-vertex
 // functions, so every decision and every force is k2d_run's):
-//   k2d_wide_cells  one thread per cell: strain, orientation, centre of mass,
+//   k2d_wide_cells  eight lanes per cell: strain, orientation, centre of mass,
 //                   bounds of the input positions;
 //   k2d_wide_cand   one wave per cell: its candidate cells, ascending (the
 //                   lanes test 64 cells at a time, a ballot keeps the order);
@@ -65,16 +65,19 @@ __device__ __forceinline__ Lds2D<float> wide_view(const Wide2D& a, const Tissue2
   l.cand = a.cand + (size_t)T.c0 * DPM2D_MAXCAND;
   l.cbits = nullptr;
   l.red = nullptr;
+  l.has_arc = l.has_vc = false;
+  l.arc = nullptr;
+  l.vc = nullptr;
   return l;
 }
 
 extern "C" __global__ void __launch_bounds__(256) k2d_wide_cells(const Wide2D a) {
-  const int gc = blockIdx.x * blockDim.x + threadIdx.x;
-  if (a.counters && gc == 0) atomicAdd(&a.counters[0], 1ull);
-  if (gc >= a.C) return;
+  const int gc = (int)((blockIdx.x * blockDim.x + threadIdx.x) / 8);
+  if (a.counters && blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&a.counters[0], 1ull);
+  if (gc >= a.C) return;  // whole groups
   const int t = a.cell_tissue[gc];
   const Tissue2DCtx<float> T = tissue_ctx(a.g, t);
-  cell_one(a.g, T, wide_view(a, T, t, a.xin, a.yin), gc - T.c0);
+  cell_group(a.g, T, wide_view(a, T, t, a.xin, a.yin), gc - T.c0, threadIdx.x & 7);
 }
 
 // The list cand_one makes (maybe_pair over the tissue's cells, ascending,
@@ -233,7 +236,7 @@ __global__ void __launch_bounds__(256) k2d_wide_step(const Wide2D a) {
   bool over = false;
   if (mask & M2_REPULSION) {
     group_candidates(w, l, ci, T.nc, [&](int cj) { return !outside_box_even(l, cj, px, py, T.pbc, L); }, [&](int cj) {
-      over = __popcll(w.bits(crossing_odd(l, cj, px, py, T.pbc, L, w.lane, G))) & 1;
+      over = __popcll(w.bits(crossing_odd(l, cj, px, py, T.pbc, L, T.invL, w.lane, G))) & 1;
       return !over;
     });
     if (over) repulsion_push(a.g, T, l, ci, px, py, fx, fy);

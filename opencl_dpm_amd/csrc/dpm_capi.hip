@@ -143,8 +143,9 @@ struct dpm_tissue {
   // ------------------------------------------------------------------ 2D
   int V = 0, NT2 = 0, NTr = 0;  // Euler threads, relax threads per tissue
   size_t lds2 = 0;
-  size_t lds_run = 0;  // k2d_run: lds2 and, where it fits, the crossing-parity pair list
+  size_t lds_run = 0;  // k2d_run's (lds2: the relaxation kernel's)
   int over_cap = 0;
+  int run_extra = 0, relax_extra = 0;  // the optional LDS arrays fit
   // arrays of the real type (rs bytes)
   void *x2 = nullptr, *y2 = nullptr, *fx2 = nullptr, *fy2 = nullptr;
   void *vx2 = nullptr, *vy2 = nullptr, *sx2 = nullptr, *sy2 = nullptr;  // FIRE / jamming
@@ -1579,6 +1580,14 @@ extern "C" int dpm3d_adjoint_f64(dpm_tissue* h, const double* lambda_final, doub
 
 static_assert(sizeof(dpm_relax_stats) == RS_COUNT * sizeof(double), "dpm_relax_stats layout");
 
+template <typename R>
+static auto relax_kernel(int mode) {
+  return mode == RELAX_EULER ? k2d_relax<R, RELAX_EULER>
+         : mode == RELAX_FIRE ? k2d_relax<R, RELAX_FIRE>
+         : mode == RELAX_JAM  ? k2d_relax<R, RELAX_JAM>
+                              : k2d_relax<R, RELAX_ENERGY>;
+}
+
 static int create2d(const dpm2d_desc* d, dpm_tissue** out, int rs) {
   if (!d || !out) return fail(DPM_EINVAL, "null argument");
   *out = nullptr;
@@ -1619,8 +1628,7 @@ static int create2d(const dpm2d_desc* d, dpm_tissue** out, int rs) {
   for (int t = 0; t < T; t++) {
     const int nc = d->cell_begin[t + 1] - d->cell_begin[t];
     const int nvt = cvb[d->cell_begin[t + 1]] - cvb[d->cell_begin[t]];
-    if (nvt <= 32 * DPM2D_CSPLIT * nc && (long long)nvt * nc <= 16LL * nt4)
-      any_pass = true;
+    if (over_split(nvt, nc, nt4)) any_pass = true;
   }
   h->NT2 = any_pass ? nt4 : std::min(1024, std::max(64, (std::max(maxv, DPM2D_CSPLIT * maxc) + 63) / 64 * 64));
   h->NTr = std::min(1024, std::max(64, (maxv / 4 + 63) / 64 * 64));
@@ -1633,13 +1641,27 @@ static int create2d(const dpm2d_desc* d, dpm_tissue** out, int rs) {
     return fail(DPM_ERANGE, "a double 2D tissue must fit the LDS of one workgroup");
   }
   if (!h->fits_wg) h->lds2 = 0;
-  // the crossing-parity pair list where a tissue can take the pass and the
-  // LDS allows it (without it the pass tests every pair where it finds it)
-  h->lds_run = h->lds2;
-  h->over_cap = 0;
-  if (h->fits_wg && any_pass && (int)(h->lds2 + lds2d_over_bytes()) <= max_lds_per_block(h->device)) {
-    h->lds_run = h->lds2 + lds2d_over_bytes();
-    h->over_cap = DPM2D_OVER_CAP;
+  // the crossing-parity pair list where a tissue can take the pass (without
+  // it the pass tests every pair where it finds it) and the optional arrays,
+  // each where the LDS allows it
+  const size_t lds_max = (size_t)max_lds_per_block(h->device);
+  auto need = [&](int over, int extra) {  // the largest tissue's
+    size_t run = 0, relax = 0;
+    for (int t = 0; t < T; t++) {
+      const int nc = d->cell_begin[t + 1] - d->cell_begin[t];
+      const int nvt = cvb[d->cell_begin[t + 1]] - cvb[d->cell_begin[t]];
+      const size_t b = lds2d_bytes(nvt, nc, rs), x = extra ? lds2d_extra_bytes(nvt, nc, rs) : 0;
+      run = std::max(run, b + run2d_list_bytes(nvt, nc, h->NT2, over) + x);
+      relax = std::max(relax, b + x);
+    }
+    return std::make_pair(run, relax);
+  };
+  if (h->fits_wg) {
+    h->over_cap = any_pass && need(DPM2D_OVER_CAP, 0).first <= lds_max ? DPM2D_OVER_CAP : 0;
+    h->run_extra = need(h->over_cap, 1).first <= lds_max;
+    h->relax_extra = need(0, 1).second <= lds_max;
+    h->lds_run = need(h->over_cap, h->run_extra).first;
+    h->lds2 = need(0, h->relax_extra).second;
   }
   h->max_cells = maxc;
   h->cvb_h = cvb;
@@ -1676,8 +1698,9 @@ static int create2d(const dpm2d_desc* d, dpm_tissue** out, int rs) {
   if (rc) { delete h; return rc; }
   if (h->fits_wg) {
     (void)hipFuncSetAttribute((const void*)k2d_run, hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->lds_run);
-    (void)hipFuncSetAttribute(rs == 8 ? (const void*)k2d_relax_f64 : (const void*)k2d_relax_f32,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->lds2);
+    for (int mode : {RELAX_EULER, RELAX_FIRE, RELAX_JAM, RELAX_ENERGY})
+      (void)hipFuncSetAttribute(rs == 8 ? (const void*)relax_kernel<double>(mode) : (const void*)relax_kernel<float>(mode),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->lds2);
   }
   *out = h;
   return DPM_OK;
@@ -1754,7 +1777,7 @@ static Wide2D wide_args(dpm_tissue* h, int in, float dt, int flags) {
 }
 
 static int launch_wide(dpm_tissue* h, const Wide2D& a) {
-  const int bc = (h->C + 255) / 256, bw = (h->C + 3) / 4;
+  const int bc = (int)((8LL * h->C + 255) / 256), bw = (h->C + 3) / 4;
   const int G = wide_group(h->V);
   const unsigned bv = (unsigned)(((long long)h->V * G + 255) / 256);
   auto step = G == 32 ? k2d_wide_step<32> : G == 16 ? k2d_wide_step<16> : k2d_wide_step<8>;
@@ -1972,6 +1995,7 @@ static Run2D run2d_args(dpm_tissue* h, int nsteps, float dt) {
   a.dt = dt;
   a.counters = h->counters;
   a.over_cap = h->over_cap;
+  a.extra = h->run_extra;
   return a;
 }
 
@@ -2039,14 +2063,12 @@ static int launch_relax(dpm_tissue* h, int mode, int threads, Edit edit) {
     a.tLout = (R*)h->tLr;
     a.res = h->res2;
     a.sum_a0 = h->sum_a0;
-    a.mode = mode;
+    a.extra = h->relax_extra;
     dpm_fire_params fd;
     dpm_fire_defaults(&fd);
     a.fire = fire_params(&fd);
     edit(a);
-    void (*k)(Relax2D<R>) = nullptr;
-    if constexpr (sizeof(R) == 8) k = k2d_relax_f64; else k = k2d_relax_f32;
-    hipLaunchKernelGGL(k, dim3(h->T), dim3(threads > 0 ? threads : h->NTr), h->lds2, h->stream, a);
+    hipLaunchKernelGGL(relax_kernel<R>(mode), dim3(h->T), dim3(threads > 0 ? threads : h->NTr), h->lds2, h->stream, a);
     HIPCHECK(hipGetLastError());
     return DPM_OK;
   };
