@@ -44,6 +44,7 @@ template <typename R>
 struct Geom2D {
   const int* tissue_cell_begin;  // [T+1]
   const int* cell_vert_begin;    // [C+1] (global vertex offsets)
+  const int* order;              // [T] the tissue of each workgroup
   const float* Ka;
   const float* Kl;
   const float* Kb;
@@ -869,7 +870,7 @@ __host__ __device__ inline size_t run2d_list_bytes(int nvt, int nc, int NT, int 
 extern "C" __global__ void __launch_bounds__(1024) k2d_run(const Run2D a) {
   extern __shared__ __align__(16) unsigned char smem[];
   const Geom2D<float>& g = a.g;
-  const Tissue2DCtx<float> T = tissue_ctx(g, blockIdx.x);
+  const Tissue2DCtx<float> T = tissue_ctx(g, g.order[blockIdx.x]);
   const int tid = threadIdx.x, NT = blockDim.x;
   const size_t base = lds2d_bytes(T.nvt, T.nc, (int)sizeof(float));
   const Lds2D<float> l = carve2d<float>(
@@ -1196,13 +1197,14 @@ template <typename R, int MODE>
 __global__ void __launch_bounds__(1024) k2d_relax(const Relax2D<R> a) {
   extern __shared__ __align__(16) unsigned char smem[];
   const Geom2D<R>& g = a.g;
-  Tissue2DCtx<R> T = tissue_ctx(g, blockIdx.x);
+  const int t = g.order[blockIdx.x];
+  Tissue2DCtx<R> T = tissue_ctx(g, t);
   const Lds2D<R> l = carve2d<R>(smem, T.nvt, T.nc, a.extra ? lds2d_bytes(T.nvt, T.nc, (int)sizeof(R)) : 0);
   const int tid = threadIdx.x, NT = blockDim.x;
   stage_tissue(g, T, l, a.x, a.y);
   double res[RS_COUNT];
   for (int i = 0; i < RS_COUNT; i++) res[i] = 0.0;
-  const double A0 = a.sum_a0[blockIdx.x];
+  const double A0 = a.sum_a0[t];
 
   if constexpr (MODE == RELAX_EULER) {
     for (int s = 0; s < a.nsteps; s++) {
@@ -1232,7 +1234,7 @@ __global__ void __launch_bounds__(1024) k2d_relax(const Relax2D<R> a) {
     const JamParams& jp = a.jam;
     R* sx = a.sx + T.v0;
     R* sy = a.sy + T.v0;
-    const double* prev = a.res + (size_t)blockIdx.x * RS_COUNT;
+    const double* prev = a.res + (size_t)t * RS_COUNT;
     double phi, phi_lo, phi_hi, iters, unconv;
     int stage, status;
     if (a.jam_start) {
@@ -1315,7 +1317,7 @@ __global__ void __launch_bounds__(1024) k2d_relax(const Relax2D<R> a) {
     a.y[T.v0 + k] = l.y[k];
   }
   if (tid == 0) {
-    for (int i = 0; i < RS_COUNT; i++) a.res[(size_t)blockIdx.x * RS_COUNT + i] = res[i];
-    a.tLout[blockIdx.x] = T.L;
+    for (int i = 0; i < RS_COUNT; i++) a.res[(size_t)t * RS_COUNT + i] = res[i];
+    a.tLout[t] = T.L;
   }
 }

@@ -152,7 +152,7 @@ struct dpm_tissue {
   void* tLr = nullptr;  // per-tissue box length
   double* res2 = nullptr;     // [T * RS_COUNT]
   double* sum_a0 = nullptr;   // [T]
-  int *tcb = nullptr, *cvb = nullptr;
+  int *tcb = nullptr, *cvb = nullptr, *order2 = nullptr;
   float *Kl = nullptr, *l0_2 = nullptr, *r0 = nullptr;
   std::vector<int> cvb_h;
   std::vector<float> a0_h;
@@ -1677,6 +1677,7 @@ static int create2d(const dpm2d_desc* d, dpm_tissue** out, int rs) {
   rc |= h->alloc(&h->sum_a0, T);
   rc |= h->alloc(&h->tcb, T + 1);
   rc |= h->alloc(&h->cvb, C + 1);
+  rc |= h->alloc(&h->order2, T);
   rc |= h->alloc(&h->Ka, C);
   rc |= h->alloc(&h->Kl, C);
   rc |= h->alloc(&h->Kb, C);
@@ -1690,6 +1691,18 @@ static int create2d(const dpm2d_desc* d, dpm_tissue** out, int rs) {
   hipStream_t s = h->stream;
   rc |= upload(h->tcb, d->cell_begin, T + 1, s);
   rc |= upload(h->cvb, cvb.data(), C + 1, s);
+  // Workgroups take the tissues largest first: one of up to 1024 threads
+  // fills a compute unit's registers, so a batch beyond the device runs in
+  // rounds, and a large tissue started late runs on alone (512 tissues of 8 to
+  // 128 cells, as given and largest first: Euler 10.1 and 8.5 ms for 50 steps,
+  // FIRE in double 31.9 and 23.7 ms for 100 iterations).
+  std::vector<int> order(T);
+  for (int t = 0; t < T; t++) order[t] = t;
+  std::stable_sort(order.begin(), order.end(), [&](int p, int q) {
+    auto nvt = [&](int t) { return cvb[d->cell_begin[t + 1]] - cvb[d->cell_begin[t]]; };
+    return nvt(p) > nvt(q);
+  });
+  rc |= upload(h->order2, order.data(), T, s);
   (void)hipMemsetAsync(h->fx2, 0, (size_t)h->V * rs, s);
   (void)hipMemsetAsync(h->fy2, 0, (size_t)h->V * rs, s);
   (void)hipMemsetAsync(h->res2, 0, sizeof(double) * T * RS_COUNT, s);
@@ -1697,8 +1710,10 @@ static int create2d(const dpm2d_desc* d, dpm_tissue** out, int rs) {
   if (!rc) rc = dpm2d_set_tissue_params(h, d->L, d->pbc, d->Kre, d->Kat, d->mask);
   if (rc) { delete h; return rc; }
   if (h->fits_wg) {
-    (void)hipFuncSetAttribute((const void*)k2d_run, hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->lds_run);
-    for (int mode : {RELAX_EULER, RELAX_FIRE, RELAX_JAM, RELAX_ENERGY})
+    // (64 KiB need no attribute)
+    if (h->lds_run > 65536)
+      (void)hipFuncSetAttribute((const void*)k2d_run, hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->lds_run);
+    if (h->lds2 > 65536) for (int mode : {RELAX_EULER, RELAX_FIRE, RELAX_JAM, RELAX_ENERGY})
       (void)hipFuncSetAttribute(rs == 8 ? (const void*)relax_kernel<double>(mode) : (const void*)relax_kernel<float>(mode),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->lds2);
   }
@@ -1970,6 +1985,7 @@ static Geom2D<R> geom2d(dpm_tissue* h) {
   Geom2D<R> g{};
   g.tissue_cell_begin = h->tcb;
   g.cell_vert_begin = h->cvb;
+  g.order = h->order2;
   g.Ka = h->Ka;
   g.Kl = h->Kl;
   g.Kb = h->Kb;
