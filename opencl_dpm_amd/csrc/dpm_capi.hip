@@ -2360,11 +2360,12 @@ extern "C" int dpm_disperse(const float* r, int n, float L, float* X, float* Y, 
   if (hipGetDeviceCount(&ndev) != hipSuccess || ndev == 0) return fail(DPM_EDEVICE, "no HIP device is visible");
   int dev = 0;
   HIPCHECK(hipGetDevice(&dev));
-  float rmax = 0.0f;
+  float rmax = 0.0f, reach = L;
   for (int i = 0; i < n; i++) {
     if (!(r[i] >= 0.0f) || !std::isfinite(r[i])) return fail(DPM_EINVAL, "dpm_disperse: radii must be finite and >= 0");
     if (!std::isfinite(X[i]) || !std::isfinite(Y[i])) return fail(DPM_ENONFINITE, "dpm_disperse: non-finite centre");
     rmax = std::max(rmax, r[i]);
+    reach = std::max(reach, std::max(std::fabs(X[i]), std::fabs(Y[i])));
   }
   // bins no narrower than the largest contact distance 2 rmax (with slack)
   int nb = rmax > 0.0f ? (int)std::floor(L / (2.0f * rmax * 1.001f + 1e-6f)) : 0;
@@ -2385,22 +2386,34 @@ extern "C" int dpm_disperse(const float* r, int n, float L, float* X, float* Y, 
   int rc = dev_alloc(&dr, n);
   rc |= dev_alloc(&dx, n);
   rc |= dev_alloc(&dy, n);
-  rc |= dev_alloc(&dout, 2);
+  rc |= dev_alloc(&dout, DISP_WORDS);
   rc |= dev_alloc(&dt, (size_t)term_cap);
-  int out[2] = {0, 0};
-  if (!rc) rc = upload(dr, r, n, s) | upload(dx, X, n, s) | upload(dy, Y, n, s);
+  int out[DISP_WORDS] = {0, 0, 1, 0};
+  const float u0 = 100.0f;
+  std::memcpy(&out[DISP_U], &u0, sizeof(u0));
+  if (!rc) rc = upload(dout, out, DISP_WORDS, s) | upload(dr, r, n, s) | upload(dx, X, n, s) | upload(dy, Y, n, s);
   if (!rc && hipFuncSetAttribute((const void*)k_disperse2d, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) !=
                  hipSuccess)
     rc = fail(DPM_EDEVICE, "hipFuncSetAttribute(k_disperse2d) failed");
   if (!rc) {
     Disperse2DArgs a{dr, dx, dy, n, L, max_count, nb, dout, dt, term_cap};
+    // the list form where its LDS fits (up to 32 neighbours, else 16) and a
+    // tenth of the skin is far above the rounding of the coordinates
+    const size_t lds32 = disp_list_layout(nullptr, n, 32).total, lds16 = disp_list_layout(nullptr, n, 16).total;
+    const float skin = 0.2f * rmax;
+    if (0.1f * skin > 4e-6f * reach && lds16 <= (size_t)maxlds) {
+      auto k = lds32 <= (size_t)maxlds ? k_disperse_list<32> : k_disperse_list<16>;
+      const size_t need = lds32 <= (size_t)maxlds ? lds32 : lds16;
+      (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)need);
+      hipLaunchKernelGGL(k, dim3(1), dim3(64 * disp_list_waves(n)), need, s, a, skin, 2.0f * reach);
+    }
     hipLaunchKernelGGL(k_disperse2d, dim3(1), dim3(threads), lds, s, a);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) rc = fail(DPM_EDEVICE, std::string("k_disperse2d: ") + hipGetErrorString(e));
   }
   if (!rc && (hipMemcpyAsync(X, dx, n * sizeof(float), hipMemcpyDeviceToHost, s) != hipSuccess ||
               hipMemcpyAsync(Y, dy, n * sizeof(float), hipMemcpyDeviceToHost, s) != hipSuccess ||
-              hipMemcpyAsync(out, dout, 2 * sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess))
+              hipMemcpyAsync(out, dout, DISP_WORDS * sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess))
     rc = fail(DPM_EDEVICE, "dpm_disperse: copy back failed");
   if (hipStreamSynchronize(s) != hipSuccess && !rc) rc = fail(DPM_EDEVICE, "dpm_disperse: stream sync failed");
   for (void* p : {(void*)dr, (void*)dx, (void*)dy, (void*)dout, (void*)dt})
@@ -2408,8 +2421,8 @@ extern "C" int dpm_disperse(const float* r, int n, float L, float* X, float* Y, 
   (void)hipStreamDestroy(s);
   if (rc) return rc;
   if (result) {
-    result[0] = out[0];
-    result[1] = out[1];
+    result[0] = out[DISP_COUNT];
+    result[1] = out[DISP_CAPPED];
   }
   return DPM_OK;
 }

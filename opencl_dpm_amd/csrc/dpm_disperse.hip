@@ -33,9 +33,17 @@ struct Disperse2DArgs {
   float L;
   int max_count;   // the loop stops once it has run more than this many iterations
   int nb;          // bins per axis (0: every centre scans all)
-  int* out;        // [0] iterations run, [1] 1 if stopped by max_count
+  int* out;        // DISP_*: the run's state, taken up by each kernel
   float* terms;    // [term_cap] U terms in (i, j) order
   int term_cap;
+};
+
+enum : int {
+  DISP_COUNT = 0,  // iterations run
+  DISP_CAPPED,     // 1 if stopped by max_count
+  DISP_LEFT,       // 1 while the relaxation is unfinished
+  DISP_U,          // bits of the last iteration's U (100 before the first)
+  DISP_WORDS
 };
 
 struct DispLds {
@@ -83,10 +91,13 @@ struct PairTerm {
 
 __device__ __forceinline__ PairTerm disp_pair(float xa, float ya, float ra, float xb, float yb, float rb, float L) {
   PairTerm t{false, 0.0f, 0.0f, 0.0f};
-  float dx = xb - xa;
-  dx -= L * roundf(dx / L);
-  float dy = yb - ya;
-  dy -= L * roundf(dy / L);
+  float dx = xb - xa, dy = yb - ya;
+  // (a component below 0.49 L rounds to image 0, which leaves it unchanged)
+  const float half = 0.49f * L;
+  if (!(fabsf(dx) < half && fabsf(dy) < half)) {
+    dx -= L * roundf(dx / L);
+    dy -= L * roundf(dy / L);
+  }
   const float dist = sqrtf(dx * dx + dy * dy);
   const float rr = ra + rb;
   if (dist <= rr) {
@@ -147,12 +158,13 @@ extern "C" __global__ void __launch_bounds__(kDispThreads) k_disperse2d(const Di
     l.y[k] = a.Y[k];
     l.r[k] = a.r[k];
   }
+  if (!a.out[DISP_LEFT]) return;  // block-uniform: k_disperse_list finished
   if (tid == 0) {
-    l.red[1] = 100.0f;  // oldU
-    l.red[2] = 100.0f;  // dU
+    l.red[1] = __int_as_float(a.out[DISP_U]);  // oldU
+    l.red[2] = 100.0f;                         // dU
   }
+  int count = a.out[DISP_COUNT];
   __syncthreads();
-  int count = 0;
   bool capped = false;
   // while (dU > 1e-6): the loop condition in double, as the reference's
   // float dU against a double literal
@@ -299,7 +311,299 @@ extern "C" __global__ void __launch_bounds__(kDispThreads) k_disperse2d(const Di
     a.Y[k] = l.y[k];
   }
   if (tid == 0) {
-    a.out[0] = count;
-    a.out[1] = capped ? 1 : 0;
+    a.out[DISP_COUNT] = count;
+    a.out[DISP_CAPPED] = capped ? 1 : 0;
+    a.out[DISP_LEFT] = 0;
+  }
+}
+
+// The same relaxation from neighbour lists, for centres that fit (below).
+// k_disperse2d's iteration is a chain of serial passes on one compute unit —
+// bins, a sort per centre, each pair's term three times, the scan of the term
+// counts, then U's float sum by one lane while the others wait.  us per
+// iteration, that one and this: 38 and 2.9 (16 centres), 57 and 4.5 (100), 89
+// and 10.4 (400, bound by U's additions).  900 centres do not fit (145).
+// Here:
+//   * each centre keeps the centres within contact + skin, ascending, until
+//     some centre has moved 0.45 skin; a pair outside the lists is out of
+//     contact, and adds nothing, as long as they hold;
+//   * eight lanes share a centre's list.  The term that row i adds to k,
+//     f(i, k), is -f(k, i) exactly (every operation of disp_pair is odd in
+//     the differences and symmetric in the radii), so one evaluation g of
+//     each pair serves the reference's three visits: k's force is the sum of
+//     g over partners below k, then over all, then over those above k;
+//   * U's terms go compacted to LDS (eight centres' rows a segment), and a
+//     wave of its own adds them while the others are at the next
+//     iteration's forces; an iteration whose predecessor turns out to have
+//     been the last is dropped before it moves anything.  The reference adds
+//     0.5 t in double and rounds to float; both addends are floats and U
+//     stays below 2^27 (t <= 1), so the double sum is exact and that is the
+//     float addition of U and 0.5 t.  Adding +0 (padding, pairs out of
+//     contact) changes neither U nor a force (no sum starts at -0).
+// Two barriers an iteration.  A list that overflows, or a centre that leaves
+// the range the skin's margin was checked for, hands the run's state over to
+// k_disperse2d, which starts where this kernel stopped.
+constexpr int kDispGroups = 8;    // centres per wave, eight lanes each
+constexpr int kDispMaxWaves = 16; // the last one adds U
+
+struct DispListLds {
+  float *x, *y, *r, *x0, *y0, *fx, *fy;
+  unsigned short *cnt, *split;  // list length; entries below the centre
+  unsigned short* list;         // [n * cap]
+  float* g;                     // [waves * 8 * 2 * cap]
+  float* term;                  // [2][segments * 8 * cap]
+  int* nterm;                   // [2][segments], padded to whole blocks of add_u
+  int* flag;                    // [4] rebuild (two, in turn), overflow, stop
+  float* u;                     // [1] U of the last finished iteration
+  size_t total;
+};
+__host__ __device__ inline int disp_list_waves(int n) {
+  const int seg = (n + kDispGroups - 1) / kDispGroups;
+  return (seg < kDispMaxWaves - 1 ? seg : kDispMaxWaves - 1) + 1;
+}
+__host__ __device__ inline DispListLds disp_list_layout(unsigned char* base, int n, int cap) {
+  DispListLds l;
+  size_t o = 0;
+  auto take = [&](size_t bytes) {
+    unsigned char* p = base + o;
+    o = (o + bytes + 15) & ~(size_t)15;
+    return p;
+  };
+  const size_t N = (size_t)n, seg = (N + kDispGroups - 1) / kDispGroups;
+  l.x = (float*)take(4 * N);
+  l.y = (float*)take(4 * N);
+  l.r = (float*)take(4 * N);
+  l.x0 = (float*)take(4 * N);
+  l.y0 = (float*)take(4 * N);
+  l.fx = (float*)take(4 * N);
+  l.fy = (float*)take(4 * N);
+  l.cnt = (unsigned short*)take(2 * N);
+  l.split = (unsigned short*)take(2 * N);
+  l.list = (unsigned short*)take(2 * N * cap);
+  l.g = (float*)take(4 * (size_t)(disp_list_waves(n) - 1) * kDispGroups * 2 * cap);
+  l.term = (float*)take(8 * seg * kDispGroups * cap);
+  l.nterm = (int*)take(8 * seg);
+  l.flag = (int*)take(16);
+  l.u = (float*)take(4);
+  l.total = o;
+  return l;
+}
+
+template <int CAP>
+__global__ void __launch_bounds__(64 * kDispMaxWaves) k_disperse_list(const Disperse2DArgs a, float skin, float range) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int n = a.n, tid = threadIdx.x, NT = blockDim.x;
+  const float L = a.L;
+  const DispListLds l = disp_list_layout(smem, n, CAP);
+  const int lane = tid & (DPM_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(tid / DPM_WAVE);
+  const int W = NT / DPM_WAVE - 1;  // waves at the forces; wave W adds U
+  const int nseg = (n + kDispGroups - 1) / kDispGroups;
+  const int sub = lane & 7, grp = lane >> 3;
+  for (int k = tid; k < n; k += NT) {
+    l.x[k] = a.X[k];
+    l.y[k] = a.Y[k];
+    l.r[k] = a.r[k];
+  }
+  if (tid < 4) l.flag[tid] = 0;
+  if (tid == 0) *l.u = 100.0f;
+  __syncthreads();
+
+  // Adds iteration it - 1's terms in order (every lane the same sum) and
+  // raises flag[3] if it was the last.
+  auto add_u = [&](int it) {
+    // Half a segment's room (padded with +0) a block, one block read ahead:
+    // the additions run back to back, the chain that bounds a large run.
+    constexpr int B = kDispGroups * CAP / 4 < 64 ? kDispGroups * CAP / 4 : 64;
+    struct Block {
+      float4 v[B / 4];
+    };
+    const int b = (it - 1) & 1;
+    const float* term = l.term + (size_t)b * nseg * kDispGroups * CAP;
+    const int* count = l.nterm + b * nseg;
+    auto read = [&](Block& k, int s, int q) {
+      const float4* t = reinterpret_cast<const float4*>(term + (size_t)s * kDispGroups * CAP + q);
+#pragma unroll
+      for (int i = 0; i < B / 4; i++) k.v[i] = t[i];
+    };
+    float U = 0.0f;
+    auto add = [&](const Block& k) {
+#pragma unroll
+      for (int i = 0; i < B / 4; i++) {
+        U += k.v[i].x;
+        U += k.v[i].y;
+        U += k.v[i].z;
+        U += k.v[i].w;
+      }
+    };
+    Block k0, k1;
+    read(k0, 0, 0);
+    int m = __builtin_amdgcn_readfirstlane(count[0]), mn;
+    for (int s = 0; s < nseg; s++, m = mn) {
+      const int sn = s + 1 < nseg ? s + 1 : s;
+      mn = count[sn];
+      int q = 0;
+      for (; q + B < m; q += B) {
+        read(k1, s, q + B);
+        add(k0);
+        k0 = k1;
+      }
+      read(k1, sn, 0);
+      add(k0);
+      k0 = k1;
+      mn = __builtin_amdgcn_readfirstlane(mn);
+    }
+    float dU = U - *l.u;
+    if ((double)dU < 0.0) dU *= -1.0f;
+    wave_lds_sync();
+    if (lane == 0) {
+      *l.u = U;
+      if (!((double)dU > 1e-6)) l.flag[3] = 1;
+    }
+  };
+
+  int it = 0;
+  bool rebuild = true, capped = false, left = false;
+  for (;;) {
+    if (rebuild) {  // block-uniform
+      if (wave < W)
+        for (int s = wave; s < nseg; s += W) {
+          const int k = s * kDispGroups + grp;
+          int m = 0, p = 0;
+          if (k < n) {  // whole groups
+            const float xk = l.x[k], yk = l.y[k], rk = l.r[k] + skin;
+            for (int i0 = 0; i0 < n; i0 += 8) {
+              const int i = i0 + sub;
+              bool in = false;
+              if (i < n && i != k) {
+                float dx = l.x[i] - xk, dy = l.y[i] - yk;
+                dx -= L * roundf(dx / L);
+                dy -= L * roundf(dy / L);
+                const float rr = rk + l.r[i];
+                in = !(dx * dx + dy * dy > rr * rr);
+              }
+              const unsigned bits = (unsigned)(__ballot(in) >> (8 * grp)) & 0xffu;
+              const int slot = m + __popc(bits & ((1u << sub) - 1u));
+              if (in && slot < CAP) l.list[k * CAP + slot] = (unsigned short)i;
+              m += __popc(bits);
+              const int below = min(max(k - i0, 0), 8);
+              p += __popc(bits & ((1u << below) - 1u));
+            }
+            if (sub == 0) {
+              l.cnt[k] = (unsigned short)min(m, CAP);
+              l.split[k] = (unsigned short)p;
+              l.x0[k] = xk;
+              l.y0[k] = yk;
+              if (m > CAP || !(fabsf(xk) <= range && fabsf(yk) <= range)) l.flag[2] = 1;
+            }
+          }
+        }
+      __syncthreads();
+      if (l.flag[2]) {  // block-uniform
+        if (it > 0 && wave == W) add_u(it);
+        __syncthreads();
+        left = !l.flag[3];
+        break;
+      }
+    }
+    if (wave == W) {
+      if (it > 0) {
+        __builtin_amdgcn_s_setprio(3);  // the longest chain of the iteration
+        add_u(it);
+        __builtin_amdgcn_s_setprio(0);
+      }
+    } else {
+      float* g = l.g + (size_t)wave * kDispGroups * 2 * CAP + grp * 2 * CAP;
+      for (int s = wave; s < nseg; s += W) {
+        const int k = s * kDispGroups + grp;
+        const int m = k < n ? l.cnt[k] : 0, p = k < n ? l.split[k] : 0;
+        const float xk = k < n ? l.x[k] : 0.0f, yk = k < n ? l.y[k] : 0.0f, rk = k < n ? l.r[k] : 0.0f;
+        float* term = l.term + ((size_t)(it & 1) * nseg + s) * kDispGroups * CAP;
+        int ns = 1;  // rounds of eight entries (wave-uniform)
+        while (ns < CAP / 8 && __ballot(m > 8 * ns)) ns++;
+        unsigned long long hits[CAP / 8];
+        float u[CAP / 8];
+#pragma unroll
+        for (int q = 0; q < CAP / 8; q++) {
+          hits[q] = 0ull;
+          if (q < ns) {
+            const int c = 8 * q + sub;
+            PairTerm t{false, 0.0f, 0.0f, 0.0f};
+            if (c < m) {
+              const int j = l.list[k * CAP + c];
+              t = disp_pair(xk, yk, rk, l.x[j], l.y[j], l.r[j], L);
+            }
+            g[c] = t.touch ? -t.fx : 0.0f;
+            g[CAP + c] = t.touch ? -t.fy : 0.0f;
+            hits[q] = __ballot(t.touch);
+            u[q] = 0.5f * t.u;
+          }
+        }
+        // the segment's terms: by centre, then by list entry
+        int total = 0, before = 0;
+        const unsigned long long lower = (1ull << (8 * grp)) - 1ull;
+#pragma unroll
+        for (int q = 0; q < CAP / 8; q++) {
+          total += __popcll(hits[q]);
+          before += __popcll(hits[q] & lower);
+        }
+#pragma unroll
+        for (int q = 0; q < CAP / 8; q++) {
+          const unsigned bits = (unsigned)(hits[q] >> (8 * grp)) & 0xffu;
+          if ((bits >> sub) & 1u) term[before + __popc(bits & ((1u << sub) - 1u))] = u[q];
+          before += __popc(bits);
+        }
+        constexpr int B = kDispGroups * CAP / 4 < 64 ? kDispGroups * CAP / 4 : 64;  // add_u's block
+        const int padded = total < B ? B : (total + B - 1) / B * B;
+        if (lane < padded - total) term[total + lane] = 0.0f;
+        if (lane == 0) l.nterm[(it & 1) * nseg + s] = padded;
+        wave_lds_sync();
+        if (sub < 2 && k < n) {  // x by the group's first lane, y by its second
+          float v[CAP];
+#pragma unroll
+          for (int c = 0; c < CAP; c++)
+            if (c / 8 < ns) v[c] = g[sub * CAP + c];
+          float F = 0.0f;
+#pragma unroll
+          for (int c = 0; c < CAP; c++)
+            if (c / 8 < ns) F += c < p ? v[c] : 0.0f;
+#pragma unroll
+          for (int c = 0; c < CAP; c++)
+            if (c / 8 < ns) F += v[c];
+#pragma unroll
+          for (int c = 0; c < CAP; c++)
+            if (c / 8 < ns) F += c >= p ? v[c] : 0.0f;
+          (sub ? l.fy : l.fx)[k] = F;
+        }
+        wave_lds_sync();
+      }
+    }
+    __syncthreads();
+    if (l.flag[3]) break;  // block-uniform: iteration it - 1 was the last
+    for (int k = tid; k < n; k += NT) {  // X[i] += 0.01 * Fx[i], in double
+      const float xk = (float)((double)l.x[k] + 0.01 * (double)l.fx[k]);
+      const float yk = (float)((double)l.y[k] + 0.01 * (double)l.fy[k]);
+      l.x[k] = xk;
+      l.y[k] = yk;
+      const float dx = xk - l.x0[k], dy = yk - l.y0[k], lim = 0.45f * skin;
+      if (!(dx * dx + dy * dy <= lim * lim)) l.flag[it & 1] = 1;
+    }
+    if (tid == 0) l.flag[(it + 1) & 1] = 0;  // read by all before the barrier above
+    __syncthreads();
+    rebuild = l.flag[it & 1] != 0;
+    it++;
+    if (it > a.max_count) {
+      capped = true;
+      break;
+    }
+  }
+  for (int k = tid; k < n; k += NT) {
+    a.X[k] = l.x[k];
+    a.Y[k] = l.y[k];
+  }
+  if (tid == 0) {
+    a.out[DISP_COUNT] = it;
+    a.out[DISP_CAPPED] = capped ? 1 : 0;
+    a.out[DISP_LEFT] = left ? 1 : 0;
+    a.out[DISP_U] = __float_as_int(*l.u);
   }
 }
