@@ -510,12 +510,18 @@ static int create3d(const dpm3d_desc* d, dpm_tissue** out, int rs) {
     if (ldsw_layout(nv, nf, cpw, rs).total <= 65536) {
       h->wave_cpw = cpw;
       h->lds_w = ldsw_layout(nv, nf, cpw, rs).total;
-      // automatic choice: the wave form once the batch gives every CU about
-      // 24 cells (measured crossover between 16 and 32 cells per CU on the
-      // 256-cell monolayer); below, the workgroup form fills the device better
+      // automatic choice, by cells per compute unit: a workgroup per cell
+      // shortens one cell's step while the device has room for every cell at
+      // once, a wave per cell takes fewer waves and no barriers.  Measured,
+      // us per step, every term, workgroup | wave form: float 162 vertices,
+      // 484 cells 31.4 | 38.7, 1024 cells 46.0 | 33.3, 4096 cells 126 | 50.5;
+      // float 42 vertices, 256 cells 27.3 | 30.0, 1352 cells 49.4 | 32.1;
+      // double 162 vertices, 256 cells 30.2 | 46.5, 1024 cells 64.3 | 61.4,
+      // 4096 cells 214 | 119; double 42 vertices, 64 cells 42.0 | 32.0
       int dev = 0, cus = 256;
       if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-      h->wave_min_cells = 24 * std::max(1, cus);
+      const int per_cu = nv > DPM_WAVE ? (rs == 8 ? 4 : 3) : (rs == 8 ? 0 : 2);
+      h->wave_min_cells = per_cu * std::max(1, cus);
       // the topology image: faces packed 10 bits per index (staged in
       // LDS), incidence and neighbour rows of 16-bit entries (0xffff: none)
       const Lds3DWave LW = ldsw_layout(nv, nf, cpw, rs);
