@@ -20,6 +20,7 @@
 #include "dpm2d_wide.hip"
 #include "dpm_disperse.hip"
 #include "dpm_measures.hip"
+#include "dpm_hostcopy.hip"
 
 namespace {
 
@@ -80,6 +81,7 @@ struct dpm_tissue {
   hipStream_t stream = nullptr;
   unsigned long long* counters = nullptr;  // device [4 * DPM_COUNTER_SLOTS]
   std::vector<void*> allocs;
+  XferSlots xfer;  // pinned slots of the vertex transfers (from the first transfer on)
 
   // ------------------------------------------------------------------ 3D
   int T = 0, C = 0, nv = 0, nf = 0, NT = 0, ncmax = 0;
@@ -186,6 +188,7 @@ struct dpm_tissue {
     if (graph) (void)hipGraphExecDestroy(graph);
     if (jam_graph) (void)hipGraphExecDestroy(jam_graph);
     if (wide_graph) (void)hipGraphExecDestroy(wide_graph);
+    xfer.release();
     for (void* p : allocs) (void)hipFree(p);
     if (stream) (void)hipStreamDestroy(stream);
   }
@@ -266,6 +269,122 @@ static int check_finite(dpm_tissue* h, const R* a, const R* b, const R* c, size_
   HIPCHECK(hipStreamSynchronize(h->stream));
   if (f) return fail(DPM_ENONFINITE, "Non-finite simulation results");
   return DPM_OK;
+}
+
+// Pinned slots for a transfer of `bytes`: one slot for what fits it, two
+// that alternate, or two per thread.
+static int ensure_slots(dpm_tissue* h, size_t bytes) {
+  XferSlots& x = h->xfer;
+  const int n = bytes >= kXferThreaded ? 2 * kXferThreads : bytes > kXferSlot ? 2 : 1;
+  const size_t slot = n > 1 ? kXferSlot : std::max<size_t>((bytes + 4095) & ~(size_t)4095, 4096);
+  if (x.host && x.n >= n && x.slot >= slot) return DPM_OK;
+  x.release();
+  if (hipHostMalloc(reinterpret_cast<void**>(&x.host), slot * n, hipHostMallocCoherent) != hipSuccess) {
+    x.host = nullptr;
+    return fail(DPM_ENOMEM, "hipHostMalloc: pinned transfer slots");
+  }
+  x.slot = slot;
+  x.n = n;
+  for (int i = 0; i < n; i++) HIPCHECK(hipEventCreateWithFlags(&x.ev[i], hipEventDisableTiming));
+  return DPM_OK;
+}
+
+// Runs body(slice range, first slot, slots) over [0, n) vertices: here, or
+// on kXferThreads threads with two slots each.
+template <typename Body>
+static int run_slices(dpm_tissue* h, size_t n, size_t bytes, Body body) {
+  if (bytes < kXferThreaded) return body((size_t)0, n, 0, h->xfer.n > 1 ? 2 : 1);
+  const size_t part = (n / kXferThreads + kXferVerts - 1) / kXferVerts * kXferVerts;
+  int rcs[kXferThreads] = {};
+  std::string msg[kXferThreads];
+  std::thread th[kXferThreads];
+  auto work = [&](int k) {
+    const size_t a = std::min(n, k * part), b = k + 1 == kXferThreads ? n : std::min(n, (k + 1) * part);
+    if (hipSetDevice(h->device) != hipSuccess) rcs[k] = fail(DPM_EDEVICE, "hipSetDevice");
+    else if (a < b) rcs[k] = body(a, b, 2 * k, 2);
+    if (rcs[k]) msg[k] = g_err;
+  };
+  int started = 1;
+  try {
+    for (; started < kXferThreads; started++) th[started] = std::thread(work, started);
+  } catch (const std::exception&) {  // no more threads: the rest runs here
+  }
+  int dev = -1;
+  (void)hipGetDevice(&dev);
+  work(0);
+  for (int k = started; k < kXferThreads; k++) work(k);
+  if (dev >= 0) (void)hipSetDevice(dev);
+  for (int k = 1; k < started; k++) th[k].join();
+  for (int k = 0; k < kXferThreads; k++)
+    if (rcs[k]) return fail(rcs[k], msg[k]);
+  return DPM_OK;
+}
+
+// Host array of n vertices, NC interleaved components -> c0, c1, c2 on the
+// device, in stream order (the caller's array is free on return).  check:
+// refuses non-finite values (what was written by then stays written).
+template <typename R, int NC, typename H>
+static int upload_split(dpm_tissue* h, const H* src, size_t n, R* c0, R* c1, R* c2, float* lo, bool check) {
+  const size_t vb = NC * sizeof(H);
+  TRY(ensure_slots(h, n * vb));
+  XferSlots& x = h->xfer;
+  const size_t per = n * vb <= x.slot ? n : x.slot / vb / kXferVerts * kXferVerts;  // vertices per slice
+  return run_slices(h, n, n * vb, [&, per](size_t a, size_t b, int s0, int ns) -> int {
+    int turn = 0;
+    for (size_t v = a; v < b;) {
+      const size_t m = std::min(per, b - v);
+      const int s = s0 + turn;
+      turn = (turn + 1) % ns;
+      if (x.pending[s]) HIPCHECK(hipEventSynchronize(x.ev[s]));
+      H* slot = reinterpret_cast<H*>(x.host + (size_t)s * x.slot);
+      const bool finite = copy_finite(slot, src + v * NC, m * NC);
+      if (check && !finite) return fail(DPM_ENONFINITE, "Non-finite vertex coordinates");
+      k_split<H, R, NC><<<(int)((m + kXferVerts - 1) / kXferVerts), 256, 0, h->stream>>>(
+          slot, c0 + v, c1 + v, NC == 3 ? c2 + v : nullptr, lo ? lo + v : nullptr, n, (int)m);
+      HIPCHECK(hipGetLastError());
+      HIPCHECK(hipEventRecord(x.ev[s], h->stream));
+      x.pending[s] = true;
+      v += m;
+    }
+    return DPM_OK;
+  });
+}
+
+// The way back: complete on return.
+template <typename R, int NC, typename H>
+static int download_merge(dpm_tissue* h, H* dst, size_t n, const R* c0, const R* c1, const R* c2, const float* lo) {
+  const size_t vb = NC * sizeof(H);
+  TRY(ensure_slots(h, n * vb));
+  XferSlots& x = h->xfer;
+  const size_t per = n * vb <= x.slot ? n : x.slot / vb / kXferVerts * kXferVerts;
+  return run_slices(h, n, n * vb, [&, per](size_t a, size_t b, int s0, int ns) -> int {
+    auto launch = [&](size_t v, int s) -> int {
+      const size_t m = std::min(per, b - v);
+      if (x.pending[s]) HIPCHECK(hipEventSynchronize(x.ev[s]));
+      k_merge<H, R, NC><<<(int)((m + kXferVerts - 1) / kXferVerts), 256, 0, h->stream>>>(
+          reinterpret_cast<H*>(x.host + (size_t)s * x.slot), c0 + v, c1 + v, NC == 3 ? c2 + v : nullptr,
+          lo ? lo + v : nullptr, n, (int)m);
+      HIPCHECK(hipGetLastError());
+      HIPCHECK(hipEventRecord(x.ev[s], h->stream));
+      x.pending[s] = true;
+      return DPM_OK;
+    };
+    size_t ahead = a;
+    for (int k = 0; k < ns && ahead < b; k++, ahead += per) TRY(launch(ahead, s0 + k));
+    int turn = 0;
+    for (size_t v = a; v < b; v += per) {
+      const int s = s0 + turn;
+      turn = (turn + 1) % ns;
+      HIPCHECK(hipEventSynchronize(x.ev[s]));
+      x.pending[s] = false;
+      std::memcpy(dst + v * NC, x.host + (size_t)s * x.slot, std::min(per, b - v) * vb);
+      if (ahead < b) {
+        TRY(launch(ahead, s));
+        ahead += per;
+      }
+    }
+    return DPM_OK;
+  });
 }
 
 // ================================================================== 3D ====
@@ -649,58 +768,31 @@ extern "C" int dpm3d_set_tissue_params(dpm_tissue* h, const float* L, const int*
   return DPM_OK;
 }
 
-// Host AoS (reference order) <-> device SoA of the handle's real type.
+// Host AoS (reference order) <-> device SoA of the handle's real type.  The
+// positions go to the other buffer set, which becomes the current one when
+// all of them are finite; residuals have one buffer and are checked first.
 template <typename In>
 static int set_positions3(dpm_tissue* h, const In* xyz, size_t n) {
   if (!h || h->dim != 3 || !xyz) return fail(DPM_EINVAL, "bad arguments");
   const size_t NVT = (size_t)h->C * h->nv;
   if (n != NVT) return fail(DPM_EINVAL, "position count does not match the tissue");
-  if (!all_finite(xyz, 3 * n)) return fail(DPM_ENONFINITE, "Non-finite vertex coordinates");
-  const int k = h->cur;
+  if (h->lo && !all_finite(xyz, 3 * n)) return fail(DPM_ENONFINITE, "Non-finite vertex coordinates");
+  const int k = 1 - h->cur;
   auto put = [&](auto tag) -> int {
     using R = decltype(tag);
-    std::vector<R> a(n), b(n), c(n);
-    for (size_t i = 0; i < n; i++) {
-      a[i] = (R)xyz[3 * i];
-      b[i] = (R)xyz[3 * i + 1];
-      c[i] = (R)xyz[3 * i + 2];
-    }
-    TRY(upload((R*)h->x[k], a.data(), n, h->stream));
-    TRY(upload((R*)h->y[k], b.data(), n, h->stream));
-    TRY(upload((R*)h->z[k], c.data(), n, h->stream));
-    HIPCHECK(hipStreamSynchronize(h->stream));
-    return DPM_OK;
+    return upload_split<R, 3>(h, xyz, n, (R*)h->x[k], (R*)h->y[k], (R*)h->z[k], (float*)h->lo, true);
   };
   TRY(h->rs == 8 ? put(0.0) : put(0.0f));
-  if (h->lo) {  // residuals: what the float positions did not keep
-    std::vector<float> r(3 * n);
-    for (size_t i = 0; i < n; i++)
-      for (int k = 0; k < 3; k++)
-        r[k * n + i] = (float)((double)xyz[3 * i + k] - (double)(float)xyz[3 * i + k]);
-    TRY(upload((float*)h->lo, r.data(), 3 * n, h->stream));
-    HIPCHECK(hipStreamSynchronize(h->stream));
-  }
+  h->cur = k;
   h->stats_valid = false;
   return DPM_OK;
 }
 
 template <typename Out>
 static int download3(dpm_tissue* h, const void* a, const void* b, const void* c, Out* xyz, size_t n) {
-  auto get = [&](auto tag) -> int {
-    using R = decltype(tag);
-    std::vector<R> A(n), B(n), Cc(n);
-    HIPCHECK(hipMemcpyAsync(A.data(), a, n * sizeof(R), hipMemcpyDeviceToHost, h->stream));
-    HIPCHECK(hipMemcpyAsync(B.data(), b, n * sizeof(R), hipMemcpyDeviceToHost, h->stream));
-    HIPCHECK(hipMemcpyAsync(Cc.data(), c, n * sizeof(R), hipMemcpyDeviceToHost, h->stream));
-    HIPCHECK(hipStreamSynchronize(h->stream));
-    for (size_t i = 0; i < n; i++) {
-      xyz[3 * i] = (Out)A[i];
-      xyz[3 * i + 1] = (Out)B[i];
-      xyz[3 * i + 2] = (Out)Cc[i];
-    }
-    return DPM_OK;
-  };
-  return h->rs == 8 ? get(0.0) : get(0.0f);
+  if (h->rs == 8)
+    return download_merge<double, 3>(h, xyz, n, (const double*)a, (const double*)b, (const double*)c, nullptr);
+  return download_merge<float, 3>(h, xyz, n, (const float*)a, (const float*)b, (const float*)c, nullptr);
 }
 
 template <typename Out>
@@ -708,13 +800,10 @@ static int get_positions3(dpm_tissue* h, Out* xyz, size_t n) {
   if (!h || h->dim != 3 || !xyz) return fail(DPM_EINVAL, "bad arguments");
   if (n != (size_t)h->C * h->nv) return fail(DPM_EINVAL, "position count does not match the tissue");
   const int k = h->cur;
-  TRY(download3(h, h->x[k], h->y[k], h->z[k], xyz, n));
-  if (h->lo && sizeof(Out) == 8) {  // compensated: x + residual
-    std::vector<Out> r(3 * n);
-    TRY(download3(h, h->lo, (float*)h->lo + n, (float*)h->lo + 2 * n, r.data(), n));
-    for (size_t i = 0; i < 3 * n; i++) xyz[i] += r[i];
-  }
-  return DPM_OK;
+  if (h->lo && sizeof(Out) == 8)  // compensated: x + residual
+    return download_merge<float, 3>(h, xyz, n, (const float*)h->x[k], (const float*)h->y[k], (const float*)h->z[k],
+                                    (const float*)h->lo);
+  return download3(h, h->x[k], h->y[k], h->z[k], xyz, n);
 }
 
 extern "C" int dpm3d_set_compensated(dpm_tissue* h, int on) {
@@ -1927,31 +2016,16 @@ template <typename In>
 static int set_positions2(dpm_tissue* h, const In* xy, size_t n) {
   if (!h || h->dim != 2 || !xy) return fail(DPM_EINVAL, "bad arguments");
   if (n != (size_t)h->V) return fail(DPM_EINVAL, "position count does not match the tissue");
-  std::vector<In> a(n), b(n);
-  for (size_t i = 0; i < n; i++) {
-    a[i] = xy[2 * i];
-    b[i] = xy[2 * i + 1];
-  }
-  TRY(upload_real(h, h->x2, a.data(), n));
-  TRY(upload_real(h, h->y2, b.data(), n));
-  return DPM_OK;
+  if (h->rs == 8)
+    return upload_split<double, 2>(h, xy, n, (double*)h->x2, (double*)h->y2, (double*)nullptr, nullptr, false);
+  return upload_split<float, 2>(h, xy, n, (float*)h->x2, (float*)h->y2, (float*)nullptr, nullptr, false);
 }
 
 template <typename Out>
 static int download2(dpm_tissue* h, const void* a, const void* b, Out* xy, size_t n) {
-  auto get = [&](auto tag) -> int {
-    using R = decltype(tag);
-    std::vector<R> A(n), B(n);
-    HIPCHECK(hipMemcpyAsync(A.data(), a, n * sizeof(R), hipMemcpyDeviceToHost, h->stream));
-    HIPCHECK(hipMemcpyAsync(B.data(), b, n * sizeof(R), hipMemcpyDeviceToHost, h->stream));
-    HIPCHECK(hipStreamSynchronize(h->stream));
-    for (size_t i = 0; i < n; i++) {
-      xy[2 * i] = (Out)A[i];
-      xy[2 * i + 1] = (Out)B[i];
-    }
-    return DPM_OK;
-  };
-  return h->rs == 8 ? get(0.0) : get(0.0f);
+  if (h->rs == 8)
+    return download_merge<double, 2>(h, xy, n, (const double*)a, (const double*)b, (const double*)nullptr, nullptr);
+  return download_merge<float, 2>(h, xy, n, (const float*)a, (const float*)b, (const float*)nullptr, nullptr);
 }
 
 template <typename Out>
