@@ -205,8 +205,9 @@ int dpm3d_energy(dpm_tissue* h, double* energy);
  * 325-364, with exact culling); 1 bins the centres of mass each step
  * (counting sort into hashed periodic bins no narrower than the step's
  * largest candidate reach) and visits the 27 surrounding bins; -1 (default)
- * chooses 1 for tissues of more than 8 x threads-per-cell cells.  Both give
- * bit-identical results. */
+ * chooses 0.  All give bit-identical results.  Where the scan runs in a tissue
+ * of more than 512 cells, a step keeps lists with a skin and the following
+ * steps test only those, until a cell has moved too far for them. */
 int dpm3d_set_cell_list(dpm_tissue* h, int mode);
 
 /* Bin width of the cell list over the step's largest candidate reach, a

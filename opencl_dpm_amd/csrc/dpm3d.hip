@@ -159,7 +159,33 @@ struct Step3D {
   const int* tbin_nb;    // per tissue: bins per axis (0: scan)
   const int* tbin_nbuck;
   const int* tbin_hoff;
+  // candidate lists (nullptr: none), see NearList
+  int* nl_cnt;            // per cell: entries of its list, -1 more than kNearList
+  int* nl_idx;            // [ncells * kNearList] ascending
+  CellStat<R>* nl_ref;    // the cell's statistics when the lists were made
+  const int* nl_stale;    // per tissue: this step makes the lists
+  int* nl_stale_out;      // the same for the next step, set here
+  int* nl_stale_clear;    // the same for the step after, cleared here
+  R nl_skin;
 };
+
+// The step kernels' arguments, read where they are used: the struct is their
+// only parameter.  Sixty pointers loaded ahead and kept do not fit the scalar
+// registers; the compiler parks them in vector lanes, an instruction for
+// every store and use.  After step_args_again() they are loaded again (a
+// scalar load each, from the cache).  126 -> 38 parked registers in the
+// 162-vertex wave form (64 x 256 cells: 154.8 -> 143.2 us a step with the
+// candidate lists' code), 162 -> 56 in the 642-vertex workgroup form.
+template <typename R>
+using Step3DArgs = const __attribute__((address_space(4))) Step3D<R>;
+template <typename R>
+__device__ __forceinline__ Step3DArgs<R>* step_args_here() {
+  return (Step3DArgs<R>*)__builtin_amdgcn_kernarg_segment_ptr();
+}
+template <typename R>
+__device__ __forceinline__ void step_args_again(Step3DArgs<R>*& a) {
+  asm volatile("" : "+s"(a));
+}
 
 // a + b = s + e exactly (Knuth's TwoSum, any magnitudes).
 template <typename R>
@@ -368,7 +394,7 @@ __device__ __forceinline__ void face_of(const Lds3D<R>& l, int f, int& i0, int& 
 // origin.
 // one_each: a thread per vertex, vertex tid in pv (cell_stats_own).
 template <typename R>
-__device__ void cell_stats_impl(const Lds3D<R>& l, int nv, int nf, CellStat<R>* st_out,
+__device__ CellStat<R> cell_stats_impl(const Lds3D<R>& l, int nv, int nf, CellStat<R>* st_out,
                                 double* vol_out, R* em_out, int ci, R l0c, bool one_each, bool has_v, V3<R> pv) {
   const int tid = threadIdx.x, NT = blockDim.x;
   double px = 0.0, py = 0.0, pz = 0.0;
@@ -418,14 +444,17 @@ __device__ void cell_stats_impl(const Lds3D<R>& l, int nv, int nf, CellStat<R>* 
     r = (R)rd;
     e2 = (R)e2d;
   }
+  CellStat<R> st{};  // thread 0's
   if (tid == 0) {
     // Slack of a few ulp so that the culling tests are never tighter than the
     // largest distance a vertex can have from C, or the longest edge.
     const R em = sqrt(e2) * R(1.000001f);
-    st_out[ci] = make_cell_stat<R>(C.x, C.y, C.z, r * R(1.0000005f) + R(1e-30f), em, l0c);
+    st = make_cell_stat<R>(C.x, C.y, C.z, r * R(1.0000005f) + R(1e-30f), em, l0c);
+    st_out[ci] = st;
     vol_out[ci] = fabs(vol / 6.0);
     em_out[ci] = em;
   }
+  return st;
 }
 template <typename R>
 __device__ void cell_stats(const Lds3D<R>& l, int nv, int nf, CellStat<R>* st_out, double* vol_out, R* em_out,
@@ -438,21 +467,21 @@ __device__ void cell_stats(const Lds3D<R>& l, int nv, int nf, CellStat<R>* st_ou
 // positions are read only by the face loop, after the first reduction's
 // barrier, so they may be written just before the call.
 template <typename R>
-__device__ void cell_stats_own(const Lds3D<R>& l, int nv, int nf, CellStat<R>* st_out, double* vol_out,
+__device__ CellStat<R> cell_stats_own(const Lds3D<R>& l, int nv, int nf, CellStat<R>* st_out, double* vol_out,
                                R* em_out, int ci, R l0c, bool has_v, V3<R> pv) {
-  cell_stats_impl(l, nv, nf, st_out, vol_out, em_out, ci, l0c, true, has_v, pv);
+  return cell_stats_impl(l, nv, nf, st_out, vol_out, em_out, ci, l0c, true, has_v, pv);
 }
 
-template <typename R>
-__device__ __forceinline__ void stage_topology(const Step3D<R>& a, const Lds3D<R>& l) {
+template <typename R, typename Args>
+__device__ __forceinline__ void stage_topology(Args& a, const Lds3D<R>& l) {
   const int tid = threadIdx.x, NT = blockDim.x;
   for (int f = tid; f < a.nf; f += NT)
     l.sf[f] = make_uint2((unsigned)a.faces[3 * f] | ((unsigned)a.faces[3 * f + 1] << 16),
                          (unsigned)a.faces[3 * f + 2]);
 }
 
-template <typename R>
-__device__ __forceinline__ void load_own(const Step3D<R>& a, const Lds3D<R>& l, size_t base) {
+template <typename R, typename Args>
+__device__ __forceinline__ void load_own(Args& a, const Lds3D<R>& l, size_t base) {
   for (int v = threadIdx.x; v < a.nv; v += blockDim.x) {
     l.sx[v] = a.xin[base + v];
     l.sy[v] = a.yin[base + v];
@@ -567,6 +596,49 @@ __device__ __forceinline__ V3<R> substrate_corner(V3<R> pos, V3<R> C, R Ks, R ks
     }
   }
   return c;
+}
+
+// ---------------------------------------------------------- candidate lists
+//
+// The scan tests every cell of the tissue for every cell and step: at 4096
+// cells of 642 vertices a third of the step (27 of 86 kcycles of a
+// workgroup).  A step that finds its tissue's lists stale scans as before and
+// also keeps, per cell, the cells within `skin` of its reach; the following
+// steps apply the scan's own test to those entries, in the same ascending
+// order, so the candidates are the scan's, bit for bit.
+// The lists hold as long as no pair can have come closer than the skin: a
+// cell's excess is its centre's displacement since the lists were made plus
+// what its radius and contact margin grew; the reach of a pair grows by no
+// more than both excesses, its minimum-image distance shrinks by no more.
+// The step that moves a cell past 0.49 of the skin marks the tissue's lists
+// stale for the next one (not below half: float rounding has 2 % of the skin,
+// which is thousands of ulp of the coordinates).  Three sets of marks: the
+// one read, the one written for the next step, the one cleared for the step
+// after.
+constexpr int kNearList = DPM_WAVE;
+
+template <typename R>
+__device__ __forceinline__ bool near_list_moved(const CellStat<R>& ref, V3<R> C, R r, R em, R skin) {
+  const V3<R> d = {C.x - ref.cx, C.y - ref.cy, C.z - ref.cz};
+  const R excess = sqrt(vdot(d, d)) + R(1.0002f) * fmax(R(0), r - ref.r) + R(0.41f) * fmax(R(0), em - ref.em);
+  return !(excess <= R(0.49f) * skin);  // a NaN is stale
+}
+
+// The scan's test with the skin: within reach + skin by either contact or
+// adhesion, or the pair takes every image.
+template <typename R>
+__device__ __forceinline__ bool near_list_takes(const CellStat<R>& sti, const CellStat<R>& stj, bool pbc, R L, R invL,
+                                                bool contact, bool adhesion, R skin) {
+  V3<R> sh = {R(0), R(0), R(0)};
+  if (pbc)
+    sh = v3(image_shift(sti.cx - stj.cx, L, invL), image_shift(sti.cy - stj.cy, L, invL),
+            image_shift(sti.cz - stj.cz, L, invL));
+  const V3<R> d = {stj.cx + sh.x - sti.cx, stj.cy + sh.y - sti.cy, stj.cz + sh.z - sti.cz};
+  R reach = R(0);
+  if (contact) reach = sti.r + stj.r + contact_margin(stj.r, stj.em);
+  if (adhesion) reach = fmax(reach, sti.r + stj.r + R(2) * fmax(sti.l0, fmax(stj.l0, R(1e-12f))));
+  const R rr = (reach + skin) * R(1.0001f) + R(1e-6f);
+  return vdot(d, d) <= rr * rr || (pbc && R(2) * rr >= R(0.999f) * L);
 }
 
 // ---------------------------------------------------------------- cell list
@@ -765,35 +837,45 @@ __device__ __forceinline__ R winding_wave(const Lds3D<R>& l, Q4<R>* ut, int nv, 
 // NVC, NFC, NTC, WWC: vertex and face counts, threads per workgroup and
 // winding waves fixed at compile time (0: taken from the arguments).
 template <typename R, int NVC, int NFC, int NTC, int WWC, bool PROBE = true>
-__device__ void k3d_step_body(const Step3D<R>& a) {
+__device__ void k3d_step_body() {
+  Step3DArgs<R>* a = step_args_here<R>();
   extern __shared__ __align__(16) unsigned char smem[];
-  const int nv = NVC > 0 ? NVC : a.nv, nf = NFC > 0 ? NFC : a.nf, NT = NTC > 0 ? NTC : (int)blockDim.x, tid = threadIdx.x;
-  const int ww = WWC > 0 ? WWC : a.ww;
+  const int nv = NVC > 0 ? NVC : a->nv, nf = NFC > 0 ? NFC : a->nf, NT = NTC > 0 ? NTC : (int)blockDim.x, tid = threadIdx.x;
+  const int ww = WWC > 0 ? WWC : a->ww;
   const int lane = tid & (DPM_WAVE - 1), wave = tid / DPM_WAVE;
   const int ci = xcd_remap(blockIdx.x, gridDim.x);
   Lds3D<R> l = carve3d<R>(smem, nv, nf, NT, ww);
 
-  const int t = a.cell_tissue[ci];
-  const int cb = a.tissue_begin[t], ce = a.tissue_begin[t + 1];
-  const R L = (R)a.tL[t];
-  const int pbc = a.tpbc[t];
-  const R Kre = (R)a.tKre[t], Kat = (R)a.tKat[t], ksg = (R)a.tksg[t];
-  const CellStat<R> sti = a.st_in[ci];
+  const int t = a->cell_tissue[ci];
+  const int cb = a->tissue_begin[t], ce = a->tissue_begin[t + 1];
+  const R L = (R)a->tL[t];
+  const int pbc = a->tpbc[t];
+  const R Kre = (R)a->tKre[t], Kat = (R)a->tKat[t], ksg = (R)a->tksg[t];
+  const CellStat<R> sti = a->st_in[ci];
   const V3<R> Ci = {sti.cx, sti.cy, sti.cz};
   const R Ri = sti.r;
-  const R Kvi = (R)a.Kv[ci], Kai = (R)a.Ka[ci], Ksi = (R)a.Ks[ci], Kbi = (R)a.Kb[ci];
-  const R v0i = (R)a.v0[ci], a0i = (R)a.a0[ci], l0i = cell_l0<R>(a.a0, ci);
-  const unsigned mask = a.mask;
+  const R Kvi = (R)a->Kv[ci], Kai = (R)a->Ka[ci], Ksi = (R)a->Ks[ci], Kbi = (R)a->Kb[ci];
+  const R v0i = (R)a->v0[ci], a0i = (R)a->a0[ci], l0i = cell_l0<R>(a->a0, ci);
+  const unsigned mask = a->mask;
   const size_t base = (size_t)ci * nv;
   const bool own = tid < nv;
   const V3<R> zero = {R(0), R(0), R(0)};
+
+  // candidate lists: made by this step, or read (nlist entries; not when
+  // there are more than a list holds)
+  const bool nl_on = a->nl_cnt && !a->bin_list;  // block-uniform
+  const bool relist = nl_on && a->nl_stale[t] != 0;
+  const int nlist = nl_on && !relist ? a->nl_cnt[ci] : -1;
+  const bool listed = nlist >= 0;
+  CellStat<R> nl_ref = sti;  // where this step makes the lists
+  if (nl_on && !relist) nl_ref = a->nl_ref[ci];
 
   // per-vertex topology rows in registers
   int vfr[DPM3D_MAXDEG], adjr[DPM3D_MAXDEG];
 #pragma unroll
   for (int k = 0; k < DPM3D_MAXDEG; k++) {
-    vfr[k] = own ? a.vf[tid * DPM3D_MAXDEG + k] : -1;
-    adjr[k] = own ? a.adj[tid * DPM3D_MAXDEG + k] : -1;
+    vfr[k] = own ? a->vf[tid * DPM3D_MAXDEG + k] : -1;
+    adjr[k] = own ? a->adj[tid * DPM3D_MAXDEG + k] : -1;
   }
   // The candidate scan's statistics (every cell of a tissue of at most NT
   // cells, no cell list) are loaded here with the cell's own data, one
@@ -801,29 +883,29 @@ __device__ void k3d_step_body(const Step3D<R>& a) {
   // the others the registers held until the scan would spill).
   const bool scan_pre = (sizeof(R) == 4 && NTC > 0) &&
                         (((mask & M_CONTACT) && Kre != R(0)) || ((mask & M_ADHESION) && Kat != R(0)));
-  const bool scan_all = scan_pre && !(a.bin_list && a.tbin_nb[t] > 0) && ce - cb <= NT;  // block-uniform
+  const bool scan_all = scan_pre && !listed && !(a->bin_list && a->tbin_nb[t] > 0) && ce - cb <= NT;  // block-uniform
   CellStat<R> st_pre{};
-  if (scan_all && tid < ce - cb) st_pre = a.st_in[cb + tid];
+  if (scan_all && tid < ce - cb) st_pre = a->st_in[cb + tid];
   if constexpr (NFC > 0 && NVC > 0 && NTC > 0) {
     // compile-time sizes: every load in flight before the first LDS store
     static_assert(NFC <= 2 * NTC, "at most two faces per thread");
     const int f0 = tid, f1 = tid + NTC;
     int a0 = 0, b0 = 0, e0 = 0, a1 = 0, b1 = 0, e1 = 0;
     if (f0 < NFC) {
-      a0 = a.faces[3 * f0];
-      b0 = a.faces[3 * f0 + 1];
-      e0 = a.faces[3 * f0 + 2];
+      a0 = a->faces[3 * f0];
+      b0 = a->faces[3 * f0 + 1];
+      e0 = a->faces[3 * f0 + 2];
     }
     if (f1 < NFC) {
-      a1 = a.faces[3 * f1];
-      b1 = a.faces[3 * f1 + 1];
-      e1 = a.faces[3 * f1 + 2];
+      a1 = a->faces[3 * f1];
+      b1 = a->faces[3 * f1 + 1];
+      e1 = a->faces[3 * f1 + 2];
     }
     R px = R(0), py = R(0), pz = R(0);
     if (own) {
-      px = a.xin[base + tid];
-      py = a.yin[base + tid];
-      pz = a.zin[base + tid];
+      px = a->xin[base + tid];
+      py = a->yin[base + tid];
+      pz = a->zin[base + tid];
     }
     if (f0 < NFC) l.sf[f0] = make_uint2((unsigned)a0 | ((unsigned)b0 << 16), (unsigned)e0);
     if (f1 < NFC) l.sf[f1] = make_uint2((unsigned)a1 | ((unsigned)b1 << 16), (unsigned)e1);
@@ -833,8 +915,8 @@ __device__ void k3d_step_body(const Step3D<R>& a) {
       l.sz[tid] = pz;
     }
   } else {
-    stage_topology(a, l);
-    load_own(a, l, base);
+    stage_topology(*a, l);
+    load_own(*a, l, base);
   }
   __syncthreads();
 
@@ -843,6 +925,8 @@ __device__ void k3d_step_body(const Step3D<R>& a) {
   bool ring_done = false;  // shape forces by the ring walk (bending's first sum in ring_sb)
   V3<R> ring_sb = zero;
 
+  step_args_again<R>(a);
+
   // ---------------------------------------------------------- shape forces
   // Per-face pass: each face's volume, edge-spring and substrate terms for
   // its three corners are computed once into LDS; every vertex then gathers
@@ -850,7 +934,7 @@ __device__ void k3d_step_body(const Step3D<R>& a) {
   if (mask & (M_VOLUME | M_SURFACE | M_SUBSTRATE)) {  // block-uniform
     // Volume strain of the current volume, in double (the residual V/v0 - 1
     // cancels when the cell is near its target).
-    const R strain = (R)(a.vol_in[ci] / (double)v0i - 1.0);
+    const R strain = (R)(a->vol_in[ci] / (double)v0i - 1.0);
     const R kvol = -Kvi * strain / R(6);
     const bool vol_on = (mask & M_VOLUME) && Kvi != R(0);
     const bool surf_on = (mask & M_SURFACE) && !(Kai < R(1e-8f));
@@ -858,7 +942,7 @@ __device__ void k3d_step_body(const Step3D<R>& a) {
     const R sc = Kai * sqrt(a0i) / l0i * R(0.3f);
     const R inv_l0 = R(1) / l0i;
     const double sub_inv_l0 = 1.0 / (double)l0i;
-    if ((sizeof(R) == 4 || NTC > 0) && a.closed) {  // block-uniform
+    if ((sizeof(R) == 4 || NTC > 0) && a->closed) {  // block-uniform
       // Closed mesh, neighbour rows in ring order (face q is (v, u_q, u_(q+1))):
       // one walk around each vertex's ring, as the wave-per-cell step takes
       // it — volume kvol sum_q d_q x d_(q+1), edge springs 2 sc sum_q s(d_q),
@@ -879,7 +963,7 @@ __device__ void k3d_step_body(const Step3D<R>& a) {
             face_of(l, f, i0, i1, i2);
             const V3<R> P0 = lds_v(l.sx, l.sy, l.sz, i0);
             dn = facing_down(vcross(vsub(lds_v(l.sx, l.sy, l.sz, i1), P0), vsub(lds_v(l.sx, l.sy, l.sz, i2), P0)));
-            if (PROBE && dn && a.p_down) a.p_down[(size_t)ci * nf + f] = 1;
+            if (PROBE && dn && a->p_down) a->p_down[(size_t)ci * nf + f] = 1;
           }
           const unsigned long long m = __ballot(dn);
           if (lane == 0) {
@@ -955,7 +1039,7 @@ __device__ void k3d_step_body(const Step3D<R>& a) {
       if (sub_on) {  // Cell3D_Kernel.cl:206-246
         const V3<R> un = vnormalize(vcross(vsub(P1, P0), vsub(P2, P0)));
         if (un.z < R(-0.1f)) {
-          if (PROBE && a.p_down) a.p_down[(size_t)ci * nf + f] = 1;
+          if (PROBE && a->p_down) a->p_down[(size_t)ci * nf + f] = 1;
           c0 = vadd(c0, substrate_corner(P0, Ci, Ksi, ksg, L, l0i, sub_inv_l0));
           c1 = vadd(c1, substrate_corner(P1, Ci, Ksi, ksg, L, l0i, sub_inv_l0));
           c2 = vadd(c2, substrate_corner(P2, Ci, Ksi, ksg, L, l0i, sub_inv_l0));
@@ -1020,6 +1104,8 @@ __device__ void k3d_step_body(const Step3D<R>& a) {
     }
   }
 
+  step_args_again<R>(a);
+
   // ------------------------------------------- contact and vertex adhesion
   const bool do_contact = (mask & M_CONTACT) && Kre != R(0);
   const bool do_adh = (mask & M_ADHESION) && Kat != R(0);
@@ -1034,9 +1120,9 @@ __device__ void k3d_step_body(const Step3D<R>& a) {
     // the 27 buckets around this cell, sorted by index (block-uniform)
     const int* src = nullptr;
     int nsrc = ce - cb;
-    if (a.bin_list && a.tbin_nb[t] > 0) {
-      const int nb = a.tbin_nb[t], nbuck = a.tbin_nbuck[t];
-      const int* bs = a.bin_start + a.tbin_hoff[t];
+    if (a->bin_list && a->tbin_nb[t] > 0) {
+      const int nb = a->tbin_nb[t], nbuck = a->tbin_nbuck[t];
+      const int* bs = a->bin_start + a->tbin_hoff[t];
       const R wb = L / (R)nb;
       int* gid = l.gath;        // [27] bucket ids
       int* gst = l.gath + 32;   // [27] bucket starts
@@ -1058,7 +1144,7 @@ __device__ void k3d_step_body(const Step3D<R>& a) {
         if (tid < n) {
           int u = 0;
           while (gof[u + 1] <= tid) u++;
-          l.glist[tid] = a.bin_list[cb + gst[u] + (tid - gof[u])];
+          l.glist[tid] = a->bin_list[cb + gst[u] + (tid - gof[u])];
         }
         __syncthreads();
         if (tid < n) {  // rank sort (indices are distinct)
@@ -1074,6 +1160,11 @@ __device__ void k3d_step_body(const Step3D<R>& a) {
         nsrc = n;
       }
     }
+    if (listed) {  // at most 64 entries: one chunk
+      src = a->nl_idx + (size_t)ci * kNearList;
+      nsrc = nlist;
+    }
+    int nnl = 0;  // entries of the list being made
     for (int c0 = 0; c0 < nsrc; c0 += NT) {
       const int k = c0 + tid;
       const int cj = k < nsrc ? (src ? src[k] : cb + k) : ce;
@@ -1083,7 +1174,7 @@ __device__ void k3d_step_body(const Step3D<R>& a) {
         if (scan_all && c0 == 0)
           stj = st_pre;
         else
-          stj = a.st_in[cj];
+          stj = a->st_in[cj];
         V3<R> sh = zero;
         if (pbc)
           sh = v3(image_shift(Ci.x - stj.cx, L, invL), image_shift(Ci.y - stj.cy, L, invL),
@@ -1103,12 +1194,19 @@ __device__ void k3d_step_body(const Step3D<R>& a) {
         const R rr = reach * R(1.0001f) + R(1e-6f);
         cand = cand || vdot(d, d) <= rr * rr;
       }
+      if (relist) {  // block-uniform
+        const bool nr = cj < ce && cj != ci && near_list_takes(sti, stj, pbc, L, invL, do_contact, do_adh, a->nl_skin);
+        const int n = block_compact(nr, cj, l.plist, l.cnt);
+        if (tid < n && nnl + tid < kNearList) a->nl_idx[(size_t)ci * kNearList + nnl + tid] = l.plist[tid];
+        nnl += n;
+        __syncthreads();  // the compaction's arrays are written again next
+      }
       const int ncand = block_compact_with(cand, cj, l.clist, l.cnt, [&](int slot) {
         if (slot < kCandStats) l.cst[slot] = stj;
       });
       n_cand += ncand;
       // candidate q's statistics (wave-uniform q)
-      auto cand_stat = [&](int q) { return q < kCandStats ? l.cst[q] : a.st_in[l.clist[q]]; };
+      auto cand_stat = [&](int q) { return q < kCandStats ? l.cst[q] : a->st_in[l.clist[q]]; };
       // Separation along the centre line n = (C_j - C_i) / D (float steps
       // and the compile-time-sized instances): every vertex p of this cell
       // has (p - C_i).n <= hi and every point x of cell j's (shifted) hull
@@ -1152,7 +1250,7 @@ __device__ void k3d_step_body(const Step3D<R>& a) {
           const size_t bj = (size_t)cjq * nv;
           for (int v = lane; v < nv; v += DPM_WAVE) {
             hi = fmax(hi, vdot(vsub(lds_v(l.sx, l.sy, l.sz, v), Ci), nC));
-            hj = fmax(hj, vdot(v3(stj.cx - a.xin[bj + v], stj.cy - a.yin[bj + v], stj.cz - a.zin[bj + v]), nC));
+            hj = fmax(hj, vdot(v3(stj.cx - a->xin[bj + v], stj.cy - a->yin[bj + v], stj.cz - a->zin[bj + v]), nC));
           }
           hi = wave_max_all(hi);
           hj = wave_max_all(hj);
@@ -1178,7 +1276,7 @@ __device__ void k3d_step_body(const Step3D<R>& a) {
       V3<R> pre = zero;
       if (nkeep > 0 && own) {
         const size_t b0 = (size_t)l.clist[entry(0) & 0x0fffffff] * nv + tid;
-        pre = v3(a.xin[b0], a.yin[b0], a.zin[b0]);
+        pre = v3(a->xin[b0], a->yin[b0], a->zin[b0]);
       }
       for (int qq = 0; qq < nkeep; qq++) {
         const int ent = entry(qq);
@@ -1198,7 +1296,7 @@ __device__ void k3d_step_body(const Step3D<R>& a) {
         __syncthreads();
         if (qq + 1 < nkeep && own) {
           const size_t b1 = (size_t)l.clist[entry(qq + 1) & 0x0fffffff] * nv + tid;
-          pre = v3(a.xin[b1], a.yin[b1], a.zin[b1]);
+          pre = v3(a->xin[b1], a->yin[b1], a->zin[b1]);
         }
         const bool skip_contact = !(passes & 1), skip_adh = !(passes & 2);
         if (do_contact && !skip_contact) {  // block-uniform
@@ -1228,31 +1326,31 @@ __device__ void k3d_step_body(const Step3D<R>& a) {
           __syncthreads();
           if (need) {
             const R wv = l.wb[tid];
-            const size_t pidx = (base + tid) * (size_t)a.ncmax + (size_t)(cj2 - cb);
-            if (PROBE && a.p_winding) a.p_winding[pidx] = (float)wv;
+            const size_t pidx = (base + tid) * (size_t)a->ncmax + (size_t)(cj2 - cb);
+            if (PROBE && a->p_winding) a->p_winding[pidx] = (float)wv;
             if (!(fabs(wv) < R(1e-6f))) {
               const V3<R> dir = vnormalize(vsub(Ci, P));
               const R mag = fabs(wv) * R(0.5f) * Kre;
               F = vadd(F, vscale(dir, mag));
               n_contact++;
               wsum += fabs(wv);
-              if (a.rec_cell) {
+              if (a->rec_cell) {
                 if (npart < DPM3D_MAXPART) {
                   const size_t r = (base + tid) * DPM3D_MAXPART + npart;
-                  a.rec_cell[r] = cj2;
-                  a.rec_w[r] = wv;
-                  a.rec_shift[3 * r] = sh.x;
-                  a.rec_shift[3 * r + 1] = sh.y;
-                  a.rec_shift[3 * r + 2] = sh.z;
+                  a->rec_cell[r] = cj2;
+                  a->rec_w[r] = wv;
+                  a->rec_shift[3 * r] = sh.x;
+                  a->rec_shift[3 * r + 1] = sh.y;
+                  a->rec_shift[3 * r + 2] = sh.z;
                 } else {
-                  atomicOr(a.rec_overflow, 1);
+                  atomicOr(a->rec_overflow, 1);
                 }
                 npart++;
               }
-              if (PROBE && a.p_contact) a.p_contact[pidx] = 1;
-              if (PROBE && a.p_contact_key) {  // count, then key sum of the partner cells
-                atomicAdd(&a.p_contact_key[2 * (base + tid)], 1u);
-                atomicAdd(&a.p_contact_key[2 * (base + tid) + 1], cell_key(cj2 - cb));
+              if (PROBE && a->p_contact) a->p_contact[pidx] = 1;
+              if (PROBE && a->p_contact_key) {  // count, then key sum of the partner cells
+                atomicAdd(&a->p_contact_key[2 * (base + tid)], 1u);
+                atomicAdd(&a->p_contact_key[2 * (base + tid) + 1], cell_key(cj2 - cb));
               }
             }
           }
@@ -1327,13 +1425,13 @@ __device__ void k3d_step_body(const Step3D<R>& a) {
                       if (own_on) {
                         Fa = adhesion_term_near(dl, y, kh_f, inv_l0i_f, Fa);
                         cnt_own++;
-                        if (PROBE && a.p_adh_hash)
-                          atomicAdd(&a.p_adh_hash[2 * (base + il[iv])], vertex_key(pj.x, pj.y, pj.z));
+                        if (PROBE && a->p_adh_hash)
+                          atomicAdd(&a->p_adh_hash[2 * (base + il[iv])], vertex_key(pj.x, pj.y, pj.z));
                       }
                       if (rev_on) {
                         Fa = adhesion_term_near(dl, y, kh_f, inv_l0j_f, Fa);
-                        if (PROBE && a.p_adh_hash)
-                          atomicAdd(&a.p_adh_hash[2 * (base + il[iv]) + 1], vertex_key(pj.x, pj.y, pj.z));
+                        if (PROBE && a->p_adh_hash)
+                          atomicAdd(&a->p_adh_hash[2 * (base + il[iv]) + 1], vertex_key(pj.x, pj.y, pj.z));
                       }
                     }
                     continue;
@@ -1342,13 +1440,13 @@ __device__ void k3d_step_body(const Step3D<R>& a) {
                 if (cut_own(d2)) {
                   Fa = vsub(Fa, adhesion_term(pj, Pv, nl, L, Kat, L0i, kh, inv_l0i));
                   cnt_own++;
-                  if (PROBE && a.p_adh_hash) atomicAdd(&a.p_adh_hash[2 * (base + il[iv])], vertex_key(pj.x, pj.y, pj.z));
+                  if (PROBE && a->p_adh_hash) atomicAdd(&a->p_adh_hash[2 * (base + il[iv])], vertex_key(pj.x, pj.y, pj.z));
                 }
                 const R d2r = vdot(dr, dr);
                 if (cut_rev(d2r)) {
                   Fa = vadd(Fa, adhesion_term(Pv, pj, nr, L, Kat, L0j, kh, inv_l0j));
-                  if (PROBE && a.p_adh_hash)
-                    atomicAdd(&a.p_adh_hash[2 * (base + il[iv]) + 1], vertex_key(pj.x, pj.y, pj.z));
+                  if (PROBE && a->p_adh_hash)
+                    atomicAdd(&a->p_adh_hash[2 * (base + il[iv]) + 1], vertex_key(pj.x, pj.y, pj.z));
                 }
               }
               acc[sl * nmine + iv] = Q4<R>{Fa.x, Fa.y, Fa.z, (R)cnt_own};
@@ -1361,42 +1459,49 @@ __device__ void k3d_step_body(const Step3D<R>& a) {
                 F = vadd(F, V3<R>{q4.x, q4.y, q4.z});
                 cnt_own += (int)q4.w;
               }
-              if (PROBE && a.p_adh) a.p_adh[base + tid] += cnt_own;
+              if (PROBE && a->p_adh) a->p_adh[base + tid] += cnt_own;
             }
           }
         }
         __syncthreads();
       }
     }
+    if (relist && tid == 0) {
+      a->nl_cnt[ci] = nnl <= kNearList ? nnl : -1;
+      a->nl_ref[ci] = sti;
+    }
   }
+  if (a->nl_cnt && ci == cb && tid == 0) a->nl_stale_clear[t] = 0;
+
+  step_args_again<R>(a);
 
   // ------------------------------------------------------- Euler and stats
-  if (own && a.w_out) a.w_out[base + tid] = wsum;
-  if (own && a.rec_cell)
-    for (int q = npart; q < DPM3D_MAXPART; q++) a.rec_cell[(base + tid) * DPM3D_MAXPART + q] = -1;
-  if (own && (a.flags & F_WRITE_FORCES)) {
-    a.fx[base + tid] = F.x;
-    a.fy[base + tid] = F.y;
-    a.fz[base + tid] = F.z;
+  if (own && a->w_out) a->w_out[base + tid] = wsum;
+  if (own && a->rec_cell)
+    for (int q = npart; q < DPM3D_MAXPART; q++) a->rec_cell[(base + tid) * DPM3D_MAXPART + q] = -1;
+  if (own && (a->flags & F_WRITE_FORCES)) {
+    a->fx[base + tid] = F.x;
+    a->fy[base + tid] = F.y;
+    a->fz[base + tid] = F.z;
   }
-  if (a.flags & F_MOVE) {  // block-uniform
+  if (a->flags & F_MOVE) {  // block-uniform
     V3<R> Pn = P;
     if (own) {
-      if (a.xlo) {
+      if (a->xlo) {
         // x + lo + F dt, the displacement rounded once onto the residual
         R ex, ey, ez;
-        Pn = v3(two_sum(P.x, fma(F.x, a.dt, a.xlo[base + tid]), ex),
-                two_sum(P.y, fma(F.y, a.dt, a.ylo[base + tid]), ey),
-                two_sum(P.z, fma(F.z, a.dt, a.zlo[base + tid]), ez));
-        a.xlo[base + tid] = ex;
-        a.ylo[base + tid] = ey;
-        a.zlo[base + tid] = ez;
+        Pn = v3(two_sum(P.x, fma(F.x, a->dt, a->xlo[base + tid]), ex),
+                two_sum(P.y, fma(F.y, a->dt, a->ylo[base + tid]), ey),
+                two_sum(P.z, fma(F.z, a->dt, a->zlo[base + tid]), ez));
+        a->xlo[base + tid] = ex;
+        a->ylo[base + tid] = ey;
+        a->zlo[base + tid] = ez;
       } else {
-        Pn = v3(fma(F.x, a.dt, P.x), fma(F.y, a.dt, P.y), fma(F.z, a.dt, P.z));
+        Pn = v3(fma(F.x, a->dt, P.x), fma(F.y, a->dt, P.y), fma(F.z, a->dt, P.z));
       }
-      a.xout[base + tid] = Pn.x;
-      a.yout[base + tid] = Pn.y;
-      a.zout[base + tid] = Pn.z;
+      a->xout[base + tid] = Pn.x;
+      a->yout[base + tid] = Pn.y;
+      a->zout[base + tid] = Pn.z;
     }
     __syncthreads();  // every read of the step's positions is done
     if (own) {
@@ -1404,9 +1509,11 @@ __device__ void k3d_step_body(const Step3D<R>& a) {
       l.sy[tid] = Pn.y;
       l.sz[tid] = Pn.z;
     }
-    cell_stats_own(l, nv, nf, a.st_out, a.vol_out, a.em_out, ci, l0i, own, Pn);
+    const CellStat<R> stn = cell_stats_own(l, nv, nf, a->st_out, a->vol_out, a->em_out, ci, l0i, own, Pn);
+    if (nl_on && tid == 0 && near_list_moved(nl_ref, v3(stn.cx, stn.cy, stn.cz), stn.r, stn.em, a->nl_skin))
+      a->nl_stale_out[t] = 1;
   }
-  if (a.counters) {
+  if (a->counters) {
     // per wave, without a workgroup barrier: the wave's contact count, its
     // winding count (kept by lane 0), and the candidates (every thread holds
     // the workgroup's count; wave 0 adds it).  Spread over
@@ -1415,7 +1522,7 @@ __device__ void k3d_step_body(const Step3D<R>& a) {
     unsigned long long c = n_contact;
     for (int o = 32; o > 0; o >>= 1) c += __shfl_down(c, o, DPM_WAVE);
     if (lane == 0) {
-      unsigned long long* slot = a.counters + 4 * ((blockIdx.x * (NT / DPM_WAVE) + wave) % DPM_COUNTER_SLOTS);
+      unsigned long long* slot = a->counters + 4 * ((blockIdx.x * (NT / DPM_WAVE) + wave) % DPM_COUNTER_SLOTS);
       if (blockIdx.x == 0 && wave == 0) atomicAdd(&slot[0], 1ull);
       if (n_wind) atomicAdd(&slot[1], n_wind);
       if (c) atomicAdd(&slot[2], c);
@@ -1883,23 +1990,23 @@ __device__ void k3d_vjp_body(const Vjp3D<R>& a) {
 
 extern "C" __global__ void __launch_bounds__(1024) k3d_stats_f32(const Step3D<float> a) { k3d_stats_body(a); }
 extern "C" __global__ void __launch_bounds__(1024) k3d_stats_f64(const Step3D<double> a) { k3d_stats_body(a); }
-extern "C" __global__ void __launch_bounds__(1024) k3d_step_f32(const Step3D<float> a) { k3d_step_body<float, 0, 0, 0, 0>(a); }
-extern "C" __global__ void __launch_bounds__(1024) k3d_step_f64(const Step3D<double> a) { k3d_step_body<double, 0, 0, 0, 0>(a); }
+extern "C" __global__ void __launch_bounds__(1024) k3d_step_f32(const Step3D<float> a) { k3d_step_body<float, 0, 0, 0, 0>(); }
+extern "C" __global__ void __launch_bounds__(1024) k3d_step_f64(const Step3D<double> a) { k3d_step_body<double, 0, 0, 0, 0>(); }
 // Instances for the icospheres of subdivision 2 and 3 (162 / 642 vertices):
 // sizes, workgroup size and winding waves fixed at compile time, so LDS
 // offsets are immediates and the register budget is that of 256 or 704
 // threads instead of 1024 (the general kernel spills at 128 registers).
 // The host takes them where the handle's nv, nf, NT and ww match.
 extern "C" __global__ void __launch_bounds__(256) k3d_step_f32_v162(const Step3D<float> a) {
-  k3d_step_body<float, 162, 320, 256, 4, false>(a);
+  k3d_step_body<float, 162, 320, 256, 4, false>();
 }
 // the same with the diagnostic outputs (dpm3d_probe*) compiled in
 extern "C" __global__ void __launch_bounds__(256) k3d_step_f32_v162_probe(const Step3D<float> a) {
-  k3d_step_body<float, 162, 320, 256, 4, true>(a);
+  k3d_step_body<float, 162, 320, 256, 4, true>();
 }
-extern "C" __global__ void __launch_bounds__(704) k3d_step_f32_v642(const Step3D<float> a) { k3d_step_body<float, 642, 1280, 704, 4>(a); }
-extern "C" __global__ void __launch_bounds__(704) k3d_step_f64_v642(const Step3D<double> a) { k3d_step_body<double, 642, 1280, 704, 2>(a); }
-extern "C" __global__ void __launch_bounds__(256) k3d_step_f64_v162(const Step3D<double> a) { k3d_step_body<double, 162, 320, 256, 4>(a); }
+extern "C" __global__ void __launch_bounds__(704) k3d_step_f32_v642(const Step3D<float> a) { k3d_step_body<float, 642, 1280, 704, 4>(); }
+extern "C" __global__ void __launch_bounds__(704) k3d_step_f64_v642(const Step3D<double> a) { k3d_step_body<double, 642, 1280, 704, 2>(); }
+extern "C" __global__ void __launch_bounds__(256) k3d_step_f64_v162(const Step3D<double> a) { k3d_step_body<double, 162, 320, 256, 4>(); }
 extern "C" __global__ void __launch_bounds__(1024) k3d_energy_f32(const Step3D<float> a) { k3d_energy_body(a); }
 extern "C" __global__ void __launch_bounds__(1024) k3d_energy_f64(const Step3D<double> a) { k3d_energy_body(a); }
 // lambda += dt * (contributions from other cells), contributions cleared.

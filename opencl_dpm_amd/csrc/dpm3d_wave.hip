@@ -152,9 +152,10 @@ __device__ __forceinline__ R winding_w(const R* nx, const R* ny, const R* nz, co
 // rolled: unrolled, their iterations' registers spill to scratch memory
 // (208 B per lane, 6x the step's HBM traffic, at the same speed).
 template <typename R, int NVC, int NFC, bool PROBE = true>
-__device__ void k3d_wstep_body(const Step3D<R>& a) {
+__device__ void k3d_wstep_body() {
+  Step3DArgs<R>* a = step_args_here<R>();
   extern __shared__ __align__(16) unsigned char smem[];
-  const int nv = NVC > 0 ? NVC : a.nv, nf = NFC > 0 ? NFC : a.nf;
+  const int nv = NVC > 0 ? NVC : a->nv, nf = NFC > 0 ? NFC : a->nf;
   // 64-vertex chunks of a cell (a bound when the size is a run-time value)
   constexpr int kChunks = NVC > 0 ? (NVC + DPM_WAVE - 1) / DPM_WAVE : kWaveMaxNv / DPM_WAVE;
   // wv, and every per-cell value derived from it, is wave-uniform: through
@@ -165,11 +166,11 @@ __device__ void k3d_wstep_body(const Step3D<R>& a) {
   const int cpw = blockDim.x / DPM_WAVE;
   const Lds3DWave LW = ldsw_layout(nv, nf, cpw, (int)sizeof(R));
   unsigned* sf = reinterpret_cast<unsigned*>(smem);
-  const uint4* rows = a.wtopo;  // 16-byte words of the topology image
+  const uint4* rows = a->wtopo;  // 16-byte words of the topology image
   for (int i = threadIdx.x; i < (int)(LW.fend / 16); i += blockDim.x) reinterpret_cast<uint4*>(smem)[i] = rows[i];
   __syncthreads();  // the only workgroup barrier
   const int ci = xcd_remap(blockIdx.x, gridDim.x) * cpw + wv;
-  if (ci >= a.ncells) return;  // whole wave
+  if (ci >= a->ncells) return;  // whole wave
 
   unsigned char* slb = smem + LW.fend + (size_t)wv * LW.slice;
   R* sx = reinterpret_cast<R*>(slb + LW.sx);
@@ -188,32 +189,40 @@ __device__ void k3d_wstep_body(const Step3D<R>& a) {
   int* cl = reinterpret_cast<int*>(slb + LW.cl);
   unsigned* down = reinterpret_cast<unsigned*>(slb + LW.down);
 
-  const int t = a.cell_tissue[ci];
-  const int cb = a.tissue_begin[t], ce = a.tissue_begin[t + 1];
-  const R L = (R)a.tL[t];
-  const int pbc = a.tpbc[t];
-  const R Kre = (R)a.tKre[t], Kat = (R)a.tKat[t], ksg = (R)a.tksg[t];
-  const CellStat<R> sti = a.st_in[ci];
+  const int t = a->cell_tissue[ci];
+  const int cb = a->tissue_begin[t], ce = a->tissue_begin[t + 1];
+  const R L = (R)a->tL[t];
+  const int pbc = a->tpbc[t];
+  const R Kre = (R)a->tKre[t], Kat = (R)a->tKat[t], ksg = (R)a->tksg[t];
+  const CellStat<R> sti = a->st_in[ci];
   const V3<R> Ci = {sti.cx, sti.cy, sti.cz};
   const R Ri = sti.r;
-  const R Kvi = (R)a.Kv[ci], Kai = (R)a.Ka[ci], Ksi = (R)a.Ks[ci], Kbi = (R)a.Kb[ci];
-  const R v0i = (R)a.v0[ci], a0i = (R)a.a0[ci], l0i = cell_l0<R>(a.a0, ci);
-  const unsigned mask = a.mask;
+  const R Kvi = (R)a->Kv[ci], Kai = (R)a->Ka[ci], Ksi = (R)a->Ks[ci], Kbi = (R)a->Kb[ci];
+  const R v0i = (R)a->v0[ci], a0i = (R)a->a0[ci], l0i = cell_l0<R>(a->a0, ci);
+  const unsigned mask = a->mask;
   const size_t base = (size_t)ci * nv;
   const V3<R> zero = {R(0), R(0), R(0)};
+  // candidate lists: made by this step, or read (nlist entries; not when
+  // there are more than a list holds); wave-uniform
+  const bool nl_on = a->nl_cnt && !a->bin_list;
+  const bool relist = nl_on && a->nl_stale[t] != 0;
+  const int nlist = nl_on && !relist ? a->nl_cnt[ci] : -1;
+  if (a->nl_cnt && ci == cb && lane == 0) a->nl_stale_clear[t] = 0;
 
-  wave_stage_cell(sx, sy, sz, a.xin, a.yin, a.zin, base, nv, lane);
+  wave_stage_cell(sx, sy, sz, a->xin, a->yin, a->zin, base, nv, lane);
   #pragma unroll 1
   for (int v = lane; v < nv; v += DPM_WAVE) {
-    if (a.w_out) a.w_out[base + v] = R(0);
-    if (a.rec_cell)
-      for (int q = 0; q < DPM3D_MAXPART; q++) a.rec_cell[(base + v) * DPM3D_MAXPART + q] = -1;
+    if (a->w_out) a->w_out[base + v] = R(0);
+    if (a->rec_cell)
+      for (int q = 0; q < DPM3D_MAXPART; q++) a->rec_cell[(base + v) * DPM3D_MAXPART + q] = -1;
   }
   wave_lds_sync();
 
+  step_args_again<R>(a);
+
   // ---------------------------------------------------------- shape forces
   const bool shape_on = (mask & (M_VOLUME | M_SURFACE | M_SUBSTRATE)) != 0;
-  const R strain = (R)(a.vol_in[ci] / (double)v0i - 1.0);
+  const R strain = (R)(a->vol_in[ci] / (double)v0i - 1.0);
   const R kvol = -Kvi * strain / R(6);
   const bool vol_on = (mask & M_VOLUME) && Kvi != R(0);
   // the ring walk sums the volume products unconditionally and scales them
@@ -247,7 +256,7 @@ __device__ void k3d_wstep_body(const Step3D<R>& a) {
           atomicAdd(&dcnt[i1], 1u);
           atomicAdd(&dcnt[i2], 1u);
         }
-        if (PROBE && dn && a.p_down) a.p_down[(size_t)ci * nf + f] = 1;
+        if (PROBE && dn && a->p_down) a->p_down[(size_t)ci * nf + f] = 1;
       }
       const unsigned long long m = __ballot(dn);
       if (lane == 0) {
@@ -262,7 +271,7 @@ __device__ void k3d_wstep_body(const Step3D<R>& a) {
   // makes the reference skip its faces' edge springs): the walk checks every
   // ring edge, and a cell with such an edge is taken again, every vertex by
   // the per-corner form (its springs skip those faces as the reference does).
-  bool ring_pass = shape_on && a.closed;  // wave-uniform
+  bool ring_pass = shape_on && a->closed;  // wave-uniform
   for (int pass = 0; pass < 2; pass++) {
   bool short_edge = false;
   #pragma unroll 1
@@ -385,6 +394,8 @@ __device__ void k3d_wstep_body(const Step3D<R>& a) {
   }
   wave_lds_sync();  // forces and scratch settled before the candidates
 
+  step_args_again<R>(a);
+
   // ------------------------------------------- contact and vertex adhesion
   const bool do_contact = (mask & M_CONTACT) && Kre != R(0);
   const bool do_adh = (mask & M_ADHESION) && Kat != R(0);
@@ -396,9 +407,9 @@ __device__ void k3d_wstep_body(const Step3D<R>& a) {
     // buckets around this cell sorted by index (held two per lane)
     bool gathered = false;
     int nsrc = ce - cb;
-    if (a.bin_list && a.tbin_nb[t] > 0) {
-      const int nb = a.tbin_nb[t], nbuck = a.tbin_nbuck[t];
-      const int* bs = a.bin_start + a.tbin_hoff[t];
+    if (a->bin_list && a->tbin_nb[t] > 0) {
+      const int nb = a->tbin_nb[t], nbuck = a->tbin_nbuck[t];
+      const int* bs = a->bin_start + a->tbin_hoff[t];
       const R wb = L / (R)nb;
       int* gst = gath + 32;
       int* gof = gath + 64;
@@ -417,14 +428,14 @@ __device__ void k3d_wstep_body(const Step3D<R>& a) {
         if (lane < n) {
           int u = 0;
           while (gof[u + 1] <= lane) u++;
-          val0 = a.bin_list[cb + gst[u] + (lane - gof[u])];
+          val0 = a->bin_list[cb + gst[u] + (lane - gof[u])];
           gl[lane] = val0;
         }
         if (lane + DPM_WAVE < n) {
           const int i = lane + DPM_WAVE;
           int u = 0;
           while (gof[u + 1] <= i) u++;
-          val1 = a.bin_list[cb + gst[u] + (i - gof[u])];
+          val1 = a->bin_list[cb + gst[u] + (i - gof[u])];
           gl[i] = val1;
         }
         wave_lds_sync();
@@ -443,13 +454,20 @@ __device__ void k3d_wstep_body(const Step3D<R>& a) {
         nsrc = n;
       }
     }
+    if (nlist >= 0) {
+      if (lane < nlist) cl[lane] = a->nl_idx[(size_t)ci * kNearList + lane];
+      wave_lds_sync();
+      gathered = true;
+      nsrc = nlist;
+    }
+    int nnl = 0;  // entries of the list being made
     int c0 = 0;
     // a chunk's source cell and statistics, loaded one chunk ahead (a gathered
     // source is read before the compaction below can overwrite it: the
     // compacted slots lie below the chunk being tested)
     int cj_nx = lane < nsrc ? (gathered ? cl[lane] : cb + lane) : ce;
     CellStat<R> st_nx{};
-    if (cj_nx < ce && cj_nx != ci) st_nx = a.st_in[cj_nx];
+    if (cj_nx < ce && cj_nx != ci) st_nx = a->st_in[cj_nx];
     while (c0 < nsrc) {  // wave-uniform: candidates in batches of at most kWaveCand
       int ncl = 0;
       while (c0 < nsrc && ncl + DPM_WAVE <= kWaveCand) {
@@ -458,7 +476,7 @@ __device__ void k3d_wstep_body(const Step3D<R>& a) {
         {
           const int k1 = c0 + DPM_WAVE + lane;
           cj_nx = k1 < nsrc ? (gathered ? cl[k1] : cb + k1) : ce;
-          if (cj_nx < ce && cj_nx != ci) st_nx = a.st_in[cj_nx];
+          if (cj_nx < ce && cj_nx != ci) st_nx = a->st_in[cj_nx];
         }
         bool cand = false;
         if (cj < ce && cj != ci) {
@@ -485,6 +503,14 @@ __device__ void k3d_wstep_body(const Step3D<R>& a) {
           const R rr = reach * R(1.0001f) + R(1e-6f);
           cand = cand || vdot(d, d) <= rr * rr;
         }
+        if (relist) {  // wave-uniform
+          const bool nr =
+              cj < ce && cj != ci && near_list_takes(sti, stj, pbc, L, invL, do_contact, do_adh, a->nl_skin);
+          const unsigned long long m = __ballot(nr);
+          const int slot = nnl + lanes_below(m);
+          if (nr && slot < kNearList) a->nl_idx[(size_t)ci * kNearList + slot] = cj;
+          nnl += __popcll(m);
+        }
         const unsigned long long cmask = __ballot(cand);
         if (cand) cl[ncl + lanes_below(cmask)] = cj;  // ascending
         ncl += __popcll(cmask);
@@ -494,7 +520,7 @@ __device__ void k3d_wstep_body(const Step3D<R>& a) {
       wave_lds_sync();
       for (int qc = 0; qc < ncl; qc++) {
         const int cj2 = cl[qc];
-        const CellStat<R> stj = a.st_in[cj2];
+        const CellStat<R> stj = a->st_in[cj2];
         // cell j's positions stay in registers through the list pass (lane l
         // holds vertices l, l + 64, ..., as its chunks of the pass); every
         // load is issued before the first use
@@ -506,9 +532,9 @@ __device__ void k3d_wstep_body(const Step3D<R>& a) {
             const int v = lane + k * DPM_WAVE;
             qx[k] = qy[k] = qz[k] = R(0);
             if (v < nv) {
-              qx[k] = a.xin[bj + v];
-              qy[k] = a.yin[bj + v];
-              qz[k] = a.zin[bj + v];
+              qx[k] = a->xin[bj + v];
+              qy[k] = a->yin[bj + v];
+              qz[k] = a->zin[bj + v];
             }
           }
         }
@@ -635,13 +661,13 @@ __device__ void k3d_wstep_body(const Step3D<R>& a) {
                     if (own_on) {
                       Fa = adhesion_term_near(dl, y, kh_f, inv_l0i_f, Fa);
                       cnt_own++;
-                      if (PROBE && a.p_adh_hash)
-                        atomicAdd(&a.p_adh_hash[2 * (base + il[iv])], vertex_key(pj.x, pj.y, pj.z));
+                      if (PROBE && a->p_adh_hash)
+                        atomicAdd(&a->p_adh_hash[2 * (base + il[iv])], vertex_key(pj.x, pj.y, pj.z));
                     }
                     if (rev_on) {
                       Fa = adhesion_term_near(dl, y, kh_f, inv_l0j_f, Fa);
-                      if (PROBE && a.p_adh_hash)
-                        atomicAdd(&a.p_adh_hash[2 * (base + il[iv]) + 1], vertex_key(pj.x, pj.y, pj.z));
+                      if (PROBE && a->p_adh_hash)
+                        atomicAdd(&a->p_adh_hash[2 * (base + il[iv]) + 1], vertex_key(pj.x, pj.y, pj.z));
                     }
                   }
                   continue;
@@ -650,12 +676,12 @@ __device__ void k3d_wstep_body(const Step3D<R>& a) {
               if (cut_own(d2)) {
                 Fa = vsub(Fa, adhesion_term(pj, Pv, nl, L, Kat, L0i, kh, inv_l0i));
                 cnt_own++;
-                if (PROBE && a.p_adh_hash) atomicAdd(&a.p_adh_hash[2 * (base + il[iv])], vertex_key(pj.x, pj.y, pj.z));
+                if (PROBE && a->p_adh_hash) atomicAdd(&a->p_adh_hash[2 * (base + il[iv])], vertex_key(pj.x, pj.y, pj.z));
               }
               if (cut_rev(d2r)) {
                 Fa = vadd(Fa, adhesion_term(Pv, pj, nr, L, Kat, L0j, kh, inv_l0j));
-                if (PROBE && a.p_adh_hash)
-                  atomicAdd(&a.p_adh_hash[2 * (base + il[iv]) + 1], vertex_key(pj.x, pj.y, pj.z));
+                if (PROBE && a->p_adh_hash)
+                  atomicAdd(&a->p_adh_hash[2 * (base + il[iv]) + 1], vertex_key(pj.x, pj.y, pj.z));
               }
             }
             ut[sl * nmine + iv] = Q4<R>{Fa.x, Fa.y, Fa.z, (R)cnt_own};
@@ -673,7 +699,7 @@ __device__ void k3d_wstep_body(const Step3D<R>& a) {
             fx[v] = F.x;
             fy[v] = F.y;
             fz[v] = F.z;
-            if (PROBE && a.p_adh) a.p_adh[base + v] += cnt_own;
+            if (PROBE && a->p_adh) a->p_adh[base + v] += cnt_own;
           }
         }
         // Contact: a point at least m_j from every face of cell j has winding
@@ -681,7 +707,7 @@ __device__ void k3d_wstep_body(const Step3D<R>& a) {
         // separation; it stages cell j's whole mesh.
         if (do_contact && any_need && !(gap >= mj)) {  // wave-uniform
           wave_lds_sync();
-          wave_stage_cell(nx, ny, nz, a.xin, a.yin, a.zin, (size_t)cj2 * nv, nv, lane);
+          wave_stage_cell(nx, ny, nz, a->xin, a->yin, a->zin, (size_t)cj2 * nv, nv, lane);
           wave_lds_sync();
           #pragma unroll 1
           for (int k0v = 0; k0v < nv; k0v += DPM_WAVE) {
@@ -706,8 +732,8 @@ __device__ void k3d_wstep_body(const Step3D<R>& a) {
               if (lane == bb) wk = w;
             }
             if (need) {
-              const size_t pidx = (base + v) * (size_t)a.ncmax + (size_t)(cj2 - cb);
-              if (PROBE && a.p_winding) a.p_winding[pidx] = (float)wk;
+              const size_t pidx = (base + v) * (size_t)a->ncmax + (size_t)(cj2 - cb);
+              if (PROBE && a->p_winding) a->p_winding[pidx] = (float)wk;
               if (!(fabs(wk) < R(1e-6f))) {
                 const V3<R> dir = vnormalize(vsub(Ci, P));
                 const R mag = fabs(wk) * R(0.5f) * Kre;
@@ -716,26 +742,26 @@ __device__ void k3d_wstep_body(const Step3D<R>& a) {
                 fy[v] = F.y;
                 fz[v] = F.z;
                 n_contact++;
-                if (a.w_out) a.w_out[base + v] += fabs(wk);
-                if (a.rec_cell) {  // the first free of the vertex's partner slots
+                if (a->w_out) a->w_out[base + v] += fabs(wk);
+                if (a->rec_cell) {  // the first free of the vertex's partner slots
                   const size_t r0 = (base + v) * DPM3D_MAXPART;
                   int q = 0;
-                  while (q < DPM3D_MAXPART && a.rec_cell[r0 + q] >= 0) q++;
+                  while (q < DPM3D_MAXPART && a->rec_cell[r0 + q] >= 0) q++;
                   if (q < DPM3D_MAXPART) {
                     const size_t r = r0 + q;
-                    a.rec_cell[r] = cj2;
-                    a.rec_w[r] = wk;
-                    a.rec_shift[3 * r] = sh.x;
-                    a.rec_shift[3 * r + 1] = sh.y;
-                    a.rec_shift[3 * r + 2] = sh.z;
+                    a->rec_cell[r] = cj2;
+                    a->rec_w[r] = wk;
+                    a->rec_shift[3 * r] = sh.x;
+                    a->rec_shift[3 * r + 1] = sh.y;
+                    a->rec_shift[3 * r + 2] = sh.z;
                   } else {
-                    atomicOr(a.rec_overflow, 1);
+                    atomicOr(a->rec_overflow, 1);
                   }
                 }
-                if (PROBE && a.p_contact) a.p_contact[pidx] = 1;
-                if (PROBE && a.p_contact_key) {  // count, then key sum of the partner cells
-                  atomicAdd(&a.p_contact_key[2 * (base + v)], 1u);
-                  atomicAdd(&a.p_contact_key[2 * (base + v) + 1], cell_key(cj2 - cb));
+                if (PROBE && a->p_contact) a->p_contact[pidx] = 1;
+                if (PROBE && a->p_contact_key) {  // count, then key sum of the partner cells
+                  atomicAdd(&a->p_contact_key[2 * (base + v)], 1u);
+                  atomicAdd(&a->p_contact_key[2 * (base + v) + 1], cell_key(cj2 - cb));
                 }
               }
             }
@@ -744,36 +770,42 @@ __device__ void k3d_wstep_body(const Step3D<R>& a) {
         wave_lds_sync();  // the candidate arrays are rewritten next
       }
     }
+    if (relist && lane == 0) {
+      a->nl_cnt[ci] = nnl <= kNearList ? nnl : -1;
+      a->nl_ref[ci] = sti;
+    }
   }
+
+  step_args_again<R>(a);
 
   // ------------------------------------------------------- Euler and stats
   double px = 0.0, py = 0.0, pz = 0.0;
   #pragma unroll 1
   for (int v = lane; v < nv; v += DPM_WAVE) {
     const V3<R> F = lds_v(fx, fy, fz, v);
-    if (a.flags & F_WRITE_FORCES) {
-      a.fx[base + v] = F.x;
-      a.fy[base + v] = F.y;
-      a.fz[base + v] = F.z;
+    if (a->flags & F_WRITE_FORCES) {
+      a->fx[base + v] = F.x;
+      a->fy[base + v] = F.y;
+      a->fz[base + v] = F.z;
     }
-    if (a.flags & F_MOVE) {
+    if (a->flags & F_MOVE) {
       const V3<R> P = lds_v(sx, sy, sz, v);
       V3<R> Pn;
-      if (a.xlo) {
+      if (a->xlo) {
         // x + lo + F dt, the displacement rounded once onto the residual
         R ex, ey, ez;
-        Pn = v3(two_sum(P.x, fma(F.x, a.dt, a.xlo[base + v]), ex),
-                two_sum(P.y, fma(F.y, a.dt, a.ylo[base + v]), ey),
-                two_sum(P.z, fma(F.z, a.dt, a.zlo[base + v]), ez));
-        a.xlo[base + v] = ex;
-        a.ylo[base + v] = ey;
-        a.zlo[base + v] = ez;
+        Pn = v3(two_sum(P.x, fma(F.x, a->dt, a->xlo[base + v]), ex),
+                two_sum(P.y, fma(F.y, a->dt, a->ylo[base + v]), ey),
+                two_sum(P.z, fma(F.z, a->dt, a->zlo[base + v]), ez));
+        a->xlo[base + v] = ex;
+        a->ylo[base + v] = ey;
+        a->zlo[base + v] = ez;
       } else {
-        Pn = v3(fma(F.x, a.dt, P.x), fma(F.y, a.dt, P.y), fma(F.z, a.dt, P.z));
+        Pn = v3(fma(F.x, a->dt, P.x), fma(F.y, a->dt, P.y), fma(F.z, a->dt, P.z));
       }
-      a.xout[base + v] = Pn.x;
-      a.yout[base + v] = Pn.y;
-      a.zout[base + v] = Pn.z;
+      a->xout[base + v] = Pn.x;
+      a->yout[base + v] = Pn.y;
+      a->zout[base + v] = Pn.z;
       sx[v] = Pn.x;
       sy[v] = Pn.y;
       sz[v] = Pn.z;
@@ -782,7 +814,7 @@ __device__ void k3d_wstep_body(const Step3D<R>& a) {
       pz += (double)Pn.z;
     }
   }
-  if (a.flags & F_MOVE) {  // wave-uniform: statistics for the next step (cell_stats)
+  if (a->flags & F_MOVE) {  // wave-uniform: statistics for the next step (cell_stats)
     wave_lds_sync();
     px = wsum_all(px);
     py = wsum_all(py);
@@ -812,16 +844,22 @@ __device__ void k3d_wstep_body(const Step3D<R>& a) {
     vol = wsum_all(vol);
     if (lane == 0) {
       const R em = sqrt((R)e2d) * R(1.000001f);
-      a.st_out[ci] = make_cell_stat<R>(C.x, C.y, C.z, (R)rd * R(1.0000005f) + R(1e-30f), em, l0i);
-      a.vol_out[ci] = fabs(vol / 6.0);
-      a.em_out[ci] = em;
+      const CellStat<R> stn = make_cell_stat<R>(C.x, C.y, C.z, (R)rd * R(1.0000005f) + R(1e-30f), em, l0i);
+      a->st_out[ci] = stn;
+      if (nl_on) {
+        CellStat<R> ref = sti;
+        if (!relist) ref = a->nl_ref[ci];
+        if (near_list_moved(ref, C, stn.r, stn.em, a->nl_skin)) a->nl_stale_out[t] = 1;
+      }
+      a->vol_out[ci] = fabs(vol / 6.0);
+      a->em_out[ci] = em;
     }
   }
-  if (a.counters) {
+  if (a->counters) {
     // n_contact counts this lane's contacts; n_wind and n_cand are wave totals
     const unsigned long long c = (unsigned long long)wsum_all((double)n_contact);
     if (lane == 0) {
-      unsigned long long* slot = a.counters + 4 * ((blockIdx.x * cpw + wv) % DPM_COUNTER_SLOTS);
+      unsigned long long* slot = a->counters + 4 * ((blockIdx.x * cpw + wv) % DPM_COUNTER_SLOTS);
       if (ci == 0) atomicAdd(&slot[0], 1ull);
       if (n_wind) atomicAdd(&slot[1], (unsigned long long)n_wind);
       if (c) atomicAdd(&slot[2], c);
@@ -831,15 +869,15 @@ __device__ void k3d_wstep_body(const Step3D<R>& a) {
 }
 
 extern "C" __global__ void __launch_bounds__(256, 4) k3d_wstep_f32(const Step3D<float> a) {
-  k3d_wstep_body<float, 0, 0>(a);
+  k3d_wstep_body<float, 0, 0>();
 }
 // the icosphere of subdivision 2 (162 vertices, 320 faces); the production
 // instance has the diagnostic outputs compiled out (their registers would
 // spill), the _probe instance of the same source records them
 extern "C" __global__ void __launch_bounds__(256, 4) k3d_wstep_f32_v162(const Step3D<float> a) {
-  k3d_wstep_body<float, 162, 320, false>(a);
+  k3d_wstep_body<float, 162, 320, false>();
 }
 extern "C" __global__ void __launch_bounds__(256, 4) k3d_wstep_f32_v162_probe(const Step3D<float> a) {
-  k3d_wstep_body<float, 162, 320, true>(a);
+  k3d_wstep_body<float, 162, 320, true>();
 }
-extern "C" __global__ void __launch_bounds__(256) k3d_wstep_f64(const Step3D<double> a) { k3d_wstep_body<double, 0, 0>(a); }
+extern "C" __global__ void __launch_bounds__(256) k3d_wstep_f64(const Step3D<double> a) { k3d_wstep_body<double, 0, 0>(); }

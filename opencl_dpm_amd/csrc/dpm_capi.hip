@@ -69,8 +69,13 @@ int max_lds_per_block(int dev) {
 // Steps replayed per hipGraph launch (even, so the position ping-pong ends
 // where it started).
 constexpr int kGraphSteps = 64;
+// cells of a handle's largest tissue above which it keeps candidate lists
+// (us per step, scan | lists: 256 cells of 162 vertices 24.2 | 25.2, 1024 of 642
+// in double 190 | 169, 4096 of 642 542 | 390; not timed in between)
+constexpr int kNearListFrom = 512;
 // reals per cell of the cached cell statistics (CellStat)
 constexpr int kStatWords = (int)(sizeof(CellStat<float>) / sizeof(float));
+static_assert(kGraphSteps % 4 == 0, "a step graph ends on the list marks it starts from");
 static_assert(sizeof(CellStat<double>) == kStatWords * sizeof(double), "CellStat layout");
 
 }  // namespace
@@ -141,6 +146,14 @@ struct dpm_tissue {
   int *bin_start = nullptr, *bin_list = nullptr, *tbin_nb = nullptr, *tbin_nbuck = nullptr,
       *tbin_hoff = nullptr;
   size_t bin_lds = 0;
+  // candidate lists (see dpm3d.hip): tissues over one wave of cells; the set
+  // of marks the next step reads (its parity follows cur); valid until the
+  // positions or a parameter change
+  int *nl_cnt = nullptr, *nl_idx = nullptr, *nl_stale = nullptr;  // marks: [4 * T]
+  void* nl_ref = nullptr;
+  float nl_skin = 0.0f;
+  int nl_phase = 0;
+  bool nl_ok = false;
 
   // ------------------------------------------------------------------ 2D
   int V = 0, NT2 = 0, NTr = 0;  // Euler threads, relax threads per tissue
@@ -577,6 +590,13 @@ static int create3d(const dpm3d_desc* d, dpm_tissue** out, int rs) {
   rc |= A(&h->tbin_nb, (size_t)T);
   rc |= A(&h->tbin_nbuck, (size_t)T);
   rc |= A(&h->tbin_hoff, (size_t)T);
+  // where the scan costs more than the lists' two dependent loads
+  if (ncmax_t > kNearListFrom) {
+    rc |= A(&h->nl_cnt, (size_t)C);
+    rc |= A(&h->nl_idx, (size_t)C * kNearList);
+    rc |= A(&h->nl_stale, 4 * (size_t)T);
+    rc |= AR(&h->nl_ref, (size_t)C * kStatWords);
+  }
   if (rc) { delete h; return DPM_ENOMEM; }
   h->tissue_begin_h.assign(d->cell_begin, d->cell_begin + T + 1);
   h->faces_h.assign(d->faces, d->faces + 3 * nf);
@@ -592,10 +612,6 @@ static int create3d(const dpm3d_desc* d, dpm_tissue** out, int rs) {
   rc |= upload(h->adj, adj.data(), adj.size(), s);
   rc |= upload(h->tbin_nbuck, nbuck.data(), (size_t)T, s);
   rc |= upload(h->tbin_hoff, hoff.data(), (size_t)T, s);
-  // automatic: the cell list pays only where a cell would scan many chunks
-  // (at 4096 cells x 642 vertices it measured 2.57 ms against the scan's
-  // 2.43 ms per step)
-  h->cells_on = ncmax_t > 8 * h->NT;
   HIPCHECK(hipMemsetAsync(h->fx, 0, NVT * rs, s));
   HIPCHECK(hipMemsetAsync(h->fy, 0, NVT * rs, s));
   HIPCHECK(hipMemsetAsync(h->fz, 0, NVT * rs, s));
@@ -693,10 +709,12 @@ extern "C" float dpm3d_bin_width(dpm_tissue* h) { return h && h->dim == 3 ? h->b
 extern "C" int dpm3d_set_cell_list(dpm_tissue* h, int mode) {
   if (!h || h->dim != 3) return fail(DPM_EINVAL, "not a 3D tissue");
   if (mode < -1 || mode > 1) return fail(DPM_EINVAL, "mode must be -1 (automatic), 0 or 1");
-  int ncmax_t = 0;
-  for (int t = 0; t < h->T; t++) ncmax_t = std::max(ncmax_t, h->tissue_begin_h[t + 1] - h->tissue_begin_h[t]);
   h->cell_list_mode = mode;
-  h->cells_on = mode == 1 || (mode == -1 && ncmax_t > 8 * h->NT);
+  // automatic: the candidate lists make the scan rare (4096 cells of 642
+  // vertices: see kNearList), so the bins, made anew every step, are for
+  // programs that ask for them
+  h->cells_on = mode == 1;
+  h->nl_ok = false;  // steps with bins do not mind the lists
   if (h->graph) {  // captured with the old arguments
     (void)hipGraphExecDestroy(h->graph);
     h->graph = nullptr;
@@ -736,6 +754,12 @@ extern "C" int dpm3d_set_cell_params(dpm_tissue* h, const float* Kv, const float
   if (Ks) TRY(upload(h->Ks, Ks, C, s));
   if (Kb) TRY(upload(h->Kb, Kb, C, s));
   if (v0) TRY(upload(h->v0, v0, C, s));
+  h->nl_ok = false;
+  if (v0) {  // the skin: 0.15 radii of the smallest cell at rest
+    float vmin = v0[0];
+    for (int c = 1; c < C; c++) vmin = std::min(vmin, v0[c]);
+    h->nl_skin = 0.15f * std::cbrt(0.2387324f * vmin);
+  }
   if (a0) {
     TRY(upload(h->a0, a0, C, s));
     h->stats_valid = false;  // the cached statistics carry each cell's l0
@@ -760,6 +784,7 @@ extern "C" int dpm3d_set_tissue_params(dpm_tissue* h, const float* L, const int*
   if (Kat) TRY(upload(h->tKat, Kat, T, s));
   if (ks_grad) TRY(upload(h->tksg, ks_grad, T, s));
   h->mask = mask & DPM3D_ALL;
+  h->nl_ok = false;
   HIPCHECK(hipStreamSynchronize(s));
   if (h->graph) {
     (void)hipGraphExecDestroy(h->graph);
@@ -784,7 +809,7 @@ static int set_positions3(dpm_tissue* h, const In* xyz, size_t n) {
   };
   TRY(h->rs == 8 ? put(0.0) : put(0.0f));
   h->cur = k;
-  h->stats_valid = false;
+  h->stats_valid = h->nl_ok = false;
   return DPM_OK;
 }
 
@@ -991,11 +1016,45 @@ static int ensure_stats(dpm_tissue* h) {
   return DPM_OK;
 }
 
-static int launch_step3d(dpm_tissue* h, int in, float dt, int flags) {
-  return launch3d(h, K_STEP, in, dt, flags, [](auto&) {});
+// The lists' marks: stale for the next step, which reads set `phase`.
+__global__ void k_lists_stale(int* marks, int T, int phase) {
+  for (int i = threadIdx.x; i < 4 * T; i += blockDim.x) marks[i] = i / T == phase;
 }
 
-// A graph of kGraphSteps steps starting from buffer 0 (ends on buffer 0).
+static int ensure_lists(dpm_tissue* h) {
+  if (!h->nl_cnt || (h->nl_ok && (h->nl_phase & 1) == h->cur)) return DPM_OK;
+  h->nl_phase = h->cur;
+  k_lists_stale<<<1, 256, 0, h->stream>>>(h->nl_stale, h->T, h->nl_phase);
+  HIPCHECK(hipGetLastError());
+  h->nl_ok = true;
+  return DPM_OK;
+}
+
+// One step from buffer `in`; phase: the set of list marks it reads.
+static int launch_step3d(dpm_tissue* h, int in, int phase, float dt, int flags) {
+  return launch3d(h, K_STEP, in, dt, flags, [&](auto& a) {
+    if (!h->nl_cnt) return;
+    using S = std::remove_reference_t<decltype(*a.nl_ref)>;
+    a.nl_cnt = h->nl_cnt;
+    a.nl_idx = h->nl_idx;
+    a.nl_ref = (S*)h->nl_ref;
+    a.nl_stale = h->nl_stale + (size_t)phase * h->T;
+    a.nl_stale_out = h->nl_stale + (size_t)((phase + 1) & 3) * h->T;
+    a.nl_stale_clear = h->nl_stale + (size_t)((phase + 2) & 3) * h->T;
+    a.nl_skin = h->nl_skin;
+  });
+}
+
+// The handle's next step (after ensure_stats and ensure_lists).
+static int next_step3d(dpm_tissue* h, float dt, int flags) {
+  TRY(launch_step3d(h, h->cur, h->nl_phase, dt, flags));
+  h->cur = 1 - h->cur;
+  h->nl_phase = (h->nl_phase + 1) & 3;
+  return DPM_OK;
+}
+
+// A graph of kGraphSteps steps starting from buffer 0 and list marks 0 (ends
+// there: kGraphSteps is a multiple of 4).
 static int build_graph3d(dpm_tissue* h, float dt) {
   if (h->graph) {
     (void)hipGraphExecDestroy(h->graph);
@@ -1004,7 +1063,7 @@ static int build_graph3d(dpm_tissue* h, float dt) {
   hipGraph_t g = nullptr;
   HIPCHECK(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
   int rc = DPM_OK;
-  for (int s = 0; s < kGraphSteps && !rc; s++) rc = launch_step3d(h, s & 1, dt, F_MOVE);
+  for (int s = 0; s < kGraphSteps && !rc; s++) rc = launch_step3d(h, s & 1, s & 3, dt, F_MOVE);
   hipError_t e = hipStreamEndCapture(h->stream, &g);
   if (rc) {
     if (g) (void)hipGraphDestroy(g);
@@ -1028,28 +1087,18 @@ static int euler3d(dpm_tissue* h, int nsteps, float dt) {
   // the step graph for this dt is captured on the first call with it (a
   // capture launches nothing), so that later calls replay it
   if (!h->graph || h->graph_dt != dt) TRY(build_graph3d(h, dt));
+  TRY(ensure_lists(h));
   int left = nsteps - 1;  // the last step also writes the forces
   if (left >= kGraphSteps) {
-    // Bring the ping-pong to buffer 0 so that the graph (captured from 0)
-    // applies.
-    if (h->cur != 0) {
-      TRY(launch_step3d(h, h->cur, dt, F_MOVE));
-      h->cur = 1 - h->cur;
+    // Bring the buffers and the lists' marks to 0, where the graph starts.
+    while (left >= kGraphSteps && (h->cur != 0 || (h->nl_cnt && h->nl_phase != 0))) {
+      TRY(next_step3d(h, dt, F_MOVE));
       left--;
     }
-    if (left >= kGraphSteps) {
-      while (left >= kGraphSteps) {
-        HIPCHECK(hipGraphLaunch(h->graph, h->stream));
-        left -= kGraphSteps;
-      }
-    }
+    for (; left >= kGraphSteps; left -= kGraphSteps) HIPCHECK(hipGraphLaunch(h->graph, h->stream));
   }
-  for (; left > 0; left--) {
-    TRY(launch_step3d(h, h->cur, dt, F_MOVE));
-    h->cur = 1 - h->cur;
-  }
-  TRY(launch_step3d(h, h->cur, dt, F_MOVE | F_WRITE_FORCES));
-  h->cur = 1 - h->cur;
+  for (; left > 0; left--) TRY(next_step3d(h, dt, F_MOVE));
+  TRY(next_step3d(h, dt, F_MOVE | F_WRITE_FORCES));
   h->forces_valid = true;
   return DPM_OK;
 }
@@ -1123,15 +1172,15 @@ extern "C" int dpm3d_autotune(dpm_tissue* h, int steps, float dt, int* best, flo
       for (int rep = 0; rep < 2 && !rc; rep++) {  // a warm-up launch, then the timed steps
         rc = copy_all(false);
         if (rc) break;
+        h->nl_ok = false;  // the state was restored
+        rc = ensure_lists(h);
+        if (rc) break;
         if (rep == 0) {
-          rc = launch_step3d(h, h->cur, dt, F_MOVE);
+          rc = launch_step3d(h, h->cur, h->nl_phase, dt, F_MOVE);
           continue;
         }
         if (hipEventRecord(e0, h->stream) != hipSuccess) rc = fail(DPM_EDEVICE, "hipEventRecord failed");
-        for (int k = 0; k < steps && !rc; k++) {
-          rc = launch_step3d(h, h->cur, dt, F_MOVE);
-          h->cur = 1 - h->cur;
-        }
+        for (int k = 0; k < steps && !rc; k++) rc = next_step3d(h, dt, F_MOVE);
         if (!rc && (hipEventRecord(e1, h->stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess))
           rc = fail(DPM_EDEVICE, "timing failed");
         float ms = 0.0f;
@@ -1151,6 +1200,7 @@ extern "C" int dpm3d_autotune(dpm_tissue* h, int steps, float dt, int* best, flo
   if (e0) (void)hipEventDestroy(e0);
   if (e1) (void)hipEventDestroy(e1);
   int rc2 = copy_all(false);
+  h->nl_ok = false;
   if (!rc && rc2) rc = rc2;
   if (hipStreamSynchronize(h->stream) != hipSuccess && !rc) rc = fail(DPM_EDEVICE, "stream sync failed");
   (void)hipFree(save);
@@ -1609,7 +1659,7 @@ static int adjoint3d(dpm_tissue* h, const In* lambda_final, double* dtheta, Out*
     TRY(copy_positions_dd(h, h->x[0], h->y[0], h->z[0], c, slot(h, c, 1), slot(h, c, 2)));
     if (h->lo)
       HIPCHECK(hipMemcpyAsync(h->lo, slot(h, c, 3), 3 * NVT * h->rs, hipMemcpyDeviceToDevice, h->stream));
-    h->stats_valid = false;
+    h->stats_valid = h->nl_ok = false;
     TRY(ensure_stats(h));
     for (int s = 0; s < every; s++) {
       void* xs = slot(h, h->seg, 3 * (size_t)s);
@@ -1652,7 +1702,7 @@ static int adjoint3d(dpm_tissue* h, const In* lambda_final, double* dtheta, Out*
   TRY(copy_positions_dd(h, h->x[0], h->y[0], h->z[0], last, slot(h, last, 1), slot(h, last, 2)));
   if (h->lo)
     HIPCHECK(hipMemcpyAsync(h->lo, slot(h, last, 3), 3 * NVT * h->rs, hipMemcpyDeviceToDevice, h->stream));
-  h->stats_valid = false;
+  h->stats_valid = h->nl_ok = false;
   if (dtheta)
     HIPCHECK(hipMemcpyAsync(dtheta, h->gtheta, sizeof(double) * h->C * 4, hipMemcpyDeviceToHost, h->stream));
   if (lambda0) TRY(download3(h, h->lam, slot(h, h->lam, 1), slot(h, h->lam, 2), lambda0, NVT));
