@@ -798,739 +798,6 @@ __device__ void k3d_stats_body(const Step3D<R>& a) {
   cell_stats(l, a.nv, a.nf, a.st_out, a.vol_out, a.em_out, ci, cell_l0<R>(a.a0, ci));
 }
 
-// Winding number of point p about the staged cell (l.nx/ny/nz shifted by sh),
-// evaluated by one wave: lanes normalise the directions to the cell's
-// vertices once into this wave's LDS table (the same bits a per-face
-// normalisation gives, so every face's `denom < 1e-8` decision is the
-// reference order's), then split the faces.  The sum is reduced in double.
-template <typename R>
-__device__ __forceinline__ R winding_wave(const Lds3D<R>& l, Q4<R>* ut, int nv, int nf, V3<R> sh,
-                                          V3<R> p) {
-  const int lane = threadIdx.x & (DPM_WAVE - 1);
-  for (int v = lane; v < nv; v += DPM_WAVE) {
-    // Verts + shift - point, in the reference's order (Cell3D_Kernel.cl:285-287)
-    const V3<R> A = {(l.nx[v] + sh.x) - p.x, (l.ny[v] + sh.y) - p.y, (l.nz[v] + sh.z) - p.z};
-    const V3<R> u = vnormalize(A);
-    ut[v] = Q4<R>{u.x, u.y, u.z, R(0)};
-  }
-  wave_lds_sync();
-  R part = R(0);
-  for (int f = lane; f < nf; f += DPM_WAVE) {
-    int ia, ib, ic;
-    face_of(l, f, ia, ib, ic);
-    const Q4<R> ua = ut[ia], ub = ut[ib], uc = ut[ic];
-    const V3<R> u = {ua.x, ua.y, ua.z};
-    const V3<R> v = {ub.x, ub.y, ub.z};
-    const V3<R> w = {uc.x, uc.y, uc.z};
-    const R denom = ((R(1) + vdot(u, v)) + vdot(v, w)) + vdot(w, u);
-    if (denom < R(1e-8f)) continue;
-    const R num = vdot(u, vcross(v, w));
-    part += R(2) * atan2(num, denom);
-  }
-  const double tot = wave_sum_d((double)part);  // every lane (DPP tree)
-  wave_lds_sync();  // this wave's table reads finish before it is rewritten
-  return (R)(tot / (double)(R(4) * R(3.14159265358979323846)));
-}
-
-// One overdamped Euler step of every cell (or, without F_MOVE, one force
-// evaluation for diagnostics).  blockDim.x >= nv, a multiple of 64.
-// NVC, NFC, NTC, WWC: vertex and face counts, threads per workgroup and
-// winding waves fixed at compile time (0: taken from the arguments).
-template <typename R, int NVC, int NFC, int NTC, int WWC, bool PROBE = true>
-__device__ void k3d_step_body() {
-  Step3DArgs<R>* a = step_args_here<R>();
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int nv = NVC > 0 ? NVC : a->nv, nf = NFC > 0 ? NFC : a->nf, NT = NTC > 0 ? NTC : (int)blockDim.x, tid = threadIdx.x;
-  const int ww = WWC > 0 ? WWC : a->ww;
-  const int lane = tid & (DPM_WAVE - 1), wave = tid / DPM_WAVE;
-  const int ci = xcd_remap(blockIdx.x, gridDim.x);
-  Lds3D<R> l = carve3d<R>(smem, nv, nf, NT, ww);
-
-  const int t = a->cell_tissue[ci];
-  const int cb = a->tissue_begin[t], ce = a->tissue_begin[t + 1];
-  const R L = (R)a->tL[t];
-  const int pbc = a->tpbc[t];
-  const R Kre = (R)a->tKre[t], Kat = (R)a->tKat[t], ksg = (R)a->tksg[t];
-  const CellStat<R> sti = a->st_in[ci];
-  const V3<R> Ci = {sti.cx, sti.cy, sti.cz};
-  const R Ri = sti.r;
-  const R Kvi = (R)a->Kv[ci], Kai = (R)a->Ka[ci], Ksi = (R)a->Ks[ci], Kbi = (R)a->Kb[ci];
-  const R v0i = (R)a->v0[ci], a0i = (R)a->a0[ci], l0i = cell_l0<R>(a->a0, ci);
-  const unsigned mask = a->mask;
-  const size_t base = (size_t)ci * nv;
-  const bool own = tid < nv;
-  const V3<R> zero = {R(0), R(0), R(0)};
-
-  // candidate lists: made by this step, or read (nlist entries; not when
-  // there are more than a list holds)
-  const bool nl_on = a->nl_cnt && !a->bin_list;  // block-uniform
-  const bool relist = nl_on && a->nl_stale[t] != 0;
-  const int nlist = nl_on && !relist ? a->nl_cnt[ci] : -1;
-  const bool listed = nlist >= 0;
-  CellStat<R> nl_ref = sti;  // where this step makes the lists
-  if (nl_on && !relist) nl_ref = a->nl_ref[ci];
-
-  // per-vertex topology rows in registers
-  int vfr[DPM3D_MAXDEG], adjr[DPM3D_MAXDEG];
-#pragma unroll
-  for (int k = 0; k < DPM3D_MAXDEG; k++) {
-    vfr[k] = own ? a->vf[tid * DPM3D_MAXDEG + k] : -1;
-    adjr[k] = own ? a->adj[tid * DPM3D_MAXDEG + k] : -1;
-  }
-  // The candidate scan's statistics (every cell of a tissue of at most NT
-  // cells, no cell list) are loaded here with the cell's own data, one
-  // memory round trip for both (float instances with compile-time sizes; in
-  // the others the registers held until the scan would spill).
-  const bool scan_pre = (sizeof(R) == 4 && NTC > 0) &&
-                        (((mask & M_CONTACT) && Kre != R(0)) || ((mask & M_ADHESION) && Kat != R(0)));
-  const bool scan_all = scan_pre && !listed && !(a->bin_list && a->tbin_nb[t] > 0) && ce - cb <= NT;  // block-uniform
-  CellStat<R> st_pre{};
-  if (scan_all && tid < ce - cb) st_pre = a->st_in[cb + tid];
-  if constexpr (NFC > 0 && NVC > 0 && NTC > 0) {
-    // compile-time sizes: every load in flight before the first LDS store
-    static_assert(NFC <= 2 * NTC, "at most two faces per thread");
-    const int f0 = tid, f1 = tid + NTC;
-    int a0 = 0, b0 = 0, e0 = 0, a1 = 0, b1 = 0, e1 = 0;
-    if (f0 < NFC) {
-      a0 = a->faces[3 * f0];
-      b0 = a->faces[3 * f0 + 1];
-      e0 = a->faces[3 * f0 + 2];
-    }
-    if (f1 < NFC) {
-      a1 = a->faces[3 * f1];
-      b1 = a->faces[3 * f1 + 1];
-      e1 = a->faces[3 * f1 + 2];
-    }
-    R px = R(0), py = R(0), pz = R(0);
-    if (own) {
-      px = a->xin[base + tid];
-      py = a->yin[base + tid];
-      pz = a->zin[base + tid];
-    }
-    if (f0 < NFC) l.sf[f0] = make_uint2((unsigned)a0 | ((unsigned)b0 << 16), (unsigned)e0);
-    if (f1 < NFC) l.sf[f1] = make_uint2((unsigned)a1 | ((unsigned)b1 << 16), (unsigned)e1);
-    if (own) {
-      l.sx[tid] = px;
-      l.sy[tid] = py;
-      l.sz[tid] = pz;
-    }
-  } else {
-    stage_topology(*a, l);
-    load_own(*a, l, base);
-  }
-  __syncthreads();
-
-  const V3<R> P = own ? lds_v(l.sx, l.sy, l.sz, tid) : zero;
-  V3<R> F = zero;
-  bool ring_done = false;  // shape forces by the ring walk (bending's first sum in ring_sb)
-  V3<R> ring_sb = zero;
-
-  step_args_again<R>(a);
-
-  // ---------------------------------------------------------- shape forces
-  // Per-face pass: each face's volume, edge-spring and substrate terms for
-  // its three corners are computed once into LDS; every vertex then gathers
-  // its incident (face, corner) entries in ascending face order.
-  if (mask & (M_VOLUME | M_SURFACE | M_SUBSTRATE)) {  // block-uniform
-    // Volume strain of the current volume, in double (the residual V/v0 - 1
-    // cancels when the cell is near its target).
-    const R strain = (R)(a->vol_in[ci] / (double)v0i - 1.0);
-    const R kvol = -Kvi * strain / R(6);
-    const bool vol_on = (mask & M_VOLUME) && Kvi != R(0);
-    const bool surf_on = (mask & M_SURFACE) && !(Kai < R(1e-8f));
-    const bool sub_on = (mask & M_SUBSTRATE) && !(Ksi < R(1e-12f));
-    const R sc = Kai * sqrt(a0i) / l0i * R(0.3f);
-    const R inv_l0 = R(1) / l0i;
-    const double sub_inv_l0 = 1.0 / (double)l0i;
-    if ((sizeof(R) == 4 || NTC > 0) && a->closed) {  // block-uniform
-      // Closed mesh, neighbour rows in ring order (face q is (v, u_q, u_(q+1))):
-      // one walk around each vertex's ring, as the wave-per-cell step takes
-      // it — volume kvol sum_q d_q x d_(q+1), edge springs 2 sc sum_q s(d_q),
-      // bending's first sum, substrate per facing-down incident face.  A
-      // ring edge shorter than 2e-12 (the reference skips such faces'
-      // springs) sends the cell back to the face pass below.  Float steps
-      // and the compile-time-sized instances only: in the general double
-      // kernel (128 registers at 1024 threads) the walk's registers push
-      // the rest of the step into spills (measured 5 % slower on 4096 x 642
-      // cells), and the face pass stays.
-      unsigned* dbits = reinterpret_cast<unsigned*>(l.fcx);  // dead until the candidates
-      if (sub_on) {
-        for (int f0 = wave * DPM_WAVE; f0 < nf; f0 += NT) {  // 64 consecutive faces per wave
-          const int f = f0 + lane;
-          bool dn = false;
-          if (f < nf) {
-            int i0, i1, i2;
-            face_of(l, f, i0, i1, i2);
-            const V3<R> P0 = lds_v(l.sx, l.sy, l.sz, i0);
-            dn = facing_down(vcross(vsub(lds_v(l.sx, l.sy, l.sz, i1), P0), vsub(lds_v(l.sx, l.sy, l.sz, i2), P0)));
-            if (PROBE && dn && a->p_down) a->p_down[(size_t)ci * nf + f] = 1;
-          }
-          const unsigned long long m = __ballot(dn);
-          if (lane == 0) {
-            dbits[f0 / 32] = (unsigned)m;
-            if (f0 / 32 + 1 < (nf + 31) / 32) dbits[f0 / 32 + 1] = (unsigned)(m >> 32);
-          }
-        }
-        __syncthreads();
-      }
-      bool bad = false;
-      V3<R> Fr = zero;
-      if (own) {
-        // (Force arithmetic, its products fused into FMAs; the short-edge
-        // test keeps a factor 2 of margin to the reference's 1e-12 cut.)
-        const V3<R> d0 = vsub(lds_v(l.sx, l.sy, l.sz, adjr[0]), P);
-        V3<R> dq = d0, Fv = zero, Fs = zero, sb = zero;
-#pragma unroll
-        for (int q = 0; q < DPM3D_MAXDEG; q++) {
-          if (surf_on) {
-            const R d2 = vdot_f(dq, dq);
-            bad = bad || d2 < R(4e-24f);
-            Fs = vmadd_f(dq, spring_factor(d2, inv_l0), Fs);
-          }
-          sb = vadd(sb, dq);
-          const int un = q + 1 < DPM3D_MAXDEG ? adjr[q + 1] : -1;
-          const V3<R> dn = un < 0 ? d0 : vsub(lds_v(l.sx, l.sy, l.sz, un), P);
-          if (vol_on) Fv = vcross_add_f(dq, dn, Fv);
-          if (un < 0) break;
-          dq = dn;
-        }
-        Fr = vadd(vscale(Fv, kvol), vscale(Fs, R(2) * sc));
-        ring_sb = sb;
-        if (sub_on) {
-          int ndown = 0;
-#pragma unroll
-          for (int k = 0; k < DPM3D_MAXDEG; k++) {
-            const int e = vfr[k];  // face*3 + corner
-            if (e < 0) break;
-            const int f = e / 3;
-            ndown += (dbits[f >> 5] >> (f & 31)) & 1u;
-          }
-          if (ndown) Fr = vadd(Fr, vscale(substrate_corner(P, Ci, Ksi, ksg, L, l0i, sub_inv_l0), (R)ndown));
-        }
-      }
-      ring_done = !__syncthreads_or(bad);  // also: every facing-down bit read
-      if (ring_done) F = Fr;
-    }
-    for (int f = tid; f < nf && !ring_done; f += NT) {
-      int i0, i1, i2;
-      face_of(l, f, i0, i1, i2);
-      const V3<R> P0 = lds_v(l.sx, l.sy, l.sz, i0);
-      const V3<R> P1 = lds_v(l.sx, l.sy, l.sz, i1);
-      const V3<R> P2 = lds_v(l.sx, l.sy, l.sz, i2);
-      V3<R> c0 = zero, c1 = zero, c2 = zero;
-      if (vol_on) {  // Cell3D_Kernel.cl:95-111
-        const V3<R> A = vsub(P1, Ci), B = vsub(P2, Ci), Cc = vsub(P0, Ci);
-        c0 = vscale(vcross(A, B), kvol);
-        c1 = vscale(vcross(B, Cc), kvol);
-        c2 = vscale(vcross(Cc, A), kvol);
-      }
-      if (surf_on) {  // Cell3D_Kernel.cl:140-176
-        const V3<R> lv0 = vsub(P1, P0), lv1 = vsub(P2, P1), lv2 = vsub(P0, P2);
-        const R len0 = sqrt(vdot(lv0, lv0)), len1 = sqrt(vdot(lv1, lv1)), len2 = sqrt(vdot(lv2, lv2));
-        if (!(len0 < R(1e-12f) || len1 < R(1e-12f) || len2 < R(1e-12f))) {
-          const V3<R> e0 = vscale(lv0, (len0 * inv_l0 - R(1)) / len0);
-          const V3<R> e1 = vscale(lv1, (len1 * inv_l0 - R(1)) / len1);
-          const V3<R> e2 = vscale(lv2, (len2 * inv_l0 - R(1)) / len2);
-          c0 = vadd(c0, vscale(vsub(e0, e2), sc));
-          c1 = vadd(c1, vscale(vsub(e1, e0), sc));
-          c2 = vadd(c2, vscale(vsub(e2, e1), sc));
-        }
-      }
-      if (sub_on) {  // Cell3D_Kernel.cl:206-246
-        const V3<R> un = vnormalize(vcross(vsub(P1, P0), vsub(P2, P0)));
-        if (un.z < R(-0.1f)) {
-          if (PROBE && a->p_down) a->p_down[(size_t)ci * nf + f] = 1;
-          c0 = vadd(c0, substrate_corner(P0, Ci, Ksi, ksg, L, l0i, sub_inv_l0));
-          c1 = vadd(c1, substrate_corner(P1, Ci, Ksi, ksg, L, l0i, sub_inv_l0));
-          c2 = vadd(c2, substrate_corner(P2, Ci, Ksi, ksg, L, l0i, sub_inv_l0));
-        }
-      }
-      l.fcx[3 * f] = c0.x;
-      l.fcy[3 * f] = c0.y;
-      l.fcz[3 * f] = c0.z;
-      l.fcx[3 * f + 1] = c1.x;
-      l.fcy[3 * f + 1] = c1.y;
-      l.fcz[3 * f + 1] = c1.z;
-      l.fcx[3 * f + 2] = c2.x;
-      l.fcy[3 * f + 2] = c2.y;
-      l.fcz[3 * f + 2] = c2.z;
-    }
-    if (!ring_done) {  // block-uniform
-      __syncthreads();
-      if (own) {
-#pragma unroll
-        for (int k = 0; k < DPM3D_MAXDEG; k++) {
-          const int e = vfr[k];  // face*3 + corner
-          if (e < 0) break;
-          F = vadd(F, V3<R>{l.fcx[e], l.fcy[e], l.fcz[e]});
-        }
-      }
-      __syncthreads();  // the shape-force bytes are reused below
-    }
-  }
-
-  // --------------------------------------------------------------- bending
-  if ((mask & M_BENDING) && Kbi != R(0)) {  // block-uniform
-    if (own) {
-      V3<R> s = zero;
-      if (ring_done) {
-        s = ring_sb;
-      } else {
-#pragma unroll
-        for (int k = 0; k < DPM3D_MAXDEG; k++) {
-          const int u = adjr[k];
-          if (u < 0) break;
-          s = vadd(s, vsub(lds_v(l.sx, l.sy, l.sz, u), P));
-        }
-      }
-      l.sb[3 * tid] = s.x;
-      l.sb[3 * tid + 1] = s.y;
-      l.sb[3 * tid + 2] = s.z;
-    }
-    __syncthreads();
-    if (own) {
-      V3<R> acc = zero;
-      int deg = 0;
-#pragma unroll
-      for (int k = 0; k < DPM3D_MAXDEG; k++) {
-        const int u = adjr[k];
-        if (u < 0) break;
-        deg++;
-        acc = vadd(acc, V3<R>{l.sb[3 * u], l.sb[3 * u + 1], l.sb[3 * u + 2]});
-      }
-      const V3<R> sv = {l.sb[3 * tid], l.sb[3 * tid + 1], l.sb[3 * tid + 2]};
-      const V3<R> lap = vsub(acc, vscale(sv, (R)deg));
-      F = vadd(F, vscale(lap, -Kbi));
-    }
-  }
-
-  step_args_again<R>(a);
-
-  // ------------------------------------------- contact and vertex adhesion
-  const bool do_contact = (mask & M_CONTACT) && Kre != R(0);
-  const bool do_adh = (mask & M_ADHESION) && Kat != R(0);
-  unsigned long long n_wind = 0, n_contact = 0, n_cand = 0;
-  R wsum = R(0);  // the contact force is wsum * Kre/2 * normalize(C_i - p)
-  int npart = 0;
-  if (do_contact || do_adh) {  // block-uniform
-    const R L0i = fmax(l0i, R(1e-12f));
-    const R invL = R(1) / L;
-    Q4<R>* ut = l.utab + (size_t)wave * nv;
-    // candidate source: every cell of the tissue in order, or the cells of
-    // the 27 buckets around this cell, sorted by index (block-uniform)
-    const int* src = nullptr;
-    int nsrc = ce - cb;
-    if (a->bin_list && a->tbin_nb[t] > 0) {
-      const int nb = a->tbin_nb[t], nbuck = a->tbin_nbuck[t];
-      const int* bs = a->bin_start + a->tbin_hoff[t];
-      const R wb = L / (R)nb;
-      int* gid = l.gath;        // [27] bucket ids
-      int* gst = l.gath + 32;   // [27] bucket starts
-      int* gof = l.gath + 64;   // [28] prefix of bucket sizes
-      if (tid < DPM_WAVE) {  // the whole first wave: distinct buckets, their cells' offsets
-        int g = 0;
-        if (tid < 27) {
-          const int bx = bin_coord(Ci.x, L, wb, nb), by = bin_coord(Ci.y, L, wb, nb),
-                    bz = bin_coord(Ci.z, L, wb, nb);
-          const int dx = tid % 3 - 1, dy = (tid / 3) % 3 - 1, dz = tid / 9 - 1;
-          g = (int)bin_bucket((bx + dx + nb) % nb, (by + dy + nb) % nb, (bz + dz + nb) % nb, nb, nbuck);
-        }
-        const int nu = distinct_buckets27(g, bs, gst, gof);
-        if (tid == 0) gid[31] = nu;
-      }
-      __syncthreads();
-      const int nu = gid[31], n = gof[nu];
-      if (n <= NT) {  // block-uniform; otherwise scan every cell
-        if (tid < n) {
-          int u = 0;
-          while (gof[u + 1] <= tid) u++;
-          l.glist[tid] = a->bin_list[cb + gst[u] + (tid - gof[u])];
-        }
-        __syncthreads();
-        if (tid < n) {  // rank sort (indices are distinct)
-          const int v = l.glist[tid];
-          int r = 0;
-          for (int u = 0; u < n; u++) r += l.glist[u] < v;
-          l.clist[r] = v;
-        }
-        __syncthreads();
-        if (tid < n) l.glist[tid] = l.clist[tid];
-        __syncthreads();
-        src = l.glist;
-        nsrc = n;
-      }
-    }
-    if (listed) {  // at most 64 entries: one chunk
-      src = a->nl_idx + (size_t)ci * kNearList;
-      nsrc = nlist;
-    }
-    int nnl = 0;  // entries of the list being made
-    for (int c0 = 0; c0 < nsrc; c0 += NT) {
-      const int k = c0 + tid;
-      const int cj = k < nsrc ? (src ? src[k] : cb + k) : ce;
-      bool cand = false;
-      CellStat<R> stj{};
-      if (cj < ce && cj != ci) {
-        if (scan_all && c0 == 0)
-          stj = st_pre;
-        else
-          stj = a->st_in[cj];
-        V3<R> sh = zero;
-        if (pbc)
-          sh = v3(image_shift(Ci.x - stj.cx, L, invL), image_shift(Ci.y - stj.cy, L, invL),
-                  image_shift(Ci.z - stj.cz, L, invL));
-        const V3<R> d = {stj.cx + sh.x - Ci.x, stj.cy + sh.y - Ci.y, stj.cz + sh.z - Ci.z};
-        R reach = R(0);
-        if (do_contact) reach = Ri + stj.r + contact_margin(stj.r, stj.em);
-        if (do_adh) {
-          const R l0m = fmax(L0i, fmax(stj.l0, R(1e-12f)));
-          const R r2 = Ri + stj.r + R(2) * l0m;
-          reach = fmax(reach, r2);
-          // Adhesion takes the minimum image per vertex pair
-          // (Cell3D_Kernel.cl:341-346), which can differ from the
-          // centre-of-mass image when the box is small: then no culling.
-          if (pbc && R(2) * r2 >= R(0.999f) * L) cand = true;
-        }
-        const R rr = reach * R(1.0001f) + R(1e-6f);
-        cand = cand || vdot(d, d) <= rr * rr;
-      }
-      if (relist) {  // block-uniform
-        const bool nr = cj < ce && cj != ci && near_list_takes(sti, stj, pbc, L, invL, do_contact, do_adh, a->nl_skin);
-        const int n = block_compact(nr, cj, l.plist, l.cnt);
-        if (tid < n && nnl + tid < kNearList) a->nl_idx[(size_t)ci * kNearList + nnl + tid] = l.plist[tid];
-        nnl += n;
-        __syncthreads();  // the compaction's arrays are written again next
-      }
-      const int ncand = block_compact_with(cand, cj, l.clist, l.cnt, [&](int slot) {
-        if (slot < kCandStats) l.cst[slot] = stj;
-      });
-      n_cand += ncand;
-      // candidate q's statistics (wave-uniform q)
-      auto cand_stat = [&](int q) { return q < kCandStats ? l.cst[q] : a->st_in[l.clist[q]]; };
-      // Separation along the centre line n = (C_j - C_i) / D (float steps
-      // and the compile-time-sized instances): every vertex p of this cell
-      // has (p - C_i).n <= hi and every point x of cell j's (shifted) hull
-      // has (C_j - x).n <= hj, so |x - p| >= D - hi - hj, less slack for the
-      // float sums (1e-4 of the cells' extent, 1e-6 of the coordinates).
-      // Contact needs a point closer than the culling margin m_j to a face
-      // of j (contact_margin), adhesion a vertex pair closer than 2 l0 — on
-      // pairs that take no periodic image (the unshifted centres and radii
-      // keep every component below 0.48 L; the shift is 0 then).  The waves
-      // take the candidates in turn (maxima by wave shuffles, cell j's
-      // vertices read from the L2), so the bound costs no workgroup barrier
-      // per candidate; the candidates that need neither pass are dropped
-      // and the rest keep their two bits (1 contact, 2 adhesion) above bit
-      // 28 of their entry.  In the general double kernel the extra
-      // registers cost more than the skipped work (spills, measured on
-      // 4096 x 642 cells), and every candidate takes both passes.
-      // the candidates that take a pass: entries q | passes << 28 (q the
-      // index in l.clist, passes 1 contact, 2 adhesion)
-      int nkeep = ncand;
-      const int* keep = nullptr;
-      bool flagged = false;
-      if constexpr (sizeof(R) == 4 || NTC > 0) {
-        const int nwaves = NT / DPM_WAVE;
-        for (int q = wave; q < ncand; q += nwaves) {  // wave-uniform
-          const int cjq = l.clist[q];
-          const CellStat<R> stj = cand_stat(q);
-          V3<R> sh = zero;
-          if (pbc)
-            sh = v3(image_shift(Ci.x - stj.cx, L, invL), image_shift(Ci.y - stj.cy, L, invL),
-                    image_shift(Ci.z - stj.cz, L, invL));
-          const V3<R> Cj = {stj.cx + sh.x, stj.cy + sh.y, stj.cz + sh.z};
-          const R l0m = fmax(L0i, fmax(stj.l0, R(1e-12f)));
-          const bool all_images = pbc && R(2) * (Ri + stj.r + R(2) * l0m) >= R(0.999f) * L;
-          const bool no_image = !pbc || (fabs(Ci.x - stj.cx) + (Ri + stj.r) < R(0.48f) * L &&
-                                         fabs(Ci.y - stj.cy) + (Ri + stj.r) < R(0.48f) * L &&
-                                         fabs(Ci.z - stj.cz) + (Ri + stj.r) < R(0.48f) * L);
-          const V3<R> dC = vsub(Cj, Ci);
-          const R D = sqrt(vdot(dC, dC));
-          const V3<R> nC = D > R(0) ? vscale(dC, R(1) / D) : zero;
-          R hi = R(-3.0e38f), hj = R(-3.0e38f);
-          const size_t bj = (size_t)cjq * nv;
-          for (int v = lane; v < nv; v += DPM_WAVE) {
-            hi = fmax(hi, vdot(vsub(lds_v(l.sx, l.sy, l.sz, v), Ci), nC));
-            hj = fmax(hj, vdot(v3(stj.cx - a->xin[bj + v], stj.cy - a->yin[bj + v], stj.cz - a->zin[bj + v]), nC));
-          }
-          hi = wave_max_all(hi);
-          hj = wave_max_all(hj);
-          bool skip_contact = false, skip_adh = false;
-          const R Mc = ((fabs(Ci.x) + fabs(Ci.y)) + fabs(Ci.z)) + ((fabs(Cj.x) + fabs(Cj.y)) + fabs(Cj.z));
-          if (D > R(0)) {
-            const R gap = ((D - hi) - hj) - (R(1e-4f) * ((Ri + stj.r) + D) + R(1e-6f) * Mc);
-            skip_contact = gap >= contact_margin(stj.r, stj.em);
-            skip_adh = !all_images && no_image && gap >= R(2) * l0m;
-          }
-          const int bits = ((do_contact && !skip_contact) ? 1 : 0) | ((do_adh && !skip_adh) ? 2 : 0);
-          if (lane == 0) l.plist[q] = q | (bits << 28);
-        }
-        __syncthreads();
-        const int ent = tid < ncand ? l.plist[tid] : 0;
-        nkeep = block_compact(tid < ncand && (ent >> 28) != 0, ent, l.glist, l.cnt);
-        keep = l.glist;
-        flagged = true;
-      }
-      // each thread stages one vertex (NT >= nv) of a kept candidate; the
-      // next candidate's vertex is loaded while the current one is processed
-      auto entry = [&](int qq) { return flagged ? keep[qq] : (qq | (3 << 28)); };
-      V3<R> pre = zero;
-      if (nkeep > 0 && own) {
-        const size_t b0 = (size_t)l.clist[entry(0) & 0x0fffffff] * nv + tid;
-        pre = v3(a->xin[b0], a->yin[b0], a->zin[b0]);
-      }
-      for (int qq = 0; qq < nkeep; qq++) {
-        const int ent = entry(qq);
-        const int q = ent & 0x0fffffff;
-        const int cj2 = l.clist[q];
-        const int passes = ent >> 28;
-        const CellStat<R> stj = cand_stat(q);
-        V3<R> sh = zero;
-        if (pbc)
-          sh = v3(image_shift(Ci.x - stj.cx, L, invL), image_shift(Ci.y - stj.cy, L, invL),
-                  image_shift(Ci.z - stj.cz, L, invL));
-        if (own) {
-          l.nx[tid] = pre.x;
-          l.ny[tid] = pre.y;
-          l.nz[tid] = pre.z;
-        }
-        __syncthreads();
-        if (qq + 1 < nkeep && own) {
-          const size_t b1 = (size_t)l.clist[entry(qq + 1) & 0x0fffffff] * nv + tid;
-          pre = v3(a->xin[b1], a->yin[b1], a->zin[b1]);
-        }
-        const bool skip_contact = !(passes & 1), skip_adh = !(passes & 2);
-        if (do_contact && !skip_contact) {  // block-uniform
-          const V3<R> Cj = {stj.cx + sh.x, stj.cy + sh.y, stj.cz + sh.z};
-          const R mj = contact_margin(stj.r, stj.em);
-          const R rj = (stj.r + mj) * R(1.0001f) + R(1e-6f);
-          bool need = false;
-          if (own) {
-            const V3<R> d = vsub(P, Cj);
-            const R d2 = vdot(d, d);
-            need = d2 <= rj * rj;
-          }
-          const int np = block_compact(need, tid, l.plist, l.cnt);
-          if (wave < ww) {
-            for (int pi = wave; pi < np; pi += ww) {  // wave-uniform
-              const int v = l.plist[pi];
-              const V3<R> Pv = lds_v(l.sx, l.sy, l.sz, v);
-              // a point beyond the margin from j's hull has winding number 0
-              R wv = R(0);
-              if (!outside_by_margin(l.nx, l.ny, l.nz, nv, stj.cx, stj.cy, stj.cz, Cj, vsub(Pv, Cj), mj, stj.r)) {
-                wv = winding_wave(l, ut, nv, nf, sh, Pv);
-                if (lane == 0) n_wind++;
-              }
-              if (lane == 0) l.wb[v] = wv;
-            }
-          }
-          __syncthreads();
-          if (need) {
-            const R wv = l.wb[tid];
-            const size_t pidx = (base + tid) * (size_t)a->ncmax + (size_t)(cj2 - cb);
-            if (PROBE && a->p_winding) a->p_winding[pidx] = (float)wv;
-            if (!(fabs(wv) < R(1e-6f))) {
-              const V3<R> dir = vnormalize(vsub(Ci, P));
-              const R mag = fabs(wv) * R(0.5f) * Kre;
-              F = vadd(F, vscale(dir, mag));
-              n_contact++;
-              wsum += fabs(wv);
-              if (a->rec_cell) {
-                if (npart < DPM3D_MAXPART) {
-                  const size_t r = (base + tid) * DPM3D_MAXPART + npart;
-                  a->rec_cell[r] = cj2;
-                  a->rec_w[r] = wv;
-                  a->rec_shift[3 * r] = sh.x;
-                  a->rec_shift[3 * r + 1] = sh.y;
-                  a->rec_shift[3 * r + 2] = sh.z;
-                } else {
-                  atomicOr(a->rec_overflow, 1);
-                }
-                npart++;
-              }
-              if (PROBE && a->p_contact) a->p_contact[pidx] = 1;
-              if (PROBE && a->p_contact_key) {  // count, then key sum of the partner cells
-                atomicAdd(&a->p_contact_key[2 * (base + tid)], 1u);
-                atomicAdd(&a->p_contact_key[2 * (base + tid) + 1], cell_key(cj2 - cb));
-              }
-            }
-          }
-        }
-        const R L0j = fmax(stj.l0, R(1e-12f));
-        const R l0m = fmax(L0i, L0j);
-        const bool all_images = pbc && R(2) * (Ri + stj.r + R(2) * l0m) >= R(0.999f) * L;
-        if (do_adh && !skip_adh) {  // block-uniform
-          // Vertices of cell j within reach of this cell (a pair closer than
-          // 2 l0 has |q - Ci| <= |q - p| + |p - Ci| < 2 l0 + Ri) and vertices
-          // of this cell within reach of cell j, the same bound reversed.
-          bool near = false, mine = false;
-          if (own) {
-            const V3<R> ds = {l.nx[tid] + sh.x - Ci.x, l.ny[tid] + sh.y - Ci.y, l.nz[tid] + sh.z - Ci.z};
-            const R rk = (Ri + R(2) * l0m) * R(1.0001f) + R(1e-6f);
-            near = all_images || vdot(ds, ds) <= rk * rk;
-            const V3<R> dp = {P.x - stj.cx - sh.x, P.y - stj.cy - sh.y, P.z - stj.cz - sh.z};
-            const R r2 = (stj.r + R(2) * l0m) * R(1.0001f) + R(1e-6f);
-            mine = all_images || vdot(dp, dp) <= r2 * r2;
-          }
-          int nnear = 0, nmine = 0, slot = 0;
-          int* jl = l.plist;
-          int* il = l.plist + NT;
-          block_compact2(near, tid, jl, mine, tid, il, l.cnt, nnear, nmine, slot);
-          if (nnear > 0 && nmine > 0) {  // block-uniform
-            // (own vertex, slice of near vertices) per thread; each thread
-            // sums its slice in order into LDS, then every own vertex adds
-            // its slices in order: deterministic, every lane busy.
-            const int S = max(1, min(nnear, NT / nmine));
-            const int per = (nnear + S - 1) / S;
-            const int iv = tid % nmine, sl = tid / nmine;
-            Q4<R>* acc = l.utab;
-            if (sl < S) {
-              const V3<R> Pv = lds_v(l.sx, l.sy, l.sz, il[iv]);
-              V3<R> Fa = zero;
-              int cnt_own = 0;
-              const R half_l = R(0.49f) * L;
-              const AdhCut<R> cut_own(L0i * R(2)), cut_rev(L0j * R(2));
-              const double kh = 0.5 * (double)Kat, inv_l0i = sti.inv_l0, inv_l0j = stj.inv_l0;
-              const float kh_f = (float)kh, inv_l0i_f = (float)inv_l0i, inv_l0j_f = (float)inv_l0j;
-              const int m1 = min(nnear, (sl + 1) * per);
-              for (int m = sl * per; m < m1; m++) {
-                const int vj = jl[m];
-                const V3<R> pj = lds_v(l.nx, l.ny, l.nz, vj);
-                // the own vertex's loop: delta = pj - p, minimum image per
-                // component (Cell3D_Kernel.cl:341-346); a component below
-                // 0.49 L rounds to image 0, which leaves it unchanged.
-                V3<R> dl = vsub(pj, Pv);
-                V3<R> dr = vsub(Pv, pj);  // the partner's loop: delta = p - pj
-                V3<R> nl = zero, nr = zero;  // image indices
-                bool imaged = false;
-                if (pbc && !(fabs(dl.x) < half_l && fabs(dl.y) < half_l && fabs(dl.z) < half_l)) {
-                  nl = v3(round(dl.x / L), round(dl.y / L), round(dl.z / L));
-                  nr = v3(round(dr.x / L), round(dr.y / L), round(dr.z / L));
-                  dl = vsub(dl, v3(L * nl.x, L * nl.y, L * nl.z));
-                  dr = vsub(dr, v3(L * nr.x, L * nr.y, L * nr.z));
-                  imaged = true;
-                }
-                // The decisions are the reference's ones (AdhCut).  The force
-                // of an accepted pair across the periodic boundary is
-                // evaluated in double on the same image, since there the
-                // float difference of two near-L numbers keeps few digits of a
-                // short vector; without an image (dr = -dl exactly, the same
-                // squared distance) a float step takes it in float
-                // (adhesion_term_near).
-                const R d2 = vdot(dl, dl);
-                if constexpr (sizeof(R) == 4) {
-                  if (!imaged) {
-                    const bool own_on = cut_own(d2), rev_on = cut_rev(d2);
-                    if (own_on || rev_on) {
-                      const R y = __builtin_amdgcn_rsqf(d2);
-                      if (own_on) {
-                        Fa = adhesion_term_near(dl, y, kh_f, inv_l0i_f, Fa);
-                        cnt_own++;
-                        if (PROBE && a->p_adh_hash)
-                          atomicAdd(&a->p_adh_hash[2 * (base + il[iv])], vertex_key(pj.x, pj.y, pj.z));
-                      }
-                      if (rev_on) {
-                        Fa = adhesion_term_near(dl, y, kh_f, inv_l0j_f, Fa);
-                        if (PROBE && a->p_adh_hash)
-                          atomicAdd(&a->p_adh_hash[2 * (base + il[iv]) + 1], vertex_key(pj.x, pj.y, pj.z));
-                      }
-                    }
-                    continue;
-                  }
-                }
-                if (cut_own(d2)) {
-                  Fa = vsub(Fa, adhesion_term(pj, Pv, nl, L, Kat, L0i, kh, inv_l0i));
-                  cnt_own++;
-                  if (PROBE && a->p_adh_hash) atomicAdd(&a->p_adh_hash[2 * (base + il[iv])], vertex_key(pj.x, pj.y, pj.z));
-                }
-                const R d2r = vdot(dr, dr);
-                if (cut_rev(d2r)) {
-                  Fa = vadd(Fa, adhesion_term(Pv, pj, nr, L, Kat, L0j, kh, inv_l0j));
-                  if (PROBE && a->p_adh_hash)
-                    atomicAdd(&a->p_adh_hash[2 * (base + il[iv]) + 1], vertex_key(pj.x, pj.y, pj.z));
-                }
-              }
-              acc[sl * nmine + iv] = Q4<R>{Fa.x, Fa.y, Fa.z, (R)cnt_own};
-            }
-            __syncthreads();
-            if (mine) {
-              int cnt_own = 0;
-              for (int s2 = 0; s2 < S; s2++) {
-                const Q4<R> q4 = acc[s2 * nmine + slot];
-                F = vadd(F, V3<R>{q4.x, q4.y, q4.z});
-                cnt_own += (int)q4.w;
-              }
-              if (PROBE && a->p_adh) a->p_adh[base + tid] += cnt_own;
-            }
-          }
-        }
-        __syncthreads();
-      }
-    }
-    if (relist && tid == 0) {
-      a->nl_cnt[ci] = nnl <= kNearList ? nnl : -1;
-      a->nl_ref[ci] = sti;
-    }
-  }
-  if (a->nl_cnt && ci == cb && tid == 0) a->nl_stale_clear[t] = 0;
-
-  step_args_again<R>(a);
-
-  // ------------------------------------------------------- Euler and stats
-  if (own && a->w_out) a->w_out[base + tid] = wsum;
-  if (own && a->rec_cell)
-    for (int q = npart; q < DPM3D_MAXPART; q++) a->rec_cell[(base + tid) * DPM3D_MAXPART + q] = -1;
-  if (own && (a->flags & F_WRITE_FORCES)) {
-    a->fx[base + tid] = F.x;
-    a->fy[base + tid] = F.y;
-    a->fz[base + tid] = F.z;
-  }
-  if (a->flags & F_MOVE) {  // block-uniform
-    V3<R> Pn = P;
-    if (own) {
-      if (a->xlo) {
-        // x + lo + F dt, the displacement rounded once onto the residual
-        R ex, ey, ez;
-        Pn = v3(two_sum(P.x, fma(F.x, a->dt, a->xlo[base + tid]), ex),
-                two_sum(P.y, fma(F.y, a->dt, a->ylo[base + tid]), ey),
-                two_sum(P.z, fma(F.z, a->dt, a->zlo[base + tid]), ez));
-        a->xlo[base + tid] = ex;
-        a->ylo[base + tid] = ey;
-        a->zlo[base + tid] = ez;
-      } else {
-        Pn = v3(fma(F.x, a->dt, P.x), fma(F.y, a->dt, P.y), fma(F.z, a->dt, P.z));
-      }
-      a->xout[base + tid] = Pn.x;
-      a->yout[base + tid] = Pn.y;
-      a->zout[base + tid] = Pn.z;
-    }
-    __syncthreads();  // every read of the step's positions is done
-    if (own) {
-      l.sx[tid] = Pn.x;
-      l.sy[tid] = Pn.y;
-      l.sz[tid] = Pn.z;
-    }
-    const CellStat<R> stn = cell_stats_own(l, nv, nf, a->st_out, a->vol_out, a->em_out, ci, l0i, own, Pn);
-    if (nl_on && tid == 0 && near_list_moved(nl_ref, v3(stn.cx, stn.cy, stn.cz), stn.r, stn.em, a->nl_skin))
-      a->nl_stale_out[t] = 1;
-  }
-  if (a->counters) {
-    // per wave, without a workgroup barrier: the wave's contact count, its
-    // winding count (kept by lane 0), and the candidates (every thread holds
-    // the workgroup's count; wave 0 adds it).  Spread over
-    // DPM_COUNTER_SLOTS slots so that workgroups do not serialise on one
-    // address; the host sums the slots.
-    unsigned long long c = n_contact;
-    for (int o = 32; o > 0; o >>= 1) c += __shfl_down(c, o, DPM_WAVE);
-    if (lane == 0) {
-      unsigned long long* slot = a->counters + 4 * ((blockIdx.x * (NT / DPM_WAVE) + wave) % DPM_COUNTER_SLOTS);
-      if (blockIdx.x == 0 && wave == 0) atomicAdd(&slot[0], 1ull);
-      if (n_wind) atomicAdd(&slot[1], n_wind);
-      if (c) atomicAdd(&slot[2], c);
-      if (wave == 0 && n_cand) atomicAdd(&slot[3], n_cand);
-    }
-  }
-}
-
 // Elastic energy of each cell at the current positions, all in double
 // (centre of mass and volume included, so that a float tissue's energy is
 // exact for its float positions): the energies whose negative gradients are
@@ -1990,23 +1257,6 @@ __device__ void k3d_vjp_body(const Vjp3D<R>& a) {
 
 extern "C" __global__ void __launch_bounds__(1024) k3d_stats_f32(const Step3D<float> a) { k3d_stats_body(a); }
 extern "C" __global__ void __launch_bounds__(1024) k3d_stats_f64(const Step3D<double> a) { k3d_stats_body(a); }
-extern "C" __global__ void __launch_bounds__(1024) k3d_step_f32(const Step3D<float> a) { k3d_step_body<float, 0, 0, 0, 0>(); }
-extern "C" __global__ void __launch_bounds__(1024) k3d_step_f64(const Step3D<double> a) { k3d_step_body<double, 0, 0, 0, 0>(); }
-// Instances for the icospheres of subdivision 2 and 3 (162 / 642 vertices):
-// sizes, workgroup size and winding waves fixed at compile time, so LDS
-// offsets are immediates and the register budget is that of 256 or 704
-// threads instead of 1024 (the general kernel spills at 128 registers).
-// The host takes them where the handle's nv, nf, NT and ww match.
-extern "C" __global__ void __launch_bounds__(256) k3d_step_f32_v162(const Step3D<float> a) {
-  k3d_step_body<float, 162, 320, 256, 4, false>();
-}
-// the same with the diagnostic outputs (dpm3d_probe*) compiled in
-extern "C" __global__ void __launch_bounds__(256) k3d_step_f32_v162_probe(const Step3D<float> a) {
-  k3d_step_body<float, 162, 320, 256, 4, true>();
-}
-extern "C" __global__ void __launch_bounds__(704) k3d_step_f32_v642(const Step3D<float> a) { k3d_step_body<float, 642, 1280, 704, 4>(); }
-extern "C" __global__ void __launch_bounds__(704) k3d_step_f64_v642(const Step3D<double> a) { k3d_step_body<double, 642, 1280, 704, 2>(); }
-extern "C" __global__ void __launch_bounds__(256) k3d_step_f64_v162(const Step3D<double> a) { k3d_step_body<double, 162, 320, 256, 4>(); }
 extern "C" __global__ void __launch_bounds__(1024) k3d_energy_f32(const Step3D<float> a) { k3d_energy_body(a); }
 extern "C" __global__ void __launch_bounds__(1024) k3d_energy_f64(const Step3D<double> a) { k3d_energy_body(a); }
 // lambda += dt * (contributions from other cells), contributions cleared.

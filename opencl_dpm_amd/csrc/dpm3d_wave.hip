@@ -152,7 +152,7 @@ __device__ __forceinline__ R winding_w(const R* nx, const R* ny, const R* nz, co
 // rolled: unrolled, their iterations' registers spill to scratch memory
 // (208 B per lane, 6x the step's HBM traffic, at the same speed).
 template <typename R, int NVC, int NFC, bool PROBE = true>
-__device__ void k3d_wstep_body() {
+__device__ __forceinline__ void k3d_wstep_body() {
   Step3DArgs<R>* a = step_args_here<R>();
   extern __shared__ __align__(16) unsigned char smem[];
   const int nv = NVC > 0 ? NVC : a->nv, nf = NFC > 0 ? NFC : a->nf;
@@ -204,7 +204,7 @@ __device__ void k3d_wstep_body() {
   const V3<R> zero = {R(0), R(0), R(0)};
   // candidate lists: made by this step, or read (nlist entries; not when
   // there are more than a list holds); wave-uniform
-  const bool nl_on = a->nl_cnt && !a->bin_list;
+  const bool nl_on = a->nl_cnt && !a->bin_list && ce - cb > kNearList;
   const bool relist = nl_on && a->nl_stale[t] != 0;
   const int nlist = nl_on && !relist ? a->nl_cnt[ci] : -1;
   if (a->nl_cnt && ci == cb && lane == 0) a->nl_stale_clear[t] = 0;

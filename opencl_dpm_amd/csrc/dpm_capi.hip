@@ -17,6 +17,7 @@
 #include "dpm2d.hip"
 #include "dpm3d.hip"
 #include "dpm3d_wave.hip"
+#include "dpm3d_group.hip"
 #include "dpm2d_wide.hip"
 #include "dpm_disperse.hip"
 #include "dpm_measures.hip"
@@ -112,6 +113,8 @@ struct dpm_tissue {
   void* wtopo = nullptr;  // LDS image of the wave form's shared topology
   int wtopo_n16 = 0;
   size_t lds_w = 0;
+  int ww_g = 1;      // workgroup-per-cell step: waves that take winding numbers, LDS
+  size_t lds_g = 0;
   unsigned mask = 0;
   int cur = 0;
   bool stats_valid = false;
@@ -418,6 +421,16 @@ static const void* wstep_kernel(int rs, int nv, int nf, bool probe = false) {
   return rs == 8 ? (const void*)k3d_wstep_f64 : (const void*)k3d_wstep_f32;
 }
 
+// The workgroup form's kernel for a handle.
+static const void* gstep_kernel(int rs, int nv, int nf, bool probe = false) {
+  if (nv == 162 && nf == 320)
+    return rs == 8 ? (const void*)k3d_step_f64_v162
+                   : probe ? (const void*)k3d_step_f32_v162_probe : (const void*)k3d_step_f32_v162;
+  if (nv == 642 && nf == 1280) return rs == 8 ? (const void*)k3d_step_f64_v642 : (const void*)k3d_step_f32_v642;
+  if (nv > kGrpThreads) return rs == 8 ? (const void*)k3d_step_f64_big : (const void*)k3d_step_f32_big;
+  return rs == 8 ? (const void*)k3d_step_f64 : (const void*)k3d_step_f32;
+}
+
 static int create3d(const dpm3d_desc* d, dpm_tissue** out, int rs) {
   if (!d || !out) return fail(DPM_EINVAL, "null argument");
   *out = nullptr;
@@ -532,6 +545,8 @@ static int create3d(const dpm3d_desc* d, dpm_tissue** out, int rs) {
   // table in LDS (at most ~48 KB of tables).
   h->ww = std::max(1, std::min(h->NT / 64, 49152 / (4 * rs * nv)));
   h->lds = lds3d_layout(nv, nf, h->NT, h->ww, rs).total;
+  h->ww_g = group_winding_waves(nv, rs);
+  h->lds_g = ldsg_layout(nv, nf, h->ww_g, rs).total;
   if ((int)h->lds > max_lds_per_block(h->device)) {
     delete h;
     return fail(DPM_ERANGE, "cell mesh does not fit the LDS of one workgroup");
@@ -627,18 +642,36 @@ static int create3d(const dpm3d_desc* d, dpm_tissue** out, int rs) {
   }
   if (!rc && hipStreamSynchronize(s) != hipSuccess) rc = fail(DPM_EDEVICE, "stream sync failed");
   if (rc) { delete h; return rc; }
-  const void* kern[2][3] = {{(const void*)k3d_step_f32, (const void*)k3d_stats_f32, (const void*)k3d_energy_f32},
-                            {(const void*)k3d_step_f64, (const void*)k3d_stats_f64, (const void*)k3d_energy_f64}};
+  const void* kern[2][2] = {{(const void*)k3d_stats_f32, (const void*)k3d_energy_f32},
+                            {(const void*)k3d_stats_f64, (const void*)k3d_energy_f64}};
   for (const void* k : kern[rs == 8 ? 1 : 0])
     (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->lds);
-  (void)hipFuncSetAttribute((const void*)k3d_step_f32_v162, hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->lds);
-  (void)hipFuncSetAttribute((const void*)k3d_step_f32_v162_probe, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)h->lds);
-  (void)hipFuncSetAttribute((const void*)k3d_step_f32_v642, hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->lds);
-  (void)hipFuncSetAttribute((const void*)k3d_step_f64_v642, hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->lds);
-  (void)hipFuncSetAttribute((const void*)k3d_step_f64_v162, hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->lds);
+  for (bool probe : {false, true})
+    (void)hipFuncSetAttribute(gstep_kernel(rs, nv, nf, probe), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)h->lds_g);
   (void)hipFuncSetAttribute(rs == 8 ? (const void*)k3d_bin_f64 : (const void*)k3d_bin_f32,
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->bin_lds);
+  // the step kernels' topology image: faces packed 10 bits per index (staged in
+  // LDS), incidence and neighbour rows of 16-bit entries (0xffff: none)
+  const Lds3DWave LW = ldsw_layout(nv, nf, 1, rs);
+  std::vector<unsigned char> img(LW.img, 0);
+  unsigned* pf = reinterpret_cast<unsigned*>(img.data());
+  for (int f = 0; f < nf; f++)
+    pf[f] = (unsigned)d->faces[3 * f] | ((unsigned)d->faces[3 * f + 1] << 10) |
+            ((unsigned)d->faces[3 * f + 2] << 20);
+  unsigned short* pv = reinterpret_cast<unsigned short*>(img.data() + LW.vf);
+  unsigned short* pa = reinterpret_cast<unsigned short*>(img.data() + LW.adj);
+  for (size_t i = 0; i < vf.size(); i++) {
+    pv[i] = (unsigned short)vf[i];
+    pa[i] = (unsigned short)adj[i];
+  }
+  h->wtopo_n16 = (int)(img.size() / 16);
+  unsigned char* q = nullptr;
+  if (h->alloc(&q, img.size()) || hipMemcpy(q, img.data(), img.size(), hipMemcpyHostToDevice) != hipSuccess) {
+    delete h;
+    return fail(DPM_EDEVICE, "topology upload failed");
+  }
+  h->wtopo = q;
   if (nv <= kWaveMaxNv) {  // cells per workgroup: as many as fit 64 KiB of LDS, at most 4
     int cpw = 4;
     while (cpw > 1 && ldsw_layout(nv, nf, cpw, rs).total > 65536) cpw /= 2;
@@ -657,27 +690,6 @@ static int create3d(const dpm3d_desc* d, dpm_tissue** out, int rs) {
       if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
       const int per_cu = nv > DPM_WAVE ? (rs == 8 ? 4 : 3) : (rs == 8 ? 0 : 2);
       h->wave_min_cells = per_cu * std::max(1, cus);
-      // the topology image: faces packed 10 bits per index (staged in
-      // LDS), incidence and neighbour rows of 16-bit entries (0xffff: none)
-      const Lds3DWave LW = ldsw_layout(nv, nf, cpw, rs);
-      std::vector<unsigned char> img(LW.img, 0);
-      unsigned* pf = reinterpret_cast<unsigned*>(img.data());
-      for (int f = 0; f < nf; f++)
-        pf[f] = (unsigned)d->faces[3 * f] | ((unsigned)d->faces[3 * f + 1] << 10) |
-                ((unsigned)d->faces[3 * f + 2] << 20);
-      unsigned short* pv = reinterpret_cast<unsigned short*>(img.data() + LW.vf);
-      unsigned short* pa = reinterpret_cast<unsigned short*>(img.data() + LW.adj);
-      for (size_t i = 0; i < vf.size(); i++) {
-        pv[i] = (unsigned short)vf[i];
-        pa[i] = (unsigned short)adj[i];
-      }
-      h->wtopo_n16 = (int)(img.size() / 16);
-      unsigned char* q = nullptr;
-      if (h->alloc(&q, img.size()) || hipMemcpy(q, img.data(), img.size(), hipMemcpyHostToDevice) != hipSuccess) {
-        delete h;
-        return fail(DPM_EDEVICE, "topology upload failed");
-      }
-      h->wtopo = q;
       for (bool probe : {false, true})
         (void)hipFuncSetAttribute(wstep_kernel(rs, nv, nf, probe), hipFuncAttributeMaxDynamicSharedMemorySize,
                                   (int)h->lds_w);
@@ -950,22 +962,8 @@ static int launch3d(dpm_tissue* h, Kind3D kind, int in, float dt, int flags, Edi
     using R = decltype(tag);
     Step3D<R> a = step_args<R>(h, in, dt, flags);
     edit(a);
-    void (*k)(Step3D<R>) = nullptr;
-    if constexpr (sizeof(R) == 8)
-      k = kind == K_STEP ? k3d_step_f64 : kind == K_STATS ? k3d_stats_f64 : k3d_energy_f64;
-    else
-      k = kind == K_STEP ? k3d_step_f32 : kind == K_STATS ? k3d_stats_f32 : k3d_energy_f32;
     // diagnostic outputs requested: the instances that record them
     const bool probe = a.p_contact || a.p_winding || a.p_down || a.p_adh || a.p_adh_hash || a.p_contact_key;
-    if constexpr (sizeof(R) == 4)
-      if (kind == K_STEP && h->ww == 4 && h->nv == 162 && h->nf == 320 && h->NT == 256)
-        k = probe ? k3d_step_f32_v162_probe : k3d_step_f32_v162;
-    if constexpr (sizeof(R) == 4)
-      if (kind == K_STEP && h->ww == 4 && h->nv == 642 && h->nf == 1280 && h->NT == 704) k = k3d_step_f32_v642;
-    if constexpr (sizeof(R) == 8)
-      if (kind == K_STEP && h->ww == 2 && h->nv == 642 && h->nf == 1280 && h->NT == 704) k = k3d_step_f64_v642;
-    if constexpr (sizeof(R) == 8)
-      if (kind == K_STEP && h->ww == 4 && h->nv == 162 && h->nf == 320 && h->NT == 256) k = k3d_step_f64_v162;
     if (kind == K_STEP && a.bin_list) {  // this step's cell list, from its input statistics
       Bin3D<R> b{};
       b.tissue_begin = h->tissue_begin;
@@ -993,7 +991,16 @@ static int launch3d(dpm_tissue* h, Kind3D kind, int in, float dt, int flags, Edi
       auto kw = reinterpret_cast<void (*)(Step3D<R>)>(const_cast<void*>(wstep_kernel(h->rs, h->nv, h->nf, probe)));
       hipLaunchKernelGGL(kw, dim3((h->C + h->wave_cpw - 1) / h->wave_cpw), dim3(64 * h->wave_cpw), h->lds_w,
                          h->stream, a);
+    } else if (kind == K_STEP) {
+      a.ww = h->ww_g;
+      auto kg = reinterpret_cast<void (*)(Step3D<R>)>(const_cast<void*>(gstep_kernel(h->rs, h->nv, h->nf, probe)));
+      hipLaunchKernelGGL(kg, dim3(h->C), dim3(kGrpThreads), h->lds_g, h->stream, a);
     } else {
+      void (*k)(Step3D<R>) = nullptr;
+      if constexpr (sizeof(R) == 8)
+        k = kind == K_STATS ? k3d_stats_f64 : k3d_energy_f64;
+      else
+        k = kind == K_STATS ? k3d_stats_f32 : k3d_energy_f32;
       hipLaunchKernelGGL(k, dim3(h->C), dim3(h->NT), h->lds, h->stream, a);
     }
     HIPCHECK(hipGetLastError());
