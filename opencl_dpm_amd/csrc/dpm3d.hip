@@ -118,6 +118,7 @@ struct Step3D {
   const int* vf;            // [nv*MAXDEG] incident (face*3 + corner), ascending, -1 pad
   const int* adj;           // [nv*MAXDEG] neighbour vertices (ring order if closed), -1 pad
   int nv, nf, ncells;
+  int one_tissue;  // ncells cells of tissue 0
   int closed;  // every edge on two faces, every vertex's faces one oriented cycle
   // the wave form's workgroup-shared topology, byte for byte its LDS image
   // (packed faces, 16-bit incidence and neighbour rows), in 16-byte words

@@ -15,8 +15,8 @@
 // registers filled a compute unit alone, and every barrier idled it.
 // Against one thread per vertex, a face pass of its own and five barriers per
 // candidate, us per step: 9 x 162 vertices 12.9 -> 9.9, 256 x 162 23.5 ->
-// 17.5, 4096 x 642 375 -> 175, in double 256 x 162 30.0 -> 24.6 and 1024 x 642
-// 158 -> 112.
+// 17.1, 4096 x 642 375 -> 133, in double 256 x 162 30.0 -> 23.7 and 1024 x 642
+// 158 -> 97.
 #pragma once
 
 constexpr int kGrpThreads = 256;
@@ -26,6 +26,7 @@ constexpr int kGrpSlots = 4;    // candidates whose vertex lists are kept at onc
 constexpr int kGrpCap = 64;     // entries of such a list
 constexpr int kGrpTasks = 512;  // partial sums of the adhesion pairs kept at once
 constexpr int kGrpSlices = 256;  // partial sums a candidate is cut into, at most
+static_assert(kGrpSlots == 4 && kGrpCap <= 127 && kGrpSlices <= kGrpTasks, "the task search and the records' fields");
 
 // LDS.  Three users of the last bytes, one after the other: the kept
 // candidates' lists and partial sums; a candidate taken by itself (its own
@@ -149,8 +150,13 @@ __device__ __forceinline__ void k3d_step_body() {
       arow[k] = rows[LT.adj / 16 + v];
     }
   }
-  const int t = a->cell_tissue[ci];
-  const int cb = a->tissue_begin[t], ce = a->tissue_begin[t + 1];
+  // (a handle of one tissue needs no look-up: two dependent loads less)
+  int t = 0, cb = 0, ce = a->ncells;
+  if (!a->one_tissue) {
+    t = a->cell_tissue[ci];
+    cb = a->tissue_begin[t];
+    ce = a->tissue_begin[t + 1];
+  }
   const R L = (R)a->tL[t];
   const int pbc = a->tpbc[t];
   const R Kre = (R)a->tKre[t], Kat = (R)a->tKat[t], ksg = (R)a->tksg[t];
@@ -350,13 +356,28 @@ __device__ __forceinline__ void k3d_step_body() {
   // centres and radii keep every component below 0.48 L; the shift is 0 then).
   // Lists: a pair closer than 2 l0 has |q - C_i| <= |q - p| + |p - C_i| <
   // 2 l0 + R_i, and the same bound reversed.
-  // rec: 1 contact | 2 adhesion | 4 the lists fit | near << 3 | own << 13.
+  // rec: 1 contact | 2 adhesion | 4 the lists fit, then near << 3 | own << 10
+  // | slices << 17 | near vertices per slice << 24 (each at most 64): the
+  // adhesion pairs are (own vertex, slice of near vertices) tasks, at most
+  // kGrpSlices of them.
   auto separate = [&](unsigned long long m) __attribute__((always_inline)) {
     int o = 0;
     for (unsigned long long w = m; w; w &= w - 1ull, o++) {
       if (o % kGrpWaves != wave) continue;  // wave-uniform
       const int b = __ffsll((long long)w) - 1;
       const int cjq = from_lane(cj_l, b);
+      const size_t bj = (size_t)cjq * nv;
+      constexpr int kAtOnce = 4;  // 64-vertex chunks whose loads are issued together
+      V3<R> q[kAtOnce];
+      auto load = [&](int v0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < kAtOnce; k++) {
+          const int v = v0 + k * DPM_WAVE + lane;
+          q[k] = zero;
+          if (v < nv) q[k] = v3(a->xin[bj + v], a->yin[bj + v], a->zin[bj + v]);
+        }
+      };
+      load(0);
       const CellStat<R> stj = from_lane(st_l, b);
       V3<R> sh = zero;
       if (pbc)
@@ -382,16 +403,8 @@ __device__ __forceinline__ void k3d_step_body() {
       const bool keep = o < kGrpSlots;
       R hi = R(-3.0e38f), hj = R(-3.0e38f);
       int nnear = 0, nmine = 0;
-      const size_t bj = (size_t)cjq * nv;
-      constexpr int kAtOnce = 4;  // 64-vertex chunks whose loads are issued together
       for (int v0 = 0; v0 < nv; v0 += kAtOnce * DPM_WAVE) {
-        V3<R> q[kAtOnce];
-#pragma unroll
-        for (int k = 0; k < kAtOnce; k++) {
-          const int v = v0 + k * DPM_WAVE + lane;
-          q[k] = zero;
-          if (v < nv) q[k] = v3(a->xin[bj + v], a->yin[bj + v], a->zin[bj + v]);
-        }
+        if (v0 > 0) load(v0);
 #pragma unroll
         for (int k = 0; k < kAtOnce; k++) {
           const int v = v0 + k * DPM_WAVE + lane;
@@ -434,7 +447,14 @@ __device__ __forceinline__ void k3d_step_body() {
       }
       const int bits = ((do_contact && !skip_contact) ? 1 : 0) | ((do_adh && !skip_adh) ? 2 : 0);
       const bool fit = keep && nnear <= kGrpCap && nmine <= kGrpCap;
-      if (lane == 0) rec[b] = bits | (fit ? 4 : 0) | (fit ? nnear << 3 | nmine << 13 : 0);
+      if (lane == 0) {
+        int e = bits;
+        if (fit && nnear > 0 && nmine > 0) {
+          const int S = max(1, min(nnear, kGrpSlices / nmine));
+          e |= 4 | nnear << 3 | nmine << 10 | S << 17 | (nnear + S - 1) / S << 24;
+        }
+        rec[b] = e;
+      }
     }
   };
   if (cmask) separate(cmask);
@@ -775,51 +795,73 @@ __device__ __forceinline__ void k3d_step_body() {
       return;
     }
     Q4<R>* acc = reinterpret_cast<Q4<R>*>(smem + LG.acc);
+    auto place_of = [&](int o) __attribute__((always_inline)) {  // lists of the o-th candidate of m
+      return smem + LG.slots + (size_t)o * LG.slot;
+    };
     while (left) {  // as many candidates as there is room for their partial sums
-      const unsigned long long from = left;
-      int total = 0;
-      while (left) {
-        const int b = __ffsll((long long)left) - 1;
-        const int rb = from_lane(r, b), nnear = (rb >> 3) & 1023, nmine = rb >> 13;
-        const int S = max(1, min(nnear, kGrpSlices / nmine)), per = (nnear + S - 1) / S, n = S * nmine;
-        if (total + n > kGrpTasks) break;
-        const unsigned char* sl = smem + LG.slots + (size_t)__popcll(m & ((1ull << b) - 1ull)) * LG.slot;
-        const R* qx = reinterpret_cast<const R*>(sl);
-        const unsigned short* own = reinterpret_cast<const unsigned short*>(qx + 3 * kGrpCap);
-        const R L0j = fmax(from_lane(st_l.l0, b), R(1e-12f));
-        const double inv_l0j = from_lane(st_l.inv_l0, b);
-        // this candidate's tasks start where the last one's ended
-        for (int i = (tid - total) & (NT - 1); i < n; i += NT) {
-          const int iv = i % nmine, s = i / nmine;
-          acc[total + i] = pair_sum(own[iv], s * per, min(nnear, (s + 1) * per), L0j, inv_l0j,
-                                    [&](int q) __attribute__((always_inline)) { return lds_v(qx, qx + kGrpCap, qx + 2 * kGrpCap, q); });
+      int n = 0, lanes[kGrpSlots] = {0, 0, 0, 0}, ends[kGrpSlots] = {0, 0, 0, 0}, total = 0;
+#pragma unroll
+      for (int c = 0; c < kGrpSlots; c++) {
+        if (left) {
+          const int b = __ffsll((long long)left) - 1, rb = from_lane(r, b);
+          const int tasks = ((rb >> 10) & 127) * ((rb >> 17) & 127);
+          if (total + tasks <= kGrpTasks) {
+            lanes[c] = b;
+            total += tasks;
+            n = c + 1;
+            left &= left - 1ull;
+          }
         }
-        total += n;
-        left &= left - 1ull;
+        ends[c] = total;
+      }
+      for (int i0 = 0; i0 < total; i0 += NT) {  // uniform: every lane takes part in the shuffles
+        const int i = i0 + tid;
+        const int c = (i >= ends[0]) + (i >= ends[1]) + (i >= ends[2]);
+        const int first = c == 0 ? 0 : c == 1 ? ends[0] : c == 2 ? ends[1] : ends[2];
+        const int b = c == 0 ? lanes[0] : c == 1 ? lanes[1] : c == 2 ? lanes[2] : lanes[3];
+        const int rb = __shfl(r, b, DPM_WAVE);
+        const R L0j = fmax(__shfl(st_l.l0, b, DPM_WAVE), R(1e-12f));
+        const double inv_l0j = __shfl(st_l.inv_l0, b, DPM_WAVE);
+        if (i < total) {
+          const int nnear = (rb >> 3) & 127, nmine = (rb >> 10) & 127, per = rb >> 24;
+          // (i - first) / nmine: at most 512 / 64, half away from an integer
+          const int s = (int)(((float)(i - first) + 0.5f) * __builtin_amdgcn_rcpf((float)nmine));
+          const int iv = i - first - s * nmine;
+          const R* qx = reinterpret_cast<const R*>(place_of(__popcll(m & ((1ull << b) - 1ull))));
+          const unsigned short* own = reinterpret_cast<const unsigned short*>(qx + 3 * kGrpCap);
+          acc[i] = pair_sum(own[iv], s * per, min(nnear, (s + 1) * per), L0j, inv_l0j,
+                            [&](int q) __attribute__((always_inline)) { return lds_v(qx, qx + kGrpCap, qx + 2 * kGrpCap, q); });
+        }
       }
       __syncthreads();
-      total = 0;
-      for (unsigned long long w = from & ~left; w; w &= w - 1ull) {
-        const int b = __ffsll((long long)w) - 1;
-        const int rb = from_lane(r, b), nnear = (rb >> 3) & 1023, nmine = rb >> 13;
-        const int S = max(1, min(nnear, kGrpSlices / nmine));
-        const unsigned char* sl = smem + LG.slots + (size_t)__popcll(m & ((1ull << b) - 1ull)) * LG.slot;
+#pragma unroll
+      for (int c = 0; c < kGrpSlots; c++) {
+        if (c >= n) break;  // block-uniform
+        const int b = lanes[c], rb = from_lane(r, b), nmine = (rb >> 10) & 127, S = (rb >> 17) & 127;
+        const Q4<R>* sums = acc + (c > 0 ? ends[c - 1] : 0);
         const unsigned short* place =
-            reinterpret_cast<const unsigned short*>(reinterpret_cast<const R*>(sl) + 3 * kGrpCap) + kGrpCap;
+            reinterpret_cast<const unsigned short*>(
+                reinterpret_cast<const R*>(place_of(__popcll(m & ((1ull << b) - 1ull)))) + 3 * kGrpCap) +
+            kGrpCap;
 #pragma unroll
         for (int k = 0; k < VPT; k++) {
           const int v = tid + k * NT;
           const int p = v < nv ? (int)place[v] : 0xffff;
           if (p == 0xffff) continue;
           int cnt_own = 0;
-          for (int s = 0; s < S; s++) {
-            const Q4<R> q4 = acc[total + s * nmine + p];
-            F[k] = vadd(F[k], V3<R>{q4.x, q4.y, q4.z});
-            cnt_own += (int)q4.w;
+          for (int s = 0; s < S; s += 4) {  // four loads in flight, added in order
+            Q4<R> q4[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) q4[j] = sums[min(s + j, S - 1) * nmine + p];
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+              if (s + j < S) {
+                F[k] = vadd(F[k], V3<R>{q4[j].x, q4[j].y, q4[j].z});
+                cnt_own += (int)q4[j].w;
+              }
           }
           if (PROBE && a->p_adh) a->p_adh[base + v] += cnt_own;
         }
-        total += S * nmine;
       }
       if (left) __syncthreads();
     }
@@ -1055,11 +1097,15 @@ __device__ __forceinline__ void k3d_step_body() {
 // with their sizes fixed; the production one of the former has the diagnostic
 // outputs compiled out, the _probe instance of the same source records them.
 extern "C" __global__ void __launch_bounds__(256) k3d_step_f32(const Step3D<float>) { k3d_step_body<float, 0, 0, 1, 0>(); }
-extern "C" __global__ void __launch_bounds__(256) k3d_step_f32_big(const Step3D<float>) { k3d_step_body<float, 0, 0, 4, 0>(); }
-extern "C" __global__ void __launch_bounds__(256) k3d_step_f64(const Step3D<double>) { k3d_step_body<double, 0, 0, 1, 0>(); }
-extern "C" __global__ void __launch_bounds__(256) k3d_step_f64_big(const Step3D<double>) { k3d_step_body<double, 0, 0, 4, 0>(); }
+extern "C" __global__ void __launch_bounds__(256, 2) k3d_step_f32_big(const Step3D<float>) { k3d_step_body<float, 0, 0, 4, 0>(); }
+extern "C" __global__ void __launch_bounds__(256, 2) k3d_step_f64(const Step3D<double>) { k3d_step_body<double, 0, 0, 1, 0>(); }
+extern "C" __global__ void __launch_bounds__(256, 2) k3d_step_f64_big(const Step3D<double>) { k3d_step_body<double, 0, 0, 4, 0>(); }
 extern "C" __global__ void __launch_bounds__(256) k3d_step_f32_v162(const Step3D<float>) { k3d_step_body<float, 162, 320, 1, 4, false>(); }
 extern "C" __global__ void __launch_bounds__(256) k3d_step_f32_v162_probe(const Step3D<float>) { k3d_step_body<float, 162, 320, 1, 4>(); }
+// 642 vertices: the _many instances keep three (double: two) cells on a
+// compute unit at the cost of spills, the others one or two without.
 extern "C" __global__ void __launch_bounds__(256) k3d_step_f32_v642(const Step3D<float>) { k3d_step_body<float, 642, 1280, 3, 1>(); }
+extern "C" __global__ void __launch_bounds__(256, 3) k3d_step_f32_v642_many(const Step3D<float>) { k3d_step_body<float, 642, 1280, 3, 1>(); }
 extern "C" __global__ void __launch_bounds__(256) k3d_step_f64_v642(const Step3D<double>) { k3d_step_body<double, 642, 1280, 3, 1>(); }
-extern "C" __global__ void __launch_bounds__(256) k3d_step_f64_v162(const Step3D<double>) { k3d_step_body<double, 162, 320, 1, 2>(); }
+extern "C" __global__ void __launch_bounds__(256, 2) k3d_step_f64_v642_many(const Step3D<double>) { k3d_step_body<double, 642, 1280, 3, 1>(); }
+extern "C" __global__ void __launch_bounds__(256, 2) k3d_step_f64_v162(const Step3D<double>) { k3d_step_body<double, 162, 320, 1, 2>(); }

@@ -115,6 +115,7 @@ struct dpm_tissue {
   size_t lds_w = 0;
   int ww_g = 1;      // workgroup-per-cell step: waves that take winding numbers, LDS
   size_t lds_g = 0;
+  bool many_g = false;  // more cells than the few-cells instances serve best
   unsigned mask = 0;
   int cur = 0;
   bool stats_valid = false;
@@ -421,12 +422,18 @@ static const void* wstep_kernel(int rs, int nv, int nf, bool probe = false) {
   return rs == 8 ? (const void*)k3d_wstep_f64 : (const void*)k3d_wstep_f32;
 }
 
-// The workgroup form's kernel for a handle.
-static const void* gstep_kernel(int rs, int nv, int nf, bool probe = false) {
+// The workgroup form's kernel for a handle.  many: the 642-vertex instances
+// for handles beyond four cells per compute unit (double: one); us per step,
+// plain | many: 1024 cells 63 | 68, 4096 cells 175 | 133; double, 64 cells
+// 31 | 38, 1024 cells 112 | 97.
+static const void* gstep_kernel(int rs, int nv, int nf, bool probe, bool many) {
   if (nv == 162 && nf == 320)
     return rs == 8 ? (const void*)k3d_step_f64_v162
                    : probe ? (const void*)k3d_step_f32_v162_probe : (const void*)k3d_step_f32_v162;
-  if (nv == 642 && nf == 1280) return rs == 8 ? (const void*)k3d_step_f64_v642 : (const void*)k3d_step_f32_v642;
+  if (nv == 642 && nf == 1280) {
+    if (rs == 8) return many ? (const void*)k3d_step_f64_v642_many : (const void*)k3d_step_f64_v642;
+    return many ? (const void*)k3d_step_f32_v642_many : (const void*)k3d_step_f32_v642;
+  }
   if (nv > kGrpThreads) return rs == 8 ? (const void*)k3d_step_f64_big : (const void*)k3d_step_f32_big;
   return rs == 8 ? (const void*)k3d_step_f64 : (const void*)k3d_step_f32;
 }
@@ -646,8 +653,12 @@ static int create3d(const dpm3d_desc* d, dpm_tissue** out, int rs) {
                             {(const void*)k3d_stats_f64, (const void*)k3d_energy_f64}};
   for (const void* k : kern[rs == 8 ? 1 : 0])
     (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->lds);
+  int dev = 0, cus = 256;
+  if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  cus = std::max(1, cus);
+  h->many_g = C > (rs == 8 ? 1 : 4) * cus;
   for (bool probe : {false, true})
-    (void)hipFuncSetAttribute(gstep_kernel(rs, nv, nf, probe), hipFuncAttributeMaxDynamicSharedMemorySize,
+    (void)hipFuncSetAttribute(gstep_kernel(rs, nv, nf, probe, h->many_g), hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)h->lds_g);
   (void)hipFuncSetAttribute(rs == 8 ? (const void*)k3d_bin_f64 : (const void*)k3d_bin_f32,
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->bin_lds);
@@ -686,10 +697,8 @@ static int create3d(const dpm3d_desc* d, dpm_tissue** out, int rs) {
       // float 42 vertices, 256 cells 27.3 | 30.0, 1352 cells 49.4 | 32.1;
       // double 162 vertices, 256 cells 30.2 | 46.5, 1024 cells 64.3 | 61.4,
       // 4096 cells 214 | 119; double 42 vertices, 64 cells 42.0 | 32.0
-      int dev = 0, cus = 256;
-      if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
       const int per_cu = nv > DPM_WAVE ? (rs == 8 ? 4 : 3) : (rs == 8 ? 0 : 2);
-      h->wave_min_cells = per_cu * std::max(1, cus);
+      h->wave_min_cells = per_cu * cus;
       for (bool probe : {false, true})
         (void)hipFuncSetAttribute(wstep_kernel(rs, nv, nf, probe), hipFuncAttributeMaxDynamicSharedMemorySize,
                                   (int)h->lds_w);
@@ -928,6 +937,7 @@ static Step3D<R> step_args(dpm_tissue* h, int in, float dt, int flags) {
   a.nv = h->nv;
   a.nf = h->nf;
   a.ncells = h->C;
+  a.one_tissue = h->T == 1;
   a.closed = h->closed;
   a.wtopo = (const uint4*)h->wtopo;
   a.wtopo_n16 = h->wtopo_n16;
@@ -993,7 +1003,7 @@ static int launch3d(dpm_tissue* h, Kind3D kind, int in, float dt, int flags, Edi
                          h->stream, a);
     } else if (kind == K_STEP) {
       a.ww = h->ww_g;
-      auto kg = reinterpret_cast<void (*)(Step3D<R>)>(const_cast<void*>(gstep_kernel(h->rs, h->nv, h->nf, probe)));
+      auto kg = reinterpret_cast<void (*)(Step3D<R>)>(const_cast<void*>(gstep_kernel(h->rs, h->nv, h->nf, probe, h->many_g)));
       hipLaunchKernelGGL(kg, dim3(h->C), dim3(kGrpThreads), h->lds_g, h->stream, a);
     } else {
       void (*k)(Step3D<R>) = nullptr;
