@@ -915,6 +915,9 @@ struct Vjp3D {
   R* cx;  // [3 * nverts] contributions to other cells' lambda (atomic)
   R* cy;
   R* cz;
+  R* px;  // the contributions the step before left: added here, then cleared
+  R* py;
+  R* pz;
   R* lx;       // adjoint: lambda_{n+1} in, lambda_n out (in place)
   R* ly;
   R* lz;
@@ -955,9 +958,28 @@ __host__ __device__ inline LdsVjpLayout ldsvjp_layout(int nv, int nf, int rsize)
   o = (o + 15u) & ~(size_t)15u;
   L.fc = o;    o += 9u * rs * (size_t)nf;
   o = (o + 7u) & ~(size_t)7u;
-  L.red = o;   o += 8u * 32u;
+  L.red = o;   o += 8u * 16u * 11u;  // three, two and six sums over at most 16 waves
   L.total = o;
   return L;
+}
+
+// N sums over the workgroup with one barrier, every thread adding the waves'
+// partial sums itself; scratch (16 N doubles) serves one reduction only.
+template <int N>
+__device__ __forceinline__ void block_sums_1b(double (&v)[N], double* scratch) {
+  const int lane = threadIdx.x & (DPM_WAVE - 1), wave = threadIdx.x / DPM_WAVE;
+  const int nw = (blockDim.x + DPM_WAVE - 1) / DPM_WAVE;
+#pragma unroll
+  for (int i = 0; i < N; i++) {
+    v[i] = wave_sum_d(v[i]);
+    if (lane == 0) scratch[16 * i + wave] = v[i];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < N; i++) {
+    v[i] = 0.0;
+    for (int w = 0; w < nw; w++) v[i] += scratch[16 * i + w];
+  }
 }
 
 template <typename R>
@@ -969,6 +991,11 @@ __device__ __forceinline__ V3<R> jnorm(V3<R> v, V3<R> l) {
   return vscale(vsub(l, vscale(u, vdot(u, l))), R(1) / n);
 }
 
+// The adjoint of one step.  With few cells it is a chain of short passes: the
+// sums take one barrier each group instead of three each, and what a step adds
+// to other cells' lambda waits for the next step's load (two sets of
+// contributions, one written while the other is read) instead of a kernel of
+// its own.
 template <typename R>
 __device__ void k3d_vjp_body(const Vjp3D<R>& a) {
   extern __shared__ __align__(16) unsigned char smem[];
@@ -998,9 +1025,10 @@ __device__ void k3d_vjp_body(const Vjp3D<R>& a) {
     l.sx[v] = a.x[base + v];
     l.sy[v] = a.y[base + v];
     l.sz[v] = a.z[base + v];
-    l.nx[v] = a.lx[base + v];  // lambda
-    l.ny[v] = a.ly[base + v];
-    l.nz[v] = a.lz[base + v];
+    l.nx[v] = a.lx[base + v] + a.dt * a.px[base + v];  // lambda
+    l.ny[v] = a.ly[base + v] + a.dt * a.py[base + v];
+    l.nz[v] = a.lz[base + v] + a.dt * a.pz[base + v];
+    a.px[base + v] = a.py[base + v] = a.pz[base + v] = R(0);
   }
   int vfr[DPM3D_MAXDEG], adjr[DPM3D_MAXDEG];
 #pragma unroll
@@ -1017,16 +1045,14 @@ __device__ void k3d_vjp_body(const Vjp3D<R>& a) {
   const unsigned mask = a.mask;
 
   // centre of mass and volume of x_n, as the forward step's statistics
-  double px = 0.0, py = 0.0, pz = 0.0;
+  double p[3] = {0.0, 0.0, 0.0};
   for (int v = tid; v < nv; v += NT) {
-    px += (double)l.sx[v];
-    py += (double)l.sy[v];
-    pz += (double)l.sz[v];
+    p[0] += (double)l.sx[v];
+    p[1] += (double)l.sy[v];
+    p[2] += (double)l.sz[v];
   }
-  px = block_sum(px, l.red);
-  py = block_sum(py, l.red);
-  pz = block_sum(pz, l.red);
-  const V3<R> C = {(R)(px / nv), (R)(py / nv), (R)(pz / nv)};
+  block_sums_1b(p, l.red);
+  const V3<R> C = {(R)(p[0] / nv), (R)(p[1] / nv), (R)(p[2] / nv)};
   double vol = 0.0, S1 = 0.0;
   const bool vol_on = (mask & M_VOLUME) && Kvi != R(0);
   for (int f = tid; f < nf; f += NT) {
@@ -1042,8 +1068,10 @@ __device__ void k3d_vjp_body(const Vjp3D<R>& a) {
             (double)vdot(vcross(P0, P1), lds_v(l.nx, l.ny, l.nz, i2));
     }
   }
-  vol = fabs(block_sum(vol, l.red) / 6.0);
-  S1 = block_sum(S1, l.red) / 6.0;
+  double vs[2] = {vol, S1};
+  block_sums_1b(vs, l.red + 48);
+  vol = fabs(vs[0] / 6.0);
+  S1 = vs[1] / 6.0;
   const R strain = (R)(vol / (double)v0i - 1.0);
 
   // per face-corner adjoint contributions (into the shape-force bytes)
@@ -1233,12 +1261,9 @@ __device__ void k3d_vjp_body(const Vjp3D<R>& a) {
       }
     }
   }
-  Lcx = block_sum(Lcx, l.red);
-  Lcy = block_sum(Lcy, l.red);
-  Lcz = block_sum(Lcz, l.red);
-  gKa = block_sum(gKa, l.red);
-  gKs = block_sum(gKs, l.red);
-  gKb = block_sum(gKb, l.red);
+  double g[6] = {Lcx, Lcy, Lcz, gKa, gKs, gKb};
+  block_sums_1b(g, l.red + 80);
+  Lcx = g[0], Lcy = g[1], Lcz = g[2], gKa = g[3], gKs = g[4], gKb = g[5];
   if (own) {
     // the centre of mass moves with each vertex by 1/nv
     mu = vadd(mu, V3<R>{(R)(Lcx / nv), (R)(Lcy / nv), (R)(Lcz / nv)});

@@ -1586,7 +1586,7 @@ extern "C" int dpm3d_trajectory(dpm_tissue* h, int nsteps, float dt, int every) 
 }
 
 template <typename R>
-static Vjp3D<R> vjp_args(dpm_tissue* h, size_t s) {
+static Vjp3D<R> vjp_args(dpm_tissue* h, size_t s, int set) {
   Vjp3D<R> a{};
   void* xs = slot(h, h->seg, 3 * s);
   a.x = (const R*)xs;
@@ -1597,9 +1597,12 @@ static Vjp3D<R> vjp_args(dpm_tissue* h, size_t s) {
   a.rec_cell = h->segcell + s * NP;
   a.rec_w = (const R*)h->segwp + s * NP;
   a.rec_shift = (const R*)h->segsh + s * NP * 3;
-  a.cx = (R*)h->cross;
-  a.cy = (R*)slot(h, h->cross, 1);
-  a.cz = (R*)slot(h, h->cross, 2);
+  a.cx = (R*)slot(h, h->cross, 3 * set);
+  a.cy = (R*)slot(h, h->cross, 3 * set + 1);
+  a.cz = (R*)slot(h, h->cross, 3 * set + 2);
+  a.px = (R*)slot(h, h->cross, 3 * (1 - set));
+  a.py = (R*)slot(h, h->cross, 3 * (1 - set) + 1);
+  a.pz = (R*)slot(h, h->cross, 3 * (1 - set) + 2);
   a.lx = (R*)h->lam;
   a.ly = (R*)slot(h, h->lam, 1);
   a.lz = (R*)slot(h, h->lam, 2);
@@ -1641,7 +1644,7 @@ static int adjoint3d(dpm_tissue* h, const In* lambda_final, double* dtheta, Out*
   TRY(ensure_real(h, &h->lam, h->lam_cap, 3 * NVT));
   TRY(ensure_real(h, &h->segwp, h->segwp_cap, (size_t)every * NVT * DPM3D_MAXPART));
   TRY(ensure_real(h, &h->segsh, h->segsh_cap, (size_t)every * NVT * DPM3D_MAXPART * 3));
-  TRY(ensure_real(h, &h->cross, h->cross_cap, 3 * NVT));
+  TRY(ensure_real(h, &h->cross, h->cross_cap, 6 * NVT));
   if (h->segcell_cap < (size_t)every * NVT * DPM3D_MAXPART) {
     if (h->segcell) {
       (void)hipFree(h->segcell);
@@ -1654,7 +1657,7 @@ static int adjoint3d(dpm_tissue* h, const In* lambda_final, double* dtheta, Out*
   if (!h->gtheta) TRY(h->alloc(&h->gtheta, (size_t)h->C * 4));
   if (!h->rec_overflow) TRY(h->alloc(&h->rec_overflow, 1));
   HIPCHECK(hipMemsetAsync(h->rec_overflow, 0, sizeof(int), h->stream));
-  HIPCHECK(hipMemsetAsync(h->cross, 0, 3 * NVT * h->rs, h->stream));
+  HIPCHECK(hipMemsetAsync(h->cross, 0, 6 * NVT * h->rs, h->stream));
   // lambda_N
   {
     std::vector<In> a(NVT), b(NVT), c(NVT);
@@ -1669,49 +1672,72 @@ static int adjoint3d(dpm_tissue* h, const In* lambda_final, double* dtheta, Out*
   }
   HIPCHECK(hipMemsetAsync(h->gtheta, 0, sizeof(double) * h->C * 4, h->stream));
   const float dt = h->traj_dt;
+  int set = 0;  // of the two sets of contributions to other cells, the one written next
   for (int sg = nseg - 1; sg >= 0; sg--) {
-    // recompute the segment from its checkpoint, keeping x_n and W_n
+    // recompute the segment from its checkpoint, keeping x_n and W_n: step s
+    // reads its positions from the segment and writes the next ones there
+    // (the last step's, the next checkpoint's, go to the handle's buffers)
     void* c = slot(h, h->ck, (size_t)ns * sg);
     h->cur = 0;
-    TRY(copy_positions_dd(h, h->x[0], h->y[0], h->z[0], c, slot(h, c, 1), slot(h, c, 2)));
+    HIPCHECK(hipMemcpyAsync(h->seg, c, 3 * NVT * h->rs, hipMemcpyDeviceToDevice, h->stream));
     if (h->lo)
       HIPCHECK(hipMemcpyAsync(h->lo, slot(h, c, 3), 3 * NVT * h->rs, hipMemcpyDeviceToDevice, h->stream));
+    auto from_segment = [&](auto& a, size_t s) {
+      using R = std::remove_const_t<std::remove_reference_t<decltype(*a.xin)>>;
+      void* xs = slot(h, h->seg, 3 * s);
+      a.xin = (const R*)xs;
+      a.yin = (const R*)slot(h, xs, 1);
+      a.zin = (const R*)slot(h, xs, 2);
+    };
+    TRY(launch3d(h, K_STATS, 0, 0.0f, 0, [&](auto& a) {
+      using S = std::remove_reference_t<decltype(*a.st_out)>;
+      using R = std::remove_reference_t<decltype(*a.em_out)>;
+      from_segment(a, 0);
+      a.st_out = (S*)h->st[0];
+      a.vol_out = h->vol[0];
+      a.em_out = (R*)h->em[0];
+    }));
     h->stats_valid = h->nl_ok = false;
-    TRY(ensure_stats(h));
     for (int s = 0; s < every; s++) {
-      void* xs = slot(h, h->seg, 3 * (size_t)s);
-      TRY(copy_positions_dd(h, xs, slot(h, xs, 1), slot(h, xs, 2), h->x[h->cur], h->y[h->cur], h->z[h->cur]));
       void* w = slot(h, h->segw, s);
       const size_t NP = NVT * DPM3D_MAXPART;
-      TRY(launch3d(h, K_STEP, h->cur, dt, F_MOVE, [&](auto& a) {
+      TRY(launch3d(h, K_STEP, s & 1, dt, F_MOVE, [&](auto& a) {
         using R = std::remove_reference_t<decltype(*a.w_out)>;
+        from_segment(a, (size_t)s);
+        if (s + 1 < every) {
+          void* xn = slot(h, h->seg, 3 * ((size_t)s + 1));
+          a.xout = (R*)xn;
+          a.yout = (R*)slot(h, xn, 1);
+          a.zout = (R*)slot(h, xn, 2);
+        }
         a.w_out = (R*)w;
         a.rec_cell = h->segcell + s * NP;
         a.rec_w = (R*)h->segwp + s * NP;
         a.rec_shift = (R*)h->segsh + s * NP * 3;
         a.rec_overflow = h->rec_overflow;
       }));
-      h->cur = 1 - h->cur;
     }
     // reverse sweep through the segment
     for (int s = every - 1; s >= 0; s--) {
-      const int cb = (int)std::min<size_t>((NVT + 255) / 256, 1024);
-      if (h->rs == 8) {
-        Vjp3D<double> a = vjp_args<double>(h, s);
-        if (h->NT == 256)
-          hipLaunchKernelGGL(k3d_vjp_f64_t256, dim3(h->C), dim3(h->NT), h->lds_vjp, h->stream, a);
-        else
-          hipLaunchKernelGGL(k3d_vjp_f64, dim3(h->C), dim3(h->NT), h->lds_vjp, h->stream, a);
-        hipLaunchKernelGGL(k3d_vjp_cross_f64, dim3(cb), dim3(256), 0, h->stream, a.lx, a.ly, a.lz, a.cx, a.cy,
-                           a.cz, (double)a.dt, NVT);
-      } else {
-        Vjp3D<float> a = vjp_args<float>(h, s);
-        hipLaunchKernelGGL(k3d_vjp_f32, dim3(h->C), dim3(h->NT), h->lds_vjp, h->stream, a);
-        hipLaunchKernelGGL(k3d_vjp_cross_f32, dim3(cb), dim3(256), 0, h->stream, a.lx, a.ly, a.lz, a.cx, a.cy,
-                           a.cz, a.dt, NVT);
-      }
+      if (h->rs == 8)
+        hipLaunchKernelGGL(h->NT == 256 ? k3d_vjp_f64_t256 : k3d_vjp_f64, dim3(h->C), dim3(h->NT), h->lds_vjp,
+                           h->stream, vjp_args<double>(h, s, set));
+      else
+        hipLaunchKernelGGL(k3d_vjp_f32, dim3(h->C), dim3(h->NT), h->lds_vjp, h->stream, vjp_args<float>(h, s, set));
       HIPCHECK(hipGetLastError());
+      set = 1 - set;
     }
+  }
+  {  // what the first step added to other cells
+    const int cb = (int)std::min<size_t>((NVT + 255) / 256, 1024);
+    auto add = [&](auto kernel, auto tag) {
+      using R = decltype(tag);
+      const Vjp3D<R> a = vjp_args<R>(h, 0, 1 - set);
+      hipLaunchKernelGGL(kernel, dim3(cb), dim3(256), 0, h->stream, a.lx, a.ly, a.lz, a.cx, a.cy, a.cz, a.dt, NVT);
+    };
+    if (h->rs == 8) add(k3d_vjp_cross_f64, 0.0);
+    else add(k3d_vjp_cross_f32, 0.0f);
+    HIPCHECK(hipGetLastError());
   }
   // back to the final state of the trajectory
   void* last = slot(h, h->ck, (size_t)ns * nseg);
