@@ -224,8 +224,8 @@ float dpm3d_bin_width(dpm_tissue* h);
  * 1 one workgroup per cell; 2 one 64-lane wave per cell (meshes of at most
  * 256 vertices, several cells per workgroup, no workgroup barriers after
  * set-up); 0 (default) chooses 2 for meshes it takes once the handle holds
- * enough cells (float: 3 per compute unit, 2 for meshes of at most 64
- * vertices; double: 4, and always for those meshes), else 1.  Both make the same
+ * enough cells (4 per compute unit; meshes of at most 64 vertices: 3, in
+ * double 2), else 1.  Both make the same
  * pair decisions; the wave form sums each vertex's edge springs once per ring
  * edge and its adhesion terms in slices, so forces agree to float rounding. */
 int dpm3d_set_step_kernel(dpm_tissue* h, int kind);

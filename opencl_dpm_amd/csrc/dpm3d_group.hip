@@ -1093,13 +1093,16 @@ __device__ __forceinline__ void k3d_step_body() {
 }
 
 // VPT 1: meshes of at most 256 vertices; VPT 4: up to 1024.  The icospheres of
-// subdivision 2 (162 vertices, 320 faces) and 3 (642, 1280) have instances
-// with their sizes fixed; the production one of the former has the diagnostic
-// outputs compiled out, the _probe instance of the same source records them.
+// subdivision 1 (42 vertices, 80 faces), 2 (162, 320) and 3 (642, 1280) have
+// instances with their sizes fixed; the production float ones of the first two
+// have the diagnostic outputs compiled out, the _probe instance of the same
+// source and the general kernel record them.
 extern "C" __global__ void __launch_bounds__(256) k3d_step_f32(const Step3D<float>) { k3d_step_body<float, 0, 0, 1, 0>(); }
 extern "C" __global__ void __launch_bounds__(256, 2) k3d_step_f32_big(const Step3D<float>) { k3d_step_body<float, 0, 0, 4, 0>(); }
 extern "C" __global__ void __launch_bounds__(256, 2) k3d_step_f64(const Step3D<double>) { k3d_step_body<double, 0, 0, 1, 0>(); }
 extern "C" __global__ void __launch_bounds__(256, 2) k3d_step_f64_big(const Step3D<double>) { k3d_step_body<double, 0, 0, 4, 0>(); }
+extern "C" __global__ void __launch_bounds__(256) k3d_step_f32_v42(const Step3D<float>) { k3d_step_body<float, 42, 80, 1, 4, false>(); }
+extern "C" __global__ void __launch_bounds__(256, 2) k3d_step_f64_v42(const Step3D<double>) { k3d_step_body<double, 42, 80, 1, 4, false>(); }
 extern "C" __global__ void __launch_bounds__(256) k3d_step_f32_v162(const Step3D<float>) { k3d_step_body<float, 162, 320, 1, 4, false>(); }
 extern "C" __global__ void __launch_bounds__(256) k3d_step_f32_v162_probe(const Step3D<float>) { k3d_step_body<float, 162, 320, 1, 4>(); }
 // 642 vertices: the _many instances keep three (double: two) cells on a

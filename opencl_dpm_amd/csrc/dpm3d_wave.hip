@@ -880,4 +880,15 @@ extern "C" __global__ void __launch_bounds__(256, 4) k3d_wstep_f32_v162(const St
 extern "C" __global__ void __launch_bounds__(256, 4) k3d_wstep_f32_v162_probe(const Step3D<float> a) {
   k3d_wstep_body<float, 162, 320, true>();
 }
+// the icosphere of subdivision 1 (42 vertices, 80 faces), and both in double;
+// without the diagnostic outputs (the general kernels record them)
+extern "C" __global__ void __launch_bounds__(256, 4) k3d_wstep_f32_v42(const Step3D<float>) {
+  k3d_wstep_body<float, 42, 80, false>();
+}
+extern "C" __global__ void __launch_bounds__(256) k3d_wstep_f64_v42(const Step3D<double>) {
+  k3d_wstep_body<double, 42, 80, false>();
+}
+extern "C" __global__ void __launch_bounds__(256) k3d_wstep_f64_v162(const Step3D<double>) {
+  k3d_wstep_body<double, 162, 320, false>();
+}
 extern "C" __global__ void __launch_bounds__(256) k3d_wstep_f64(const Step3D<double> a) { k3d_wstep_body<double, 0, 0>(); }

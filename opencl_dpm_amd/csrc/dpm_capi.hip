@@ -413,12 +413,14 @@ static bool all_finite(const R* p, size_t n) {
   return true;
 }
 
-// The wave-per-cell step kernel of a precision.
-// The wave form's kernel for a handle: the compile-time-sized instance for
-// float 162-vertex, 320-face meshes, else the general one.
+// The wave form's kernel for a handle: the compile-time-sized instance of an
+// icosphere of 42 or 162 vertices, else the general one.
 static const void* wstep_kernel(int rs, int nv, int nf, bool probe = false) {
-  if (rs == 4 && nv == 162 && nf == 320) return probe ? (const void*)k3d_wstep_f32_v162_probe
-                                                      : (const void*)k3d_wstep_f32_v162;
+  if (nv == 162 && nf == 320) {
+    if (rs == 4) return probe ? (const void*)k3d_wstep_f32_v162_probe : (const void*)k3d_wstep_f32_v162;
+    if (!probe) return (const void*)k3d_wstep_f64_v162;
+  }
+  if (nv == 42 && nf == 80 && !probe) return rs == 8 ? (const void*)k3d_wstep_f64_v42 : (const void*)k3d_wstep_f32_v42;
   return rs == 8 ? (const void*)k3d_wstep_f64 : (const void*)k3d_wstep_f32;
 }
 
@@ -430,6 +432,7 @@ static const void* gstep_kernel(int rs, int nv, int nf, bool probe, bool many) {
   if (nv == 162 && nf == 320)
     return rs == 8 ? (const void*)k3d_step_f64_v162
                    : probe ? (const void*)k3d_step_f32_v162_probe : (const void*)k3d_step_f32_v162;
+  if (nv == 42 && nf == 80 && !probe) return rs == 8 ? (const void*)k3d_step_f64_v42 : (const void*)k3d_step_f32_v42;
   if (nv == 642 && nf == 1280) {
     if (rs == 8) return many ? (const void*)k3d_step_f64_v642_many : (const void*)k3d_step_f64_v642;
     return many ? (const void*)k3d_step_f32_v642_many : (const void*)k3d_step_f32_v642;
@@ -693,11 +696,12 @@ static int create3d(const dpm3d_desc* d, dpm_tissue** out, int rs) {
       // shortens one cell's step while the device has room for every cell at
       // once, a wave per cell takes fewer waves and no barriers.  Measured,
       // us per step, every term, workgroup | wave form: float 162 vertices,
-      // 484 cells 31.4 | 38.7, 1024 cells 46.0 | 33.3, 4096 cells 126 | 50.5;
-      // float 42 vertices, 256 cells 27.3 | 30.0, 1352 cells 49.4 | 32.1;
-      // double 162 vertices, 256 cells 30.2 | 46.5, 1024 cells 64.3 | 61.4,
-      // 4096 cells 214 | 119; double 42 vertices, 64 cells 42.0 | 32.0
-      const int per_cu = nv > DPM_WAVE ? (rs == 8 ? 4 : 3) : (rs == 8 ? 0 : 2);
+      // 768 cells 26.4 | 32.9, 1024 cells 35.4 | 33.7, 2048 cells 50.4 | 36.9;
+      // float 42 vertices, 484 cells 26.6 | 26.8, 845 cells 25.1 | 24.3, 1352
+      // cells 35.8 | 26.0; double 162 vertices, 512 cells 36.4 | 44.9, 1024
+      // cells 53.0 | 53.7, 1536 cells 77.3 | 54.8; double 42 vertices, 256 cells
+      // 28.6 | 32.4, 512 cells 31.0 | 31.5, 3887 cells 154 | 64
+      const int per_cu = nv > DPM_WAVE ? 4 : rs == 8 ? 2 : 3;
       h->wave_min_cells = per_cu * cus;
       for (bool probe : {false, true})
         (void)hipFuncSetAttribute(wstep_kernel(rs, nv, nf, probe), hipFuncAttributeMaxDynamicSharedMemorySize,
