@@ -284,84 +284,55 @@ __device__ __forceinline__ bool facing_down(V3<R> n) {
   return vnormalize(n).z < R(-0.1f);
 }
 
-// LDS layout (byte offsets), shared by host (sizing) and device (carving).
-// The per-(face, corner) shape forces are dead once every vertex gathered
-// them, so they share their bytes with the tables of the later passes
-// (bending, neighbour cell, winding directions).
+// LDS of the statistics and energy kernels (byte offsets).
 struct Lds3DLayout {
-  size_t own, faces, clist, plist, glist, gath, cnt, red, cst, nbr, bend, wnum, utab, fc, total;
+  size_t own, faces, red, total;
 };
-// Statistics of the first kCandStats candidates of a scan chunk are kept in
-// LDS (the rest are read from global memory).
-constexpr int kCandStats = 64;
-__host__ __device__ inline Lds3DLayout lds3d_layout(int nv, int nf, int nt, int ww, int rsize) {
+__host__ __device__ inline Lds3DLayout lds3d_layout(int nv, int nf, int rsize) {
   Lds3DLayout L;
   const size_t rs = (size_t)rsize;
   size_t o = 0;
   L.own = o;     o += 3u * rs * (size_t)nv;
   o = (o + 7u) & ~(size_t)7u;
   L.faces = o;   o += 8u * (size_t)nf;  // (i0 | i1 << 16, i2) per face
-  o = (o + 3u) & ~(size_t)3u;
-  L.clist = o;   o += 4u * (size_t)nt;
-  L.plist = o;   o += 8u * (size_t)nt;  // two lists of nt
-  L.glist = o;   o += 4u * (size_t)nt;  // candidate cells gathered from the cell list
-  L.gath = o;    o += 4u * 96u;         // 27 buckets: ids, starts, prefix
-  L.cnt = o;     o += 4u * 48u;
-  o = (o + 7u) & ~(size_t)7u;
   L.red = o;     o += 8u * 192u;  // three 64-double regions (cell_stats alternates them)
-  o = (o + 31u) & ~(size_t)31u;
-  L.cst = o;     o += 8u * rs * (size_t)kCandStats;  // CellStat<R> of the candidates
-  o = (o + 31u) & ~(size_t)31u;
-  L.fc = o;  // union: shape pass | later passes
-  const size_t fc_end = o + 9u * rs * (size_t)nf;
-  L.nbr = o;     o += 3u * rs * (size_t)nv;
-  L.bend = o;    o += 3u * rs * (size_t)nv;
-  L.wnum = o;    o += rs * (size_t)nv;
-  o = (o + 31u) & ~(size_t)31u;
-  L.utab = o;    o += 4u * rs * (size_t)nv * (size_t)ww;
-  // the adhesion pass's per-(slice, vertex) partial sums share the winding
-  // directions' bytes (the two passes are separated by barriers)
-  const size_t adh_end = L.utab + 4u * rs * (size_t)nt;
-  if (o < adh_end) o = adh_end;
-  L.total = o > fc_end ? o : fc_end;
+  L.total = o;
   return L;
 }
 
+// The bound on meshes: what a workgroup of a thread per vertex holds with nine
+// reals per face, or the winding directions of its waves, beside its vertices.
+// No kernel here takes that much; it keeps the meshes that are refused.
+inline size_t mesh_lds_bound(int nv, int nf, int nt, int rsize) {
+  const size_t rs = (size_t)rsize, n = (size_t)nv, t = (size_t)nt;
+  const size_t ww = std::max<size_t>(1, std::min<size_t>(t / DPM_WAVE, 49152 / (4 * rs * n)));
+  size_t o = (3 * rs * n + 7) & ~(size_t)7;
+  o = ((o + 8 * (size_t)nf + 16 * t + 4 * 144 + 7) & ~(size_t)7) + 8 * 192;
+  o = ((o + 31) & ~(size_t)31) + 8 * rs * 64;
+  o = (o + 31) & ~(size_t)31;
+  const size_t faces = o + 9 * rs * (size_t)nf;
+  o = (o + 7 * rs * n + 31) & ~(size_t)31;
+  return std::max(faces, o + std::max(4 * rs * n * ww, 4 * rs * t));
+}
+
+// Pointers into a workgroup's LDS (the adjoint's kernel has a layout of its
+// own and fills the rest: lambda in nx, bending sums, per-corner terms).
 template <typename R>
 struct Lds3D {
-  R *sx, *sy, *sz, *nx, *ny, *nz, *sb, *wb, *fcx, *fcy, *fcz;
-  Q4<R>* utab;
-  CellStat<R>* cst;
+  R *sx, *sy, *sz, *nx, *ny, *nz, *sb, *fcx, *fcy, *fcz;
   uint2* sf;
-  int *clist, *plist, *glist, *gath, *cnt;
   double* red;
 };
 template <typename R>
-__device__ __forceinline__ Lds3D<R> carve3d(unsigned char* smem, int nv, int nf, int nt, int ww) {
-  const Lds3DLayout L = lds3d_layout(nv, nf, nt, ww, (int)sizeof(R));
-  Lds3D<R> l;
+__device__ __forceinline__ Lds3D<R> carve3d(unsigned char* smem, int nv, int nf) {
+  const Lds3DLayout L = lds3d_layout(nv, nf, (int)sizeof(R));
+  Lds3D<R> l{};
   R* o = reinterpret_cast<R*>(smem + L.own);
   l.sx = o;
   l.sy = o + nv;
   l.sz = o + 2 * nv;
-  R* n = reinterpret_cast<R*>(smem + L.nbr);
-  l.nx = n;
-  l.ny = n + nv;
-  l.nz = n + 2 * nv;
-  l.sb = reinterpret_cast<R*>(smem + L.bend);
-  l.wb = reinterpret_cast<R*>(smem + L.wnum);
   l.sf = reinterpret_cast<uint2*>(smem + L.faces);
-  l.clist = reinterpret_cast<int*>(smem + L.clist);
-  l.plist = reinterpret_cast<int*>(smem + L.plist);
-  l.glist = reinterpret_cast<int*>(smem + L.glist);
-  l.gath = reinterpret_cast<int*>(smem + L.gath);
-  l.cnt = reinterpret_cast<int*>(smem + L.cnt);
-  l.utab = reinterpret_cast<Q4<R>*>(smem + L.utab);
-  l.fcx = reinterpret_cast<R*>(smem + L.fc);
-  l.fcy = l.fcx + 3 * nf;
-  l.fcz = l.fcy + 3 * nf;
   l.red = reinterpret_cast<double*>(smem + L.red);
-  l.cst = reinterpret_cast<CellStat<R>*>(smem + L.cst);
   return l;
 }
 
@@ -393,38 +364,22 @@ __device__ __forceinline__ void face_of(const Lds3D<R>& l, int f, int& i0, int& 
 // absolute-coordinate triple products in float (getVolume,
 // Cell3D_Kernel.cl:46-64), which cancels catastrophically far from the
 // origin.
-// one_each: a thread per vertex, vertex tid in pv (cell_stats_own).
 template <typename R>
-__device__ CellStat<R> cell_stats_impl(const Lds3D<R>& l, int nv, int nf, CellStat<R>* st_out,
-                                double* vol_out, R* em_out, int ci, R l0c, bool one_each, bool has_v, V3<R> pv) {
+__device__ void cell_stats(const Lds3D<R>& l, int nv, int nf, CellStat<R>* st_out, double* vol_out, R* em_out,
+                           int ci, R l0c) {
   const int tid = threadIdx.x, NT = blockDim.x;
   double px = 0.0, py = 0.0, pz = 0.0;
-  if (one_each) {
-    if (has_v) {
-      px = (double)pv.x;
-      py = (double)pv.y;
-      pz = (double)pv.z;
-    }
-  } else {
-    for (int v = tid; v < nv; v += NT) {
-      px += (double)l.sx[v];
-      py += (double)l.sy[v];
-      pz += (double)l.sz[v];
-    }
+  for (int v = tid; v < nv; v += NT) {
+    px += (double)l.sx[v];
+    py += (double)l.sy[v];
+    pz += (double)l.sz[v];
   }
   block_sum3_1b(px, py, pz, l.red + 64);  // the two reductions alternate scratch regions
   const V3<R> C = {(R)(px / nv), (R)(py / nv), (R)(pz / nv)};
   R r = R(0);
-  if (one_each) {
-    if (has_v) {
-      const V3<R> d = vsub(pv, C);
-      r = sqrt(vdot(d, d));
-    }
-  } else {
-    for (int v = tid; v < nv; v += NT) {
-      const V3<R> d = vsub(lds_v(l.sx, l.sy, l.sz, v), C);
-      r = fmax(r, sqrt(vdot(d, d)));
-    }
+  for (int v = tid; v < nv; v += NT) {
+    const V3<R> d = vsub(lds_v(l.sx, l.sy, l.sz, v), C);
+    r = fmax(r, sqrt(vdot(d, d)));
   }
   double vol = 0.0;
   R e2 = R(0);
@@ -445,32 +400,14 @@ __device__ CellStat<R> cell_stats_impl(const Lds3D<R>& l, int nv, int nf, CellSt
     r = (R)rd;
     e2 = (R)e2d;
   }
-  CellStat<R> st{};  // thread 0's
   if (tid == 0) {
     // Slack of a few ulp so that the culling tests are never tighter than the
     // largest distance a vertex can have from C, or the longest edge.
     const R em = sqrt(e2) * R(1.000001f);
-    st = make_cell_stat<R>(C.x, C.y, C.z, r * R(1.0000005f) + R(1e-30f), em, l0c);
-    st_out[ci] = st;
+    st_out[ci] = make_cell_stat<R>(C.x, C.y, C.z, r * R(1.0000005f) + R(1e-30f), em, l0c);
     vol_out[ci] = fabs(vol / 6.0);
     em_out[ci] = em;
   }
-  return st;
-}
-template <typename R>
-__device__ void cell_stats(const Lds3D<R>& l, int nv, int nf, CellStat<R>* st_out, double* vol_out, R* em_out,
-                           int ci, R l0c) {
-  cell_stats_impl(l, nv, nf, st_out, vol_out, em_out, ci, l0c, false, false, V3<R>{R(0), R(0), R(0)});
-}
-// The same from a workgroup with a thread per vertex (NT >= nv): thread v
-// holds vertex v (has_v) in registers, and the centre of mass and radius are
-// taken from them (the sums and maxima of cell_stats, bit for bit); the LDS
-// positions are read only by the face loop, after the first reduction's
-// barrier, so they may be written just before the call.
-template <typename R>
-__device__ CellStat<R> cell_stats_own(const Lds3D<R>& l, int nv, int nf, CellStat<R>* st_out, double* vol_out,
-                               R* em_out, int ci, R l0c, bool has_v, V3<R> pv) {
-  return cell_stats_impl(l, nv, nf, st_out, vol_out, em_out, ci, l0c, true, has_v, pv);
 }
 
 template <typename R, typename Args>
@@ -792,7 +729,7 @@ template <typename R>
 __device__ void k3d_stats_body(const Step3D<R>& a) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int ci = xcd_remap(blockIdx.x, gridDim.x);
-  Lds3D<R> l = carve3d<R>(smem, a.nv, a.nf, blockDim.x, a.ww);
+  Lds3D<R> l = carve3d<R>(smem, a.nv, a.nf);
   stage_topology(a, l);
   load_own(a, l, (size_t)ci * a.nv);
   __syncthreads();
@@ -812,7 +749,7 @@ __device__ void k3d_energy_body(const Step3D<R>& a) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int nv = a.nv, nf = a.nf, NT = blockDim.x, tid = threadIdx.x;
   const int ci = xcd_remap(blockIdx.x, gridDim.x);
-  Lds3D<R> l = carve3d<R>(smem, nv, nf, NT, a.ww);
+  Lds3D<R> l = carve3d<R>(smem, nv, nf);
   stage_topology(a, l);
   load_own(a, l, (size_t)ci * nv);
   __syncthreads();

@@ -105,7 +105,6 @@ struct dpm_tissue {
   float *tL = nullptr, *tKre = nullptr, *tKat = nullptr, *tksg = nullptr;
   int* tpbc = nullptr;
   int *faces = nullptr, *vf = nullptr, *adj = nullptr;
-  int ww = 1;
   int closed = 0;
   // wave-per-cell step (meshes of <= 256 vertices): cells per workgroup
   // (0: not available), LDS; step_kernel 0 automatic, 1 workgroup, 2 wave
@@ -551,13 +550,10 @@ static int create3d(const dpm3d_desc* d, dpm_tissue** out, int rs) {
   h->closed = closed ? 1 : 0;
   h->ncmax = ncmax;
   h->NT = std::max(256, (nv + 63) / 64 * 64);
-  // Waves that evaluate winding numbers, each with an nv-entry direction
-  // table in LDS (at most ~48 KB of tables).
-  h->ww = std::max(1, std::min(h->NT / 64, 49152 / (4 * rs * nv)));
-  h->lds = lds3d_layout(nv, nf, h->NT, h->ww, rs).total;
+  h->lds = lds3d_layout(nv, nf, rs).total;
   h->ww_g = group_winding_waves(nv, rs);
   h->lds_g = ldsg_layout(nv, nf, h->ww_g, rs).total;
-  if ((int)h->lds > max_lds_per_block(h->device)) {
+  if ((int)std::max(h->lds_g, mesh_lds_bound(nv, nf, h->NT, rs)) > max_lds_per_block(h->device)) {
     delete h;
     return fail(DPM_ERANGE, "cell mesh does not fit the LDS of one workgroup");
   }
@@ -937,7 +933,7 @@ static Step3D<R> step_args(dpm_tissue* h, int in, float dt, int flags) {
   a.faces = h->faces;
   a.vf = h->vf;
   a.adj = h->adj;
-  a.ww = h->ww;
+  a.ww = h->ww_g;
   a.nv = h->nv;
   a.nf = h->nf;
   a.ncells = h->C;
@@ -1006,7 +1002,6 @@ static int launch3d(dpm_tissue* h, Kind3D kind, int in, float dt, int flags, Edi
       hipLaunchKernelGGL(kw, dim3((h->C + h->wave_cpw - 1) / h->wave_cpw), dim3(64 * h->wave_cpw), h->lds_w,
                          h->stream, a);
     } else if (kind == K_STEP) {
-      a.ww = h->ww_g;
       auto kg = reinterpret_cast<void (*)(Step3D<R>)>(const_cast<void*>(gstep_kernel(h->rs, h->nv, h->nf, probe, h->many_g)));
       hipLaunchKernelGGL(kg, dim3(h->C), dim3(kGrpThreads), h->lds_g, h->stream, a);
     } else {

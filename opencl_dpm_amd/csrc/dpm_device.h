@@ -213,39 +213,8 @@ __device__ __forceinline__ double block_sum(double v, double* scratch) {
   __syncthreads();
   return r;
 }
-// Three block-wide sums in one pass (every thread gets them); scratch: >= 52
-// doubles of LDS.  Contains __syncthreads.
-__device__ __forceinline__ void block_sum3(double& a, double& b, double& c, double* scratch) {
-  const int lane = threadIdx.x & (DPM_WAVE - 1), wave = threadIdx.x / DPM_WAVE;
-  const int nw = (blockDim.x + DPM_WAVE - 1) / DPM_WAVE;
-  a = wave_sum(a);
-  b = wave_sum(b);
-  c = wave_sum(c);
-  if (lane == 0) {
-    scratch[wave] = a;
-    scratch[16 + wave] = b;
-    scratch[32 + wave] = c;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double sa = 0.0, sb = 0.0, sc = 0.0;
-    for (int w = 0; w < nw; w++) {
-      sa += scratch[w];
-      sb += scratch[16 + w];
-      sc += scratch[32 + w];
-    }
-    scratch[48] = sa;
-    scratch[49] = sb;
-    scratch[50] = sc;
-  }
-  __syncthreads();
-  a = scratch[48];
-  b = scratch[49];
-  c = scratch[50];
-  __syncthreads();
-}
 
-// block_sum3 with one workgroup barrier: every thread adds the waves'
+// Three sums with one workgroup barrier: every thread adds the waves'
 // partial sums itself, in wave order (the same result as one thread adding
 // them and broadcasting).  scratch (>= 48 doubles) must not be written by
 // another reduction until every thread has passed a later barrier: callers
@@ -273,7 +242,8 @@ __device__ __forceinline__ void block_sum3_1b(double& a, double& b, double& c, d
   c = sc;
 }
 
-// block_max_sum_max with one workgroup barrier (as block_sum3_1b).
+// Max, sum, max of three per-thread values with one workgroup barrier (as
+// block_sum3_1b).
 // FLOAT_MAX: the maxima hold float values (exact as floats: DPP maxima);
 // otherwise double maxima by shuffles.  The sum by the DPP tree.
 template <bool FLOAT_MAX>
@@ -303,70 +273,6 @@ __device__ __forceinline__ void block_max_sum_max_1b(double& m1, double& s, doub
   m1 = a;
   s = b;
   m2 = c;
-}
-
-// max, sum, max of three per-thread values in one pass (every thread gets
-// them); scratch: >= 52 doubles of LDS.  Contains __syncthreads.
-__device__ __forceinline__ void block_max_sum_max(double& m1, double& s, double& m2, double* scratch) {
-  const int lane = threadIdx.x & (DPM_WAVE - 1), wave = threadIdx.x / DPM_WAVE;
-  const int nw = (blockDim.x + DPM_WAVE - 1) / DPM_WAVE;
-  for (int o = 32; o > 0; o >>= 1) {
-    m1 = fmax(m1, __shfl_down(m1, o, DPM_WAVE));
-    s += __shfl_down(s, o, DPM_WAVE);
-    m2 = fmax(m2, __shfl_down(m2, o, DPM_WAVE));
-  }
-  if (lane == 0) {
-    scratch[wave] = m1;
-    scratch[16 + wave] = s;
-    scratch[32 + wave] = m2;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double a = scratch[0], b = 0.0, c = scratch[32];
-    for (int w = 0; w < nw; w++) {
-      a = fmax(a, scratch[w]);
-      b += scratch[16 + w];
-      c = fmax(c, scratch[32 + w]);
-    }
-    scratch[48] = a;
-    scratch[49] = b;
-    scratch[50] = c;
-  }
-  __syncthreads();
-  m1 = scratch[48];
-  s = scratch[49];
-  m2 = scratch[50];
-  __syncthreads();
-}
-
-// Two block-wide maxima in one pass (every thread gets them); scratch: >= 34
-// values of LDS.  Contains __syncthreads: call from all threads.
-template <typename R>
-__device__ __forceinline__ void block_max2(R& a, R& b, R* scratch) {
-  const int lane = threadIdx.x & (DPM_WAVE - 1), wave = threadIdx.x / DPM_WAVE;
-  const int nw = (blockDim.x + DPM_WAVE - 1) / DPM_WAVE;
-  for (int o = 32; o > 0; o >>= 1) {
-    a = fmax(a, __shfl_down(a, o, DPM_WAVE));
-    b = fmax(b, __shfl_down(b, o, DPM_WAVE));
-  }
-  if (lane == 0) {
-    scratch[wave] = a;
-    scratch[16 + wave] = b;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    R x = scratch[0], y = scratch[16];
-    for (int w = 1; w < nw; w++) {
-      x = fmax(x, scratch[w]);
-      y = fmax(y, scratch[16 + w]);
-    }
-    scratch[32] = x;
-    scratch[33] = y;
-  }
-  __syncthreads();
-  a = scratch[32];
-  b = scratch[33];
-  __syncthreads();
 }
 
 template <typename R>
@@ -406,62 +312,6 @@ __device__ __forceinline__ int block_compact(bool flag, int value, int* list, in
   if (flag) list[off + __popcll(m & ((1ull << lane) - 1ull))] = value;
   __syncthreads();  // the list is complete; every read of counts is done
   return total;
-}
-
-// block_compact that also calls also(slot) on every flagged thread, with
-// the thread's index in the list, before the closing barrier (so what it
-// writes to LDS is visible to every thread on return).
-template <typename Fn>
-__device__ __forceinline__ int block_compact_with(bool flag, int value, int* list, int* counts, Fn&& also) {
-  const int lane = threadIdx.x & (DPM_WAVE - 1), wave = threadIdx.x / DPM_WAVE;
-  const int nw = (blockDim.x + DPM_WAVE - 1) / DPM_WAVE;
-  const unsigned long long m = __ballot(flag);
-  if (lane == 0) counts[wave] = __popcll(m);
-  __syncthreads();
-  int off = 0, total = 0;
-  for (int w = 0; w < nw; w++) {
-    const int c = counts[w];
-    off += w < wave ? c : 0;
-    total += c;
-  }
-  if (flag) {
-    const int slot = off + __popcll(m & ((1ull << lane) - 1ull));
-    list[slot] = value;
-    also(slot);
-  }
-  __syncthreads();
-  return total;
-}
-
-// Two stream compactions in one pass: threads with fa append va to la,
-// threads with fb append vb to lb, in thread order; slot_b is the calling
-// thread's index in lb (meaningful where fb).  counts holds >= 34 ints.
-__device__ __forceinline__ void block_compact2(bool fa, int va, int* la, bool fb, int vb, int* lb, int* counts,
-                                               int& na, int& nb, int& slot_b) {
-  const int lane = threadIdx.x & (DPM_WAVE - 1), wave = threadIdx.x / DPM_WAVE;
-  const int nw = (blockDim.x + DPM_WAVE - 1) / DPM_WAVE;
-  const unsigned long long ma = __ballot(fa), mb = __ballot(fb);
-  const unsigned long long below = (1ull << lane) - 1ull;
-  if (lane == 0) {
-    counts[wave] = __popcll(ma);
-    counts[16 + wave] = __popcll(mb);
-  }
-  __syncthreads();
-  int oa = 0, ob = 0, sa = 0, sb = 0;
-  for (int w = 0; w < nw; w++) {
-    const int ca = counts[w], cb = counts[16 + w];
-    oa += w < wave ? ca : 0;
-    ob += w < wave ? cb : 0;
-    sa += ca;
-    sb += cb;
-  }
-  const int pa = oa + __popcll(ma & below);
-  slot_b = ob + __popcll(mb & below);
-  if (fa) la[pa] = va;
-  if (fb) lb[slot_b] = vb;
-  na = sa;
-  nb = sb;
-  __syncthreads();
 }
 
 // Workgroups are dispatched round-robin over the 8 XCDs of an MI355X
