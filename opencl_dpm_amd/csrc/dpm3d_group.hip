@@ -10,7 +10,7 @@
 //   each) | barrier | substrate, bending, the pair tests of all kept
 //   candidates together | barrier | their sums, in order | barrier | Euler
 //   step | barrier | volume, radius, longest edge | barrier | statistics.
-// Contact, long lists and many candidates take the candidates one by one.
+// Long lists and many candidates take the candidates one by one.
 // Four waves, not one thread per vertex: 11 waves of a 642-vertex cell at 141
 // registers filled a compute unit alone, and every barrier idled it.
 // Against one thread per vertex, a face pass of its own and five barriers per
@@ -25,6 +25,7 @@ constexpr int kGrpSeg = 16;     // candidates of one wave's 64 cells kept ahead 
 constexpr int kGrpSlots = 4;    // candidates whose vertex lists are kept at once
 constexpr int kGrpCap = 64;     // entries of such a list
 constexpr int kGrpTasks = 512;  // partial sums of the adhesion pairs kept at once
+constexpr int kGrpPoints = 512;  // (candidate, vertex) points whose winding numbers are taken together
 constexpr int kGrpSlices = 256;  // partial sums a candidate is cut into, at most
 static_assert(kGrpSlots == 4 && kGrpCap <= 127 && kGrpSlices <= kGrpTasks, "the task search and the records' fields");
 
@@ -33,7 +34,7 @@ static_assert(kGrpSlots == 4 && kGrpCap <= 127 && kGrpSlices <= kGrpTasks, "the 
 // vertices over the bending sums); within that, winding directions, then
 // partial sums.
 struct LdsGroup {
-  size_t own, sb, faces, down, rec, seg, segst, clist, glist, plist, gath, cnt, red, slots, slot, acc, wb, nlist, mlist,
+  size_t own, sb, faces, down, rec, seg, segst, clist, glist, plist, gath, cnt, red, slots, slot, pw, acc, wb, nlist, mlist,
       smap, ut, total;
 };
 __host__ __device__ inline int group_winding_waves(int nv, int rsize) {
@@ -59,17 +60,19 @@ __host__ __device__ inline LdsGroup ldsg_layout(int nv, int nf, int ww, int rsiz
   L.cnt = o;   o = al(o + 4u * 48u);
   L.red = o;   o = al(o + 8u * 6u * kGrpWaves);
   const size_t z = o;
+  const size_t wind = 4u * rs * n * (size_t)ww;
+  const bool points = nv <= kGrpThreads;  // contact points of all candidates together
   L.slots = o;
   L.slot = al(3u * rs * kGrpCap + 2u * kGrpCap + 2u * n);  // positions, own vertices, vertex -> place
-  L.acc = al(o + kGrpSlots * L.slot);
-  const size_t fast = L.acc + 4u * rs * kGrpTasks;
+  L.pw = al(o + kGrpSlots * L.slot);  // the points' winding numbers
+  L.acc = al(L.pw + (points ? rs * kGrpPoints : 0u));  // winding directions, then partial sums
+  const size_t fast = L.acc + (points && wind > 4u * rs * kGrpTasks ? wind : 4u * rs * kGrpTasks);
   o = z;
   L.wb = o;    o = al(o + rs * n);
   L.nlist = o; o = al(o + 2u * n);
   L.mlist = o; o = al(o + 2u * n);
   L.smap = o;  o = al(o + 2u * n);
   L.ut = o;
-  const size_t wind = 4u * rs * n * (size_t)ww;
   const size_t sums = 4u * rs * (n > (size_t)kGrpSlices ? n : (size_t)kGrpSlices);
   o += wind > sums ? wind : sums;
   L.total = al(o > fast ? o : fast);
@@ -189,7 +192,10 @@ __device__ __forceinline__ void k3d_step_body() {
   }
   for (int f = tid; f < nf; f += NT) sf[f] = reinterpret_cast<const unsigned*>(rows)[f];
   for (int i = tid; i < (nv + 3) / 4; i += NT) down4[i] = 0u;
-  if (tid == 0) *short_edge = 0;
+  if (tid == 0) {
+    *short_edge = 0;
+    one[3] = 0;
+  }
 #pragma unroll
   for (int k = 0; k < VPT; k++) {
     const int v = tid + k * NT;
@@ -635,6 +641,41 @@ __device__ __forceinline__ void k3d_step_body() {
     }
     return Q4<R>{Fa.x, Fa.y, Fa.z, (R)cnt_own};
   };
+  // Own vertex k's contact with cell cj2 at winding number wv.
+  auto touch = [&](int k, int cj2, R wv, V3<R> sh) __attribute__((always_inline)) {
+    const int v = tid + k * NT;
+    const size_t pidx = (base + v) * (size_t)a->ncmax + (size_t)(cj2 - cb);
+    if (PROBE && a->p_winding) a->p_winding[pidx] = (float)wv;
+    if (fabs(wv) < R(1e-6f)) return;
+    const V3<R> dir = vnormalize(vsub(Ci, P[k]));
+    const R mag = fabs(wv) * R(0.5f) * Kre;
+    F[k] = vadd(F[k], vscale(dir, mag));
+    n_contact++;
+    wsum[k] += fabs(wv);
+    if (a->rec_cell) {
+      if (npart[k] < DPM3D_MAXPART) {
+        const size_t r = (base + v) * DPM3D_MAXPART + npart[k];
+        a->rec_cell[r] = cj2;
+        a->rec_w[r] = wv;
+        a->rec_shift[3 * r] = sh.x;
+        a->rec_shift[3 * r + 1] = sh.y;
+        a->rec_shift[3 * r + 2] = sh.z;
+      } else {
+        atomicOr(a->rec_overflow, 1);
+      }
+      npart[k]++;
+    }
+    if (PROBE && a->p_contact) a->p_contact[pidx] = 1;
+    if (PROBE && a->p_contact_key) {  // count, then key sum of the partner cells
+      atomicAdd(&a->p_contact_key[2 * (base + v)], 1u);
+      atomicAdd(&a->p_contact_key[2 * (base + v) + 1], cell_key(cj2 - cb));
+    }
+  };
+  auto shift_to = [&](const CellStat<R>& stj) __attribute__((always_inline)) -> V3<R> {
+    if (!pbc) return V3<R>{R(0), R(0), R(0)};
+    return V3<R>{image_shift(Ci.x - stj.cx, L, invL), image_shift(Ci.y - stj.cy, L, invL),
+                 image_shift(Ci.z - stj.cz, L, invL)};
+  };
   // A candidate by itself: lane b of cj_l, st_l; passes 1 contact, 2 adhesion.
   auto take_one = [&](int b, int passes) __attribute__((always_inline)) {
     const int cj2 = from_lane(cj_l, b);
@@ -694,37 +735,8 @@ __device__ __forceinline__ void k3d_step_body() {
       }
       __syncthreads();
 #pragma unroll
-      for (int k = 0; k < VPT; k++) {
-        if (!need[k]) continue;
-        const int v = tid + k * NT;
-        const R wv = wb[v];
-        const size_t pidx = (base + v) * (size_t)a->ncmax + (size_t)(cj2 - cb);
-        if (PROBE && a->p_winding) a->p_winding[pidx] = (float)wv;
-        if (fabs(wv) < R(1e-6f)) continue;
-        const V3<R> dir = vnormalize(vsub(Ci, P[k]));
-        const R mag = fabs(wv) * R(0.5f) * Kre;
-        F[k] = vadd(F[k], vscale(dir, mag));
-        n_contact++;
-        wsum[k] += fabs(wv);
-        if (a->rec_cell) {
-          if (npart[k] < DPM3D_MAXPART) {
-            const size_t r = (base + v) * DPM3D_MAXPART + npart[k];
-            a->rec_cell[r] = cj2;
-            a->rec_w[r] = wv;
-            a->rec_shift[3 * r] = sh.x;
-            a->rec_shift[3 * r + 1] = sh.y;
-            a->rec_shift[3 * r + 2] = sh.z;
-          } else {
-            atomicOr(a->rec_overflow, 1);
-          }
-          npart[k]++;
-        }
-        if (PROBE && a->p_contact) a->p_contact[pidx] = 1;
-        if (PROBE && a->p_contact_key) {  // count, then key sum of the partner cells
-          atomicAdd(&a->p_contact_key[2 * (base + v)], 1u);
-          atomicAdd(&a->p_contact_key[2 * (base + v) + 1], cell_key(cj2 - cb));
-        }
-      }
+      for (int k = 0; k < VPT; k++)
+        if (need[k]) touch(k, cj2, wb[tid + k * NT], sh);
     }
     if (passes & 2) {  // block-uniform
       const R L0j = fmax(stj.l0, R(1e-12f));
@@ -787,13 +799,95 @@ __device__ __forceinline__ void k3d_step_body() {
     n_cand += (unsigned)__popcll(m);
     const int r = ((m >> lane) & 1ull) ? rec[lane] : 0;
     unsigned long long left = __ballot((r & 3) != 0);
-    if (__ballot((r & 1) || ((r & 2) && !(r & 4)))) {  // block-uniform: contact, or lists that do not fit
+    const unsigned long long touching = __ballot((r & 1) != 0);
+    const unsigned long long below = (1ull << lane) - 1ull;
+    // block-uniform: lists that do not fit, or contact beyond the kept slots
+    // (and any contact of a cell of several vertices a thread: the registers of
+    // its points cost the 642-vertex step 133 -> 166 us at 4096 cells)
+    constexpr bool kTogether = VPT == 1;
+    bool each = __ballot(((r & 2) && !(r & 4)) || ((r & 1) && (!kTogether || __popcll(m & below) >= kGrpSlots))) != 0ull;
+    // Contact: the points of all touching candidates in one list, the waves
+    // taking them in turn; a candidate's vertices come from the L2.  (Taken
+    // candidate after candidate, each with its own staging and barriers, a
+    // cell with contacts held a step of 256 cells for 24 us against 16.)
+    int at[VPT][kGrpSlots];
+#pragma unroll
+    for (int k = 0; k < VPT; k++)
+#pragma unroll
+      for (int c = 0; c < kGrpSlots; c++) at[k][c] = -1;
+    if (kTogether && touching && !each) {
+      unsigned short* points = reinterpret_cast<unsigned short*>(smem + LG.plist);
+      R* pw = reinterpret_cast<R*>(smem + LG.pw);
+      unsigned long long w = m;
+#pragma unroll
+      for (int c = 0; c < kGrpSlots; c++) {
+        const int b = w ? __ffsll((long long)w) - 1 : 0;
+        if (w && ((touching >> b) & 1ull)) {
+          const CellStat<R> stj = from_lane(st_l, b);
+          const V3<R> sh = shift_to(stj);
+          const V3<R> Cj = {stj.cx + sh.x, stj.cy + sh.y, stj.cz + sh.z};
+          const R rj = (stj.r + contact_margin(stj.r, stj.em)) * R(1.0001f) + R(1e-6f);
+#pragma unroll
+          for (int k = 0; k < VPT; k++) {
+            const int v = tid + k * NT;
+            bool need = false;
+            if (v < nv) {
+              const V3<R> d = vsub(P[k], Cj);
+              need = vdot(d, d) <= rj * rj;
+            }
+            const unsigned long long mn = __ballot(need);
+            if (mn) {
+              int p = 0;
+              if (lane == 0) p = atomicAdd(&one[3], (int)__popcll(mn));
+              p = __builtin_amdgcn_readfirstlane(p) + lanes_below(mn);
+              if (need) {
+                at[k][c] = p;
+                if (p < kGrpPoints) points[p] = (unsigned short)(c << 10 | v);
+              }
+            }
+          }
+        }
+        w &= w - 1ull;
+      }
+      __syncthreads();
+      const int np = one[3];
+      each = np > kGrpPoints;  // block-uniform
+      if (!each) {
+        if (wave < ww) {
+          Q4<R>* ut = reinterpret_cast<Q4<R>*>(smem + LG.acc) + (size_t)wave * nv;
+          for (int pi = wave; pi < np; pi += ww) {  // wave-uniform
+            const int e = __builtin_amdgcn_readfirstlane((int)points[pi]), c = e >> 10;
+            unsigned long long u = m;
+            for (int q = 0; q < c; q++) u &= u - 1ull;
+            const int b = __ffsll((long long)u) - 1;
+            const CellStat<R> stj = from_lane(st_l, b);
+            const V3<R> sh = shift_to(stj);
+            const V3<R> Cj = {stj.cx + sh.x, stj.cy + sh.y, stj.cz + sh.z};
+            const R mj = contact_margin(stj.r, stj.em);
+            const size_t bj = (size_t)from_lane(cj_l, b) * nv;
+            const V3<R> Pv = lds_v(sx, sy, sz, e & 1023);
+            // a point beyond the margin from j's hull has winding number 0
+            R wv = R(0);
+            if (!outside_by_margin(a->xin + bj, a->yin + bj, a->zin + bj, nv, stj.cx, stj.cy, stj.cz, Cj,
+                                   vsub(Pv, Cj), mj, stj.r)) {
+              wv = winding_w(a->xin + bj, a->yin + bj, a->zin + bj, sf, ut, nv, nf, sh, Pv);
+              n_wind++;
+            }
+            if (lane == 0) pw[pi] = wv;
+          }
+        }
+      }
+      __syncthreads();  // the winding numbers are there, the count is read
+      if (tid == 0) one[3] = 0;  // for the next candidates (a barrier ahead of them)
+    }
+    if (each) {  // block-uniform
       for (; left; left &= left - 1ull) {
         const int b = __ffsll((long long)left) - 1;
         take_one(b, from_lane(r, b) & 3);
       }
       return;
     }
+    const R* pw = reinterpret_cast<const R*>(smem + LG.pw);
     Q4<R>* acc = reinterpret_cast<Q4<R>*>(smem + LG.acc);
     auto place_of = [&](int o) __attribute__((always_inline)) {  // lists of the o-th candidate of m
       return smem + LG.slots + (size_t)o * LG.slot;
@@ -804,7 +898,7 @@ __device__ __forceinline__ void k3d_step_body() {
       for (int c = 0; c < kGrpSlots; c++) {
         if (left) {
           const int b = __ffsll((long long)left) - 1, rb = from_lane(r, b);
-          const int tasks = ((rb >> 10) & 127) * ((rb >> 17) & 127);
+          const int tasks = rb & 2 ? ((rb >> 10) & 127) * ((rb >> 17) & 127) : 0;
           if (total + tasks <= kGrpTasks) {
             lanes[c] = b;
             total += tasks;
@@ -838,6 +932,16 @@ __device__ __forceinline__ void k3d_step_body() {
       for (int c = 0; c < kGrpSlots; c++) {
         if (c >= n) break;  // block-uniform
         const int b = lanes[c], rb = from_lane(r, b), nmine = (rb >> 10) & 127, S = (rb >> 17) & 127;
+        if (kTogether && (rb & 1)) {  // block-uniform; at[][] by the candidate's slot
+          const int cj2 = from_lane(cj_l, b), o = __popcll(m & ((1ull << b) - 1ull));
+          const V3<R> sh = shift_to(from_lane(st_l, b));
+#pragma unroll
+          for (int k = 0; k < VPT; k++) {
+            const int p = o == 0 ? at[k][0] : o == 1 ? at[k][1] : o == 2 ? at[k][2] : at[k][3];
+            if (p >= 0) touch(k, cj2, pw[p], sh);
+          }
+        }
+        if (!(rb & 2)) continue;
         const Q4<R>* sums = acc + (c > 0 ? ends[c - 1] : 0);
         const unsigned short* place =
             reinterpret_cast<const unsigned short*>(
