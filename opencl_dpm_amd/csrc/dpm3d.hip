@@ -167,7 +167,7 @@ struct Step3D {
   const int* nl_stale;    // per tissue: this step makes the lists
   int* nl_stale_out;      // the same for the next step, set here
   int* nl_stale_clear;    // the same for the step after, cleared here
-  R nl_skin;
+  const R* nl_skin;       // in device memory: a captured step reads the current one
 };
 
 // The step kernels' arguments, read where they are used: the struct is their

@@ -1038,7 +1038,7 @@ __device__ __forceinline__ void k3d_step_body() {
             cand = in_reach(stj);
           }
           if (relist) {
-            const bool nr = cj < ce && cj != ci && near_list_takes(sti, stj, pbc, L, invL, do_contact, do_adh, a->nl_skin);
+            const bool nr = cj < ce && cj != ci && near_list_takes(sti, stj, pbc, L, invL, do_contact, do_adh, *a->nl_skin);
             const int n = block_compact(nr, cj, plist, cnt);
             if (tid < n && nnl + tid < kNearList) a->nl_idx[(size_t)ci * kNearList + nnl + tid] = plist[tid];
             nnl += n;
@@ -1178,7 +1178,7 @@ __device__ __forceinline__ void k3d_step_body() {
       a->st_out[ci] = make_cell_stat<R>(C.x, C.y, C.z, r, em, l0i);
       a->vol_out[ci] = fabs(vol / 6.0);
       a->em_out[ci] = em;
-      if (nl_on && near_list_moved(nl_ref, C, r, em, a->nl_skin)) a->nl_stale_out[t] = 1;
+      if (nl_on && near_list_moved(nl_ref, C, r, em, *a->nl_skin)) a->nl_stale_out[t] = 1;
     }
   }
   if (a->counters) {

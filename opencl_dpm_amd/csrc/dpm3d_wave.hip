@@ -504,7 +504,7 @@ __device__ __forceinline__ void k3d_wstep_body() {
         }
         if (relist) {  // wave-uniform
           const bool nr =
-              cj < ce && cj != ci && near_list_takes(sti, stj, pbc, L, invL, do_contact, do_adh, a->nl_skin);
+              cj < ce && cj != ci && near_list_takes(sti, stj, pbc, L, invL, do_contact, do_adh, *a->nl_skin);
           const unsigned long long m = __ballot(nr);
           const int slot = nnl + lanes_below(m);
           if (nr && slot < kNearList) a->nl_idx[(size_t)ci * kNearList + slot] = cj;
@@ -848,7 +848,7 @@ __device__ __forceinline__ void k3d_wstep_body() {
       if (nl_on) {
         CellStat<R> ref = sti;
         if (!relist) ref = a->nl_ref[ci];
-        if (near_list_moved(ref, C, stn.r, stn.em, a->nl_skin)) a->nl_stale_out[t] = 1;
+        if (near_list_moved(ref, C, stn.r, stn.em, *a->nl_skin)) a->nl_stale_out[t] = 1;
       }
       a->vol_out[ci] = fabs(vol / 6.0);
       a->em_out[ci] = em;

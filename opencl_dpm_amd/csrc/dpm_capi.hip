@@ -154,7 +154,7 @@ struct dpm_tissue {
   // positions or a parameter change
   int *nl_cnt = nullptr, *nl_idx = nullptr, *nl_stale = nullptr;  // marks: [4 * T]
   void* nl_ref = nullptr;
-  float nl_skin = 0.0f;
+  void* nl_skin = nullptr;  // one real: read by captured steps too, so not a kernel argument
   int nl_phase = 0;
   bool nl_ok = false;
 
@@ -617,6 +617,7 @@ static int create3d(const dpm3d_desc* d, dpm_tissue** out, int rs) {
     rc |= A(&h->nl_idx, (size_t)C * kNearList);
     rc |= A(&h->nl_stale, 4 * (size_t)T);
     rc |= AR(&h->nl_ref, (size_t)C * kStatWords);
+    rc |= AR(&h->nl_skin, 1);
   }
   if (rc) { delete h; return DPM_ENOMEM; }
   h->tissue_begin_h.assign(d->cell_begin, d->cell_begin + T + 1);
@@ -776,10 +777,14 @@ extern "C" int dpm3d_set_cell_params(dpm_tissue* h, const float* Kv, const float
   if (Kb) TRY(upload(h->Kb, Kb, C, s));
   if (v0) TRY(upload(h->v0, v0, C, s));
   h->nl_ok = false;
-  if (v0) {  // the skin: 0.15 radii of the smallest cell at rest
+  double skin_d = 0.0;
+  float skin = 0.0f;
+  if (v0 && h->nl_skin) {  // the skin: 0.15 radii of the smallest cell at rest
     float vmin = v0[0];
     for (int c = 1; c < C; c++) vmin = std::min(vmin, v0[c]);
-    h->nl_skin = 0.15f * std::cbrt(0.2387324f * vmin);
+    skin = 0.15f * std::cbrt(0.2387324f * vmin);
+    skin_d = (double)skin;
+    TRY(h->rs == 8 ? upload((double*)h->nl_skin, &skin_d, 1, s) : upload((float*)h->nl_skin, &skin, 1, s));
   }
   if (a0) {
     TRY(upload(h->a0, a0, C, s));
@@ -1057,7 +1062,7 @@ static int launch_step3d(dpm_tissue* h, int in, int phase, float dt, int flags) 
     a.nl_stale = h->nl_stale + (size_t)phase * h->T;
     a.nl_stale_out = h->nl_stale + (size_t)((phase + 1) & 3) * h->T;
     a.nl_stale_clear = h->nl_stale + (size_t)((phase + 2) & 3) * h->T;
-    a.nl_skin = h->nl_skin;
+    a.nl_skin = (decltype(a.nl_skin))h->nl_skin;
   });
 }
 
