@@ -2104,6 +2104,10 @@ extern "C" int dpm2d_set_tissue_params(dpm_tissue* h, const float* L, const int*
   if (pbc) TRY(upload(h->tpbc, pbc, T, s));
   if (Kre) TRY(upload(h->tKre, Kre, T, s));
   if (Kat) TRY(upload(h->tKat, Kat, T, s));
+  if (h->wide_graph && h->mask != (mask & DPM2D_ALL_TERMS)) {  // captured with the old terms
+    (void)hipGraphExecDestroy(h->wide_graph);
+    h->wide_graph = nullptr;
+  }
   h->mask = mask & DPM2D_ALL_TERMS;
   HIPCHECK(hipStreamSynchronize(s));
   return DPM_OK;
