@@ -878,24 +878,28 @@ struct Vjp3D {
 };
 
 // LDS of the adjoint kernel (byte offsets): positions, lambda, bending
-// scratch [3 nv] each, face table, per (face, corner) contributions, and
-// reduction scratch — disjoint, as every region is live at once.
+// scratch [3 nv] each, face table, per (face, corner) contributions, and 32
+// doubles for two sums.  The other sums' waves (at most 16) write where
+// nothing is read any more: the first three to the bending scratch, before
+// bending; the last six to the contributions after bending (gathered ahead of
+// its barrier), without bending to the unused bending scratch.
 struct LdsVjpLayout {
   size_t x, lam, sb, faces, fc, red, total;
 };
 __host__ __device__ inline LdsVjpLayout ldsvjp_layout(int nv, int nf, int rsize) {
   LdsVjpLayout L;
-  const size_t rs = (size_t)rsize;
+  const size_t rs = (size_t)rsize, sums = 8u * 16u * 6u;
+  auto room = [&](size_t n) { return n > sums ? n : sums; };
   size_t o = 0;
   L.x = o;     o += 3u * rs * (size_t)nv;
   L.lam = o;   o += 3u * rs * (size_t)nv;
-  L.sb = o;    o += 3u * rs * (size_t)nv;
+  L.sb = o;    o += room(3u * rs * (size_t)nv);
   o = (o + 7u) & ~(size_t)7u;
   L.faces = o; o += 8u * (size_t)nf;
   o = (o + 15u) & ~(size_t)15u;
-  L.fc = o;    o += 9u * rs * (size_t)nf;
+  L.fc = o;    o += room(9u * rs * (size_t)nf);
   o = (o + 7u) & ~(size_t)7u;
-  L.red = o;   o += 8u * 16u * 11u;  // three, two and six sums over at most 16 waves
+  L.red = o;   o += 8u * 32u;
   L.total = o;
   return L;
 }
@@ -988,7 +992,7 @@ __device__ void k3d_vjp_body(const Vjp3D<R>& a) {
     p[1] += (double)l.sy[v];
     p[2] += (double)l.sz[v];
   }
-  block_sums_1b(p, l.red);
+  block_sums_1b(p, reinterpret_cast<double*>(l.sb));
   const V3<R> C = {(R)(p[0] / nv), (R)(p[1] / nv), (R)(p[2] / nv)};
   double vol = 0.0, S1 = 0.0;
   const bool vol_on = (mask & M_VOLUME) && Kvi != R(0);
@@ -1006,7 +1010,7 @@ __device__ void k3d_vjp_body(const Vjp3D<R>& a) {
     }
   }
   double vs[2] = {vol, S1};
-  block_sums_1b(vs, l.red + 48);
+  block_sums_1b(vs, l.red);
   vol = fabs(vs[0] / 6.0);
   S1 = vs[1] / 6.0;
   const R strain = (R)(vol / (double)v0i - 1.0);
@@ -1112,7 +1116,8 @@ __device__ void k3d_vjp_body(const Vjp3D<R>& a) {
 
   // bending: mu += -Kb L (L lambda); dL/dKb = -(L lambda).(L x)
   double gKb = 0.0;
-  if ((mask & M_BENDING) && Kbi != R(0)) {
+  const bool bend_on = (mask & M_BENDING) && Kbi != R(0);
+  if (bend_on) {
     if (own) {
       V3<R> sl = zero, sx = zero;
       const V3<R> P = lds_v(l.sx, l.sy, l.sz, tid), lt = lds_v(l.nx, l.ny, l.nz, tid);
@@ -1199,7 +1204,7 @@ __device__ void k3d_vjp_body(const Vjp3D<R>& a) {
     }
   }
   double g[6] = {Lcx, Lcy, Lcz, gKa, gKs, gKb};
-  block_sums_1b(g, l.red + 80);
+  block_sums_1b(g, reinterpret_cast<double*>(bend_on ? l.fcx : l.sb));
   Lcx = g[0], Lcy = g[1], Lcz = g[2], gKa = g[3], gKs = g[4], gKb = g[5];
   if (own) {
     // the centre of mass moves with each vertex by 1/nv
