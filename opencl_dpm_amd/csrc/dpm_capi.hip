@@ -336,6 +336,15 @@ static int run_slices(dpm_tissue* h, size_t n, size_t bytes, Body body) {
   return DPM_OK;
 }
 
+// Launches a transfer kernel; its own error only (hipGetLastError would also
+// give what an earlier call of this thread left).
+template <typename... A>
+static hipError_t launch_slice(void (*kernel)(A...), size_t verts, hipStream_t s, std::common_type_t<A>... args) {
+  void* p[] = {&args...};
+  return hipLaunchKernel(reinterpret_cast<const void*>(kernel), dim3((unsigned)((verts + kXferVerts - 1) / kXferVerts)),
+                         dim3(256), p, 0, s);
+}
+
 // Host array of n vertices, NC interleaved components -> c0, c1, c2 on the
 // device, in stream order (the caller's array is free on return).  check:
 // refuses non-finite values (what was written by then stays written).
@@ -355,9 +364,9 @@ static int upload_split(dpm_tissue* h, const H* src, size_t n, R* c0, R* c1, R* 
       H* slot = reinterpret_cast<H*>(x.host + (size_t)s * x.slot);
       const bool finite = copy_finite(slot, src + v * NC, m * NC);
       if (check && !finite) return fail(DPM_ENONFINITE, "Non-finite vertex coordinates");
-      k_split<H, R, NC><<<(int)((m + kXferVerts - 1) / kXferVerts), 256, 0, h->stream>>>(
-          slot, c0 + v, c1 + v, NC == 3 ? c2 + v : nullptr, lo ? lo + v : nullptr, n, (int)m);
-      HIPCHECK(hipGetLastError());
+      HIPCHECK(launch_slice(
+          &k_split<H, R, NC>, m, h->stream, slot, c0 + v, c1 + v, NC == 3 ? c2 + v : nullptr, lo ? lo + v : nullptr, n,
+          (int)m));
       HIPCHECK(hipEventRecord(x.ev[s], h->stream));
       x.pending[s] = true;
       v += m;
@@ -377,10 +386,9 @@ static int download_merge(dpm_tissue* h, H* dst, size_t n, const R* c0, const R*
     auto launch = [&](size_t v, int s) -> int {
       const size_t m = std::min(per, b - v);
       if (x.pending[s]) HIPCHECK(hipEventSynchronize(x.ev[s]));
-      k_merge<H, R, NC><<<(int)((m + kXferVerts - 1) / kXferVerts), 256, 0, h->stream>>>(
-          reinterpret_cast<H*>(x.host + (size_t)s * x.slot), c0 + v, c1 + v, NC == 3 ? c2 + v : nullptr,
-          lo ? lo + v : nullptr, n, (int)m);
-      HIPCHECK(hipGetLastError());
+      HIPCHECK(launch_slice(
+          &k_merge<H, R, NC>, m, h->stream, reinterpret_cast<H*>(x.host + (size_t)s * x.slot), c0 + v, c1 + v,
+          NC == 3 ? c2 + v : nullptr, lo ? lo + v : nullptr, n, (int)m));
       HIPCHECK(hipEventRecord(x.ev[s], h->stream));
       x.pending[s] = true;
       return DPM_OK;
@@ -660,8 +668,9 @@ static int create3d(const dpm3d_desc* d, dpm_tissue** out, int rs) {
   for (bool probe : {false, true})
     (void)hipFuncSetAttribute(gstep_kernel(rs, nv, nf, probe, h->many_g), hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)h->lds_g);
-  (void)hipFuncSetAttribute(rs == 8 ? (const void*)k3d_bin_f64 : (const void*)k3d_bin_f32,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->bin_lds);
+  if ((int)h->bin_lds <= max_lds_per_block(h->device))  // (beyond, steps with bins fail at their launch)
+    (void)hipFuncSetAttribute(rs == 8 ? (const void*)k3d_bin_f64 : (const void*)k3d_bin_f32,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->bin_lds);
   // the step kernels' topology image: faces packed 10 bits per index (staged in
   // LDS), incidence and neighbour rows of 16-bit entries (0xffff: none)
   const Lds3DWave LW = ldsw_layout(nv, nf, 1, rs);
@@ -706,11 +715,13 @@ static int create3d(const dpm3d_desc* d, dpm_tissue** out, int rs) {
     }
   }
   h->lds_vjp = ldsvjp_layout(nv, nf, rs).total;
-  (void)hipFuncSetAttribute(rs == 8 ? (const void*)k3d_vjp_f64 : (const void*)k3d_vjp_f32,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->lds_vjp);
-  if (rs == 8)
-    (void)hipFuncSetAttribute((const void*)k3d_vjp_f64_t256, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)h->lds_vjp);
+  if ((int)h->lds_vjp <= max_lds_per_block(h->device)) {  // (beyond, dpm3d_trajectory refuses)
+    (void)hipFuncSetAttribute(rs == 8 ? (const void*)k3d_vjp_f64 : (const void*)k3d_vjp_f32,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->lds_vjp);
+    if (rs == 8)
+      (void)hipFuncSetAttribute((const void*)k3d_vjp_f64_t256, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)h->lds_vjp);
+  }
   *out = h;
   return DPM_OK;
 }

@@ -1,5 +1,5 @@
 """The double adjoint takes closed meshes up to the LDS of one workgroup, 706
-vertices.  One step's J_x^T lambda there against central
+vertices, and refuses one more.  One step's J_x^T lambda there against central
 differences of the oracle's forces in double, with and without bending (the
 kernel's last sums lie in other scratch then)."""
 import numpy as np
@@ -62,3 +62,13 @@ def test_largest_mesh(mask):
         print(f"mask {mask}: adjoint {ad:.10e} differences {fd:.10e}", flush=True)
         # the differences' rounding: forces of order 1 with 1e-16 over 1e-6, about 4000 terms
         assert abs(ad - fd) < 1e-6 * abs(fd) + 1e-7
+
+
+def test_a_vertex_more_is_refused_by_the_adjoint_only():
+    t, X, force = tissue(707, SHAPE)
+    t.set_positions(X)
+    t.euler(1, 0.002)
+    # grouping of the sums, forces of order 1 (test_gpu_group_form's bound)
+    np.testing.assert_allclose(t.forces(), force(X), atol=1e-9)
+    with pytest.raises(capi.DPMError, match="adjoint kernel"):
+        t.trajectory(1, 0.002, 1)
