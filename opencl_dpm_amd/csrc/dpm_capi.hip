@@ -295,13 +295,22 @@ static int ensure_slots(dpm_tissue* h, size_t bytes) {
   const size_t slot = n > 1 ? kXferSlot : std::max<size_t>((bytes + 4095) & ~(size_t)4095, 4096);
   if (x.host && x.n >= n && x.slot >= slot) return DPM_OK;
   x.release();
-  if (hipHostMalloc(reinterpret_cast<void**>(&x.host), slot * n, hipHostMallocCoherent) != hipSuccess) {
+  // the events belong to the current device and are recorded on the handle's
+  // stream, which may be another's: a thread starts with device 0
+  int dev = h->device;
+  (void)hipGetDevice(&dev);
+  if (dev != h->device) HIPCHECK(hipSetDevice(h->device));
+  hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&x.host), slot * n, hipHostMallocCoherent);
+  if (e == hipSuccess) {
+    x.slot = slot;
+    x.n = n;
+    for (int i = 0; i < n && e == hipSuccess; i++) e = hipEventCreateWithFlags(&x.ev[i], hipEventDisableTiming);
+    if (e != hipSuccess) x.release();
+  } else {
     x.host = nullptr;
-    return fail(DPM_ENOMEM, "hipHostMalloc: pinned transfer slots");
   }
-  x.slot = slot;
-  x.n = n;
-  for (int i = 0; i < n; i++) HIPCHECK(hipEventCreateWithFlags(&x.ev[i], hipEventDisableTiming));
+  if (dev != h->device) (void)hipSetDevice(dev);
+  if (e != hipSuccess) return fail(DPM_ENOMEM, std::string("pinned transfer slots: ") + hipGetErrorString(e));
   return DPM_OK;
 }
 
