@@ -27,7 +27,7 @@
 //   AllVertAttraction       :313-364  (not launched by the reference host)
 //   EulerPosition           :371-381
 // plus graph-Laplacian bending, which has no reference kernel.
-#include "dpm_device.h"
+#include "dpm3d_pairs.h"
 
 using namespace dpm;
 
@@ -46,38 +46,6 @@ enum : int {
   F_WRITE_FORCES = 1,
   F_MOVE = 2,
 };
-
-// Per-cell statistics of a step's input positions (written by the previous
-// step's epilogue or k3d_stats): centre of mass, bounding radius, longest
-// edge, target edge length l0, and 1 / max(l0, 1e-12) in double (the
-// adhesion term's, divided once per cell instead of once per pair).  Eight
-// reals either way (32 bytes in float, 64 in double).
-template <typename R>
-struct CellStat;
-template <>
-struct CellStat<float> {
-  float cx, cy, cz, r;
-  float em, l0;
-  double inv_l0;
-};
-template <>
-struct CellStat<double> {
-  double cx, cy, cz, r;
-  double em, l0;
-  double inv_l0, pad;
-};
-template <typename R>
-__host__ __device__ inline CellStat<R> make_cell_stat(R cx, R cy, R cz, R r, R em, R l0) {
-  CellStat<R> s{};
-  s.cx = cx;
-  s.cy = cy;
-  s.cz = cz;
-  s.r = r;
-  s.em = em;
-  s.l0 = l0;
-  s.inv_l0 = 1.0 / (double)(l0 > R(1e-12f) ? l0 : R(1e-12f));
-  return s;
-}
 
 template <typename R>
 struct alignas(4 * sizeof(R)) Q4 {
@@ -203,36 +171,6 @@ __device__ __forceinline__ R two_sum(R a, R b, R& e) {
 template <typename R>
 __device__ __forceinline__ R cell_l0(const float* a0, int c) {
   return sqrt(R(4) * (R)a0[c]) / sqrt(R(3));
-}
-
-// Periodic shift of cell j toward cell i along one axis, L round(d / L)
-// with d = C_i - C_j (Cell3D_Kernel.cl:279-281).  The quotient is taken as
-// a product with 1/L (within two ulp of the quotient); only where that
-// product lies within 1e-5 (relative) of a half-integer can the two round
-// differently, and there the division itself decides.
-template <typename R>
-__device__ __forceinline__ R image_shift(R d, R L, R invL) {
-  const R q = d * invL;
-  R n = round(q);
-  if (fabs(fabs(q - n) - R(0.5f)) < R(1e-5f) * (R(1) + fabs(q))) n = round(d / L);
-  return L * n;
-}
-
-// Culling reach added to a cell's bounding radius for the winding-number
-// test.  Every face of cell j lies inside its bounding sphere R_j, so a
-// point p outside R_j + m_j is at least m_j from every face and edge of j,
-// and outside j's convex hull: its exact winding number is 0.  An edge of
-// length <= e seen from distance >= d subtends at most 2 atan(e / 2d); with
-// d >= 0.4 e that is <= 102.7 degrees, so every pair of the unit vectors
-// u, v, w toward a face's corners has a dot product >= -0.2195 and the
-// reference's denominator 1 + u.v + v.w + w.u (Cell3D_Kernel.cl:293) is
-// >= 0.34: no face is skipped (denom < 1e-8), and the float sum of the
-// face angles is rounding noise about a true 0, far below the 1e-6 pair
-// threshold (Cell3D_Kernel.cl:303) — the pair is absent in the reference
-// arithmetic too.  m_j = 0.4 e_max(j) (with slack for float rounding).
-template <typename R>
-__device__ __forceinline__ R contact_margin(R Rj, R emax_j) {
-  return emax_j * R(0.4004f) + R(1e-6f) * Rj;
 }
 
 // Exact outside test ahead of a winding number, evaluated by one whole wave
@@ -534,49 +472,6 @@ __device__ __forceinline__ V3<R> substrate_corner(V3<R> pos, V3<R> C, R Ks, R ks
     }
   }
   return c;
-}
-
-// ---------------------------------------------------------- candidate lists
-//
-// The scan tests every cell of the tissue for every cell and step: at 4096
-// cells of 642 vertices a third of the step (27 of 86 kcycles of a
-// workgroup).  A step that finds its tissue's lists stale scans as before and
-// also keeps, per cell, the cells within `skin` of its reach; the following
-// steps apply the scan's own test to those entries, in the same ascending
-// order, so the candidates are the scan's, bit for bit.
-// The lists hold as long as no pair can have come closer than the skin: a
-// cell's excess is its centre's displacement since the lists were made plus
-// what its radius and contact margin grew; the reach of a pair grows by no
-// more than both excesses, its minimum-image distance shrinks by no more.
-// The step that moves a cell past 0.49 of the skin marks the tissue's lists
-// stale for the next one (not below half: float rounding has 2 % of the skin,
-// which is thousands of ulp of the coordinates).  Three sets of marks: the
-// one read, the one written for the next step, the one cleared for the step
-// after.
-constexpr int kNearList = DPM_WAVE;
-
-template <typename R>
-__device__ __forceinline__ bool near_list_moved(const CellStat<R>& ref, V3<R> C, R r, R em, R skin) {
-  const V3<R> d = {C.x - ref.cx, C.y - ref.cy, C.z - ref.cz};
-  const R excess = sqrt(vdot(d, d)) + R(1.0002f) * fmax(R(0), r - ref.r) + R(0.41f) * fmax(R(0), em - ref.em);
-  return !(excess <= R(0.49f) * skin);  // a NaN is stale
-}
-
-// The scan's test with the skin: within reach + skin by either contact or
-// adhesion, or the pair takes every image.
-template <typename R>
-__device__ __forceinline__ bool near_list_takes(const CellStat<R>& sti, const CellStat<R>& stj, bool pbc, R L, R invL,
-                                                bool contact, bool adhesion, R skin) {
-  V3<R> sh = {R(0), R(0), R(0)};
-  if (pbc)
-    sh = v3(image_shift(sti.cx - stj.cx, L, invL), image_shift(sti.cy - stj.cy, L, invL),
-            image_shift(sti.cz - stj.cz, L, invL));
-  const V3<R> d = {stj.cx + sh.x - sti.cx, stj.cy + sh.y - sti.cy, stj.cz + sh.z - sti.cz};
-  R reach = R(0);
-  if (contact) reach = sti.r + stj.r + contact_margin(stj.r, stj.em);
-  if (adhesion) reach = fmax(reach, sti.r + stj.r + R(2) * fmax(sti.l0, fmax(stj.l0, R(1e-12f))));
-  const R rr = (reach + skin) * R(1.0001f) + R(1e-6f);
-  return vdot(d, d) <= rr * rr || (pbc && R(2) * rr >= R(0.999f) * L);
 }
 
 // ---------------------------------------------------------------- cell list

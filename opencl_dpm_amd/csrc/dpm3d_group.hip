@@ -1178,7 +1178,7 @@ __device__ __forceinline__ void k3d_step_body() {
       a->st_out[ci] = make_cell_stat<R>(C.x, C.y, C.z, r, em, l0i);
       a->vol_out[ci] = fabs(vol / 6.0);
       a->em_out[ci] = em;
-      if (nl_on && near_list_moved(nl_ref, C, r, em, *a->nl_skin)) a->nl_stale_out[t] = 1;
+      if (nl_on && near_list_moved(nl_ref, C, r, em, pbc != 0, L, *a->nl_skin)) a->nl_stale_out[t] = 1;
     }
   }
   if (a->counters) {

@@ -848,7 +848,7 @@ __device__ __forceinline__ void k3d_wstep_body() {
       if (nl_on) {
         CellStat<R> ref = sti;
         if (!relist) ref = a->nl_ref[ci];
-        if (near_list_moved(ref, C, stn.r, stn.em, *a->nl_skin)) a->nl_stale_out[t] = 1;
+        if (near_list_moved(ref, C, stn.r, stn.em, pbc != 0, L, *a->nl_skin)) a->nl_stale_out[t] = 1;
       }
       a->vol_out[ci] = fabs(vol / 6.0);
       a->em_out[ci] = em;

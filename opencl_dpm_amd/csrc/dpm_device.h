@@ -53,7 +53,7 @@ struct V3 {
   R x, y, z;
 };
 template <typename R>
-__device__ __forceinline__ V3<R> v3(R x, R y, R z) { return {x, y, z}; }
+__host__ __device__ __forceinline__ V3<R> v3(R x, R y, R z) { return {x, y, z}; }
 template <typename R>
 __device__ __forceinline__ V3<R> vsub(V3<R> a, V3<R> b) { return {a.x - b.x, a.y - b.y, a.z - b.z}; }
 template <typename R>
@@ -61,7 +61,7 @@ __device__ __forceinline__ V3<R> vadd(V3<R> a, V3<R> b) { return {a.x + b.x, a.y
 template <typename R>
 __device__ __forceinline__ V3<R> vscale(V3<R> a, R s) { return {a.x * s, a.y * s, a.z * s}; }
 template <typename R>
-__device__ __forceinline__ R vdot(V3<R> a, V3<R> b) { return (a.x * b.x + a.y * b.y) + a.z * b.z; }
+__host__ __device__ __forceinline__ R vdot(V3<R> a, V3<R> b) { return (a.x * b.x + a.y * b.y) + a.z * b.z; }
 template <typename R>
 __device__ __forceinline__ V3<R> vcross(V3<R> a, V3<R> b) {
   return {a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
