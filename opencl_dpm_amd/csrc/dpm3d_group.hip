@@ -31,7 +31,7 @@ constexpr int kGrpTasks = 512;  // partial sums of the adhesion pairs kept at on
 // without the limit, 12.6 with it; 256 cells, 100 steps: 2.01 ms either way)
 constexpr int kGrpPoints = 16;
 constexpr int kGrpSlices = 256;  // partial sums a candidate is cut into, at most
-static_assert(kGrpSlots == 4 && kGrpCap <= 127 && kGrpSlices <= kGrpTasks, "the task search and the records' fields");
+static_assert(kGrpWaves == 4 && kGrpSlots == 4 && kGrpCap <= 127 && kGrpSlices <= kGrpTasks, "the task search and the records' fields");
 
 // LDS.  Three users of the last bytes, one after the other: the kept
 // candidates' lists and partial sums; a candidate taken by itself (its own
@@ -41,10 +41,6 @@ struct LdsGroup {
   size_t own, sb, faces, down, rec, seg, segst, clist, glist, plist, gath, cnt, red, slots, slot, pw, acc, wb, nlist, mlist,
       smap, ut, total;
 };
-__host__ __device__ inline int group_winding_waves(int nv, int rsize) {
-  const int n = 12288 / (4 * rsize * nv);
-  return n < 1 ? 1 : n > kGrpWaves ? kGrpWaves : n;
-}
 __host__ __device__ inline LdsGroup ldsg_layout(int nv, int nf, int ww, int rsize) {
   LdsGroup L;
   const size_t rs = (size_t)rsize, n = (size_t)nv;
@@ -81,6 +77,25 @@ __host__ __device__ inline LdsGroup ldsg_layout(int nv, int nf, int ww, int rsiz
   o += wind > sums ? wind : sums;
   L.total = al(o > fast ? o : fast);
   return L;
+}
+
+// Waves that take winding numbers, a point each; 1: all four on one point at a
+// time.  A cell in contact waits for hundreds of them: the more waves the
+// better, as long as their directions (four reals a vertex) do not keep cells
+// off a compute unit that its registers would hold.  Meshes of up to 256
+// vertices have room for four.  Above, floats take four where two cells still
+// fit a compute unit or the device holds all cells one a unit; doubles, the
+// instance that keeps three cells, and larger meshes have all waves on one
+// point, a barrier more each.  us per step, cells packed into contact, with one
+// to three waves at them (in brackets) | with these: 252 vertices, 256 cells (3)
+// 207 | 158, in double (1) 690 | 208; 162 in double (2) 192 | 113; 642 vertices,
+// 256 cells (1) 2705 | 768 (all on one point 863), in double (1) 3660 | 1111;
+// 4096 cells (1) 6853 | 2696.
+inline int group_winding_waves(int nv, int nf, int rsize, bool many, int cells, int cus, int lds_max) {
+  if (nv <= kGrpThreads) return kGrpWaves;
+  if (rsize == 8 || (many && nv == 642 && nf == 1280)) return 1;
+  const int fit = lds_max / (int)ldsg_layout(nv, nf, kGrpWaves, rsize).total;  // cells per compute unit
+  return fit >= 2 || cells <= fit * cus ? kGrpWaves : 1;
 }
 
 __device__ __forceinline__ int from_lane(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
@@ -698,7 +713,7 @@ __device__ __forceinline__ void k3d_step_body() {
       by[v] = a->yin[(size_t)cj2 * nv + v];
       bz[v] = a->zin[(size_t)cj2 * nv + v];
     }
-    if (tid == 0) one[0] = 0;
+    if (tid == 0) one[0] = one[1] = 0;
     __syncthreads();
     if (passes & 1) {  // block-uniform
       const V3<R> Cj = {stj.cx + sh.x, stj.cy + sh.y, stj.cz + sh.z};
@@ -723,14 +738,39 @@ __device__ __forceinline__ void k3d_step_body() {
       }
       __syncthreads();
       const int np = one[0];
-      if (wave < ww) {
-        Q4<R>* ut = reinterpret_cast<Q4<R>*>(smem + LG.ut) + (size_t)wave * nv;
+      // a point beyond the margin from j's hull has winding number 0
+      auto outside = [&](V3<R> Pv) __attribute__((always_inline)) {
+        return outside_by_margin(bx, by, bz, nv, stj.cx, stj.cy, stj.cz, Cj, vsub(Pv, Cj), mj, stj.r);
+      };
+      Q4<R>* ut = reinterpret_cast<Q4<R>*>(smem + LG.ut);
+      if (VPT > 1 && ww == 1) {  // block-uniform: the whole workgroup on one point at a time
+        for (int pi = wave; pi < np; pi += kGrpWaves) {  // wave-uniform
+          const int v = nl[pi];
+          const bool out = outside(lds_v(sx, sy, sz, v));
+          if (lane == 0) {
+            if (out) wb[v] = R(0);
+            else ml[atomicAdd(&one[1], 1)] = (unsigned short)v;  // in any order
+          }
+          n_wind += !out;
+        }
+        __syncthreads();
+        const int nw = one[1];
+        for (int q = 0; q < nw; q++) {  // block-uniform
+          const int v = ml[q];
+          const double w = winding_part(bx, by, bz, sf, ut, nv, nf, sh, lds_v(sx, sy, sz, v), tid, NT,
+                                        []() __attribute__((always_inline)) { __syncthreads(); });
+          double* sums = red + (q & 1) * kGrpWaves;
+          if (lane == 0) sums[wave] = w;
+          __syncthreads();  // the sums are there, the directions read
+          if (tid == 0) wb[v] = winding_of<R>(((sums[0] + sums[1]) + sums[2]) + sums[3]);
+        }
+      } else if (wave < ww) {
+        ut += (size_t)wave * nv;
         for (int pi = wave; pi < np; pi += ww) {  // wave-uniform
           const int v = nl[pi];
           const V3<R> Pv = lds_v(sx, sy, sz, v);
-          // a point beyond the margin from j's hull has winding number 0
           R wv = R(0);
-          if (!outside_by_margin(bx, by, bz, nv, stj.cx, stj.cy, stj.cz, Cj, vsub(Pv, Cj), mj, stj.r)) {
+          if (!outside(Pv)) {
             wv = winding_w(bx, by, bz, sf, ut, nv, nf, sh, Pv);
             n_wind++;
           }
@@ -1215,8 +1255,8 @@ extern "C" __global__ void __launch_bounds__(256) k3d_step_f32_v162(const Step3D
 extern "C" __global__ void __launch_bounds__(256) k3d_step_f32_v162_probe(const Step3D<float>) { k3d_step_body<float, 162, 320, 1, 4>(); }
 // 642 vertices: the _many instances keep three (double: two) cells on a
 // compute unit at the cost of spills, the others one or two without.
-extern "C" __global__ void __launch_bounds__(256) k3d_step_f32_v642(const Step3D<float>) { k3d_step_body<float, 642, 1280, 3, 1>(); }
+extern "C" __global__ void __launch_bounds__(256) k3d_step_f32_v642(const Step3D<float>) { k3d_step_body<float, 642, 1280, 3, 4>(); }
 extern "C" __global__ void __launch_bounds__(256, 3) k3d_step_f32_v642_many(const Step3D<float>) { k3d_step_body<float, 642, 1280, 3, 1>(); }
 extern "C" __global__ void __launch_bounds__(256) k3d_step_f64_v642(const Step3D<double>) { k3d_step_body<double, 642, 1280, 3, 1>(); }
 extern "C" __global__ void __launch_bounds__(256, 2) k3d_step_f64_v642_many(const Step3D<double>) { k3d_step_body<double, 642, 1280, 3, 1>(); }
-extern "C" __global__ void __launch_bounds__(256, 2) k3d_step_f64_v162(const Step3D<double>) { k3d_step_body<double, 162, 320, 1, 2>(); }
+extern "C" __global__ void __launch_bounds__(256, 2) k3d_step_f64_v162(const Step3D<double>) { k3d_step_body<double, 162, 320, 1, 4>(); }

@@ -116,19 +116,24 @@ __device__ __forceinline__ void wave_stage_cell(R* dx, R* dy, R* dz, const R* x,
 
 // winding_wave over per-wave arrays and packed faces (same arithmetic).
 template <typename R>
-__device__ __forceinline__ R winding_w(const R* nx, const R* ny, const R* nz, const unsigned* sf, Q4<R>* ut,
-                                       int nv, int nf, V3<R> sh, V3<R> p) {
-  const int lane = threadIdx.x & (DPM_WAVE - 1);
+__device__ __forceinline__ R winding_of(double sum) {
+  return (R)(sum / (double)(R(4) * R(3.14159265358979323846)));
+}
+// This wave's part of the sum: threads first, first + stride, ... of the
+// vertices and faces; ready() waits for the directions of all.
+template <typename R, typename Ready>
+__device__ __forceinline__ double winding_part(const R* nx, const R* ny, const R* nz, const unsigned* sf, Q4<R>* ut,
+                                               int nv, int nf, V3<R> sh, V3<R> p, int first, int stride, Ready ready) {
   #pragma unroll 1
-  for (int v = lane; v < nv; v += DPM_WAVE) {
+  for (int v = first; v < nv; v += stride) {
     const V3<R> A = {(nx[v] + sh.x) - p.x, (ny[v] + sh.y) - p.y, (nz[v] + sh.z) - p.z};
     const V3<R> u = vnormalize(A);
     ut[v] = Q4<R>{u.x, u.y, u.z, R(0)};
   }
-  wave_lds_sync();
+  ready();
   R part = R(0);
   #pragma unroll 1
-  for (int f = lane; f < nf; f += DPM_WAVE) {
+  for (int f = first; f < nf; f += stride) {
     int ia, ib, ic;
     wface(sf, f, ia, ib, ic);
     const Q4<R> ua = ut[ia], ub = ut[ib], uc = ut[ic];
@@ -140,9 +145,15 @@ __device__ __forceinline__ R winding_w(const R* nx, const R* ny, const R* nz, co
     const R num = vdot(u, vcross(v, w));
     part += R(2) * atan2(num, denom);
   }
-  const double tot = wave_sum_d((double)part);  // every lane (DPP tree)
+  return wave_sum_d((double)part);  // every lane (DPP tree)
+}
+template <typename R>
+__device__ __forceinline__ R winding_w(const R* nx, const R* ny, const R* nz, const unsigned* sf, Q4<R>* ut,
+                                       int nv, int nf, V3<R> sh, V3<R> p) {
+  const double tot = winding_part(nx, ny, nz, sf, ut, nv, nf, sh, p, (int)(threadIdx.x & (DPM_WAVE - 1)), DPM_WAVE,
+                                  []() __attribute__((always_inline)) { wave_lds_sync(); });
   wave_lds_sync();
-  return (R)(tot / (double)(R(4) * R(3.14159265358979323846)));
+  return winding_of<R>(tot);
 }
 
 // NVC, NFC: vertex and face counts fixed at compile time (0: taken from the

@@ -568,7 +568,11 @@ static int create3d(const dpm3d_desc* d, dpm_tissue** out, int rs) {
   h->ncmax = ncmax;
   h->NT = std::max(256, (nv + 63) / 64 * 64);
   h->lds = lds3d_layout(nv, nf, rs).total;
-  h->ww_g = group_winding_waves(nv, rs);
+  int cus = 256;
+  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device);
+  cus = std::max(1, cus);
+  h->many_g = C > (rs == 8 ? 1 : 4) * cus;
+  h->ww_g = group_winding_waves(nv, nf, rs, h->many_g, C, cus, max_lds_per_block(h->device));
   h->lds_g = ldsg_layout(nv, nf, h->ww_g, rs).total;
   if ((int)std::max(h->lds_g, mesh_lds_bound(nv, nf, h->NT, rs)) > max_lds_per_block(h->device)) {
     delete h;
@@ -670,10 +674,6 @@ static int create3d(const dpm3d_desc* d, dpm_tissue** out, int rs) {
                             {(const void*)k3d_stats_f64, (const void*)k3d_energy_f64}};
   for (const void* k : kern[rs == 8 ? 1 : 0])
     (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->lds);
-  int dev = 0, cus = 256;
-  if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  cus = std::max(1, cus);
-  h->many_g = C > (rs == 8 ? 1 : 4) * cus;
   for (bool probe : {false, true})
     (void)hipFuncSetAttribute(gstep_kernel(rs, nv, nf, probe, h->many_g), hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)h->lds_g);
