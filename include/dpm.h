@@ -224,9 +224,11 @@ float dpm3d_bin_width(dpm_tissue* h);
  * 1 one workgroup per cell; 2 one 64-lane wave per cell (meshes of at most
  * 256 vertices, several cells per workgroup, no workgroup barriers after
  * set-up); 0 (default) chooses 2 for meshes it takes once the handle holds
- * enough cells (4 per compute unit; meshes of at most 64 vertices: 3, in
- * double 2), else 1.  Both make the same
- * pair decisions; the wave form sums each vertex's edge springs once per ring
+ * enough cells per compute unit (12 for meshes of at most 162 vertices, 5 up to
+ * 64 vertices; in double 16, 6 up to 128 and 3 up to 64; 24 for larger ones),
+ * else 1: from there on 2 is no slower even where the cells are packed into
+ * contact.  Cells that keep apart gain from a third of these counts on;
+ * dpm3d_autotune finds that.  Both make the same pair decisions; the wave form sums each vertex's edge springs once per ring
  * edge and its adhesion terms in slices, so forces agree to float rounding. */
 int dpm3d_set_step_kernel(dpm_tissue* h, int kind);
 

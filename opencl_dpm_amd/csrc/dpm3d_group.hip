@@ -1242,21 +1242,31 @@ __device__ __forceinline__ void k3d_step_body() {
 
 // VPT 1: meshes of at most 256 vertices; VPT 4: up to 1024.  The icospheres of
 // subdivision 1 (42 vertices, 80 faces), 2 (162, 320) and 3 (642, 1280) have
-// instances with their sizes fixed; the production float ones of the first two
-// have the diagnostic outputs compiled out, the _probe instance of the same
-// source and the general kernel record them.
-extern "C" __global__ void __launch_bounds__(256) k3d_step_f32(const Step3D<float>) { k3d_step_body<float, 0, 0, 1, 0>(); }
+// instances with their sizes fixed.  The production instances up to 256
+// vertices have the diagnostic outputs compiled out, the _probe ones record
+// them.
+extern "C" __global__ void __launch_bounds__(256) k3d_step_f32(const Step3D<float>) { k3d_step_body<float, 0, 0, 1, 0, false>(); }
+extern "C" __global__ void __launch_bounds__(256) k3d_step_f32_probe(const Step3D<float>) { k3d_step_body<float, 0, 0, 1, 0>(); }
 extern "C" __global__ void __launch_bounds__(256, 2) k3d_step_f32_big(const Step3D<float>) { k3d_step_body<float, 0, 0, 4, 0>(); }
-extern "C" __global__ void __launch_bounds__(256, 2) k3d_step_f64(const Step3D<double>) { k3d_step_body<double, 0, 0, 1, 0>(); }
+extern "C" __global__ void __launch_bounds__(256, 2) k3d_step_f64(const Step3D<double>) { k3d_step_body<double, 0, 0, 1, 0, false>(); }
+extern "C" __global__ void __launch_bounds__(256, 2) k3d_step_f64_probe(const Step3D<double>) { k3d_step_body<double, 0, 0, 1, 0>(); }
 extern "C" __global__ void __launch_bounds__(256, 2) k3d_step_f64_big(const Step3D<double>) { k3d_step_body<double, 0, 0, 4, 0>(); }
 extern "C" __global__ void __launch_bounds__(256) k3d_step_f32_v42(const Step3D<float>) { k3d_step_body<float, 42, 80, 1, 4, false>(); }
 extern "C" __global__ void __launch_bounds__(256, 2) k3d_step_f64_v42(const Step3D<double>) { k3d_step_body<double, 42, 80, 1, 4, false>(); }
 extern "C" __global__ void __launch_bounds__(256) k3d_step_f32_v162(const Step3D<float>) { k3d_step_body<float, 162, 320, 1, 4, false>(); }
 extern "C" __global__ void __launch_bounds__(256) k3d_step_f32_v162_probe(const Step3D<float>) { k3d_step_body<float, 162, 320, 1, 4>(); }
-// 642 vertices: the _many instances keep three (double: two) cells on a
-// compute unit at the cost of spills, the others one or two without.
+extern "C" __global__ void __launch_bounds__(256, 2) k3d_step_f64_v162(const Step3D<double>) { k3d_step_body<double, 162, 320, 1, 4>(); }
+// Handles with many cells (group_many): registers bounded so that a compute
+// unit keeps a cell more, at the cost of a few spills.  us per step, plain |
+// bounded: 42 vertices, 1024 cells in contact 54 | 39; 162 vertices, 1024 cells
+// in contact 163 | 130, apart 34 | 28, 512 cells apart 21 | 22; 642 vertices,
+// 1024 cells apart 63 | 68, 4096 cells 175 | 133; in double, 64 cells 31 | 38,
+// 1024 cells 112 | 97.  The general double instance gains nothing (92 vertices,
+// 1024 cells in contact 1.2 times slower).
+extern "C" __global__ void __launch_bounds__(256, 4) k3d_step_f32_many(const Step3D<float>) { k3d_step_body<float, 0, 0, 1, 0, false>(); }
+extern "C" __global__ void __launch_bounds__(256, 4) k3d_step_f32_v42_many(const Step3D<float>) { k3d_step_body<float, 42, 80, 1, 4, false>(); }
+extern "C" __global__ void __launch_bounds__(256, 4) k3d_step_f32_v162_many(const Step3D<float>) { k3d_step_body<float, 162, 320, 1, 4, false>(); }
 extern "C" __global__ void __launch_bounds__(256) k3d_step_f32_v642(const Step3D<float>) { k3d_step_body<float, 642, 1280, 3, 4>(); }
 extern "C" __global__ void __launch_bounds__(256, 3) k3d_step_f32_v642_many(const Step3D<float>) { k3d_step_body<float, 642, 1280, 3, 1>(); }
 extern "C" __global__ void __launch_bounds__(256) k3d_step_f64_v642(const Step3D<double>) { k3d_step_body<double, 642, 1280, 3, 1>(); }
 extern "C" __global__ void __launch_bounds__(256, 2) k3d_step_f64_v642_many(const Step3D<double>) { k3d_step_body<double, 642, 1280, 3, 1>(); }
-extern "C" __global__ void __launch_bounds__(256, 2) k3d_step_f64_v162(const Step3D<double>) { k3d_step_body<double, 162, 320, 1, 4>(); }

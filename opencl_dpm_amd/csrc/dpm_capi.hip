@@ -440,21 +440,32 @@ static const void* wstep_kernel(int rs, int nv, int nf, bool probe = false) {
   return rs == 8 ? (const void*)k3d_wstep_f64 : (const void*)k3d_wstep_f32;
 }
 
-// The workgroup form's kernel for a handle.  many: the 642-vertex instances
-// for handles beyond four cells per compute unit (double: one); us per step,
-// plain | many: 1024 cells 63 | 68, 4096 cells 175 | 133; double, 64 cells
-// 31 | 38, 1024 cells 112 | 97.
+// The workgroup form's kernel for a handle (many: group_many).
 static const void* gstep_kernel(int rs, int nv, int nf, bool probe, bool many) {
-  if (nv == 162 && nf == 320)
-    return rs == 8 ? (const void*)k3d_step_f64_v162
-                   : probe ? (const void*)k3d_step_f32_v162_probe : (const void*)k3d_step_f32_v162;
-  if (nv == 42 && nf == 80 && !probe) return rs == 8 ? (const void*)k3d_step_f64_v42 : (const void*)k3d_step_f32_v42;
+  const bool d = rs == 8;
+  if (nv == 162 && nf == 320) {
+    if (d) return (const void*)k3d_step_f64_v162;
+    return probe ? (const void*)k3d_step_f32_v162_probe : many ? (const void*)k3d_step_f32_v162_many
+                                                               : (const void*)k3d_step_f32_v162;
+  }
+  if (nv == 42 && nf == 80 && !probe) {
+    if (d) return (const void*)k3d_step_f64_v42;
+    return many ? (const void*)k3d_step_f32_v42_many : (const void*)k3d_step_f32_v42;
+  }
   if (nv == 642 && nf == 1280) {
-    if (rs == 8) return many ? (const void*)k3d_step_f64_v642_many : (const void*)k3d_step_f64_v642;
+    if (d) return many ? (const void*)k3d_step_f64_v642_many : (const void*)k3d_step_f64_v642;
     return many ? (const void*)k3d_step_f32_v642_many : (const void*)k3d_step_f32_v642;
   }
-  if (nv > kGrpThreads) return rs == 8 ? (const void*)k3d_step_f64_big : (const void*)k3d_step_f32_big;
-  return rs == 8 ? (const void*)k3d_step_f64 : (const void*)k3d_step_f32;
+  if (nv > kGrpThreads) return d ? (const void*)k3d_step_f64_big : (const void*)k3d_step_f32_big;
+  if (probe) return d ? (const void*)k3d_step_f64_probe : (const void*)k3d_step_f32_probe;
+  if (d) return (const void*)k3d_step_f64;
+  return many ? (const void*)k3d_step_f32_many : (const void*)k3d_step_f32;
+}
+// Whether a handle takes the instances that keep a cell more on a compute unit:
+// beyond the cells that the others keep there.
+static bool group_many(int rs, int nv, int nf, int cells, int cus) {
+  const int keep = nv == 642 && nf == 1280 ? (rs == 8 ? 1 : 4) : rs == 8 ? 2 : 3;
+  return cells > keep * cus;
 }
 
 static int create3d(const dpm3d_desc* d, dpm_tissue** out, int rs) {
@@ -571,7 +582,7 @@ static int create3d(const dpm3d_desc* d, dpm_tissue** out, int rs) {
   int cus = 256;
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device);
   cus = std::max(1, cus);
-  h->many_g = C > (rs == 8 ? 1 : 4) * cus;
+  h->many_g = group_many(rs, nv, nf, C, cus);
   h->ww_g = group_winding_waves(nv, nf, rs, h->many_g, C, cus, max_lds_per_block(h->device));
   h->lds_g = ldsg_layout(nv, nf, h->ww_g, rs).total;
   if ((int)std::max(h->lds_g, mesh_lds_bound(nv, nf, h->NT, rs)) > max_lds_per_block(h->device)) {
@@ -707,16 +718,21 @@ static int create3d(const dpm3d_desc* d, dpm_tissue** out, int rs) {
     if (ldsw_layout(nv, nf, cpw, rs).total <= 65536) {
       h->wave_cpw = cpw;
       h->lds_w = ldsw_layout(nv, nf, cpw, rs).total;
-      // automatic choice, by cells per compute unit: a workgroup per cell
-      // shortens one cell's step while the device has room for every cell at
-      // once, a wave per cell takes fewer waves and no barriers.  Measured,
-      // us per step, every term, workgroup | wave form: float 162 vertices,
-      // 768 cells 26.4 | 32.9, 1024 cells 35.4 | 33.7, 2048 cells 50.4 | 36.9;
-      // float 42 vertices, 484 cells 26.6 | 26.8, 845 cells 25.1 | 24.3, 1352
-      // cells 35.8 | 26.0; double 162 vertices, 512 cells 36.4 | 44.9, 1024
-      // cells 53.0 | 53.7, 1536 cells 77.3 | 54.8; double 42 vertices, 256 cells
-      // 28.6 | 32.4, 512 cells 31.0 | 31.5, 3887 cells 154 | 64
-      const int per_cu = nv > DPM_WAVE ? 4 : rs == 8 ? 2 : 3;
+      // automatic choice, by cells per compute unit: a workgroup per cell puts
+      // four waves on a cell's chain of passes and on its winding numbers, a
+      // wave per cell takes fewer waves and no barriers.  The line lies where the
+      // wave form is no slower even for cells packed into contact (apart it
+      // gains from a third of these counts on).  us per step, workgroup | wave:
+      // float 42 vertices, 1024 cells in contact 39 | 52, apart 24 | 25, 1280 cells
+      // in contact 55 | 58, apart 33 | 26; float 162, 2048 cells in contact 220 |
+      // 293, apart 46 | 39, 3072 cells in contact 311 | 336, apart 59 | 41 (before
+      // the bounded instances 354 and 98: the wave form loses to neither); float
+      // 192, 5120 cells in contact 664 | 796, apart 111 | 83; double 42, 768 cells
+      // in contact 68 | 69, apart 44 | 33; double 92, 1536 cells in contact 220 |
+      // 210; double 162, 3072 cells in contact 693 | 770, apart 122 | 81, 4096
+      // cells in contact 922 | 894, apart 161 | 95
+      const int per_cu = rs == 8 ? (nv <= 64 ? 3 : nv <= 128 ? 6 : nv <= 162 ? 16 : 24)
+                                 : (nv <= 64 ? 5 : nv <= 162 ? 12 : 24);
       h->wave_min_cells = per_cu * cus;
       for (bool probe : {false, true})
         (void)hipFuncSetAttribute(wstep_kernel(rs, nv, nf, probe), hipFuncAttributeMaxDynamicSharedMemorySize,
