@@ -207,7 +207,8 @@ int dpm3d_energy(dpm_tissue* h, double* energy);
  * largest candidate reach) and visits the 27 surrounding bins; -1 (default)
  * chooses 0.  All give bit-identical results.  Where the scan runs in a tissue
  * of more than 512 cells, a step keeps lists with a skin and the following
- * steps test only those, until a cell has moved too far for them. */
+ * steps test only those, until a cell has moved too far for them (not the
+ * first call of one step after an upload or a change of parameters). */
 int dpm3d_set_cell_list(dpm_tissue* h, int mode);
 
 /* Bin width of the cell list over the step's largest candidate reach, a

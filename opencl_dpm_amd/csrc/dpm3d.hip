@@ -132,7 +132,7 @@ struct Step3D {
   int* nl_cnt;            // per cell: entries of its list, -1 more than kNearList
   int* nl_idx;            // [ncells * kNearList] ascending
   CellStat<R>* nl_ref;    // the cell's statistics when the lists were made
-  const int* nl_stale;    // per tissue: this step makes the lists
+  const int* nl_stale;    // per tissue: the mark of this step (near_list_mark)
   int* nl_stale_out;      // the same for the next step, set here
   int* nl_stale_clear;    // the same for the step after, cleared here
   const R* nl_skin;       // in device memory: a captured step reads the current one

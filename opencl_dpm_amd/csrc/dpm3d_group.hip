@@ -194,11 +194,12 @@ __device__ __forceinline__ void k3d_step_body() {
   // candidate lists: made by this step, or read (nlist entries; not when
   // there are more than a list holds)
   const bool nl_on = a->nl_cnt && !a->bin_list && ce - cb > kNearList;
-  const bool relist = nl_on && a->nl_stale[t] != 0;
-  const int nlist = nl_on && !relist ? a->nl_cnt[ci] : -1;
+  const int stale = nl_on ? a->nl_stale[t] : 0;  // 1: make them; more: scan
+  const bool relist = stale == 1;
+  const int nlist = nl_on && stale == 0 ? a->nl_cnt[ci] : -1;
   const bool listed = nlist >= 0;
   CellStat<R> nl_ref = sti;  // where this step makes the lists
-  if (nl_on && !relist) nl_ref = a->nl_ref[ci];
+  if (nl_on && stale == 0) nl_ref = a->nl_ref[ci];
   const bool binned = a->bin_list && a->tbin_nb[t] > 0;
   // the candidates among at most 256 cells are found ahead of the first
   // barrier: each wave keeps those among its 64 cells
@@ -1218,7 +1219,13 @@ __device__ __forceinline__ void k3d_step_body() {
       a->st_out[ci] = make_cell_stat<R>(C.x, C.y, C.z, r, em, l0i);
       a->vol_out[ci] = fabs(vol / 6.0);
       a->em_out[ci] = em;
-      if (nl_on && near_list_moved(nl_ref, C, r, em, pbc != 0, L, *a->nl_skin)) a->nl_stale_out[t] = 1;
+      if (nl_on) {
+        if (stale > 1) {
+          if (ci == cb) a->nl_stale_out[t] = stale - 1;
+        } else if (near_list_moved(nl_ref, C, r, em, pbc != 0, L, *a->nl_skin)) {
+          a->nl_stale_out[t] = near_list_mark(relist);
+        }
+      }
     }
   }
   if (a->counters) {

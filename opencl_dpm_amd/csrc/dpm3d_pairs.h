@@ -87,9 +87,18 @@ __host__ __device__ __forceinline__ R contact_margin(R Rj, R emax_j) {
 // differences, squares and the reach round by u times a few reaches.  Without
 // periodic images the coordinates' size does not enter.  A tissue far from the
 // origin, or with one cell far smaller than the others (the skin follows the
-// smallest), thus scans on every step.  Four sets of marks in turn: the one
-// read, the one written for the next step, the one cleared for the step after.
+// smallest), thus scans.  A tissue whose lists went stale in the step that made
+// them has kNearPause - 1 steps without them: there the entries cost and serve
+// nothing (10000 cells of 162 vertices that pass the skin at every step: 1062 us
+// a step with lists made at each, 924 now, 925 by the scan alone).  Four sets of
+// marks in turn: the one read, the one written for the next step, the
+// one cleared for the step after.
 constexpr int kNearList = DPM_WAVE;
+constexpr int kNearPause = 8;
+
+// The mark that a cell past the skin leaves for the next step: 0 lists in
+// force, 1 the step makes them, more: it scans, and the mark counts down.
+__host__ __device__ __forceinline__ int near_list_mark(bool made_now) { return made_now ? kNearPause : 1; }
 
 template <typename R>
 __host__ __device__ __forceinline__ bool near_list_moved(const CellStat<R>& ref, V3<R> C, R r, R em, bool pbc, R L,

@@ -215,8 +215,9 @@ __device__ __forceinline__ void k3d_wstep_body() {
   // candidate lists: made by this step, or read (nlist entries; not when
   // there are more than a list holds); wave-uniform
   const bool nl_on = a->nl_cnt && !a->bin_list && ce - cb > kNearList;
-  const bool relist = nl_on && a->nl_stale[t] != 0;
-  const int nlist = nl_on && !relist ? a->nl_cnt[ci] : -1;
+  const int stale = nl_on ? a->nl_stale[t] : 0;  // 1: make them; more: scan
+  const bool relist = stale == 1;
+  const int nlist = nl_on && stale == 0 ? a->nl_cnt[ci] : -1;
   if (a->nl_cnt && ci == cb && lane == 0) a->nl_stale_clear[t] = 0;
 
   wave_stage_cell(sx, sy, sz, a->xin, a->yin, a->zin, base, nv, lane);
@@ -858,8 +859,12 @@ __device__ __forceinline__ void k3d_wstep_body() {
       a->st_out[ci] = stn;
       if (nl_on) {
         CellStat<R> ref = sti;
-        if (!relist) ref = a->nl_ref[ci];
-        if (near_list_moved(ref, C, stn.r, stn.em, pbc != 0, L, *a->nl_skin)) a->nl_stale_out[t] = 1;
+        if (stale == 0) ref = a->nl_ref[ci];
+        if (stale > 1) {
+          if (ci == cb) a->nl_stale_out[t] = stale - 1;
+        } else if (near_list_moved(ref, C, stn.r, stn.em, pbc != 0, L, *a->nl_skin)) {
+          a->nl_stale_out[t] = near_list_mark(relist);
+        }
       }
       a->vol_out[ci] = fabs(vol / 6.0);
       a->em_out[ci] = em;

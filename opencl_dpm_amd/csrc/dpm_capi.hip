@@ -70,9 +70,13 @@ int max_lds_per_block(int dev) {
 // Steps replayed per hipGraph launch (even, so the position ping-pong ends
 // where it started).
 constexpr int kGraphSteps = 64;
-// cells of a handle's largest tissue above which it keeps candidate lists
-// (us per step, scan | lists: 256 cells of 162 vertices 24.2 | 25.2, 1024 of 642
-// in double 190 | 169, 4096 of 642 542 | 390; not timed in between)
+// cells of a handle's largest tissue above which it keeps candidate lists (us
+// per step, scan | lists, cells apart: 42 vertices, 169 cells 21.7 | 22.2, 576
+// 25.9 | 23.9; 162 vertices, 169 cells 23.5 | 24.3, 576 27.7 | 24.0, 1024 33.9 |
+// 29.3; 642 in double, 169 cells 39.1 | 39.8, 576 85 | 75, 1024 121 | 104; in
+// contact 169 cells 1 per cent slower, 1024 cells 1 to 7 faster.  The scan's cost
+// steps up past 256 cells, one test a thread; 289 to 484 cells gain 2 to 19 per
+// cent already, which this line leaves)
 constexpr int kNearListFrom = 512;
 // reals per cell of the cached cell statistics (CellStat)
 constexpr int kStatWords = (int)(sizeof(CellStat<float>) / sizeof(float));
@@ -156,7 +160,7 @@ struct dpm_tissue {
   void* nl_ref = nullptr;
   void* nl_skin = nullptr;  // one real: read by captured steps too, so not a kernel argument
   int nl_phase = 0;
-  bool nl_ok = false;
+  bool nl_ok = false, nl_wait = false;  // nl_wait: a single step went without lists, the next call makes them
 
   // ------------------------------------------------------------------ 2D
   int V = 0, NT2 = 0, NTr = 0;  // Euler threads, relax threads per tissue
@@ -768,11 +772,12 @@ extern "C" int dpm3d_set_cell_list(dpm_tissue* h, int mode) {
   if (!h || h->dim != 3) return fail(DPM_EINVAL, "not a 3D tissue");
   if (mode < -1 || mode > 1) return fail(DPM_EINVAL, "mode must be -1 (automatic), 0 or 1");
   h->cell_list_mode = mode;
-  // automatic: the candidate lists make the scan rare (4096 cells of 642
-  // vertices: see kNearList), so the bins, made anew every step, are for
-  // programs that ask for them
+  // automatic: the candidate lists make the scan rare, so the bins, made anew
+  // every step by one workgroup a tissue, are for programs that ask for them
+  // (us per step, bins | lists: 2304 cells of 42 vertices 179 | 27, 4096 of 162
+  // 259 | 46; a single step of 4096, which makes no lists, 303 | 126)
   h->cells_on = mode == 1;
-  h->nl_ok = false;  // steps with bins do not mind the lists
+  h->nl_ok = h->nl_wait = false;  // steps with bins do not mind the lists
   if (h->graph) {  // captured with the old arguments
     (void)hipGraphExecDestroy(h->graph);
     h->graph = nullptr;
@@ -812,7 +817,7 @@ extern "C" int dpm3d_set_cell_params(dpm_tissue* h, const float* Kv, const float
   if (Ks) TRY(upload(h->Ks, Ks, C, s));
   if (Kb) TRY(upload(h->Kb, Kb, C, s));
   if (v0) TRY(upload(h->v0, v0, C, s));
-  h->nl_ok = false;
+  h->nl_ok = h->nl_wait = false;
   double skin_d = 0.0;
   float skin = 0.0f;
   if (v0 && h->nl_skin) {  // the skin: 0.15 radii of the smallest cell at rest
@@ -846,7 +851,7 @@ extern "C" int dpm3d_set_tissue_params(dpm_tissue* h, const float* L, const int*
   if (Kat) TRY(upload(h->tKat, Kat, T, s));
   if (ks_grad) TRY(upload(h->tksg, ks_grad, T, s));
   h->mask = mask & DPM3D_ALL;
-  h->nl_ok = false;
+  h->nl_ok = h->nl_wait = false;
   HIPCHECK(hipStreamSynchronize(s));
   if (h->graph) {
     (void)hipGraphExecDestroy(h->graph);
@@ -871,7 +876,7 @@ static int set_positions3(dpm_tissue* h, const In* xyz, size_t n) {
   };
   TRY(h->rs == 8 ? put(0.0) : put(0.0f));
   h->cur = k;
-  h->stats_valid = h->nl_ok = false;
+  h->stats_valid = h->nl_ok = h->nl_wait = false;
   return DPM_OK;
 }
 
@@ -1087,10 +1092,11 @@ static int ensure_lists(dpm_tissue* h) {
   return DPM_OK;
 }
 
-// One step from buffer `in`; phase: the set of list marks it reads.
+// One step from buffer `in`; phase: the set of list marks it reads (negative:
+// without lists).
 static int launch_step3d(dpm_tissue* h, int in, int phase, float dt, int flags) {
   return launch3d(h, K_STEP, in, dt, flags, [&](auto& a) {
-    if (!h->nl_cnt) return;
+    if (!h->nl_cnt || phase < 0) return;
     using S = std::remove_reference_t<decltype(*a.nl_ref)>;
     a.nl_cnt = h->nl_cnt;
     a.nl_idx = h->nl_idx;
@@ -1144,6 +1150,16 @@ static int euler3d(dpm_tissue* h, int nsteps, float dt) {
   // the step graph for this dt is captured on the first call with it (a
   // capture launches nothing), so that later calls replay it
   if (!h->graph || h->graph_dt != dt) TRY(build_graph3d(h, dt));
+  // The first call of one step after an upload or a change scans without making
+  // lists that another upload may discard (10000 cells of 162 vertices: 538 us
+  // with them, 376 without); a second one makes them.
+  if (nsteps == 1 && h->nl_cnt && !h->nl_ok && !h->nl_wait) {
+    TRY(launch_step3d(h, h->cur, -1, dt, F_MOVE | F_WRITE_FORCES));
+    h->cur = 1 - h->cur;
+    h->nl_wait = true;
+    h->forces_valid = true;
+    return DPM_OK;
+  }
   TRY(ensure_lists(h));
   int left = nsteps - 1;  // the last step also writes the forces
   if (left >= kGraphSteps) {
@@ -1229,7 +1245,7 @@ extern "C" int dpm3d_autotune(dpm_tissue* h, int steps, float dt, int* best, flo
       for (int rep = 0; rep < 2 && !rc; rep++) {  // a warm-up launch, then the timed steps
         rc = copy_all(false);
         if (rc) break;
-        h->nl_ok = false;  // the state was restored
+        h->nl_ok = h->nl_wait = false;  // the state was restored
         rc = ensure_lists(h);
         if (rc) break;
         if (rep == 0) {
@@ -1257,7 +1273,7 @@ extern "C" int dpm3d_autotune(dpm_tissue* h, int steps, float dt, int* best, flo
   if (e0) (void)hipEventDestroy(e0);
   if (e1) (void)hipEventDestroy(e1);
   int rc2 = copy_all(false);
-  h->nl_ok = false;
+  h->nl_ok = h->nl_wait = false;
   if (!rc && rc2) rc = rc2;
   if (hipStreamSynchronize(h->stream) != hipSuccess && !rc) rc = fail(DPM_EDEVICE, "stream sync failed");
   (void)hipFree(save);
@@ -1737,7 +1753,7 @@ static int adjoint3d(dpm_tissue* h, const In* lambda_final, double* dtheta, Out*
       a.vol_out = h->vol[0];
       a.em_out = (R*)h->em[0];
     }));
-    h->stats_valid = h->nl_ok = false;
+    h->stats_valid = h->nl_ok = h->nl_wait = false;
     for (int s = 0; s < every; s++) {
       void* w = slot(h, h->segw, s);
       const size_t NP = NVT * DPM3D_MAXPART;
@@ -1785,7 +1801,7 @@ static int adjoint3d(dpm_tissue* h, const In* lambda_final, double* dtheta, Out*
   TRY(copy_positions_dd(h, h->x[0], h->y[0], h->z[0], last, slot(h, last, 1), slot(h, last, 2)));
   if (h->lo)
     HIPCHECK(hipMemcpyAsync(h->lo, slot(h, last, 3), 3 * NVT * h->rs, hipMemcpyDeviceToDevice, h->stream));
-  h->stats_valid = h->nl_ok = false;
+  h->stats_valid = h->nl_ok = h->nl_wait = false;
   if (dtheta)
     HIPCHECK(hipMemcpyAsync(dtheta, h->gtheta, sizeof(double) * h->C * 4, hipMemcpyDeviceToHost, h->stream));
   if (lambda0) TRY(download3(h, h->lam, slot(h, h->lam, 1), slot(h, h->lam, 2), lambda0, NVT));
