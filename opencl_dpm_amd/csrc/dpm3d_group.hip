@@ -1,5 +1,6 @@
 // Workgroup-per-cell form of the 3D step: 256 threads own one cell, thread t
-// its vertices t, t + 256, ... (VPT of them).
+// its vertices t, t + 256, ... (VPT of them); 512 threads in small handles of
+// 257 to 512 vertices.
 //
 // The form serves what the wave-per-cell form does not: handles with few
 // cells, where a step is one chain of dependent passes on a mostly idle
@@ -31,7 +32,7 @@ constexpr int kGrpTasks = 512;  // partial sums of the adhesion pairs kept at on
 // without the limit, 12.6 with it; 256 cells, 100 steps: 2.01 ms either way)
 constexpr int kGrpPoints = 16;
 constexpr int kGrpSlices = 256;  // partial sums a candidate is cut into, at most
-static_assert(kGrpWaves == 4 && kGrpSlots == 4 && kGrpCap <= 127 && kGrpSlices <= kGrpTasks, "the task search and the records' fields");
+static_assert(kGrpSlots == 4 && kGrpCap <= 127 && kGrpSlices <= kGrpTasks, "the task search and the records' fields");
 
 // LDS.  Three users of the last bytes, one after the other: the kept
 // candidates' lists and partial sums; a candidate taken by itself (its own
@@ -41,8 +42,9 @@ struct LdsGroup {
   size_t own, sb, faces, down, rec, seg, segst, clist, glist, plist, gath, cnt, red, slots, slot, pw, acc, wb, nlist, mlist,
       smap, ut, total;
 };
-__host__ __device__ inline LdsGroup ldsg_layout(int nv, int nf, int ww, int rsize) {
+__host__ __device__ inline LdsGroup ldsg_layout(int nv, int nf, int ww, int rsize, int nt = kGrpThreads) {
   LdsGroup L;
+  const size_t threads = (size_t)nt, waves = threads / DPM_WAVE;
   const size_t rs = (size_t)rsize, n = (size_t)nv;
   auto al = [](size_t o) { return (o + 31u) & ~(size_t)31u; };
   size_t o = 0;
@@ -51,17 +53,17 @@ __host__ __device__ inline LdsGroup ldsg_layout(int nv, int nf, int ww, int rsiz
   L.faces = o; o = al(o + 4u * (size_t)nf);
   L.down = o;  o = al(o + (n + 3u) / 4u * 4u);  // facing-down faces per vertex, a byte each
   L.rec = o;   o = al(o + 4u * DPM_WAVE);
-  L.seg = o;   o = al(o + 4u * kGrpWaves * kGrpSeg);
-  L.segst = o; o = al(o + 8u * rs * kGrpWaves * kGrpSeg);
-  L.clist = o; o = al(o + 4u * kGrpThreads);
-  L.glist = o; o = al(o + 4u * kGrpThreads);
-  L.plist = o; o = al(o + 4u * kGrpThreads);
+  L.seg = o;   o = al(o + 4u * waves * kGrpSeg);
+  L.segst = o; o = al(o + 8u * rs * waves * kGrpSeg);
+  L.clist = o; o = al(o + 4u * threads);
+  L.glist = o; o = al(o + 4u * threads);
+  L.plist = o; o = al(o + 4u * threads);
   L.gath = o;  o = al(o + 4u * 96u);
   L.cnt = o;   o = al(o + 4u * 48u);
-  L.red = o;   o = al(o + 8u * 6u * kGrpWaves);
+  L.red = o;   o = al(o + 8u * 6u * waves);
   const size_t z = o;
   const size_t wind = 4u * rs * n * (size_t)ww;
-  const bool points = nv <= kGrpThreads;  // contact points of all candidates together
+  const bool points = nv <= nt;  // contact points of all candidates together
   L.slots = o;
   L.slot = al(3u * rs * kGrpCap + 2u * kGrpCap + 2u * n);  // positions, own vertices, vertex -> place
   L.pw = al(o + kGrpSlots * L.slot);  // the points' winding numbers
@@ -91,8 +93,14 @@ __host__ __device__ inline LdsGroup ldsg_layout(int nv, int nf, int ww, int rsiz
 // 207 | 158, in double (1) 690 | 208; 162 in double (2) 192 | 113; 642 vertices,
 // 256 cells (1) 2705 | 768 (all on one point 863), in double (1) 3660 | 1111;
 // 4096 cells (1) 6853 | 2696.
-inline int group_winding_waves(int nv, int nf, int rsize, bool many, int cells, int cus, int lds_max) {
+// Workgroups of 512 threads take what fits.
+inline int group_winding_waves(int nv, int nf, int rsize, bool many, int cells, int cus, int lds_max, int nt) {
   if (nv <= kGrpThreads) return kGrpWaves;
+  if (nt > kGrpThreads) {
+    int n = nt / DPM_WAVE;
+    while (n > 1 && (int)ldsg_layout(nv, nf, n, rsize, nt).total > lds_max) n--;
+    return n;
+  }
   if (rsize == 8 || (many && nv == 642 && nf == 1280)) return 1;
   const int fit = lds_max / (int)ldsg_layout(nv, nf, kGrpWaves, rsize).total;  // cells per compute unit
   return fit >= 2 || cells <= fit * cus ? kGrpWaves : 1;
@@ -124,17 +132,18 @@ __device__ __forceinline__ CellStat<R> from_lane(const CellStat<R>& s, int l) {
 // One overdamped Euler step of every cell (or, without F_MOVE, one force
 // evaluation for diagnostics), nv <= VPT * 256.
 // NVC, NFC, WWC: vertex and face counts and winding waves fixed at compile
-// time (0: taken from the arguments).
-template <typename R, int NVC, int NFC, int VPT, int WWC, bool PROBE = true>
+// time (0: taken from the arguments).  NT threads.
+template <typename R, int NVC, int NFC, int VPT, int WWC, bool PROBE = true, int NT = kGrpThreads>
 __device__ __forceinline__ void k3d_step_body() {
   Step3DArgs<R>* a = step_args_here<R>();
   extern __shared__ __align__(16) unsigned char smem[];
-  constexpr int NT = kGrpThreads;
+  constexpr int W = NT / DPM_WAVE;
+  static_assert(W <= 8, "the counters' words");
   const int nv = NVC > 0 ? NVC : a->nv, nf = NFC > 0 ? NFC : a->nf, ww = WWC > 0 ? WWC : a->ww;
   const int tid = threadIdx.x, lane = tid & (DPM_WAVE - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid / DPM_WAVE);
   const int ci = xcd_remap(blockIdx.x, gridDim.x);
-  const LdsGroup LG = ldsg_layout(nv, nf, ww, (int)sizeof(R));
+  const LdsGroup LG = ldsg_layout(nv, nf, ww, (int)sizeof(R), NT);
   R* sx = reinterpret_cast<R*>(smem + LG.own);
   R* sy = sx + nv;
   R* sz = sy + nv;
@@ -269,7 +278,7 @@ __device__ __forceinline__ void k3d_step_body() {
   {
     int off = 0, src = -1;
 #pragma unroll
-    for (int w = 0; w < kGrpWaves; w++) {
+    for (int w = 0; w < W; w++) {
       const int n = seg_n[w];
       if (n > kGrpSeg) ahead = false;
       if (src < 0 && lane < off + n && n <= kGrpSeg) src = w * kGrpSeg + (lane - off);
@@ -389,7 +398,7 @@ __device__ __forceinline__ void k3d_step_body() {
   auto separate = [&](unsigned long long m) __attribute__((always_inline)) {
     int o = 0;
     for (unsigned long long w = m; w; w &= w - 1ull, o++) {
-      if (o % kGrpWaves != wave) continue;  // wave-uniform
+      if (o % W != wave) continue;  // wave-uniform
       const int b = __ffsll((long long)w) - 1;
       const int cjq = from_lane(cj_l, b);
       const size_t bj = (size_t)cjq * nv;
@@ -745,7 +754,7 @@ __device__ __forceinline__ void k3d_step_body() {
       };
       Q4<R>* ut = reinterpret_cast<Q4<R>*>(smem + LG.ut);
       if (VPT > 1 && ww == 1) {  // block-uniform: the whole workgroup on one point at a time
-        for (int pi = wave; pi < np; pi += kGrpWaves) {  // wave-uniform
+        for (int pi = wave; pi < np; pi += W) {  // wave-uniform
           const int v = nl[pi];
           const bool out = outside(lds_v(sx, sy, sz, v));
           if (lane == 0) {
@@ -760,10 +769,14 @@ __device__ __forceinline__ void k3d_step_body() {
           const int v = ml[q];
           const double w = winding_part(bx, by, bz, sf, ut, nv, nf, sh, lds_v(sx, sy, sz, v), tid, NT,
                                         []() __attribute__((always_inline)) { __syncthreads(); });
-          double* sums = red + (q & 1) * kGrpWaves;
+          double* sums = red + (q & 1) * W;
           if (lane == 0) sums[wave] = w;
           __syncthreads();  // the sums are there, the directions read
-          if (tid == 0) wb[v] = winding_of<R>(((sums[0] + sums[1]) + sums[2]) + sums[3]);
+          if (tid == 0) {
+            double tot = sums[0];
+            for (int k = 1; k < W; k++) tot += sums[k];
+            wb[v] = winding_of<R>(tot);
+          }
         }
       } else if (wave < ww) {
         ut += (size_t)wave * nv;
@@ -1164,16 +1177,16 @@ __device__ __forceinline__ void k3d_step_body() {
     }
     if (lane == 0) {
       red[wave] = px;
-      red[kGrpWaves + wave] = py;
-      red[2 * kGrpWaves + wave] = pz;
+      red[W + wave] = py;
+      red[2 * W + wave] = pz;
     }
     __syncthreads();
     px = py = pz = 0.0;
 #pragma unroll
-    for (int w = 0; w < kGrpWaves; w++) {
+    for (int w = 0; w < W; w++) {
       px += red[w];
-      py += red[kGrpWaves + w];
-      pz += red[2 * kGrpWaves + w];
+      py += red[W + w];
+      pz += red[2 * W + w];
     }
     const V3<R> C = {(R)(px / nv), (R)(py / nv), (R)(pz / nv)};
     R rr2 = R(0), e2 = R(0);  // max |d|^2, then one square root (monotonic, correctly rounded)
@@ -1199,19 +1212,19 @@ __device__ __forceinline__ void k3d_step_body() {
     e2 = wave_max_all(e2);
     vol = wave_sum_d(vol);
     if (lane == 0) {
-      red[3 * kGrpWaves + wave] = vol;
-      red[4 * kGrpWaves + wave] = (double)rr2;
-      red[5 * kGrpWaves + wave] = (double)e2;
+      red[3 * W + wave] = vol;
+      red[4 * W + wave] = (double)rr2;
+      red[5 * W + wave] = (double)e2;
     }
     __syncthreads();
     if (tid == 0) {
       double r2d = 0.0, e2d = 0.0;
       vol = 0.0;
 #pragma unroll
-      for (int w = 0; w < kGrpWaves; w++) {
-        vol += red[3 * kGrpWaves + w];
-        r2d = fmax(r2d, red[4 * kGrpWaves + w]);
-        e2d = fmax(e2d, red[5 * kGrpWaves + w]);
+      for (int w = 0; w < W; w++) {
+        vol += red[3 * W + w];
+        r2d = fmax(r2d, red[4 * W + w]);
+        e2d = fmax(e2d, red[5 * W + w]);
       }
       // slack of a few ulp so that the culling tests are never tighter than
       // the largest distance a vertex can have from C, or the longest edge
@@ -1238,7 +1251,7 @@ __device__ __forceinline__ void k3d_step_body() {
     if (any)
       for (int o = 32; o > 0; o >>= 1) c += __shfl_down(c, o, DPM_WAVE);
     if (lane == 0) {
-      unsigned long long* slot = a->counters + 4 * ((blockIdx.x * kGrpWaves + wave) % DPM_COUNTER_SLOTS);
+      unsigned long long* slot = a->counters + 4 * ((blockIdx.x * W + wave) % DPM_COUNTER_SLOTS);
       if (blockIdx.x == 0 && wave == 0) atomicAdd(&slot[0], 1ull);
       if (n_wind) atomicAdd(&slot[1], (unsigned long long)n_wind);
       if (c) atomicAdd(&slot[2], (unsigned long long)c);
@@ -1247,7 +1260,8 @@ __device__ __forceinline__ void k3d_step_body() {
   }
 }
 
-// VPT 1: meshes of at most 256 vertices; VPT 4: up to 1024.  The icospheres of
+// VPT 1: meshes of at most 256 vertices; VPT 2 (_mid): up to 512, in float; VPT
+// 4: up to 1024; _t512: 512 threads (group_threads).  The icospheres of
 // subdivision 1 (42 vertices, 80 faces), 2 (162, 320) and 3 (642, 1280) have
 // instances with their sizes fixed.  The production instances up to 256
 // vertices have the diagnostic outputs compiled out, the _probe ones record
@@ -1255,6 +1269,9 @@ __device__ __forceinline__ void k3d_step_body() {
 extern "C" __global__ void __launch_bounds__(256) k3d_step_f32(const Step3D<float>) { k3d_step_body<float, 0, 0, 1, 0, false>(); }
 extern "C" __global__ void __launch_bounds__(256) k3d_step_f32_probe(const Step3D<float>) { k3d_step_body<float, 0, 0, 1, 0>(); }
 extern "C" __global__ void __launch_bounds__(256, 2) k3d_step_f32_big(const Step3D<float>) { k3d_step_body<float, 0, 0, 4, 0>(); }
+extern "C" __global__ void __launch_bounds__(256, 3) k3d_step_f32_mid(const Step3D<float>) { k3d_step_body<float, 0, 0, 2, 0>(); }
+extern "C" __global__ void __launch_bounds__(512) k3d_step_f32_t512(const Step3D<float>) { k3d_step_body<float, 0, 0, 1, 0, true, 512>(); }
+extern "C" __global__ void __launch_bounds__(512) k3d_step_f64_t512(const Step3D<double>) { k3d_step_body<double, 0, 0, 1, 0, true, 512>(); }
 extern "C" __global__ void __launch_bounds__(256, 2) k3d_step_f64(const Step3D<double>) { k3d_step_body<double, 0, 0, 1, 0, false>(); }
 extern "C" __global__ void __launch_bounds__(256, 2) k3d_step_f64_probe(const Step3D<double>) { k3d_step_body<double, 0, 0, 1, 0>(); }
 extern "C" __global__ void __launch_bounds__(256, 2) k3d_step_f64_big(const Step3D<double>) { k3d_step_body<double, 0, 0, 4, 0>(); }

@@ -116,7 +116,8 @@ struct dpm_tissue {
   void* wtopo = nullptr;  // LDS image of the wave form's shared topology
   int wtopo_n16 = 0;
   size_t lds_w = 0;
-  int ww_g = 1;      // workgroup-per-cell step: waves that take winding numbers, LDS
+  int nt_g = 256;    // workgroup-per-cell step: threads, waves that take winding numbers, LDS
+  int ww_g = 1;
   size_t lds_g = 0;
   bool many_g = false;  // more cells than the few-cells instances serve best
   unsigned mask = 0;
@@ -445,7 +446,7 @@ static const void* wstep_kernel(int rs, int nv, int nf, bool probe = false) {
 }
 
 // The workgroup form's kernel for a handle (many: group_many).
-static const void* gstep_kernel(int rs, int nv, int nf, bool probe, bool many) {
+static const void* gstep_kernel(int rs, int nv, int nf, bool probe, bool many, int nt) {
   const bool d = rs == 8;
   if (nv == 162 && nf == 320) {
     if (d) return (const void*)k3d_step_f64_v162;
@@ -460,6 +461,8 @@ static const void* gstep_kernel(int rs, int nv, int nf, bool probe, bool many) {
     if (d) return many ? (const void*)k3d_step_f64_v642_many : (const void*)k3d_step_f64_v642;
     return many ? (const void*)k3d_step_f32_v642_many : (const void*)k3d_step_f32_v642;
   }
+  if (nt > kGrpThreads) return d ? (const void*)k3d_step_f64_t512 : (const void*)k3d_step_f32_t512;
+  if (nv > kGrpThreads && nv <= 2 * kGrpThreads && !d) return (const void*)k3d_step_f32_mid;
   if (nv > kGrpThreads) return d ? (const void*)k3d_step_f64_big : (const void*)k3d_step_f32_big;
   if (probe) return d ? (const void*)k3d_step_f64_probe : (const void*)k3d_step_f32_probe;
   if (d) return (const void*)k3d_step_f64;
@@ -470,6 +473,16 @@ static const void* gstep_kernel(int rs, int nv, int nf, bool probe, bool many) {
 static bool group_many(int rs, int nv, int nf, int cells, int cus) {
   const int keep = nv == 642 && nf == 1280 ? (rs == 8 ? 1 : 4) : rs == 8 ? 2 : 3;
   return cells > keep * cus;
+}
+
+// Threads of the workgroup form: 512 for 257 to 512 vertices while every cell has
+// a compute unit to itself; beyond, two cells of 256 threads keep as many waves
+// there.  us per step, 256 cells, 256 threads | 512 (a thread per vertex, the
+// form before): 362 vertices in contact 239 | 155 (176), apart 40 | 28 (36); 492
+// in contact 380 | 237 (263); 492 in double, in contact 576 | 457 (636), apart 57
+// | 42 (72).
+static int group_threads(int nv, int cells, int cus) {
+  return nv > kGrpThreads && nv <= 2 * kGrpThreads && cells <= cus ? 2 * kGrpThreads : kGrpThreads;
 }
 
 static int create3d(const dpm3d_desc* d, dpm_tissue** out, int rs) {
@@ -587,8 +600,9 @@ static int create3d(const dpm3d_desc* d, dpm_tissue** out, int rs) {
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device);
   cus = std::max(1, cus);
   h->many_g = group_many(rs, nv, nf, C, cus);
-  h->ww_g = group_winding_waves(nv, nf, rs, h->many_g, C, cus, max_lds_per_block(h->device));
-  h->lds_g = ldsg_layout(nv, nf, h->ww_g, rs).total;
+  h->nt_g = group_threads(nv, C, cus);
+  h->ww_g = group_winding_waves(nv, nf, rs, h->many_g, C, cus, max_lds_per_block(h->device), h->nt_g);
+  h->lds_g = ldsg_layout(nv, nf, h->ww_g, rs, h->nt_g).total;
   if ((int)std::max(h->lds_g, mesh_lds_bound(nv, nf, h->NT, rs)) > max_lds_per_block(h->device)) {
     delete h;
     return fail(DPM_ERANGE, "cell mesh does not fit the LDS of one workgroup");
@@ -690,7 +704,7 @@ static int create3d(const dpm3d_desc* d, dpm_tissue** out, int rs) {
   for (const void* k : kern[rs == 8 ? 1 : 0])
     (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->lds);
   for (bool probe : {false, true})
-    (void)hipFuncSetAttribute(gstep_kernel(rs, nv, nf, probe, h->many_g), hipFuncAttributeMaxDynamicSharedMemorySize,
+    (void)hipFuncSetAttribute(gstep_kernel(rs, nv, nf, probe, h->many_g, h->nt_g), hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)h->lds_g);
   if ((int)h->bin_lds <= max_lds_per_block(h->device))  // (beyond, steps with bins fail at their launch)
     (void)hipFuncSetAttribute(rs == 8 ? (const void*)k3d_bin_f64 : (const void*)k3d_bin_f32,
@@ -775,7 +789,7 @@ extern "C" int dpm3d_set_cell_list(dpm_tissue* h, int mode) {
   // automatic: the candidate lists make the scan rare, so the bins, made anew
   // every step by one workgroup a tissue, are for programs that ask for them
   // (us per step, bins | lists: 2304 cells of 42 vertices 179 | 27, 4096 of 162
-  // 259 | 46; a single step of 4096, which makes no lists, 303 | 126)
+  // 259 | 46; a single step of 4096, which makes no lists, 303 | 120)
   h->cells_on = mode == 1;
   h->nl_ok = h->nl_wait = false;  // steps with bins do not mind the lists
   if (h->graph) {  // captured with the old arguments
@@ -1048,8 +1062,8 @@ static int launch3d(dpm_tissue* h, Kind3D kind, int in, float dt, int flags, Edi
       hipLaunchKernelGGL(kw, dim3((h->C + h->wave_cpw - 1) / h->wave_cpw), dim3(64 * h->wave_cpw), h->lds_w,
                          h->stream, a);
     } else if (kind == K_STEP) {
-      auto kg = reinterpret_cast<void (*)(Step3D<R>)>(const_cast<void*>(gstep_kernel(h->rs, h->nv, h->nf, probe, h->many_g)));
-      hipLaunchKernelGGL(kg, dim3(h->C), dim3(kGrpThreads), h->lds_g, h->stream, a);
+      auto kg = reinterpret_cast<void (*)(Step3D<R>)>(const_cast<void*>(gstep_kernel(h->rs, h->nv, h->nf, probe, h->many_g, h->nt_g)));
+      hipLaunchKernelGGL(kg, dim3(h->C), dim3(h->nt_g), h->lds_g, h->stream, a);
     } else {
       void (*k)(Step3D<R>) = nullptr;
       if constexpr (sizeof(R) == 8)

@@ -5,6 +5,7 @@ Forces agree to rounding, contact sets are the same, and every copy of the
 tissue is the same bit for bit."""
 import numpy as np
 import pytest
+from scipy.spatial import ConvexHull
 
 from opencl_dpm_amd import capi
 from opencl_dpm_amd import workloads as W
@@ -13,27 +14,26 @@ pytestmark = pytest.mark.gpu
 
 
 def mesh(nv):
-    """The largest icosphere of at most nv vertices, with a vertex more inside
-    some faces that share none."""
-    m = W.icosphere(max(k for k in range(4) if 10 * 4**k + 2 <= nv))
-    V, F, used = [*m.unit.astype(np.float64)], [tuple(f) for f in m.faces], set()
-    for f in list(F):
-        if len(V) < nv and used.isdisjoint(f):
-            used.update(f)
-            V.append(sum(V[i] for i in f) / np.linalg.norm(sum(V[i] for i in f)))
-            a, b, c = f
-            n = len(V) - 1
-            F.remove(f)
-            F += [(a, b, n), (b, c, n), (c, a, n)]
-    assert len(V) == nv
-    return np.array(V), np.array(F, np.int32)
+    """An icosphere, or the hull of nv points along a spiral."""
+    if nv in (12, 42, 162, 642):
+        m = W.icosphere({12: 0, 42: 1, 162: 2, 642: 3}[nv])
+        return m.unit.astype(np.float64), m.faces
+    z = 1 - (2 * np.arange(nv) + 1) / nv
+    phi = np.arange(nv) * np.pi * (3 - 5**0.5)
+    V = np.stack([np.cos(phi) * np.sqrt(1 - z * z), np.sin(phi) * np.sqrt(1 - z * z), z], 1)
+    F = ConvexHull(V).simplices
+    inward = np.einsum("ij,ij->i", np.cross(V[F[:, 1]] - V[F[:, 0]], V[F[:, 2]] - V[F[:, 0]]), V[F[:, 0]]) < 0
+    F[inward] = F[inward][:, ::-1]
+    return V, np.ascontiguousarray(F, dtype=np.int32)
 
 
 # vertices, and copies of the tissue of 9 cells: beyond 1024 cells (642 vertices: the
 # instance that keeps three cells on a compute unit; 162 and general: four), beyond 256
-# (a cell a compute unit: general meshes over 690 vertices, doubles over 256)
-@pytest.mark.parametrize("nv,T,bits", [(12, 120, 32), (42, 120, 32), (162, 120, 32), (190, 120, 32), (700, 40, 32),
-                                       (642, 120, 32), (42, 60, 64), (190, 60, 64), (642, 40, 64)])
+# (a cell a compute unit: general meshes over 690 vertices, doubles over 256, 257 to 512
+# vertices on 512 threads)
+@pytest.mark.parametrize("nv,T,bits", [(12, 120, 32), (42, 120, 32), (162, 120, 32), (190, 120, 32), (257, 40, 32),
+                                       (330, 40, 32), (512, 40, 32), (700, 40, 32), (642, 120, 32), (42, 60, 64),
+                                       (190, 60, 64), (257, 40, 64), (512, 40, 64), (642, 40, 64)])
 def test_few_and_many_cells(nv, T, bits):
     V, F = mesh(nv)
     rng = np.random.default_rng(nv)
