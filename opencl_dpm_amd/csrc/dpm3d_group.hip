@@ -28,8 +28,10 @@ constexpr int kGrpCap = 64;     // entries of such a list
 constexpr int kGrpTasks = 512;  // partial sums of the adhesion pairs kept at once
 // (candidate, vertex) points whose winding numbers are taken together: beyond
 // that, re-reading a candidate's vertices from the L2 for every point costs more
-// than staging it (64 cells in contact, 200 steps forward and back: 13.4 ms
-// without the limit, 12.6 with it; 256 cells, 100 steps: 2.01 ms either way)
+// than staging it.  16 to 512 cells of 12 to 252 vertices packed into contact, 120
+// workloads: a limit of 64 loses up to 8 per cent (92 vertices, 16 cells 45.8 ->
+// 49.6 us a step), one of 1 up to 16 (12 vertices, 64 cells 19.1 -> 22.1); the
+// means are alike.
 constexpr int kGrpPoints = 16;
 constexpr int kGrpSlices = 256;  // partial sums a candidate is cut into, at most
 static_assert(kGrpSlots == 4 && kGrpCap <= 127 && kGrpSlices <= kGrpTasks, "the task search and the records' fields");
