@@ -895,6 +895,8 @@ extern "C" __global__ void __launch_bounds__(1024) k2d_run(const Run2D a) {
     if (a.p_overlap) a.p_overlap[T.v0 + k] = no;
     if (a.p_attr) a.p_attr[T.v0 + k] = na;
   };
+  const bool one = T.nvt <= NT;  // block-uniform
+  float rx = 0.0f, ry = 0.0f;
   for (int s = 0; s < nevals; s++) {
     cell_pass(g, T, l);
     __syncthreads();
@@ -914,20 +916,33 @@ extern "C" __global__ void __launch_bounds__(1024) k2d_run(const Run2D a) {
       __syncthreads();
       if (tid == 0 && listed) *oqmax = 0;  // every thread read it before the barrier above
     }
-    // The forces wait in global memory (written and read by the same thread)
-    // for the barrier before the move: in registers, up to DPM2D_VPT per
-    // thread, they need the loop unrolled, sixteen copies of force_vertex.
+    // A thread's one vertex keeps its force in registers for the barrier before
+    // the move.  More of them wait in global memory (written and read by the
+    // same thread): in registers, up to DPM2D_VPT per thread, they need the loop
+    // unrolled, sixteen copies of force_vertex.
     for (int k = tid; k < T.nvt; k += NT) {
       float fx, fy;
       force(k, fx, fy);
-      a.fx[T.v0 + k] = fx;
-      a.fy[T.v0 + k] = fy;
+      rx = fx;
+      ry = fy;
+      if (!one || s + 1 >= nevals) {
+        a.fx[T.v0 + k] = fx;
+        a.fy[T.v0 + k] = fy;
+      }
     }
     __syncthreads();
     if (nsteps > 0) {
-      for (int k = tid; k < T.nvt; k += NT) {
-        l.x[k] = fmaf(a.fx[T.v0 + k], a.dt, l.x[k]);
-        l.y[k] = fmaf(a.fy[T.v0 + k], a.dt, l.y[k]);
+      if (one) {
+        if (tid < T.nvt) {
+          l.x[tid] = fmaf(rx, a.dt, l.x[tid]);
+          l.y[tid] = fmaf(ry, a.dt, l.y[tid]);
+        }
+      } else {
+#pragma unroll 4
+        for (int k = tid; k < T.nvt; k += NT) {
+          l.x[k] = fmaf(a.fx[T.v0 + k], a.dt, l.x[k]);
+          l.y[k] = fmaf(a.fy[T.v0 + k], a.dt, l.y[k]);
+        }
       }
       __syncthreads();
     }
