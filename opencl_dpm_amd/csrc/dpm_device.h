@@ -125,11 +125,6 @@ __device__ __forceinline__ double wave_sum(double v) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, DPM_WAVE);
   return v;
 }
-__device__ __forceinline__ float wave_max(float v) {
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_down(v, o, DPM_WAVE));
-  return v;
-}
-
 // Wave-wide maximum and minimum of a float, every lane receiving the result
 // (a wave-uniform value), by DPP row operations: quad swaps, the half-row
 // and row mirrors, then the row broadcasts, which leave the full result in
