@@ -1916,8 +1916,12 @@ static int create2d(const dpm2d_desc* d, dpm_tissue** out, int rs) {
   };
   if (h->fits_wg) {
     h->over_cap = any_pass && need(DPM2D_OVER_CAP, 0).first <= lds_max ? DPM2D_OVER_CAP : 0;
-    h->run_extra = need(h->over_cap, 1).first <= lds_max;
-    h->relax_extra = need(0, 1).second <= lds_max;
+    // not for cells of a single arc or little more (us per step, with | without:
+    // 64 tissues of 60 cells, 3 to 8 vertices 73 | 66, 1 of 2 cells 10.2 | 9.6; 64
+    // of 30 cells, 8 to 16 vertices 78 | 80 a FIRE iteration)
+    const bool arcs = cvb[C] >= 12 * C;
+    h->run_extra = arcs && need(h->over_cap, 1).first <= lds_max;
+    h->relax_extra = arcs && need(0, 1).second <= lds_max;
     h->lds_run = need(h->over_cap, h->run_extra).first;
     h->lds2 = need(0, h->relax_extra).second;
   }
