@@ -2649,10 +2649,12 @@ extern "C" int dpm_disperse(const float* r, int n, float L, float* X, float* Y, 
   if (!rc) {
     Disperse2DArgs a{dr, dx, dy, n, L, max_count, nb, dout, dt, term_cap};
     // the list form where its LDS fits (up to 32 neighbours, else 16) and a
-    // tenth of the skin is far above the rounding of the coordinates
+    // tenth of the skin is far above the rounding of the coordinates; one or two
+    // centres have no list to gain from (us a call of 60 iterations, with |
+    // without: 2 centres 402 | 350, 3 centres 390 | 420)
     const size_t lds32 = disp_list_layout(nullptr, n, 32).total, lds16 = disp_list_layout(nullptr, n, 16).total;
     const float skin = 0.2f * rmax;
-    if (0.1f * skin > 4e-6f * reach && lds16 <= (size_t)maxlds) {
+    if (n > 2 && 0.1f * skin > 4e-6f * reach && lds16 <= (size_t)maxlds) {
       auto k = lds32 <= (size_t)maxlds ? k_disperse_list<32> : k_disperse_list<16>;
       const size_t need = lds32 <= (size_t)maxlds ? lds32 : lds16;
       (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)need);
