@@ -1,13 +1,14 @@
 // 3D DPM timestep kernels for gfx950.
 //
-// One workgroup owns one cell for a whole step (grid = cells of all tissues,
-// workgroups spread over the 8 XCDs so that neighbouring cells share an L2).
-// The cell's vertices and the mesh's face table live in LDS for the step.
-// Every force term of the reference's per-face kernels is evaluated once per
-// face into LDS and *gathered* by each vertex over its incident faces in a
-// fixed order, so no float atomics are used and a step is bit-reproducible
-// run to run (the reference scatters with a compare-and-swap float add,
-// Cell3D_Kernel.cl:10-32, whose order varies).
+// One workgroup (dpm3d_group.hip) or one wave (dpm3d_wave.hip) owns one cell for
+// a whole step (grid = cells of all tissues, workgroups spread over the 8 XCDs so
+// that neighbouring cells share an L2).  The cell's vertices and the mesh's face
+// table live in LDS for the step.  Each vertex *gathers* its force terms in a
+// fixed order, by one walk around its ring of neighbours (an open mesh or a cell
+// with degenerate edges: face by face), so no float atomics are used and a step
+// is bit-reproducible run to run (the reference scatters with a compare-and-swap
+// float add, Cell3D_Kernel.cl:10-32, whose order varies).  This file holds what
+// both forms share, the statistics, energy, bin and adjoint kernels.
 //
 // Positions are double-buffered (read set -> write set) and the per-cell
 // statistics the next step needs (centre of mass, bounding radius, volume,

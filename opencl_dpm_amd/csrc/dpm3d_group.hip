@@ -2,16 +2,18 @@
 // its vertices t, t + 256, ... (VPT of them); 512 threads in small handles of
 // 257 to 512 vertices.
 //
-// The form serves what the wave-per-cell form does not: handles with few
-// cells, where a step is one chain of dependent passes on a mostly idle
-// device, and meshes over 256 vertices.  Both are bound by latency, so the
-// passes are arranged for few barriers and independent loads:
+// The form serves what the wave-per-cell form does not: handles of few or a
+// middling number of cells, where a step is one chain of dependent passes on a
+// device that has room for more waves, and meshes over 256 vertices.  Both are
+// bound by latency, so the passes are arranged for few barriers and independent
+// loads:
 //   loads and the candidate test of up to 256 cells | barrier | facing-down
 //   faces, ring walk, separation and vertex lists of the candidates (a wave
 //   each) | barrier | substrate, bending, the pair tests of all kept
 //   candidates together | barrier | their sums, in order | barrier | Euler
 //   step | barrier | volume, radius, longest edge | barrier | statistics.
-// Long lists and many candidates take the candidates one by one.
+// Long lists, many candidates and contact of many points or of cells with more
+// than a vertex a thread take the candidates one by one.
 // Four waves, not one thread per vertex: 11 waves of a 642-vertex cell at 141
 // registers filled a compute unit alone, and every barrier idled it.
 // Against one thread per vertex, a face pass of its own and five barriers per
